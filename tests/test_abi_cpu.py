@@ -195,3 +195,24 @@ int main(void) {
         assert done.returncode == 0, done.stderr
         ran = subprocess.run([str(exe)], capture_output=True, text=True)
         assert ran.returncode == 0, ran.stderr
+
+
+@pytest.mark.skipif(os.path.exists("/dev/kfd"), reason="gives host arrays to launchers, which fail only where there is no device")
+@pytest.mark.parametrize("xs,ws,ys", [((2, 20, 0, 8), (6, 20, 2, 3), (2, 6, 1, 8)), ((2, 3, 0, 8), (6, 3, 2, 3), (2, 6, 1, 8)),
+                                      ((2, 0, 8, 8), (6, 0, 3, 3), (2, 6, 8, 8)), ((2, 6, 8, 8), (0, 6, 3, 3), (2, 0, 8, 8))])
+def test_convolutions_without_elements_reach_their_launch(xs, ws, ys):
+    """An image, a filter or a gradient without elements: the host side divides by none of those counts.  Without a device the
+    call then fails at its launch (an error code, no signal)."""
+    import subprocess
+    import sys
+    code = f"""
+from tsplit_amd import gpu_links as L, ndarray as nd
+x, w, y = (nd.empty(s, nd.cpu(0)) for s in ({xs}, {ws}, {ys}))
+for call, args in ((L.CuDNN_conv2d, (x, w, y)), (L.CuDNN_conv2d_gradient_of_data, (w, y, x)), (L.CuDNN_conv2d_gradient_of_filter, (x, y, w))):
+    try:
+        call(*args, 1, 1, 1)
+    except RuntimeError:
+        pass
+"""
+    ran = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert ran.returncode == 0, (ran.returncode, ran.stderr)

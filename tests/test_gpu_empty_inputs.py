@@ -69,6 +69,30 @@ def test_pooling_and_convolution_on_an_empty_batch():
         assert not dw.asnumpy().any(), (C, O, k, pad, s, H)
 
 
+# x, filter, padding, stride: images without rows, without channels, filters without taps; the output has elements
+OVER_NOTHING = [((2, 20, 0, 8), (6, 20, 2, 3), 1, 1), ((2, 3, 0, 8), (6, 3, 2, 3), 1, 1), ((2, 0, 8, 8), (6, 0, 3, 3), 1, 1),
+                ((2, 0, 8, 8), (64, 0, 1, 1), 0, 2), ((2, 32, 6, 6), (16, 32, 0, 0), 0, 1)]
+
+
+@pytest.mark.parametrize("xs,ws,pad,s", OVER_NOTHING)
+def test_convolutions_that_sum_over_nothing(xs, ws, pad, s, monkeypatch):
+    L, nd, ctx = _env()
+    ys = (xs[0], ws[0], (xs[2] + 2 * pad - ws[2]) // s + 1, (xs[3] + 2 * pad - ws[3]) // s + 1)
+    for forced in (None, "0", "1"):          # whichever routine the dispatcher would ask
+        if forced:
+            monkeypatch.setenv("TSPLIT_CONV_WINOGRAD", forced)
+        y, stats = nd.array(np.full(ys, 7, np.float32), ctx), nd.array(np.full(4 * ws[0], 7, np.float32), ctx)
+        L.CuDNN_conv2d(nd.empty(xs, ctx), nd.empty(ws, ctx), y, pad, pad, s)
+        assert not y.asnumpy().any()
+        L.conv2d_batch_norm_stats(nd.empty(xs, ctx), nd.empty(ws, ctx), y, stats, 0, pad, pad, s)
+        assert not y.asnumpy().any() and not stats.asnumpy().any()
+        # the same arrays the other way round: a gradient of no output channels, or of none through a filter without taps
+        dx = nd.array(np.full(ys, 7, np.float32), ctx)
+        back = ((0, ys[1], 1, 1), (ys[0], 0) + ys[2:]) if ws[2] else ((5, ys[1], 0, 0), (ys[0], 5, ys[2] + 1, ys[3] + 1))
+        L.CuDNN_conv2d_gradient_of_data(nd.empty(back[0], ctx), nd.empty(back[1], ctx), dx, 0, 0, 1)
+        assert not dx.asnumpy().any()
+
+
 def test_matrix_products_with_an_empty_dimension():
     L, nd, ctx = _env()
     e = lambda *s: nd.empty(tuple(s), ctx)

@@ -810,9 +810,10 @@ inline int64_t conv_reach_bytes() {
 }
 
 // The tile kernel addresses the gathered tensor with 32-bit byte offsets.  One beyond 2 GiB is taken in runs of whole images, one
-// launch each (images are independent in the forward and backward-data passes): -> images per launch, 0 if not even one fits.
+// launch each (images are independent in the forward and backward-data passes): -> images per launch, 0 if not even one fits or
+// an image has no elements.
 inline int tile_kernel_images(const ConvGeo &g, int64_t src_elems_per_img) {
-  if (g.imgs <= 0) return 0;
+  if (g.imgs <= 0 || src_elems_per_img <= 0) return 0;
   const int64_t room = conv_reach_bytes() - 4 * (static_cast<int64_t>(g.kH) * g.W + g.kW + g.ph * g.W + g.pw);
   const int64_t fit = room / (src_elems_per_img * 4);
   if (fit < 1) return 0;
@@ -1384,6 +1385,12 @@ __global__ __launch_bounds__(256) void conv_stats_final_kernel(const double *__r
 
 constexpr int kStatsSlices = 64;
 
+// a result that sums over nothing: no images, no channels, no positions or no taps on the other side
+void zero_fill(DLArray *a, hipStream_t st) {
+  const int64_t n = numel(a);
+  hipLaunchKernelGGL(zero_fill_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, mf(a), n);
+}
+
 // `stats_dst` (optional): per-channel (sum, sum of squares) of y as doubles, [O][2], for a BatchNorm that
 // follows.  The Winograd routine and the tap-major kernels produce them in their epilogues; the other
 // routes by a pass over y.
@@ -1403,7 +1410,8 @@ int conv_forward(const char *who, const DLArray *x, const DLArray *w, DLArray *y
   // images per launch of the tile kernel
   const int per = conv_tile_takes(g, false) ? tile_kernel_images(g, static_cast<int64_t>(g.C) * g.H * g.W) : 0;
   // routes whose epilogue sums the output per channel at (almost) no cost
-  const bool sums_in_epilogue = numel(y) > 0 && !thin_fwd_ok(g) && (winograd_pays(g, g.C) || per > 0);
+  const bool nothing = numel(x) == 0 || numel(w) == 0;
+  const bool sums_in_epilogue = numel(y) > 0 && !nothing && !thin_fwd_ok(g) && (winograd_pays(g, g.C) || per > 0);
   double *note_dst = nullptr;
   // (a BatchNorm over at most 16384 values per channel holds them in registers and reads its input once
   // anyway, so an output that small gets no note: the fold launch behind the epilogue would be paid for
@@ -1424,7 +1432,9 @@ int conv_forward(const char *who, const DLArray *x, const DLArray *w, DLArray *y
     sk = &sink;
   }
   if (numel(y) > 0) {
-    if (thin_fwd_ok(g)) {
+    if (nothing) {
+      zero_fill(y, st);
+    } else if (thin_fwd_ok(g)) {
       const int rc = launch_conv_thin_fwd(g, cf(x), cf(w), mf(y), st);
       if (rc) return rc;
     } else if (winograd_pays(g, g.C)) {
@@ -1492,7 +1502,9 @@ int conv_bwd_data(const char *who, const DLArray *w, const DLArray *dy, DLArray 
   if (geo_from(who, dx, w, dy, ph, pw, s, g)) return -1;
   hipStream_t st = stream_of(sh);
   ProfileScope ps(p, st, numel(dy) + numel(w), numel(dx), numel(w));
-  if (numel(dx) > 0 && winograd_pays(g, g.O)) {
+  if (numel(dx) > 0 && (numel(dy) == 0 || numel(w) == 0)) {
+    zero_fill(dx, st);
+  } else if (numel(dx) > 0 && winograd_pays(g, g.O)) {
     const int rc = conv_winograd_3x3(cf(dy), cf(w), mf(dx), g.imgs, g.O, g.C, g.H, g.W, true, st);
     if (rc) return rc;
   } else if (numel(dx) > 0) {
@@ -1544,9 +1556,7 @@ int conv_bwd_filter(const char *who, const DLArray *x, const DLArray *dy, DLArra
   ProfileScope ps(p, st, numel(x) + numel(dy), numel(dw), 0);
   int rc = 0;
   if (numel(dw) > 0 && (numel(x) == 0 || numel(dy) == 0)) {
-    // a sum over no positions (an empty batch: the last of more micro-tensors than there are images)
-    const int64_t n = numel(dw);
-    hipLaunchKernelGGL(zero_fill_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, mf(dw), n);
+    zero_fill(dw, st);   // (an empty batch: the last of more micro-tensors than there are images)
   } else if (numel(dw) > 0) {
     if (wgrad_narrow_ok(g)) {
       rc = launch_wgrad_narrow(g, cf(x), cf(dy), mf(dw), st, &ws);
