@@ -73,3 +73,20 @@ def test_infinities_stay_in_their_rows(case, rng, monkeypatch):
     rest = np.ones(shape[:2], bool)
     rest[11, :] = rest[:, 5] = False
     assert finite[rest].all() and not finite[11, 5]
+
+
+def test_steps_that_span_more_images_than_a_block_reaches(rng):
+    """2 x 2 positions of images of 300 MB: a 32-deep step covers all eight images, 32-bit offsets four of them."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    N, C, H, Oc, s = 8, 300, 512, 16, 256
+    x = np.resize(rng.normal(size=1000003).astype(np.float32), (N, C, H, H))
+    dy = rng.normal(size=(N, Oc, 2, 2)).astype(np.float32)
+    dw = nd.array(np.full((Oc, C, 3, 3), 7, np.float32), nd.gpu(0))
+    L.CuDNN_conv2d_gradient_of_filter(nd.array(x, nd.gpu(0)), nd.array(dy, nd.gpu(0)), dw, 1, 1, s)
+    got = dw.asnumpy()
+    for u in range(3):
+        for v in range(3):
+            rows, cols = [r for r in range(2) if r * s + u >= 1], [c for c in range(2) if c * s + v >= 1]
+            a = dy[:, :, rows][:, :, :, cols].transpose(1, 0, 2, 3).reshape(Oc, -1).astype(np.float64)
+            b = np.stack([x[:, :, r * s - 1 + u, c * s - 1 + v] for r in rows for c in cols], 2).transpose(0, 2, 1).reshape(-1, C).astype(np.float64)
+            assert (np.abs(got[:, :, u, v] - a @ b) <= 36 * 2.0 ** -24 * (np.abs(a) @ np.abs(b)) + 1e-30).all(), (u, v)

@@ -110,9 +110,7 @@ struct StatsSink {
 };
 
 // Convolution forward and data gradient on the tile kernel (conv_tile.hip), for tensors within reach of 32-bit byte offsets.
-struct ConvTileGeo {
-  int imgs, C, H, W, O, kH, kW, ph, pw, s, oH, oW;
-};
+struct ConvTileGeo;   // conv_reach.h
 bool conv_tile_takes(const ConvTileGeo &g, bool bwd);
 int conv_tile_forward(const float *x, const float *w, float *y, const ConvTileGeo &g, hipStream_t st, StatsSink *sink);
 int conv_tile_bwd_data(const float *dy, const float *w, float *dx, const ConvTileGeo &g, hipStream_t st);

@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "common.h"
+#include "conv_reach.h"
 #include "fastdiv.h"
 #include "mfma_gemm.h"
 
@@ -809,18 +810,8 @@ inline int64_t conv_reach_bytes() {
   return full;
 }
 
-// The tile kernel addresses the gathered tensor with 32-bit byte offsets.  One beyond 2 GiB is taken in runs of whole images, one
-// launch each (images are independent in the forward and backward-data passes): -> images per launch, 0 if not even one fits or
-// an image has no elements.
-inline int tile_kernel_images(const ConvGeo &g, int64_t src_elems_per_img) {
-  if (g.imgs <= 0 || src_elems_per_img <= 0) return 0;
-  const int64_t room = conv_reach_bytes() - 4 * (static_cast<int64_t>(g.kH) * g.W + g.kW + g.ph * g.W + g.pw);
-  const int64_t fit = room / (src_elems_per_img * 4);
-  if (fit < 1) return 0;
-  if (fit >= g.imgs) return g.imgs;
-  const int64_t launches = (g.imgs + fit - 1) / fit;          // equal runs rather than a short last one
-  return static_cast<int>((g.imgs + launches - 1) / launches);
-}
+// images per launch of the tile kernel, 0: it cannot take them
+inline int tile_kernel_images(const ConvGeo &g, int64_t src_elems_per_img) { return images_per_launch(g, src_elems_per_img, conv_reach_bytes()); }
 
 // Runs f(geometry of the run, first image) over runs of `per` images.
 template <class F>

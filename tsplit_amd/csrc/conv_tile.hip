@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "conv_reach.h"
 #include "tile_plan.h"
 
 namespace tsplit {

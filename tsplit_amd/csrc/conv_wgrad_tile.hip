@@ -4,6 +4,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "conv_reach.h"
 #include "tile_plan.h"
 
 namespace tsplit {
@@ -47,13 +48,6 @@ void launch_tile(const Params &P, int tile, const mg::TileGrid &tg, unsigned gri
   }
 }
 
-// Images of both tensors that lie within `reach` bytes of the first one, rows past the last channel included.
-int64_t span_images(const ConvTileGeo &g, int64_t reach) {
-  const int64_t dy = static_cast<int64_t>(g.O + 128) * g.oH * g.oW * 4, x = static_cast<int64_t>(g.C + 128) * g.H * g.W * 4;
-  return reach / std::max<int64_t>(1, std::max(dy, x));
-}
-int64_t padded_depth(const ConvTileGeo &g) { return (static_cast<int64_t>(g.oH) * g.oW + 3) / 4 * 4 * g.imgs; }
-
 }  // namespace
 
 void conv_fold_tap_major(const float *part, float *dw, int O, int C, int taps, int S, hipStream_t st) {
@@ -61,10 +55,7 @@ void conv_fold_tap_major(const float *part, float *dw, int O, int C, int taps, i
   hipLaunchKernelGGL(fold_tap_major_kernel, dim3(static_cast<unsigned>((mn + 63) / 64)), dim3(256), 0, st, part, dw, O, C, taps, mn, S);
 }
 
-// three images within reach: a range of at least one image's positions stays addressable
-bool conv_tile_bwd_filter_takes(const ConvTileGeo &g, int64_t reach) {
-  return span_images(g, reach) >= 3 && padded_depth(g) < (1ll << 31) - 64 && static_cast<int64_t>(g.O) * (g.C + 16) * g.kH * g.kW < (1ll << 31) - 256;
-}
+bool conv_tile_bwd_filter_takes(const ConvTileGeo &g, int64_t reach) { return filter_gradient_in_reach(g, reach); }
 
 int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvTileGeo &g, int64_t reach, hipStream_t st, int64_t *ws_elems) {
   const int taps = g.kH * g.kW;
@@ -78,9 +69,8 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   P.cols = taps * g.C;
   P.plane = g.oH * g.oW;
   P.dy_img = g.O * P.plane;
-  const int positions = (P.plane + 3) / 4 * 4;
   P.K = static_cast<int>(padded_depth(g));
-  P.image = FastDiv(positions);
+  P.image = FastDiv(depth_per_image(g));
   P.width = FastDiv(g.oW);
   P.blocks = FastDiv((g.C + 15) / 16);
   P.kw = FastDiv(g.kW);
@@ -97,9 +87,7 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   const int steps = (P.K + BK - 1) / BK;
   const TilePlan plan = plan_tiles(g.O, &cols, &steps, 1, 1, 1024, static_cast<double>(values), point ? kDense : kGathered);
   const TileKind &k = kTiles[plan.tile];
-  P.kchunk = (steps + plan.S - 1) / plan.S * BK;
-  const int64_t room = (span_images(g, reach) - 2) * positions;
-  if (P.kchunk > room) P.kchunk = std::max<int>(BK, static_cast<int>(room / BK * BK));
+  P.kchunk = range_depth(g, reach, plan.S);
   const int S = std::max(1, (P.K + P.kchunk - 1) / P.kchunk);
   const int tm = (g.O + k.bm - 1) / k.bm, tn = static_cast<int>((cols + k.bn - 1) / k.bn);
   TS_REQUIRE(static_cast<int64_t>(tm) * tn * S < (1ll << 31) - 8, "conv: too many tiles");
