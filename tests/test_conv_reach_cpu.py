@@ -64,3 +64,21 @@ def test_ranges_of_depth_stay_within_what_a_block_addresses(host):
         g = _geo(rng.randint(1, 64), rng.randint(1, 600), rng.randint(8, 300), rng.randint(8, 300), rng.randint(1, 600), 3, 3, 1, 1, rng.choice((1, 2, 8)))
         for reach in (FULL, 1 << 24):
             _ranges_stay_in_reach(host, g, reach, rng.choice((1, 3, 50)))
+
+
+def test_runs_of_images_stay_in_reach_with_the_base_moved_back(host):
+    """Both passes move the base of the gathered tensor back and address the run's bytes and that distance.  Wide padding of narrow
+    images makes the data gradient's distance, a filter's height times the OUTPUT's width, the larger one."""
+    rng, narrow = random.Random(6), 0
+    for _ in range(4000):
+        kh, kw = rng.choice(((64, 1), (32, 2), (8, 8), (7, 7), (3, 3), (1, 1)))
+        h, w, ph, pw = rng.randint(1, 40), rng.randint(1, 40), rng.randint(0, 40), rng.randint(0, 120)
+        if h + 2 * ph < kh or w + 2 * pw < kw:
+            continue
+        g = _geo(1 << 20, rng.randint(1, 64), h, w, rng.randint(1, 64), kh, kw, ph, pw, rng.choice((1, 1, 2, 3)))
+        for values, back in ((g[1] * h * w, ph * w + pw), (g[4] * g[10] * g[11], (kh - 1) * g[11] + kw - 1)):
+            for reach in (FULL, 1 << 20):
+                per = host.images(g, ctypes.c_longlong(values), ctypes.c_longlong(reach))
+                assert per == 0 or 4 * (per * values + back) <= reach, (tuple(g), per)
+                narrow += per > 0 and back > ph * w + pw + kh * w + kw
+    assert narrow > 100

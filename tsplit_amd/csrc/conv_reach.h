@@ -15,7 +15,9 @@ struct ConvTileGeo {
 // an image has no elements.
 inline int images_per_launch(const ConvTileGeo &g, int64_t src_elems_per_img, int64_t reach) {
   if (g.imgs <= 0 || src_elems_per_img <= 0) return 0;
-  const int64_t room = reach - 4 * (static_cast<int64_t>(g.kH) * g.W + g.kW + g.ph * g.W + g.pw);
+  // what the base is moved back by, so that no offset is negative: the padding (forward), the last tap (data gradient)
+  const int64_t back = std::max(static_cast<int64_t>(g.kH + g.ph) * g.W + g.kW + g.pw, static_cast<int64_t>(g.kH - 1) * g.oW + g.kW - 1);
+  const int64_t room = reach - 4 * back;
   const int64_t fit = room / (src_elems_per_img * 4);
   if (fit < 1) return 0;
   if (fit >= g.imgs) return g.imgs;
