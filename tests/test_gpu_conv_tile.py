@@ -76,3 +76,21 @@ def test_channels_past_the_last_beyond_32_bit_offsets(rng):
         rows[:, :, lo - row + 1:hi - row + 1] = x[:, :, lo:hi]
         ref, mag = O.conv2d(rows, w, 0, 1, 1), O.conv2d(np.abs(rows), np.abs(w), 0, 1, 1)
         assert (np.abs(got[:, :, row:row + 1] - ref) <= _bound(mag, C * 9 + 32)).all(), row
+
+
+def test_infinities_behind_the_channels_past_the_last(rng):
+    """A layer of one tap on large planes, 33 channels in two steps of 32: the offsets of the missing ones leave 32 bits, and folded
+    back they would lie inside the image.  Infinities there stay in their own columns."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    ctx, C, Oc, H = nd.gpu(0), 33, 8, 3900
+    x = np.resize(rng.normal(size=1009).astype(np.float32), (1, C, H, H))
+    at = [k * H * H - (1 << 29) for k in range(C, 64) if 0 <= k * H * H - (1 << 29) < x.size]   # 2^31 + 4 k H H - 2^32 bytes
+    for a in at:
+        x.reshape(-1)[a:a + 4] = np.inf
+    y = nd.empty((1, Oc, H, H), ctx)
+    L.CuDNN_conv2d(nd.array(x, ctx), nd.array(rng.normal(size=(Oc, C, 1, 1)).astype(np.float32), ctx), y, 0, 0, 1)
+    own = np.zeros(H * H, bool)
+    for a in at:
+        own[np.arange(a, a + 4) % (H * H)] = True
+    finite = np.isfinite(y.asnumpy()).reshape(Oc, -1)
+    assert len(at) > 9 and finite[:, ~own].all() and not finite[:, own].any()

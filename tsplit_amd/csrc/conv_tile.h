@@ -167,11 +167,17 @@ struct Pointwise {
     voff = n < f.N ? (img * p.img_stride + row * p.chan_stride + nn - img * f.plane.d) * 4u : kOobOffset;
   }
   __device__ __forceinline__ void load(int k0, int kend, unsigned lds) const {
+    lds += wave * kLoads * 1024;
+    const int k1 = k0 + wave * kLoads * kRows;
+    if (k0 + BK <= kend) {
 #pragma unroll
-    for (int s = 0; s < kLoads; ++s) {
-      const int k = k0 + (wave * kLoads + s) * kRows;
-      // channels past the last one are the next image's
-      gt::load_to_lds(rsrc, k0 + BK <= kend || k + row < kend ? voff : kOobOffset, k * row_bytes, lds + (wave * kLoads + s) * 1024);
+      for (int s = 0; s < kLoads; ++s) gt::load_to_lds(rsrc, voff, (k1 + s * kRows) * row_bytes, lds + s * 1024);
+    } else {   // channels past the last one are the next image's, and of large planes beyond 32-bit offsets
+#pragma unroll
+      for (int s = 0; s < kLoads; ++s) {
+        const int k = k1 + s * kRows;
+        gt::load_to_lds(rsrc, k + row < kend ? voff : kOobOffset, k < kend ? k * row_bytes : 0, lds + s * 1024);
+      }
     }
   }
   __device__ __forceinline__ bool cut(int, int) const { return false; }
