@@ -41,17 +41,21 @@ __device__ __forceinline__ i32x4 raw_buffer(const float *p, int64_t bytes) {
 // 64 lanes x 16 bytes from the buffer straight into LDS, at `lds` + 16 * lane (bytes); voff: the lane's byte offset, soff:
 // the wave's.  Lanes out of range write zeros.  The compiler does not see the LDS write (lds_ready() orders it) nor that a vector
 // memory instruction reads the scalar registers, which may have been written by a vector instruction just before: five wait states.
+// (m0 is declared although the compiler never keeps a value of its own there and says so: it does merge equal writes of it.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_to_lds(i32x4 rsrc, unsigned voff, int soff, unsigned lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff),
                "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soff))
-               : "memory");
+               : "memory", "m0");
 }
 // the same with 4 bytes a lane, at `lds` + 4 * lane
 __device__ __forceinline__ void load_word_to_lds(i32x4 rsrc, unsigned voff, int soff, unsigned lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dword %1, %2, %3 offen lds" ::"s"(__builtin_amdgcn_readfirstlane(lds)), "v"(voff),
                "s"(rsrc), "s"(__builtin_amdgcn_readfirstlane(soff))
-               : "memory");
+               : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // Everything this wave has asked for lies in LDS, every operand word it has read is in registers; then the block's barrier.
 // The wait comes twice: the compiler counts LDS reads only from the one it knows.  Without it scalar loads from before the
 // k-loop counted as outstanding through every step, and each half's reads were waited for in full before the half before
