@@ -71,3 +71,28 @@ def test_rows_of_the_result_beyond_32_bit_offsets(rng):
     for row in range(M):
         a64 = a[row:row + 1].astype(np.float64)
         assert (np.abs(got[row] - (a64 @ b64)[0]) <= _bound(a64, b64)[0]).all(), row
+
+
+@pytest.mark.parametrize("M,N,ta,batched", [(48, 512, False, False), (130, 512, True, False), (40, 512, True, True), (512, 40, False, True), (130, 512, True, True)])
+def test_operands_beyond_32_bit_offsets(M, N, ta, batched, rng):
+    """An operand of more than 2 GiB, K far longer than the result is wide.  Whole numbers of at most 1, so that every sum is exact in
+    fp32 in whatever order; a plain product is cut into ranges of K (they leave a workspace)."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    from tsplit_amd.profiler import Profiler
+    ctx, K = nd.gpu(0), (1 << 29) // max(M, N) + 4321
+    wide = rng.randint(-1, 2, size=(K, max(M, N))).astype(np.float32)
+    slim = rng.randint(-1, 2, size=(K, min(M, N))).astype(np.float32)
+    want = np.zeros((min(M, N), max(M, N)), np.float32)
+    for at in range(0, K, 1 << 16):
+        want += slim[at:at + (1 << 16)].T @ wide[at:at + (1 << 16)]
+    a, b, want = (slim, wide, want) if M < N else (wide, slim, want.T)
+    a = a if ta else np.ascontiguousarray(a.T)
+    if batched:
+        c = nd.empty((1, M, N), ctx)
+        L.batch_matrix_multiply(nd.array(a[None], ctx), ta, nd.array(b[None], ctx), False, c)
+        np.testing.assert_array_equal(c.asnumpy()[0], want)
+    else:
+        c, p = nd.empty((M, N), ctx), Profiler()
+        L.matrix_multiply(nd.array(a, ctx), ta, nd.array(b, ctx), False, c, profiler=p)
+        np.testing.assert_array_equal(c.asnumpy(), want)
+        assert p.workspace_memory > 0

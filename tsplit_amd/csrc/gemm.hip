@@ -6,8 +6,8 @@
 // The tile (128x128, 64x128, 128x64 or 64x64) and the number of ranges K is cut into come from a
 // small model of the chip (tile_plan.h); the ranges' results are added in ascending order by a
 // second kernel.  The batched form runs every leading index as one more grid dimension of the same
-// kernel.  Operands of 2 GiB and more, and results whose 64 rows
-// reach that far, stay on the engine of mfma_gemm.h, which takes 64-bit addresses.
+// kernel.  Operands of 2 GiB and more, and results whose 64 rows reach that far, stay on the engine
+// of mfma_gemm.h, which takes 64-bit addresses, with its own tiles and ranges.
 #include <algorithm>
 
 #include "common.h"
@@ -88,18 +88,57 @@ int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, flo
   return 0;
 }
 
-// operands or rows of the result beyond 32-bit offsets: 64-bit addresses, 128x128 tiles
-template <bool TA, bool TB>
-int launch_far(const float *A, int64_t lda, int64_t sa, const float *B, int64_t ldb, int64_t sb, float *C, int batch, int M, int N, int K,
-               hipStream_t s) {
-  using AL = typename std::conditional<TA, MnContigLoader<128>, KContigLoader<128>>::type;
-  using BL = typename std::conditional<TB, KContigLoader<128>, MnContigLoader<128>>::type;
-  const typename AL::Params ap{A, lda, M, lda % 4 == 0 && sa % 4 == 0 && aligned16(A)};
-  const typename BL::Params bp{B, ldb, N, ldb % 4 == 0 && sb % 4 == 0 && aligned16(B)};
-  const int tm = (M + 127) / 128, tn = (N + 127) / 128;
-  hipLaunchKernelGGL((mfma_batched_gemm_kernel<128, 128, 2, 2, AL, BL>), dim3(grid_blocks(tm, tn, batch)), dim3(kThreads), 0, s, ap, bp, C, sa,
-                     sb, static_cast<int64_t>(M) * N, M, N, K, TileGrid{tm, tn, tm * tn * batch});
+// operands or rows of the result beyond 32-bit offsets: the loaders with 64-bit addresses
+template <int BM, int BN, bool TA, bool TB>
+struct Far {
+  using AL = typename std::conditional<TA, MnContigLoader<BM>, KContigLoader<BM>>::type;
+  using BL = typename std::conditional<TB, KContigLoader<BN>, MnContigLoader<BN>>::type;
+  typename AL::Params ap;
+  typename BL::Params bp;
+  int tm, tn;
+  Far(const float *A, int64_t lda, int64_t sa, const float *B, int64_t ldb, int64_t sb, int M, int N)
+      : ap{A, lda, M, lda % 4 == 0 && sa % 4 == 0 && aligned16(A)},
+        bp{B, ldb, N, ldb % 4 == 0 && sb % 4 == 0 && aligned16(B)},
+        tm((M + BM - 1) / BM),
+        tn((N + BN - 1) / BN) {}
+};
+
+// K in ranges where the tiles alone leave the chip idle (512 x 512 over 1.1 million rows is 16 tiles: 5.2 ms in ranges, 101 whole)
+template <int BM, int BN, int WM, int WN, bool TA, bool TB>
+int launch_far(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws_elems) {
+  using F = Far<BM, BN, TA, TB>;
+  const F f(A, lda, 0, B, ldb, 0, M, N);
+  static const int occ = blocks_per_cu(mfma_gemm_kernel<BM, BN, WM, WN, typename F::AL, typename F::BL, RowMajorCols>);
+  int S, kchunk;
+  plan_splitk(f.tm * f.tn, K, 64, occ, S, kchunk);
+  float *out = C;
+  const int64_t mn = static_cast<int64_t>(M) * N;
+  if (S > 1) {
+    out = static_cast<float *>(scratch_get(s, 2, static_cast<size_t>(S) * mn * 4));
+    TS_REQUIRE(out, "DLGpuMatrixMultiply: no scratch memory for split-K");
+    *ws_elems = S * mn;
+  }
+  hipLaunchKernelGGL((mfma_gemm_kernel<BM, BN, WM, WN, typename F::AL, typename F::BL, RowMajorCols>), dim3(grid_blocks(f.tm, f.tn, S)),
+                     dim3(kThreads), 0, s, f.ap, f.bp, out, mn, static_cast<int64_t>(N), RowMajorCols{}, M, N, K, kchunk,
+                     TileGrid{f.tm, f.tn, f.tm * f.tn * S});
+  if (S > 1) gt::launch_fold(out, C, mn, S, s);
   return 0;
+}
+
+template <int BM, int BN, int WM, int WN, bool TA, bool TB>
+int launch_far_batched(const float *A, int64_t lda, int64_t sa, const float *B, int64_t ldb, int64_t sb, float *C, int batch, int M, int N,
+                       int K, hipStream_t s) {
+  using F = Far<BM, BN, TA, TB>;
+  const F f(A, lda, sa, B, ldb, sb, M, N);
+  hipLaunchKernelGGL((mfma_batched_gemm_kernel<BM, BN, WM, WN, typename F::AL, typename F::BL>), dim3(grid_blocks(f.tm, f.tn, batch)),
+                     dim3(kThreads), 0, s, f.ap, f.bp, C, sa, sb, static_cast<int64_t>(M) * N, M, N, K, TileGrid{f.tm, f.tn, f.tm * f.tn * batch});
+  return 0;
+}
+
+template <bool TA, bool TB>
+int dispatch_far(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws) {
+  if (M <= 64) return launch_far<64, 256, 1, 4, TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
+  return launch_far<128, 128, 2, 2, TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
 }
 
 // the same product with split-bf16 terms (opt-in): 128 x 128 tiles whatever M, the split-K plan and fold of above
@@ -137,10 +176,10 @@ bool rows_reach(int N) { return 65ll * 4 * N < (1ll << 31); }
 
 template <bool TA, bool TB>
 int dispatch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws) {
-  if (!near<TA, TB>(lda, ldb, M, N, K)) return launch_far<TA, TB>(A, lda, 0, B, ldb, 0, C, 1, M, N, K, s);
+  if (!near<TA, TB>(lda, ldb, M, N, K)) return dispatch_far<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
   // split-bf16 products where asked for: K a multiple of 4 (a loaded word lies inside a row or outside it)
   if (split_bf16_enabled() && K % 4 == 0 && K >= BK) return launch_gemm_split<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
-  if (!rows_reach(N)) return launch_far<TA, TB>(A, lda, 0, B, ldb, 0, C, 1, M, N, K, s);
+  if (!rows_reach(N)) return dispatch_far<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
   return launch_product<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
 }
 
@@ -149,7 +188,11 @@ int dispatch_batched(const float *A, int64_t lda, int64_t sa, const float *B, in
                      int batch, int M, int N, int K, hipStream_t s) {
   const int64_t tiles = static_cast<int64_t>((M + 63) / 64) * ((N + 63) / 64) * batch;
   TS_REQUIRE(tiles < (1ll << 31) - 8, "DLGpuBatchMatrixMultiply: too many tiles");
-  if (!near<TA, TB>(lda, ldb, M, N, K) || !rows_reach(N)) return launch_far<TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
+  if (!near<TA, TB>(lda, ldb, M, N, K) || !rows_reach(N)) {   // (batches of 1.1M x 64 x 512 on 256 x 64 tiles 0.79 ms, on 128 x 128 0.92)
+    if (M <= 64) return launch_far_batched<64, 256, 1, 4, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
+    if (N <= 64) return launch_far_batched<256, 64, 4, 1, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
+    return launch_far_batched<128, 128, 2, 2, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
+  }
   Plan plan = plan_product(M, N, K, batch, false);
   launch_planned<TA, TB>(A, lda, sa, B, ldb, sb, C, static_cast<int64_t>(M) * N, batch, M, N, K, plan, s);
   return 0;
