@@ -1,4 +1,4 @@
-"""The filter gradient's tile kernel (csrc/conv_wgrad_tile.h) at the edges of its tiles, of its blocks of 16 channels, of its 16-byte
+"""The filter gradient's tile kernel (csrc/conv_wgrad_tile.h) at the edges of its tiles, of its groups of 16, 4 and 2 channels, of its 16-byte
 words and of the images its depth runs over: against float64.
 
 Bar: an output is a sum of K = images x positions fp32 products, in whatever order: within K * 2^-24 of the sum of their
@@ -25,6 +25,11 @@ CASES = [
     (2, 96, 5, 17, 40, 1, 7, 0, 3, 1),     # a row of taps
     (4, 64, 23, 29, 192, 3, 3, 0, 0, 2),   # whole tiles and a ragged last one
     (40, 160, 20, 20, 96, 3, 1, 1, 0, 1),  # many ranges
+    (3, 3, 17, 19, 70, 7, 7, 3, 3, 2),     # groups of 4 channels, one of them padding: four taps a block of 16 columns
+    (2, 20, 9, 9, 33, 3, 3, 1, 1, 1),      # groups of 4 without padding; the last block of columns is not full
+    (2, 5, 11, 13, 129, 5, 5, 2, 2, 2),    # groups of 2, one channel padding
+    (3, 18, 8, 7, 40, 1, 3, 0, 1, 1),      # groups of 2 without padding
+    (5, 6, 30, 30, 353, 3, 3, 1, 1, 1),    # groups of 2 on wide tiles
 ]
 
 
@@ -58,7 +63,8 @@ def test_ranges_shortened_to_what_a_block_reaches(rng, monkeypatch):
     _check(case, *_gradients(case, rng))
 
 
-@pytest.mark.parametrize("case", [(3, 40, 7, 7, 20, 1, 1, 0, 0, 1), (3, 40, 7, 7, 20, 3, 3, 1, 1, 1)])
+@pytest.mark.parametrize("case", [(3, 40, 7, 7, 20, 1, 1, 0, 0, 1), (3, 40, 7, 7, 20, 3, 3, 1, 1, 1), (3, 12, 7, 7, 20, 3, 3, 1, 1, 1),
+                                  (3, 9, 7, 7, 20, 3, 3, 1, 1, 1)])
 def test_infinities_stay_in_their_rows(case, rng, monkeypatch):
     """A cut word holds the next channel's first values: they must not reach this channel's sums, not even times zero."""
     from tsplit_amd import gpu_links as L, ndarray as nd

@@ -1,8 +1,12 @@
 // Convolution filter gradient as a product on the tile kernel of gemm_tile.h: dw[o, (tap, c)] = sum over positions of
 // dy[o, position] x[c, position shifted by the tap].
 //
-//   M = O, N = taps x C (a tap's channels in whole blocks of 16), depth = images x positions, an image's positions padded to a
-//   multiple of 4.  Both operands have the depth contiguous.
+//   M = O, N = taps x C (a tap's channels in whole groups of 16, 4 or 2), depth = images x positions, an image's positions padded to
+//   a multiple of 4.  Both operands have the depth contiguous.
+//
+// Groups of 16 test a position against the image's edge once for eight loads, groups of 4 or 2 once for two loads or each one; but
+// 3 channels padded to 16 are five times the products and loads (64 x 3 x 224 x 224, 64 filters of 7x7, stride 2: 770 us in groups of
+// 16, 284 in groups of 4).
 //
 // A step's position is worked out once a lane (from the step's before it; by division only where an image begins, which as much
 // as doubles what a 64 x 64 tile spends on it) and serves every row the lane loads: rows are
@@ -41,9 +45,9 @@ struct Params {
   int64_t dy_bytes, x_bytes;
   int M, C, cols;                // O; channels of x; columns of one row of the output, taps * C
   int K, kchunk;                 // depth; one range of it (a multiple of 32)
-  FastDiv image, width, blocks;  // padded positions of an image; positions in a row; 16-channel blocks of a tap
+  FastDiv image, width, groups;  // padded positions of an image; positions in a row; groups of channels of a tap
   FastDiv kw;
-  int n_blocks;                  // 16-column blocks of N
+  int n_groups;                  // of N
   int plane, dy_img;             // positions of an image; values of an image of dy
   int x_plane, x_img, x_h, x_w;
   int ph, pw, s;
@@ -120,14 +124,14 @@ struct Words {
   }
 };
 
-// BN columns of x by tap, 4 bytes a lane.  LDS: two rows of a load in 64 floats and 4 to spare.
-template <int BN, int T>
+// BN columns of x, in groups of G channels of one tap, 4 bytes a lane.  LDS: two rows of a load in 64 floats and 4 to spare.
+template <int BN, int T, int G>
 struct Taps {
-  static constexpr int kPair = 68, kBlocks = BN / 64, kFloats = BN / 2 * kPair;   // a wave's blocks of 16 columns
+  static constexpr int kPair = 68, kGroups = BN / 4 / G, kFloats = BN / 2 * kPair;   // a wave's groups
   i32x4 rsrc;
   FastDiv image, width;
   int wave, img0, img_values, plane, x_plane, x_h, x_w, s;
-  int down[kBlocks], right[kBlocks], shift[kBlocks], chan_at[kBlocks];
+  int down[kGroups], right[kGroups], shift[kGroups], chan_at[kGroups];
   // this lane's position in its image; the input row and column its tap (0, 0) reads before padding, their byte offset
   int pos, row, col;
   unsigned at;
@@ -145,13 +149,13 @@ struct Taps {
     x_w = p.x_w;
     s = p.s;
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b) {
-      const int nb = min(n0 / 16 + wave * kBlocks + b, p.n_blocks - 1);   // blocks past the last: its values once more, never stored
-      const int tap = p.blocks.div(nb), cb = nb - tap * p.blocks.d, u = p.kw.div(tap), v = tap - u * p.kw.d;
-      down[b] = __builtin_amdgcn_readfirstlane(u - p.ph);
-      right[b] = __builtin_amdgcn_readfirstlane(v - p.pw);
-      shift[b] = (down[b] * x_w + right[b]) * 4;
-      chan_at[b] = __builtin_amdgcn_readfirstlane(16 * cb * p.x_plane * 4);
+    for (int g = 0; g < kGroups; ++g) {
+      const int ng = min(n0 / G + wave * kGroups + g, p.n_groups - 1);   // groups past the last: its values once more, never stored
+      const int tap = p.groups.div(ng), cg = ng - tap * p.groups.d, u = p.kw.div(tap), v = tap - u * p.kw.d;
+      down[g] = __builtin_amdgcn_readfirstlane(u - p.ph);
+      right[g] = __builtin_amdgcn_readfirstlane(v - p.pw);
+      shift[g] = (down[g] * x_w + right[g]) * 4;
+      chan_at[g] = __builtin_amdgcn_readfirstlane(G * cg * p.x_plane * 4);
     }
     const int rows = width.div(BK), cols = BK - rows * width.d;
     row_step = rows * s;
@@ -172,14 +176,14 @@ struct Taps {
   // steps come in order
   __device__ __forceinline__ void load(int k0, int kend, unsigned lds) {
     const bool ok = k0 + static_cast<int>(threadIdx.x & 31) < kend && pos < plane;
-    lds += wave * kBlocks * 8 * kPair * 4;
+    lds += wave * kGroups * (G / 2) * kPair * 4;
 #pragma unroll
-    for (int b = 0; b < kBlocks; ++b) {
-      const bool in = ok && static_cast<unsigned>(row + down[b]) < static_cast<unsigned>(x_h) &&
-                      static_cast<unsigned>(col + right[b]) < static_cast<unsigned>(x_w);
-      const unsigned from = in ? at + shift[b] : kOobOffset;
+    for (int g = 0; g < kGroups; ++g) {
+      const bool in = ok && static_cast<unsigned>(row + down[g]) < static_cast<unsigned>(x_h) &&
+                      static_cast<unsigned>(col + right[g]) < static_cast<unsigned>(x_w);
+      const unsigned from = in ? at + shift[g] : kOobOffset;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) gt::load_word_to_lds(rsrc, from, chan_at[b] + 2 * j * x_plane * 4, lds + (8 * b + j) * kPair * 4);
+      for (int j = 0; j < G / 2; ++j) gt::load_word_to_lds(rsrc, from, chan_at[g] + 2 * j * x_plane * 4, lds + (G / 2 * g + j) * kPair * 4);
     }
     pos += BK;
     row += row_step;
@@ -205,12 +209,12 @@ struct Taps {
   }
 };
 
-// POINT: one tap, stride 1, no padding, C a multiple of 16 or not (the columns are then the channels themselves)
-template <int TM, int TN, bool POINT>
+// G: channels of a group, the columns of one tap; 0: one tap, stride 1, no padding (the columns are the channels themselves)
+template <int TM, int TN, int G>
 __global__ __launch_bounds__(gt::kThreads, 2) void conv_wgrad_tile_kernel(Params P, mg::TileGrid tg) {
-  constexpr int BM = 32 * TM, BN = 32 * TN;
+  constexpr int BM = 32 * TM, BN = 32 * TN, kGroup = G ? G : 16;
   using AL = Words<BM, TM>;
-  using BL = typename std::conditional<POINT, Words<BN, TN>, Taps<BN, TN>>::type;
+  using BL = typename std::conditional<G == 0, Words<BN, TN>, Taps<BN, TN, kGroup>>::type;
   using C = gt::Core<TM, TN, 2, 2, AL, BL>;
   __shared__ __attribute__((aligned(1024))) float lds[C::kLdsFloats];
   int z, tile_m, tile_n;
@@ -220,7 +224,7 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_wgrad_tile_kernel(Params
   AL la;
   BL lb;
   la.init(P.dy, P.dy_bytes, P.image, P.plane, P.dy_img, m0, first_image, kbegin);
-  if constexpr (POINT)
+  if constexpr (G == 0)
     lb.init(P.x, P.x_bytes, P.image, P.plane, P.x_img, n0, first_image, kbegin);
   else
     lb.init(P, n0, first_image, kbegin);
@@ -231,8 +235,8 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_wgrad_tile_kernel(Params
   const int lane = threadIdx.x & 63, m = m0 + C::wave_m0() + C::lane_row();
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const int nb = (n0 + C::wave_n0()) / 16 + j, tap = P.blocks.div(nb), c = (nb - tap * P.blocks.d) * 16 + (lane & 15);
-    if (nb >= P.n_blocks || c >= P.C) continue;
+    const int n = n0 + C::wave_n0() + 16 * j + (lane & 15), ng = n / kGroup, tap = P.groups.div(ng), c = (ng - tap * P.groups.d) * kGroup + n % kGroup;
+    if (ng >= P.n_groups || c >= P.C) continue;
     float *to = out + static_cast<int64_t>(m) * P.cols + tap * P.C + c;
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)

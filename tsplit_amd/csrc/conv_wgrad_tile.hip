@@ -38,14 +38,23 @@ __global__ __launch_bounds__(256) void fold_tap_major_kernel(const float *__rest
   }
 }
 
-template <bool POINT>
+template <int G>
 void launch_tile(const Params &P, int tile, const mg::TileGrid &tg, unsigned grid, hipStream_t st) {
   switch (tile) {
-    case 0: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 4, POINT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
-    case 1: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 4, POINT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
-    case 2: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 2, POINT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
-    default: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 2, POINT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    case 0: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 4, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    case 1: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 4, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    case 2: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 2, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    default: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 2, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
   }
+}
+
+// Channels of a group: a smaller group where it leaves a tenth of the columns out.  32 images, 7x7 filters, stride 1, 112 x 112, 353
+// filters, in groups of 16 / 4 / 2: 3 channels 2039 / 737 / - us, 6 channels 2038 / 1182 / 891.  Where it leaves out less: 29 channels,
+// 5x5, stride 2, 361 filters at 98 x 98 299 us in 16 and 327 in twos; 33 channels, 200 filters of 7x7 at 56 x 56 227 in fours and 257 in twos.
+int group_size(int chans) {
+  const int in16 = (chans + 15) / 16 * 16, in4 = (chans + 3) / 4 * 4, in2 = (chans + 1) / 2 * 2;
+  if (in2 * 10 <= in4 * 9) return 2;
+  return in4 * 10 <= in16 * 9 ? 4 : 16;
 }
 
 }  // namespace
@@ -72,9 +81,7 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   P.K = static_cast<int>(padded_depth(g));
   P.image = FastDiv(depth_per_image(g));
   P.width = FastDiv(g.oW);
-  P.blocks = FastDiv((g.C + 15) / 16);
   P.kw = FastDiv(g.kW);
-  P.n_blocks = taps * static_cast<int>(P.blocks.d);
   P.x_plane = g.H * g.W;
   P.x_img = g.C * P.x_plane;
   P.x_h = g.H;
@@ -83,7 +90,10 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   P.pw = g.pw;
   P.s = g.s;
   const bool point = taps == 1 && g.s == 1 && g.ph == 0 && g.pw == 0;
-  const int64_t cols = 16ll * P.n_blocks, values = static_cast<int64_t>(g.O) * P.cols;
+  const int group = point ? 16 : group_size(g.C);
+  P.groups = FastDiv((g.C + group - 1) / group);
+  P.n_groups = taps * static_cast<int>(P.groups.d);
+  const int64_t cols = static_cast<int64_t>(group) * P.n_groups, values = static_cast<int64_t>(g.O) * P.cols;
   const int steps = (P.K + BK - 1) / BK;
   const TilePlan plan = plan_tiles(g.O, &cols, &steps, 1, 1, 1024, static_cast<double>(values), point ? kDense : kGathered);
   const TileKind &k = kTiles[plan.tile];
@@ -102,9 +112,13 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   const mg::TileGrid tg{tm, tn, tm * tn * S};
   const unsigned grid = mg::grid_blocks(tm, tn, S);
   if (point)
-    launch_tile<true>(P, plan.tile, tg, grid, st);
+    launch_tile<0>(P, plan.tile, tg, grid, st);
+  else if (group == 16)
+    launch_tile<16>(P, plan.tile, tg, grid, st);
+  else if (group == 4)
+    launch_tile<4>(P, plan.tile, tg, grid, st);
   else
-    launch_tile<false>(P, plan.tile, tg, grid, st);
+    launch_tile<2>(P, plan.tile, tg, grid, st);
   if (taps == 1 && S > 1 && S < 8)   // (four lanes share an output's ranges in the other)
     gt::launch_fold(P.out, dw, values, S, st);
   else if (!direct)
