@@ -6,7 +6,7 @@
 //
 // Groups of 16 test a position against the image's edge once for eight loads, groups of 4 or 2 once for two loads or each one; but
 // 3 channels padded to 16 are five times the products and loads (64 x 3 x 224 x 224, 64 filters of 7x7, stride 2: 770 us in groups of
-// 16, 284 in groups of 4).
+// 16, 259 in groups of 4).
 //
 // A step's position is worked out once a lane (from the step's before it; by division only where an image begins, which as much
 // as doubles what a 64 x 64 tile spends on it) and serves every row the lane loads: rows are
@@ -19,11 +19,11 @@
 // by value, positions outside the image as zeros.  Rows past the last channel hold values of the next image: they belong to
 // rows or columns of dw that do not exist.
 //
-// What bounds it is the matrix pipe where the tiles fill the chip (1x1 layers: 64 x 512 x 28 x 28 -> 128 in 63 us, 104 TFLOP/s) and
+// What bounds it is the matrix pipe where the tiles fill the chip (1x1 layers: 64 x 512 x 28 x 28 -> 128 in 62 us, 106 TFLOP/s) and
 // the gathered loads, 4 bytes a lane, elsewhere.  Against 16-deep steps whose operands went through vector registers: 1x1 layers of
-// ResNet-50 73, 63, 70, 79 us (were 91, 90, 88, 91), 35x35 and 8x8 ones of Inception-v4 30 and 32 (52 and 52), 3x3 at 147x147
-// 278 (396), 2x2 40 (83), 3x3 stride 2 of 96 -> 200 channels 19 (33); but 1x7 of 256 -> 256 at 17x17 104 (95) and 3x3 of
-// 512 -> 512 at 28x28, 18 images, 604 (548), where the loads count most.
+// ResNet-50 66, 62, 76, 76 us (were 90, 87, 90, 90), its first layer 259 (411), 1x7 of 256 -> 256 at 17x17 93 (96), 3x3 of 512 -> 512 at
+// 4x4 71 (79), 3x3 stride 2 of 96 -> 200 channels 17 (32); but 3x3 of 512 -> 512 at 28x28, 18 images, 570 (549), where the loads count
+// most.
 #pragma once
 #include <hip/hip_runtime.h>
 

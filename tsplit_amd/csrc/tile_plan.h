@@ -1,35 +1,54 @@
 // Which tile of the tile kernel (gemm_tile.h) a product runs on and into how many ranges its depth is cut: a small model of
 // the chip, with figures measured on it.
 //
-// One CU multiplies 16 x 16 x 4 on each of its four matrix pipes in 32 clocks (2.4 GHz): a 32-deep step of a tile takes
-// `step` microseconds of it.  A block alone on its CU adds about 0.22 us a step (barrier and latencies, measured: 2.0 / 1.07 /
-// 0.65 us a step for the three tile sizes); blocks that share a CU hide that and reach `rate` of the pipe (148 TFLOP/s of 157
-// for 128 x 128 at 8192^3, 147 for 64 x 128, 135 for 64 x 64).  A launch costs 2.5 us, each round of resident blocks `round`
-// more (first loads, stores), the fold of the ranges 2.2 us and its traffic.
-// Measured against the model: 8192x512x512 35.8 us (34.5 in the model) on 64x128, 8192x512x2048 124 (127), 512x512x8192 39
-// (41) on 64x64 in 8 ranges, 64x1000x4096 13.6 (12.6) in 16, 128x256x784 8.2 (8.6) in 8.  128x128 and 64x256 tiles only, cut
-// to fill the chip with at least 16 k-steps a range, took 62, 183, 60, 34 and 34 us for these five.
+// A CU takes its blocks in rounds of as many as are resident at once.  A 32-deep step of a round takes what it takes with that many
+// blocks on the CU: one block alone waits for its barriers and loads, several fill each other's gaps (a 64 x 64 tile: 0.49 us alone,
+// 2.5 for five; the matrix pipes need 0.43 for each).  Every round costs its first loads and its stores on top, and the ranges cost
+// a second launch, which folds them, and its traffic.
+//
+// The figures come from the times of 617 launches (products and convolutions of ResNet-50, Inception-v4, VGG, a Transformer and drawn
+// shapes, on each of the four tiles with up to 30 counts of ranges): a least-squares fit without negative figures, then moved by up to
+// a quarter where that makes the choices better.  What a choice costs over the best of the four tiles and all counts, averaged: products
+// and layers of one tap 0.95 %, gathered 0.9, pairs of phases 0.5, filter gradients 1.1 (x in words) and 0.7.  A model whose step took
+// the same time however many blocks shared the CU, fitted to one count of ranges and with five 64 x 64 blocks resident everywhere, cost
+// 1.9, 2.9, 4.0, 2.2 and 3.3 %, at worst 40 (18 x 25088 x 4096 with the second operand transposed: 153 us on 64 x 128, 109 on 64 x 64;
+// 3x3 of 512 -> 512 at 7 x 7, data gradient: 181 us in 5 ranges, 156 in 6).
 #pragma once
 #include <algorithm>
 #include <cstdint>
 
 namespace tsplit {
 
-//
-// Gathered operands (convolutions with several taps) cost a load and a row of LDS for every 64 values instead of every 256, and
-// the gather is repeated for every row of tiles: the second set of figures, fitted to the four tiles' times on 117 layers of
-// ResNet-50, Inception-v4, a VGG on 32 x 32 images and ragged ones.  Its choice costs 0.7 % over the best of the four on the
-// average, the dense set's choice 2.2 %.
 struct TileKind {
-  int bm, bn, resident;
-  double step;
+  int bm, bn;
 };
-constexpr TileKind kTiles[] = {{128, 128, 2, 1.707}, {64, 128, 3, 0.853}, {128, 64, 3, 0.853}, {64, 64, 5, 0.427}};
+constexpr TileKind kTiles[] = {{128, 128}, {64, 128}, {128, 64}, {64, 64}};
 struct TileCost {
-  double alone[4], rate[4], round[4];
+  int resident[4];       // blocks a CU holds of each tile
+  double step[4][5];     // us of a step with 1, 2, ... of them on the CU
+  double round[4];       // us
+  double fold, fold_tb;  // us; TB/s
 };
-constexpr TileCost kDense = {{0.22, 0.22, 0.22, 0.22}, {0.93, 0.93, 0.91, 0.85}, {2.5, 1.5, 1.5, 1.0}};
-constexpr TileCost kGathered = {{0.95, 0.87, 0.95, 0.95}, {0.70, 0.64, 0.73, 0.71}, {5.6, 4.9, 3.9, 4.3}};
+// both operands in words: products, convolutions of one tap
+constexpr TileCost kDense = {{2, 3, 3, 5},
+                             {{2.66, 3.66}, {1.28, 2.05, 2.80}, {1.19, 2.00, 2.80}, {0.49, 0.87, 1.25, 1.95, 2.47}},
+                             {2.7, 1.8, 1.9, 1.6}, 2.1, 9.5};
+// one operand gathered by tap: a load and a row of LDS for every 64 values instead of every 256
+constexpr TileCost kGathered = {{2, 3, 3, 5},
+                                {{2.44, 4.63}, {1.34, 2.34, 3.57}, {1.44, 2.68, 3.27}, {0.82, 1.25, 1.77, 2.36, 3.07}},
+                                {1.9, 1.7, 0.7, 0.9}, 2.5, 8.1};
+// the same in pairs of phases (data gradients of stride 2)
+constexpr TileCost kPairs = {{2, 3, 3, 5},
+                             {{4.10, 6.99}, {1.87, 3.79, 4.41}, {1.62, 2.98, 4.18}, {0.82, 1.34, 1.92, 3.02, 4.00}},
+                             {3.6, 2.9, 0.8, 1.3}, 1.1, 4.9};
+// filter gradients, x in words and by tap: rows of LDS are padded (34 KB for 64 x 64: four blocks, not five).  With several taps
+// the ranges are folded even if there is one.
+constexpr TileCost kFilterDense = {{2, 3, 3, 4},
+                                   {{2.50, 4.25}, {1.22, 2.00, 3.00}, {1.30, 2.40, 3.20}, {0.65, 1.14, 1.67, 2.19}},
+                                   {1.5, 1.5, 1.0, 0.3}, 2.0, 7.5};
+constexpr TileCost kFilterGathered = {{2, 3, 3, 4},
+                                      {{3.38, 4.57}, {1.44, 3.07, 3.68}, {1.35, 2.40, 3.34}, {0.85, 1.36, 2.04, 2.49}},
+                                      {0.6, 0.5, 0, 0}, 2.0, 6.2};
 struct TilePlan {
   int tile, S;
 };
@@ -37,13 +56,14 @@ struct TilePlan {
 // A launch of `parts` products of M rows each (the phases of a strided data gradient; 1 otherwise), every one `batch` times:
 // part i has cols[i] columns and a depth of steps[i] x 32.  max_split 1: the depth stays whole.
 inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int parts, int64_t batch, int max_split, double out_values,
-                           const TileCost &cost = kDense) {
+                           const TileCost &cost) {
   TilePlan best{0, 1};
   double least = 1e300;
   int deepest = 1;
   for (int i = 0; i < parts; ++i) deepest = std::max(deepest, steps[i]);
   for (int t = 0; t < 4; ++t) {
     const TileKind &k = kTiles[t];
+    const int resident = cost.resident[t];
     int64_t tiles = 0;
     double work = 0;   // steps of all tiles
     for (int i = 0; i < parts; ++i) {
@@ -51,18 +71,27 @@ inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int
       tiles += n;
       work += static_cast<double>(n) * steps[i];
     }
-    for (int S = 1; S <= max_split && S <= deepest; S += std::max(1, S / 4)) {
-      if (S > 1 && tiles > 1024) break;
+    auto consider = [&](int S) {
       const int per = (deepest + S - 1) / S;
-      const double n = static_cast<double>((tiles * S + 255) / 256), rounds = static_cast<double>((static_cast<int64_t>(n) + k.resident - 1) / k.resident);
+      S = (deepest + per - 1) / per;
+      const int64_t n = (tiles * S + 255) / 256, whole = n / resident, rest = n - whole * resident;   // blocks of the busiest CU
       const double mean = parts == 1 ? per : std::max(1.0, work / (static_cast<double>(tiles) * S));
-      double us = std::max(per * (k.step + cost.alone[t]), n > 1 ? n * mean * k.step / cost.rate[t] : 0.0) + 2.5 + cost.round[t] * rounds;
-      if (S > 1) us += 2.2 + (2 * S + 1) * out_values * 4 / 5e6;
+      double us = whole * (mean * cost.step[t][resident - 1] + cost.round[t]);
+      if (rest) us += mean * cost.step[t][rest - 1] + cost.round[t];
+      if (S > 1) us += cost.fold + (2 * S + 1) * out_values * 4 / (cost.fold_tb * 1e6);
       if (us < least) {
         least = us;
         best = {t, S};
       }
+    };
+    const int most = tiles > 1024 ? 1 : std::min(max_split, deepest);
+    for (int S = 1, by = 1; S <= most; S += by) {   // 1 to 8, then four to every doubling
+      if (S == 8 * by) by *= 2;
+      consider(S);
     }
+    // as many ranges as give every CU the same number of blocks
+    for (int n = 1; n <= 10; ++n)
+      if (const int64_t S = tiles > 0 ? 256 * n / tiles : 0; S > 1 && S <= most) consider(static_cast<int>(S));
   }
   return best;
 }
