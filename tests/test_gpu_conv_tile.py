@@ -60,6 +60,38 @@ def test_convolutions_at_the_edges(case, sums, rng, monkeypatch):
     assert (np.abs(dx.asnumpy() - want) <= _bound(size, Oc * kh * kw + 32)).all(), case
 
 
+@pytest.mark.parametrize("case", [
+    (3, 34, 8, 8, 35, 1, 1, 0, 0, 1),      # words
+    (3, 33, 7, 7, 35, 1, 1, 0, 0, 1),      # planes that are not whole words
+    (3, 33, 9, 7, 35, 1, 1, 0, 0, 2),
+    (3, 17, 9, 10, 19, 3, 3, 1, 1, 1),     # 24 = 17 + 7 padded channels, 24 = 19 + 5
+    (3, 17, 9, 10, 19, 3, 3, 1, 1, 2),     # pairs of phases
+    (3, 5, 11, 13, 9, 5, 5, 2, 2, 1),      # depth in the filter's order
+    (3, 9, 12, 11, 16, 8, 8, 4, 3, 3),     # single phases
+])
+def test_infinities_stay_in_their_images_and_channels(case, rng, monkeypatch):
+    """The channels that pad the depth are the next image's or the next filter's first values: they must not reach a sum, not even
+    times zero, in either pass."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    monkeypatch.setenv("TSPLIT_CONV_WINOGRAD", "0")
+    ctx, (N, C, H, W, Oc, kh, kw, ph, pw, s) = nd.gpu(0), case
+    ys = (N, Oc, (H + 2 * ph - kh) // s + 1, (W + 2 * pw - kw) // s + 1)
+    x, w, dy = (rng.normal(size=shape).astype(np.float32) for shape in ((N, C, H, W), (Oc, C, kh, kw), ys))
+    x[1] = dy[1] = np.inf
+    y, dx = nd.empty(ys, ctx), nd.empty(x.shape, ctx)
+
+    def run():
+        L.CuDNN_conv2d(nd.array(x, ctx), nd.array(w, ctx), y, ph, pw, s)
+        L.CuDNN_conv2d_gradient_of_data(nd.array(w, ctx), nd.array(dy, ctx), dx, ph, pw, s)
+        return np.isfinite(y.asnumpy()), np.isfinite(dx.asnumpy())
+    for finite in run():
+        assert finite[[0, 2]].all() and not finite[1].all()
+    w[3, 4] = np.nan                             # one channel of one filter: the output's channel 3, the gradient's channel 4
+    fy, fdx = run()
+    assert np.delete(fy, 3, 1)[[0, 2]].all() and not fy[0, 3].any(), "forward"
+    assert np.delete(fdx, 4, 1)[[0, 2]].all() and not fdx[0, 4].all(), "data gradient"
+
+
 def test_channels_past_the_last_beyond_32_bit_offsets(rng):
     """Eight output channels in a tile of 64 rows or more, planes so large that the missing ones lie past 32-bit offsets: nothing
     is stored for them anywhere."""

@@ -47,7 +47,7 @@ def test_products_at_the_edges(shape, ta, tb, rng):
         assert (np.abs(got - a64 @ b64) <= _bound(a64, b64)).all(), (shape, ta, tb, shift)
 
 
-@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("shape", [(3, 1, 1, 1), (5, 77, 50, 64), (40, 129, 65, 33), (20, 64, 128, 77)])
 def test_batched_products_at_the_edges(shape, ta, tb, rng):
     from tsplit_amd import gpu_links as L, ndarray as nd
@@ -58,6 +58,27 @@ def test_batched_products_at_the_edges(shape, ta, tb, rng):
     c = nd.array(np.full((B, M, N), 7, np.float32), ctx)
     L.batch_matrix_multiply(nd.array(a, ctx), ta, nd.array(b, ctx), tb, c)
     assert (np.abs(c.asnumpy() - a64 @ b64) <= _bound(a64, b64)).all(), (shape, ta, tb)
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("shape", [(70, 45, 5), (40, 130, 33), (65, 66, 1030)])
+def test_infinities_stay_in_their_rows_and_columns(shape, ta, tb, rng):
+    """A word that the end of K cuts holds the next row's first values, and behind a batch's last row lies the next batch: neither may
+    reach another row's sums, not even times zero."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    ctx, (M, N, K) = nd.gpu(0), shape
+    a, b = rng.normal(size=(2, M, K)).astype(np.float32), rng.normal(size=(2, K, N)).astype(np.float32)
+    a[0, 7, 0], b[0, 0, 5] = np.inf, np.nan
+    a[1, 0, :], b[1, :, 0] = np.inf, np.nan      # behind the first batch
+    ga, gb = (np.ascontiguousarray(v.transpose(0, 2, 1)) if t else v for v, t in ((a, ta), (b, tb)))
+    c, batched = nd.empty((M, N), ctx), nd.empty((2, M, N), ctx)
+    L.matrix_multiply(nd.array(ga[0], ctx), ta, nd.array(gb[0], ctx), tb, c)
+    L.batch_matrix_multiply(nd.array(ga, ctx), ta, nd.array(gb, ctx), tb, batched)
+    for got, row, col in ((c.asnumpy(), 7, 5), (batched.asnumpy()[0], 7, 5), (batched.asnumpy()[1], 0, 0)):
+        own = np.zeros((M, N), bool)
+        own[row, :] = own[:, col] = True
+        finite = np.isfinite(got)
+        assert finite[~own].all() and not finite[own].any()
 
 
 def test_rows_of_the_result_beyond_32_bit_offsets(rng):
