@@ -7,7 +7,7 @@ import subprocess
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tsplit_amd", "csrc")
-COSTS = ["kDense", "kGathered", "kPairs", "kFilterDense", "kFilterGathered"]
+COSTS = ["kProductCost", "kOneTapCost", "kGatheredCost", "kPairsCost", "kFilterWordsCost", "kFilterTapsCost"]
 SOURCE = """
 #include "tile_plan.h"
 using namespace tsplit;
@@ -23,47 +23,47 @@ extern "C" void plan(int cost, long long M, const long long *cols, const int *st
 
 # name, cost, rows, columns and steps of each part, most ranges, values of the result, us by ranges on 128x128, 64x128, 128x64, 64x64
 MEASURED = [
-    ("18 x 25088 x 4096, second operand transposed", "kDense", 18, [25088], [128], 64, 451584,
+    ("18 x 25088 x 4096, second operand transposed", "kProductCost", 18, [25088], [128], 64, 451584,
      [{2: 240, 4: 244, 5: 203, 7: 223, 8: 228, 9: 236, 10: 210, 12: 224, 13: 208, 14: 206, 16: 231, 20: 240, 24: 235, 28: 227, 32: 241, 40: 241},
       {2: 128, 3: 129, 4: 139, 6: 134, 7: 120, 8: 126, 9: 141, 10: 126, 11: 121, 12: 135, 14: 135, 16: 133, 20: 131, 24: 135, 28: 136, 32: 143, 40: 143, 48: 146},
       {1: 245, 3: 211, 4: 223, 5: 206, 6: 220, 7: 210, 8: 212, 10: 215, 12: 219, 14: 213, 16: 216, 20: 231, 24: 231, 28: 234, 32: 242, 40: 244},
       {2: 129, 4: 130, 5: 108, 6: 129, 7: 121, 8: 122, 10: 117, 12: 126, 14: 119, 16: 127, 24: 131}]),
-    ("64 x 25088 x 4096, the same", "kDense", 64, [25088], [128], 64, 1605632,
+    ("64 x 25088 x 4096, the same", "kProductCost", 64, [25088], [128], 64, 1605632,
      [{2: 242, 4: 249, 5: 209, 7: 230, 8: 236, 9: 246, 10: 222, 12: 239, 13: 222, 14: 219, 16: 246, 28: 250},
       {2: 133, 3: 134, 4: 146, 6: 143, 7: 131, 8: 141, 9: 151, 10: 139, 11: 136, 12: 158, 14: 152, 16: 154, 20: 156},
       {1: 246, 3: 212, 4: 227, 5: 208, 6: 224, 7: 218, 8: 220, 10: 223, 12: 230, 14: 227, 16: 231, 20: 246, 24: 250},
       {1: 137, 2: 138, 4: 135, 5: 123, 6: 137, 7: 131, 8: 134, 10: 131, 12: 146, 14: 139}]),
-    ("1x1, 2048 -> 512 at 7 x 7", "kDense", 512, [3136], [64], 32, 1605632,
+    ("1x1, 2048 -> 512 at 7 x 7", "kOneTapCost", 512, [3136], [64], 32, 1605632,
      [{2: 89, 4: 80, 5: 74},
       {2: 76, 3: 83, 4: 88, 5: 85, 6: 79, 7: 88, 8: 87, 10: 92},
       {1: 90, 2: 85, 3: 82, 4: 84, 5: 82, 6: 74, 7: 79, 8: 79, 9: 80, 10: 81, 11: 81, 12: 81, 14: 86, 16: 89, 20: 89},
       {1: 69, 2: 75, 3: 78, 4: 71, 5: 69, 6: 73, 7: 75, 8: 76, 10: 83, 12: 82}]),
-    ("3x3, 512 -> 512 at 7 x 7, data gradient", "kGathered", 512, [3136], [144], 32, 1605632,
+    ("3x3, 512 -> 512 at 7 x 7, data gradient", "kGatheredCost", 512, [3136], [144], 32, 1605632,
      [{2: 202, 4: 195, 5: 166, 6: 201, 7: 183, 8: 200, 10: 184, 12: 192},
       {2: 202, 3: 195, 4: 202, 5: 170, 6: 183, 7: 185, 8: 186, 10: 186, 12: 195, 14: 199, 16: 203},
       {3: 179, 4: 186, 5: 181, 6: 161, 7: 164, 8: 171, 9: 158, 10: 168, 12: 174, 13: 173, 14: 177, 16: 178, 20: 177, 24: 192, 28: 190},
       {2: 190, 3: 172, 4: 171, 5: 162, 6: 170, 7: 167, 8: 172, 10: 178, 12: 177, 14: 187, 16: 186, 20: 188}]),
-    ("3x3 stride 2, 224 -> 256 at 35 x 35", "kGathered", 256, [9248], [63], 32, 2367488,
+    ("3x3 stride 2, 224 -> 256 at 35 x 35", "kGatheredCost", 256, [9248], [63], 32, 2367488,
      [{3: 120, 4: 135, 5: 118, 6: 129, 7: 116, 8: 125, 10: 132, 12: 136, 14: 139},
       {2: 133, 3: 128, 4: 122, 5: 119, 6: 123, 7: 120, 8: 130, 10: 130, 12: 135, 14: 139},
       {2: 119, 3: 115, 4: 110, 5: 108, 6: 110, 7: 108, 8: 119, 10: 118, 12: 126, 14: 127},
       {1: 129, 2: 117, 3: 109, 4: 116, 5: 116, 6: 119, 7: 117, 8: 124, 10: 125}]),
-    ("3x3 stride 2, 384 -> 384 at 35 x 35, data gradient", "kPairs", 384, [10368, 9792], [72, 36], 32, 15052800,
+    ("3x3 stride 2, 384 -> 384 at 35 x 35, data gradient", "kPairsCost", 384, [10368, 9792], [72, 36], 32, 15052800,
      [{1: 375, 2: 441},
       {1: 384, 2: 424, 3: 455},
       {1: 357, 2: 387, 3: 406, 4: 418, 5: 435},
       {1: 360, 2: 378, 3: 405, 4: 426, 5: 439}]),
-    ("1x1, 64 -> 256 at 56 x 56, filter gradient", "kFilterDense", 256, [64], [6272], 1024, 16384,
+    ("1x1, 64 -> 256 at 56 x 56, filter gradient", "kFilterWordsCost", 256, [64], [6272], 1024, 16384,
      [{128: 121, 256: 120, 512: 130},
       {64: 134, 128: 113, 192: 113, 256: 134, 384: 124},
       {128: 72, 256: 71, 384: 73},
       {64: 84, 128: 70, 192: 70, 256: 69, 384: 72, 448: 74}]),
-    ("3x3, 512 -> 512 at 28 x 28, filter gradient", "kFilterGathered", 512, [4608], [441], 1024, 2359296,
+    ("3x3, 512 -> 512 at 28 x 28, filter gradient", "kFilterTapsCost", 512, [4608], [441], 1024, 2359296,
      [{3: 658, 5: 615, 6: 667, 7: 575, 8: 639, 10: 620, 12: 603, 14: 593, 16: 578, 17: 603, 20: 642, 24: 639, 28: 640, 32: 632, 40: 657, 48: 700},
       {3: 707, 4: 658, 5: 620, 6: 619, 7: 602, 8: 601, 10: 646, 12: 622, 14: 624, 16: 608, 20: 649, 24: 650, 28: 669, 32: 662, 40: 686, 48: 715},
       {3: 673, 4: 626, 5: 599, 6: 592, 7: 576, 8: 579, 10: 619, 12: 601, 14: 600, 16: 584, 20: 623, 24: 622, 28: 636, 32: 632, 40: 657, 48: 687},
       {2: 700, 3: 626, 4: 607, 5: 641, 6: 626, 7: 616, 8: 615, 10: 635, 12: 614, 14: 634, 16: 621, 20: 646, 24: 656, 28: 665, 32: 666, 40: 688, 48: 723}]),
-    ("3x3 stride 2, 64 -> 96 at 147 x 147, filter gradient", "kFilterGathered", 96, [576], [5332], 1024, 55296,
+    ("3x3 stride 2, 64 -> 96 at 147 x 147, filter gradient", "kFilterTapsCost", 96, [576], [5332], 1024, 55296,
      [{48: 302, 51: 288, 96: 276, 102: 262, 128: 313, 153: 276, 204: 275, 256: 278, 307: 285, 358: 285},
       {48: 305, 51: 287, 64: 308, 76: 267, 96: 289, 102: 277, 128: 273, 153: 272, 179: 279, 204: 284, 230: 286, 256: 284},
       {56: 245, 80: 234, 85: 223, 96: 270, 113: 238, 128: 253, 142: 238, 170: 235, 199: 237, 227: 244, 256: 240},

@@ -52,7 +52,7 @@ int run_phases(Params &P, bool bwd, int gather, bool across, bool pairs, float *
     cols[parts] = P.phase[i].N;
     steps[parts] = (P.phase[i].K + BK - 1) / BK + (pairs ? (P.phase[i + 1].K + BK - 1) / BK : 0);
   }
-  const TileCost &cost = gather == kWords || gather == kOneTap ? kDense : pairs ? kPairs : kGathered;
+  const TileCost &cost = gather == kWords || gather == kOneTap ? kOneTapCost : pairs ? kPairsCost : kGatheredCost;
   const TilePlan plan = plan_tiles(P.M, cols, steps, parts, 1, out_values < 0 ? 1 : 32, static_cast<double>(out_values), cost);
   const TileKind &k = kTiles[plan.tile];
   int S = 1;

@@ -95,7 +95,7 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   P.n_groups = taps * static_cast<int>(P.groups.d);
   const int64_t cols = static_cast<int64_t>(group) * P.n_groups, values = static_cast<int64_t>(g.O) * P.cols;
   const int steps = (P.K + BK - 1) / BK;
-  const TilePlan plan = plan_tiles(g.O, &cols, &steps, 1, 1, 1024, static_cast<double>(values), point ? kFilterDense : kFilterGathered);
+  const TilePlan plan = plan_tiles(g.O, &cols, &steps, 1, 1, 1024, static_cast<double>(values), point ? kFilterWordsCost : kFilterTapsCost);
   const TileKind &k = kTiles[plan.tile];
   P.kchunk = range_depth(g, reach, plan.S);
   const int S = std::max(1, (P.K + P.kchunk - 1) / P.kchunk);

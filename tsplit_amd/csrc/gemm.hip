@@ -31,7 +31,7 @@ struct Plan {
 Plan best_plan(int M, int N, int K, int batch, bool may_split) {
   const int64_t cols = N;
   const int steps = std::max(1, (K + gt::BK - 1) / gt::BK);
-  const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, kDense);
+  const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, kProductCost);
   Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK};
   p.S = std::max(1, (K + p.kchunk - 1) / p.kchunk);
   if (p.S == 1) p.kchunk = K;

@@ -2,14 +2,14 @@
 // the chip, with figures measured on it.
 //
 // A CU takes its blocks in rounds of as many as are resident at once.  A 32-deep step of a round takes what it takes with that many
-// blocks on the CU: one block alone waits for its barriers and loads, several fill each other's gaps (a 64 x 64 tile: 0.49 us alone,
+// blocks on the CU: one block alone waits for its barriers and loads, several fill each other's gaps (a 64 x 64 tile: 0.52 us alone,
 // 2.5 for five; the matrix pipes need 0.43 for each).  Every round costs its first loads and its stores on top, and the ranges cost
 // a second launch, which folds them, and its traffic.
 //
 // The figures come from the times of 617 launches (products and convolutions of ResNet-50, Inception-v4, VGG, a Transformer and drawn
 // shapes, on each of the four tiles with up to 30 counts of ranges): a least-squares fit without negative figures, then moved by up to
 // a quarter where that makes the choices better.  What a choice costs over the best of the four tiles and all counts, averaged: products
-// and layers of one tap 0.95 %, gathered 0.9, pairs of phases 0.5, filter gradients 1.1 (x in words) and 0.7.  A model whose step took
+// and layers of one tap 0.9 %, gathered 0.9, pairs of phases 0.5, filter gradients 1.1 (x in words) and 0.7.  A model whose step took
 // the same time however many blocks shared the CU, fitted to one count of ranges and with five 64 x 64 blocks resident everywhere, cost
 // 1.9, 2.9, 4.0, 2.2 and 3.3 %, at worst 40 (18 x 25088 x 4096 with the second operand transposed: 153 us on 64 x 128, 109 on 64 x 64;
 // 3x3 of 512 -> 512 at 7 x 7, data gradient: 181 us in 5 ranges, 156 in 6).
@@ -29,24 +29,28 @@ struct TileCost {
   double round[4];       // us
   double fold, fold_tb;  // us; TB/s
 };
-// both operands in words: products, convolutions of one tap
-constexpr TileCost kDense = {{2, 3, 3, 5},
-                             {{2.66, 3.66}, {1.28, 2.05, 2.80}, {1.19, 2.00, 2.80}, {0.49, 0.87, 1.25, 1.95, 2.47}},
-                             {2.7, 1.8, 1.9, 1.6}, 2.1, 9.5};
+// products
+constexpr TileCost kProductCost = {{2, 3, 3, 5},
+                                   {{2.59, 3.73}, {1.35, 1.93, 2.82}, {1.21, 2.19, 2.85}, {0.52, 0.96, 1.37, 2.03, 2.47}},
+                                   {2.0, 1.3, 2.0, 1.2}, 2.2, 7.2};
+// convolutions of one tap
+constexpr TileCost kOneTapCost = {{2, 3, 3, 5},
+                                  {{1.88, 3.76}, {1.41, 2.28, 2.84}, {0.89, 1.77, 2.84}, {0.48, 0.90, 1.25, 1.74, 2.46}},
+                                  {4.2, 2.5, 2.6, 2.3}, 0.5, 11.8};
 // one operand gathered by tap: a load and a row of LDS for every 64 values instead of every 256
-constexpr TileCost kGathered = {{2, 3, 3, 5},
-                                {{2.44, 4.63}, {1.34, 2.34, 3.57}, {1.44, 2.68, 3.27}, {0.82, 1.25, 1.77, 2.36, 3.07}},
-                                {1.9, 1.7, 0.7, 0.9}, 2.5, 8.1};
+constexpr TileCost kGatheredCost = {{2, 3, 3, 5},
+                                    {{2.44, 4.63}, {1.34, 2.34, 3.57}, {1.44, 2.68, 3.27}, {0.82, 1.25, 1.77, 2.36, 3.07}},
+                                    {1.9, 1.7, 0.7, 0.9}, 2.5, 8.1};
 // the same in pairs of phases (data gradients of stride 2)
-constexpr TileCost kPairs = {{2, 3, 3, 5},
-                             {{4.10, 6.99}, {1.87, 3.79, 4.41}, {1.62, 2.98, 4.18}, {0.82, 1.34, 1.92, 3.02, 4.00}},
-                             {3.6, 2.9, 0.8, 1.3}, 1.1, 4.9};
+constexpr TileCost kPairsCost = {{2, 3, 3, 5},
+                                 {{4.10, 6.99}, {1.87, 3.79, 4.41}, {1.62, 2.98, 4.18}, {0.82, 1.34, 1.92, 3.02, 4.00}},
+                                 {3.6, 2.9, 0.8, 1.3}, 1.1, 4.9};
 // filter gradients, x in words and by tap: rows of LDS are padded (34 KB for 64 x 64: four blocks, not five).  With several taps
 // the ranges are folded even if there is one.
-constexpr TileCost kFilterDense = {{2, 3, 3, 4},
-                                   {{2.50, 4.25}, {1.22, 2.00, 3.00}, {1.30, 2.40, 3.20}, {0.65, 1.14, 1.67, 2.19}},
-                                   {1.5, 1.5, 1.0, 0.3}, 2.0, 7.5};
-constexpr TileCost kFilterGathered = {{2, 3, 3, 4},
+constexpr TileCost kFilterWordsCost = {{2, 3, 3, 4},
+                                       {{2.50, 4.25}, {1.22, 2.00, 3.00}, {1.30, 2.40, 3.20}, {0.65, 1.14, 1.67, 2.19}},
+                                       {1.5, 1.5, 1.0, 0.3}, 2.0, 7.5};
+constexpr TileCost kFilterTapsCost = {{2, 3, 3, 4},
                                       {{3.38, 4.57}, {1.44, 3.07, 3.68}, {1.35, 2.40, 3.34}, {0.85, 1.36, 2.04, 2.49}},
                                       {0.6, 0.5, 0, 0}, 2.0, 6.2};
 struct TilePlan {
