@@ -4,9 +4,9 @@
 // computed on the fly while tiles are staged into LDS.
 //
 // Which kernels run: first layers (few reduction indices) the thin ones below; wide 3x3 layers the
-// Winograd routine (winograd.hip); every other forward and backward-data pass the tile kernel
-// (conv_tile.h).  The gather loaders below serve what the tile kernel does not take (more than 64
-// taps, an image beyond 2 GiB) and the filter gradients.
+// Winograd routine (winograd.hip); every other pass the tile kernels (conv_tile.h, conv_wgrad_tile.h).
+// The gather loaders below serve what those do not take: more than 64 taps, an image beyond 2 GiB, a
+// filter gradient whose three images, or whose one step, lie further apart.
 //
 //   forward     y[img,o,p]  : M = O,  N = imgs*oH*oW, K = C*kH*kW
 //                 A = filter [O][K] as it lies in memory (K contiguous)
@@ -1383,8 +1383,8 @@ void zero_fill(DLArray *a, hipStream_t st) {
 }
 
 // `stats_dst` (optional): per-channel (sum, sum of squares) of y as doubles, [O][2], for a BatchNorm that
-// follows.  The Winograd routine and the tap-major kernels produce them in their epilogues; the other
-// routes by a pass over y.
+// follows.  The Winograd routine and the tile kernel produce them in their epilogues (the latter unless it
+// adds up ranges of the depth); the other routes by a pass over y.
 int conv_forward(const char *who, const DLArray *x, const DLArray *w, DLArray *y, int ph, int pw, int s,
                  DLStreamHandle sh, ProfilerHandle p, double *stats_dst = nullptr) {
   ConvGeo g;
