@@ -130,3 +130,26 @@ def test_convolutions_of_values_without_a_split(layer, kind, where, rng, monkeyp
                 ok = np.ones(so, bool)
             want = ref(finite(a), finite(b))
             assert (np.abs(got[ok] - want[ok]) <= (depth + 64) * 2.0 ** -24 * size[ok] + 1e-37).all(), (name, first, kind)
+
+
+@pytest.mark.parametrize("scales", [(1.0, 1.0), (1e-36, 1e20), (1e20, 1e-36), (1e-41, 1e30), (1e35, 1e-3)])
+@pytest.mark.parametrize("layer", [(2, 144, 14, 18, 200), (3, 272, 7, 9, 130)])
+def test_winograd_gemms_hold_every_scale(layer, scales, rng, monkeypatch):
+    """Layers whose transformed tensors go through the prepared and the twice-split GEMMs (more than 64 channels on both sides, the
+    forms with both sides at most 256 switched to them by the ragged channel counts), with operands that have no split."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    monkeypatch.setenv("TSPLIT_CONV_WINOGRAD", "1")
+    ctx, (n, c, h, w, o) = nd.gpu(0), layer
+    x, f, dy = [rng.normal(size=s) for s in ((n, c, h, w), (o, c, 3, 3), (n, o, h, w))]
+    x32, f32, dy32 = (x * scales[0]).astype(np.float32), (f * scales[1]).astype(np.float32), (dy * scales[1]).astype(np.float32)
+    y, dx, dw = nd.empty((n, o, h, w), ctx), nd.empty((n, c, h, w), ctx), nd.empty((o, c, 3, 3), ctx)
+    L.CuDNN_conv2d(nd.array(x32, ctx), nd.array(f32, ctx), y, 1, 1, 1)
+    L.CuDNN_conv2d_gradient_of_filter(nd.array(x32, ctx), nd.array(dy32, ctx), dw, 1, 1, 1)
+    L.CuDNN_conv2d_gradient_of_data(nd.array(f32, ctx), nd.array((dy * scales[0]).astype(np.float32), ctx), dx, 1, 1, 1)
+    size = scales[0] * scales[1]
+    # the transforms' own share is 2e-5; subnormal operands come with fewer bits of their own
+    tol = 1e-4 if min(scales) > 1e-38 else 1e-2
+    for got, want in ((y, O.conv2d(x32, f32, 1, 1, 1)), (dw, O.conv2d_grad_filter(x32, dy32, f.shape, 1, 1, 1)),
+                      (dx, O.conv2d_grad_data(f32, (dy * scales[0]).astype(np.float32), x.shape, 1, 1, 1))):
+        want = want / size
+        assert np.abs(got.asnumpy().astype(np.float64) / size - want).max() <= tol * np.abs(want).max()

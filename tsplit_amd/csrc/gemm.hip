@@ -104,13 +104,13 @@ void launch_split_tile(const st::PlanesParams &rows, const st::DenseRows &src, c
                        int K, const Plan &plan, hipStream_t s) {
   const int tm = (P + 16 * TM * WM - 1) / (16 * TM * WM), tn = (X + 16 * TN * WN - 1) / (16 * TN * WN);
   hipLaunchKernelGGL((st::gemm_split_kernel<TM, TN, WM, WN, XMN, ACROSS>), dim3(grid_blocks(tm, tn, plan.S)), dim3(gt::kThreads), 0, s, rows, src, xp,
-                     out, mn, wide, P, X, K, plan.kchunk, TileGrid{tm, tn, tm * tn * plan.S});
+                     out, st::SplitStrides{0, 0, 0, mn}, wide, P, X, K, plan.kchunk, TileGrid{tm, tn, tm * tn * plan.S});
 }
 template <bool XMN, bool ACROSS>
 void launch_prepared(const st::DenseRows &src, const DenseParams &xp, char *planes, float *out, int P, int X, int K, const Plan &plan, hipStream_t s) {
   const int steps = (K + gt::BK - 1) / gt::BK, tiles = (P + 15) / 16, total = tiles * steps * 64;
   const int64_t mn = static_cast<int64_t>(P) * X;
-  hipLaunchKernelGGL(st::planes_kernel, dim3((total + 255) / 256), dim3(256), 0, s, src, planes, FastDiv(steps), total);
+  hipLaunchKernelGGL(st::planes_kernel, dim3((total + 255) / 256), dim3(256), 0, s, src, 0, planes, FastDiv(steps), total);
   const st::PlanesParams rows{planes, tiles, steps};
   const bool wide = (ACROSS ? P : X) % 4 == 0 && aligned16(out);
   switch (plan.tile) {

@@ -297,18 +297,25 @@ __device__ __forceinline__ void put_planes(const Src &src, int row, int k, char 
 #pragma unroll
   for (int s = 0; s < 3; ++s) *reinterpret_cast<bf16x8 *>(chunk + 1024 * s + 16 * lane) = w[s];
 }
-static __global__ __launch_bounds__(256) void planes_kernel(DenseRows src, char *__restrict__ out, FastDiv steps, int total) {
+// blockIdx.y: one of a batch of operands, `stride` values apart, and its planes
+static __global__ __launch_bounds__(256) void planes_kernel(DenseRows src, int64_t stride, char *__restrict__ out, FastDiv steps, int total) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
+  src.p += blockIdx.y * stride;
+  out += static_cast<int64_t>(blockIdx.y) * (total / 64) * kChunk;
   const int lane = i & 63, chunk = i >> 6, tile = steps.div(chunk);
   put_planes(src, 16 * tile + (lane & 15), (chunk - tile * steps.d) * BK + 4 * (lane >> 4), out + static_cast<int64_t>(chunk) * kChunk, lane);
 }
 
 // ---- dense products.  C[M,N] = rows x columns: the rows of A and the columns of B, or (ACROSS) the columns of B and the rows of A.
-// XMN: the columns' operand is stored with the depth as its rows.
+// XMN: the columns' operand is stored with the depth as its rows.  Batch z's operands and result begin z strides further on; with
+// kchunk < K (a batch of one) z is a range of the depth.
+struct SplitStrides {
+  int64_t planes, src, x, out;
+};
 template <int TM, int TN, int WM, int WN, bool XMN, bool ACROSS>
 __global__ __launch_bounds__(gt::kThreads, 2) void gemm_split_kernel(PlanesParams rows, DenseRows src, mg::DenseParams xp, float *__restrict__ out,
-                                                                     int64_t z_stride, bool wide, int P, int X, int K, int kchunk, mg::TileGrid tg) {
+                                                                     SplitStrides zs, bool wide, int P, int X, int K, int kchunk, mg::TileGrid tg) {
   using BL = typename std::conditional<XMN, gt::MnContig<16 * TN * WN, TN>, gt::KContig<16 * TN * WN, TN, !ACROSS>>::type;
   using C = Core<TM, TN, WM, WN, BL>;
   __shared__ __attribute__((aligned(1024))) float lds_f[C::kLdsFloats];
@@ -316,6 +323,9 @@ __global__ __launch_bounds__(gt::kThreads, 2) void gemm_split_kernel(PlanesParam
   int z, tile_m, tile_n;
   if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
   const int m0 = tile_m * C::BM, n0 = tile_n * C::BN, kbegin = kchunk < K ? z * kchunk : 0, kend = min(K, kbegin + kchunk);
+  rows.p += z * zs.planes;
+  src.p += z * zs.src;
+  xp.p += z * zs.x;
   typename C::AL la;
   BL lb;
   la.init(rows, m0);
@@ -323,7 +333,7 @@ __global__ __launch_bounds__(gt::kThreads, 2) void gemm_split_kernel(PlanesParam
   f32x4 acc[TM][TN];
   if (!C::run(la, lb, kbegin, kend, lds, acc)) C::exact(src, m0, lb, kbegin, kend, lds, acc);
 
-  float *o = out + z * z_stride;
+  float *o = out + z * zs.out;
   const int lane = threadIdx.x & 63, idx = lane & 15;
   if constexpr (!ACROSS) {
     const int64_t ldc = X;
@@ -373,6 +383,31 @@ __global__ __launch_bounds__(gt::kThreads, 2) void gemm_split_kernel(PlanesParam
       }
     }
   }
+}
+
+// Both operands split by the waves: batch z % batch of operands `zs.a` and `zs.b` values apart, range z / batch of the depth; result z begins
+// z * zs.c values further on.
+template <int TM, int TN, int WM, int WN, bool TA, bool TB>
+__global__ __launch_bounds__(gt::kThreads, 2) void gemm_both_kernel(mg::DenseParams ap, mg::DenseParams bp, float *__restrict__ out, gt::Strides zs, int batch,
+                                                                    bool wide, int M, int N, int K, int kchunk, mg::TileGrid tg) {
+  using T = gt::Tile<TM, TN, WM, WN, TA, TB>;
+  using C = CoreBoth<TM, TN, WM, WN, typename T::AL, typename T::BL>;
+  __shared__ __attribute__((aligned(1024))) float lds[T::C::kLdsFloats];
+  int z, tile_m, tile_n;
+  if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
+  const int range = z / batch, m0 = tile_m * T::BM, n0 = tile_n * T::BN, kbegin = range * kchunk, kend = min(K, kbegin + kchunk);
+  ap.p += (z - range * batch) * zs.a;
+  bp.p += (z - range * batch) * zs.b;
+  typename T::AL la;
+  typename T::BL lb;
+  la.init(ap, m0);
+  lb.init(bp, n0);
+  f32x4 acc[TM][TN];
+  if (!C::run(la, lb, kbegin, kend, lds, acc)) {
+    __syncthreads();   // the verdict lies where the first step goes
+    C::F::run(la, lb, kbegin, kend, lds, acc);
+  }
+  T::store(acc, out + z * zs.c, N, wide, M, N, m0, n0);
 }
 
 }  // namespace st
