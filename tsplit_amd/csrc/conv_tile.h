@@ -94,6 +94,19 @@ struct FilterRows {
     const int u = kw.div(tap), v = tap - u * kw.d;
     return row < M && k < K && ch < chans ? w[row * w_row + ch * w_chan + (tap_a + w_s * u) * w_width + tap_b + w_s * v] : 0.f;
   }
+  // values k to k + 3 of a row, k a multiple of 4; in blocks of channels they are of one tap
+  __device__ __forceinline__ void four(int row, int k, float (&v)[4]) const {
+    if (plain) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = at(row, k + j);
+      return;
+    }
+    const int block = k >> 3, cb = taps.div(block), tap = block - cb * taps.d, ch = 8 * cb + (k & 7), u = kw.div(tap);
+    const bool in = row < M && k < K;
+    const float *from = w + (in ? row * w_row + ch * w_chan + (tap_a + w_s * u) * w_width + tap_b + w_s * (tap - u * static_cast<int>(kw.d)) : 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = in && ch + j < chans ? from[j * w_chan] : 0.f;
+  }
 };
 
 // B, gathered.  BWD: element (k = (ch, u, v), position (r, c)) at [ch][r + ph - u][c + pw - v], else at
@@ -488,10 +501,9 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_pair_kernel(Params 
     }
 }
 
-// The filter's planes, every phase
-static __global__ __launch_bounds__(256) void conv_planes_kernel(Params P, char *__restrict__ out, int chunks) {
-  const int i = blockIdx.x * 256 + threadIdx.x, lane = i & 63, chunk = i >> 6;
-  if (chunk >= chunks) return;
+// The filter's planes, every phase: a block a chunk
+static __global__ __launch_bounds__(64) void conv_planes_kernel(Params P, char *__restrict__ out) {
+  const int lane = threadIdx.x, chunk = blockIdx.x;
   int ip = 0;
   while (ip + 1 < P.phases && chunk >= P.phase[ip + 1].w_at) ++ip;
   const Phase &F = P.phase[ip];

@@ -64,7 +64,7 @@ bool prepare_filter(Params &P, bool optional, hipStream_t st) {
   char *planes = static_cast<char *>(scratch_get(st, 3, static_cast<size_t>(std::max(1, chunks)) * st::kChunk, optional));
   if (!planes) return false;
   P.planes = planes;
-  if (chunks > 0) hipLaunchKernelGGL(conv_planes_kernel, dim3((chunks + 3) / 4), dim3(256), 0, st, P, planes, chunks);
+  if (chunks > 0) hipLaunchKernelGGL(conv_planes_kernel, dim3(chunks), dim3(64), 0, st, P, planes);
   return true;
 }
 

@@ -108,9 +108,9 @@ void launch_split_tile(const st::PlanesParams &rows, const st::DenseRows &src, c
 }
 template <bool XMN, bool ACROSS>
 void launch_prepared(const st::DenseRows &src, const DenseParams &xp, char *planes, float *out, int P, int X, int K, const Plan &plan, hipStream_t s) {
-  const int steps = (K + gt::BK - 1) / gt::BK, tiles = (P + 15) / 16, total = tiles * steps * 64;
+  const int steps = (K + gt::BK - 1) / gt::BK, tiles = (P + 15) / 16;
   const int64_t mn = static_cast<int64_t>(P) * X;
-  hipLaunchKernelGGL(st::planes_kernel, dim3((total + 255) / 256), dim3(256), 0, s, src, 0, planes, FastDiv(steps), total);
+  hipLaunchKernelGGL(st::planes_kernel, dim3(tiles * steps), dim3(64), 0, s, src, 0, planes, FastDiv(steps));
   const st::PlanesParams rows{planes, tiles, steps};
   const bool wide = (ACROSS ? P : X) % 4 == 0 && aligned16(out);
   switch (plan.tile) {
@@ -139,9 +139,9 @@ int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, flo
   }
   if (plan.prepared) {
     if (plan.across)
-      launch_prepared<TA, true>(st::DenseRows{B, TB ? ldb : 1, TB ? 1 : ldb, N, K}, DenseParams{A, lda, M, K}, planes, out, N, M, K, plan, s);
+      launch_prepared<TA, true>(st::dense_rows(B, TB ? ldb : 1, TB ? 1 : ldb, N, K), DenseParams{A, lda, M, K}, planes, out, N, M, K, plan, s);
     else
-      launch_prepared<!TB, false>(st::DenseRows{A, TA ? 1 : lda, TA ? lda : 1, M, K}, DenseParams{B, ldb, N, K}, planes, out, M, N, K, plan, s);
+      launch_prepared<!TB, false>(st::dense_rows(A, TA ? 1 : lda, TA ? lda : 1, M, K), DenseParams{B, ldb, N, K}, planes, out, M, N, K, plan, s);
   } else {
     launch_planned<TA, TB>(A, lda, 0, B, ldb, 0, out, mn, 1, M, N, K, plan, s);
   }

@@ -278,18 +278,30 @@ struct DenseRows {
   const float *p;
   int64_t row, step;   // distance of rows and of values along the depth
   int rows, depth;
+  bool words;          // four values from a multiple of 4 on are one aligned word
   __device__ __forceinline__ float at(int r, int k) const { return r < rows && k < depth ? p[r * row + k * step] : 0.f; }
+  // values k to k + 3 of a row, k a multiple of 4
+  __device__ __forceinline__ void four(int r, int k, float (&v)[4]) const {
+    if (words) {
+      const f32x4 w = r < rows && k < depth ? *reinterpret_cast<const f32x4 *>(p + r * row + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = w[j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = at(r, k + j);
+    }
+  }
 };
+inline DenseRows dense_rows(const float *p, int64_t row, int64_t step, int rows, int depth) {
+  return DenseRows{p, row, step, rows, depth, step == 1 && row % 4 == 0 && depth % 4 == 0 && (reinterpret_cast<uintptr_t>(p) & 15) == 0};
+}
 
 // one lane's eight values of a chunk, row and first k as they fall to it
 template <class Src>
 __device__ __forceinline__ void put_planes(const Src &src, int row, int k, char *chunk, int lane) {
   float lo[4], hi[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    lo[j] = src.at(row, k + j);
-    hi[j] = src.at(row, k + 16 + j);
-  }
+  src.four(row, k, lo);
+  src.four(row, k + 16, hi);
   bf16x8 w[3];
   unsigned least = ~0u;
   split(lo, hi, w, least);
@@ -297,13 +309,11 @@ __device__ __forceinline__ void put_planes(const Src &src, int row, int k, char 
 #pragma unroll
   for (int s = 0; s < 3; ++s) *reinterpret_cast<bf16x8 *>(chunk + 1024 * s + 16 * lane) = w[s];
 }
-// blockIdx.y: one of a batch of operands, `stride` values apart, and its planes
-static __global__ __launch_bounds__(256) void planes_kernel(DenseRows src, int64_t stride, char *__restrict__ out, FastDiv steps, int total) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= total) return;
+// A block a chunk, so that small operands spread over the chip.  blockIdx.y: one of a batch of operands, `stride` values apart, and its planes
+static __global__ __launch_bounds__(64) void planes_kernel(DenseRows src, int64_t stride, char *__restrict__ out, FastDiv steps) {
   src.p += blockIdx.y * stride;
-  out += static_cast<int64_t>(blockIdx.y) * (total / 64) * kChunk;
-  const int lane = i & 63, chunk = i >> 6, tile = steps.div(chunk);
+  out += static_cast<int64_t>(blockIdx.y) * gridDim.x * kChunk;
+  const int lane = threadIdx.x, chunk = blockIdx.x, tile = steps.div(chunk);
   put_planes(src, 16 * tile + (lane & 15), (chunk - tile * steps.d) * BK + 4 * (lane >> 4), out + static_cast<int64_t>(chunk) * kChunk, lane);
 }
 

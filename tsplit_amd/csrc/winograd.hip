@@ -692,15 +692,14 @@ int conv_winograd_3x3(const float *x, const float *w, float *y, int imgs, int ga
       const double flop = 2.0 * kXi * produced * static_cast<double>(gi.ld) * gathered;
       const double bytes = 4.0 * kXi * (static_cast<double>(produced) * gathered + static_cast<double>(gathered + produced) * gi.ld);
       if (prepared && first == 0)
-        hipLaunchKernelGGL(st::planes_kernel, dim3((row_tiles * steps + 3) / 4, kXi), dim3(256), 0, st,
-                           st::DenseRows{U, gathered, 1, produced, gathered}, static_cast<int64_t>(produced) * gathered, planes, FastDiv(steps),
-                           row_tiles * steps * 64);
+        hipLaunchKernelGGL(st::planes_kernel, dim3(row_tiles * steps, kXi), dim3(64), 0, st, st::dense_rows(U, gathered, 1, produced, gathered),
+                           static_cast<int64_t>(produced) * gathered, planes, FastDiv(steps));
       const bool asked = prepared && (gathered & 7) == 0 && split_bf16_enabled();
       GemmTiming timed(st, asked ? 3 : prepared ? 0 : 2, flop, bytes);
       if (prepared) {
         const int tm = (produced + 127) / 128, tn = (gi.ld + 127) / 128;
         hipLaunchKernelGGL((st::gemm_split_kernel<4, 4, 2, 2, true, false>), dim3(grid_blocks(tm, tn, kXi)), dim3(gt::kThreads), 0, st,
-                           st::PlanesParams{planes, row_tiles, steps}, st::DenseRows{U, gathered, 1, produced, gathered}, DenseParams{V, gi.ld, gi.ld, gathered},
+                           st::PlanesParams{planes, row_tiles, steps}, st::dense_rows(U, gathered, 1, produced, gathered), DenseParams{V, gi.ld, gi.ld, gathered},
                            M, st::SplitStrides{static_cast<int64_t>(plane_bytes), static_cast<int64_t>(produced) * gathered,
                            static_cast<int64_t>(gathered) * gi.ld, static_cast<int64_t>(produced) * gi.ld}, true, produced, gi.ld, gathered, gathered,
                            TileGrid{tm, tn, tm * tn * kXi});
