@@ -1,5 +1,5 @@
-// Convolution forward and data gradient as implicit products on the tile kernel of split_tile.h (small layers of one tap on that of
-// gemm_tile.h).
+// Convolution forward and data gradient as implicit products on the tile kernel of split_tile.h (small layers whose filter can be
+// read where it lies on that of gemm_tile.h).
 //
 //   forward        y[img,o,p]  : M = O, N = imgs * oH * oW, depth (c, tap)   A = filter [O][depth]
 //   data gradient  dx[img,c,q] : M = C, N = imgs * H * W,   depth (o, tap)   A = filter [C][depth]
@@ -249,8 +249,8 @@ struct Shape<TILE, false> {
   static constexpr int TM = TILE == 0 || TILE == 2 ? 4 : 2, TN = TILE <= 1 ? 4 : 2, WM = 2;
 };
 
-// PREPARED: the filter as planes (split_tile.h).  Else, for layers of one tap, the fp32 instruction and the filter as it lies in memory,
-// [M][depth] or (data gradient) [depth][M].
+// PREPARED: the filter as planes (split_tile.h).  Else, for layers of one tap and forward ones in the filter's own order, the fp32 instruction and
+// the filter as it lies in memory, [M][depth] or (data gradient) [depth][M].
 template <int TILE, bool BWD, int GATHER, bool PREPARED>
 struct Pass : Shape<TILE, PREPARED> {
   using S = Shape<TILE, PREPARED>;

@@ -71,9 +71,10 @@ bool prepare_filter(Params &P, bool optional, hipStream_t st) {
 // Runs the phases of P; tiles and ranges are filled in here.  out_values: elements of the output, negative if this launch does
 // not write all of them (the fold of ranges adds whole tensors).
 //
-// A filter of several taps has to be re-laid, and is prepared for the bf16 products on the way.  For one tap the preparing is a launch
-// more, and the model says whether the products win back the 3 us and 0.5 ns a chunk: 64 x 64 x 56 x 56 -> 256 does (101 -> 80 us), 32 x 1536 x 8 x 8
-// -> 256, data gradient, does not (17 -> 23).  Over 71 layers the choice takes 3149 us, the better of the two each time 3146, fp32 alone 3809.
+// A filter that has to be re-laid is prepared for the bf16 products on the way.  For one that can be read where it lies, of one tap or (forward) in its own
+// order, the preparing is a launch more, and the model says whether the products win back the 3 or 2 us and 0.5 ns a chunk: 64 x 64 x 56 x 56 -> 256 does
+// (101 -> 80 us), 32 x 1536 x 8 x 8 -> 256, data gradient, does not (17 -> 23).  Over 71 layers of one tap the choice takes 3149 us, the better of the
+// two each time 3146, fp32 alone 3809; over 20 layers of few channels 583, 583 and 647, all prepared 629.
 int run_phases(Params &P, bool bwd, int gather, bool pairs, float *out, int64_t out_values, hipStream_t st, StatsSink *sink) {
   int64_t cols[kMaxPhases];
   int steps[kMaxPhases], chunks = 0;
@@ -84,14 +85,14 @@ int run_phases(Params &P, bool bwd, int gather, bool pairs, float *out, int64_t 
     steps[parts] = (P.phase[i].K + BK - 1) / BK + (pairs ? (P.phase[i + 1].K + BK - 1) / BK : 0);
     chunks += (P.M + 15) / 16 * steps[parts];
   }
-  const bool one_tap = gather == kWords || gather == kOneTap;
+  const bool one_tap = gather == kWords || gather == kOneTap, in_place = one_tap || (gather == kTaps64 && !bwd);
   const int ranges = out_values < 0 ? 1 : 32;
   auto planned = [&](const TileCost &cost) { return plan_tiles(P.M, cols, steps, parts, 1, ranges, static_cast<double>(out_values), cost); };
   TilePlan plan = planned(one_tap ? kOneTapSplitCost : pairs ? kPairsSplitCost : kGatheredSplitCost);
   bool prepared = true;
-  if (one_tap) {
-    const TilePlan plain = planned(kOneTapCost);
-    prepared = plan.us + 3.0 + 5e-4 * chunks < plain.us && prepare_filter(P, true, st);   // without room for it: fp32
+  if (in_place) {
+    const TilePlan plain = planned(one_tap ? kOneTapCost : kGatheredCost);
+    prepared = plan.us + (one_tap ? 3.0 : 2.0) + 5e-4 * chunks < plain.us && prepare_filter(P, true, st);   // without room for it: fp32
     if (!prepared) plan = plain;
   } else {
     TS_REQUIRE(prepare_filter(P, false, st), "conv: no scratch memory for the prepared filter");
@@ -147,7 +148,12 @@ int run_phases(Params &P, bool bwd, int gather, bool pairs, float *out, int64_t 
         break;
       case kBlocks32: launch_tile<false, kBlocks32>(P, plan.tile, grid, total, st); break;
       case kBlocks64: launch_tile<false, kBlocks64>(P, plan.tile, grid, total, st); break;
-      default: launch_tile<false, kTaps64>(P, plan.tile, grid, total, st); break;
+      default:
+        if (prepared)
+          launch_tile<false, kTaps64>(P, plan.tile, grid, total, st);
+        else
+          launch_tile<false, kTaps64, false>(P, plan.tile, grid, total, st);
+        break;
     }
   } else {
     switch (gather) {

@@ -41,7 +41,8 @@ constexpr TileCost kProductCost = {{2, 3, 3, 5},
 constexpr TileCost kOneTapCost = {{2, 3, 3, 5},
                                   {{1.88, 3.76}, {1.41, 2.28, 2.84}, {0.89, 1.77, 2.84}, {0.48, 0.90, 1.25, 1.74, 2.46}},
                                   {4.2, 2.5, 2.6, 2.3}, 0.5, 11.8};
-// one operand gathered by tap, fp32 instruction (no such kernel is left; the model is tested against its times): a load and a row of LDS for every 64 values instead of every 256
+// one operand gathered by tap, fp32 instruction (small forward layers of few channels; the pairs' and taps' figures below only serve the
+// test of this model, their kernels are gone): a load and a row of LDS for every 64 values instead of every 256
 constexpr TileCost kGatheredCost = {{2, 3, 3, 5},
                                     {{2.44, 4.63}, {1.34, 2.34, 3.57}, {1.44, 2.68, 3.27}, {0.82, 1.25, 1.77, 2.36, 3.07}},
                                     {1.9, 1.7, 0.7, 0.9}, 2.5, 8.1};
