@@ -1324,11 +1324,11 @@ inline bool winograd_pays(const ConvGeo &g, int gathered) {
   return forced == 1 || winograd_wide(g, 16 * 1024);
 }
 
-// (64 channels on a side: 64 -> 128 at 32 x 32, 16 images 59 us, direct 34; at 56 x 56, 18 images 78 and 72; at 112 x 112, 8 images 68 and 109)
+// (64 channels on a side: 64 -> 128 at 32 x 32, 16 images 59 us, direct 34; at 112 x 112, 4 images 69 and 63, 8 images 68 and 109)
 inline bool winograd_filter_grad_pays(const ConvGeo &g) {
   const int forced = winograd_forced();
   if (!winograd_shape(g) || forced == 0) return false;
-  return forced == 1 || winograd_wide(g, std::min(g.C, g.O) < 96 ? 60 * 1024 : 16 * 1024);
+  return forced == 1 || winograd_wide(g, std::min(g.C, g.O) < 96 ? 48 * 1024 : 16 * 1024);
 }
 
 // ------------------------------------------------------------------ statistics of the output
