@@ -272,8 +272,8 @@ def main():
         "metric": "train samples/s, fp32, 1 MI355X; conv MFMA util %; BN/relu HBM GB/s",
         "value": a.batch * a.steps / dt, "unit": "samples/s", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f32 (the larger products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation: error below the f32 instruction's)",
-        "data": "synthetic",
+        "dtype": "f32 (products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)" if a.split_bf16 else "f32", "data": "synthetic",
+        "arithmetic": "f32 in memory and accumulation; the larger products as six bf16 x bf16 terms of exact operand splits, error below the f32 instruction's",
         "config": {"workload": "VGG-16 training step (fwd+bwd+momentum SGD), fp32 NCHW, batch %d, 3x224x224, "
                                "1000 classes, He init, %s%s" % (a.batch, "4 batch micro-tensors on the 4 largest conv layers"
                                                                 if split else "no micro-tensor split",

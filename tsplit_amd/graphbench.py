@@ -287,8 +287,8 @@ def layer_list(a, ctx):
     print(json.dumps({"net": a.net, "workload": desc, "samples_per_s": n * steps / dt,
                       "ms_per_step": dt / steps * 1e3, "steps": steps, "warmup": a.warmup, "final_loss": t.loss_value(),
                       "recorded": bool(a.record),
-                      "dtype": "f32 (the larger products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)",
-                      "data": "synthetic"}))
+                      "dtype": "f32 (products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)" if a.split_bf16 else "f32",
+                      "arithmetic": "the larger products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation", "data": "synthetic"}))
 
 
 if __name__ == "__main__":
