@@ -263,7 +263,14 @@ struct Tile {
   using BL = typename std::conditional<TB, KContig<BN, TN, true>, MnContig<BN, TN>>::type;
   using C = Core<TM, TN, WM, WN, AL, BL>;
 
-  static __device__ __forceinline__ void store(const f32x4 (&acc)[TM][TN], float *__restrict__ o, int64_t ldc, bool wide, int M, int N, int m0, int n0) {
+  static __device__ __forceinline__ void run(const mg::DenseParams &ap, const mg::DenseParams &bp, float *__restrict__ o, int64_t ldc,
+                                             bool wide, int M, int N, int m0, int n0, int kbegin, int kend, float *lds) {
+    AL la;
+    BL lb;
+    la.init(ap, m0);
+    lb.init(bp, n0);
+    f32x4 acc[TM][TN];
+    C::run(la, lb, kbegin, kend, lds, acc);
     // the wave's rows to the end of C: rows past it are out of range
     const int m = m0 + C::wave_m0(), n = n0 + C::wave_n0() + TN * (threadIdx.x & 15);
     if (m >= M) return;
@@ -305,14 +312,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(mg::DenseParams 
   if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
   ap.p += z * zs.a;
   bp.p += z * zs.b;
-  const int kbegin = kchunk < K ? z * kchunk : 0, m0 = tile_m * T::BM, n0 = tile_n * T::BN;
-  typename T::AL la;
-  typename T::BL lb;
-  la.init(ap, m0);
-  lb.init(bp, n0);
-  f32x4 acc[TM][TN];
-  T::C::run(la, lb, kbegin, min(K, kbegin + kchunk), lds, acc);
-  T::store(acc, out + z * zs.c, N, wide, M, N, m0, n0);
+  const int kbegin = kchunk < K ? z * kchunk : 0;
+  T::run(ap, bp, out + z * zs.c, N, wide, M, N, tile_m * T::BM, tile_n * T::BN, kbegin, min(K, kbegin + kchunk), lds);
 }
 
 // out[i] = sum_z part[z * n + i], z ascending, four values a thread (n a multiple of 4)
