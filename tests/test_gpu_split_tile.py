@@ -13,7 +13,7 @@ from oracle import ops as O
 pytestmark = pytest.mark.gpu
 
 # M, N, K of products large enough that one operand is prepared: rows or columns the fewer, ragged in every direction, depths that a step cuts
-SHAPES = [(2048, 512, 512), (515, 2047, 1031), (2050, 516, 1001), (100, 4096, 4096), (4096, 100, 4093), (4099, 257, 130)]
+SHAPES = [(2048, 512, 512), (515, 2047, 1031), (2050, 516, 1001), (100, 4096, 4096), (4096, 100, 4093), (4099, 257, 130), (4098, 4100, 65)]
 
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
@@ -82,7 +82,7 @@ def test_products_of_values_without_a_split(kind, where, prepared, rng):
 
 # N, C, H, W, O, kh, kw, ph, pw, s: blocks of channels and the filter's own order, 1 x 1, stride 2 in pairs of phases, few channels
 LAYERS = [(3, 40, 13, 11, 72, 3, 3, 1, 1, 1), (4, 3, 21, 19, 33, 5, 5, 2, 2, 1), (2, 24, 17, 15, 130, 3, 3, 0, 0, 2), (16, 512, 28, 28, 128, 1, 1, 0, 0, 1),
-          (3, 40, 20, 21, 48, 1, 7, 0, 3, 1)]
+          (3, 40, 20, 21, 48, 1, 7, 0, 3, 1), (6, 10, 50, 50, 375, 5, 5, 2, 2, 1)]   # the second and the last: few channels, forward without and with planes
 
 
 @pytest.mark.parametrize("kind,where", [("inf", "some"), ("nan", "some"), ("huge", "some"), ("small", "rows"), ("subnormal", "rows")])

@@ -44,19 +44,19 @@ Plan best_plan(int M, int N, int K, int batch, bool may_split, const TileCost &c
 }
 
 // The operand with fewer rows is the one to prepare, unless the result then leaves in single words, which takes long with the columns
-// prepared (3930 x 3702 over 113: 58 us, fp32 44).  The preparing costs a launch, 2.5 us and 1 ns a chunk, and below four steps a product is
-// its stores (25088 x 4096 over 18: 110 us, fp32 88; over 64: 151 and 143).  Else the model decides: over 276 products its choice takes
-// 7683 us, the better of the two each time 7637, fp32 alone 9809.
+// prepared (3930 x 3702 over 113: 58 us, fp32 44).  The preparing costs a launch, 3.5 us and 1 ns a chunk, and below two steps a product is
+// its stores (25088 x 4096 over 18: 110 us, fp32 88; over 64 139 and 153, over 66 160 and 191).  Else the model decides: over 276 products its
+// choice takes 7.69 ms, the better of the two each time 7.64, fp32 alone 9.81; the seven that 2.5 us took as well 148 us, fp32 146.
 Plan choose_plan(int M, int N, int K, int batch, bool may_split) {
   const Plan plain = best_plan(M, N, K, batch, may_split, kProductCost);
-  if (!may_split || K < 4 * gt::BK) return plain;
+  if (!may_split || K < 2 * gt::BK) return plain;
   const bool across = N % 4 == 0 ? M > N : M > 4ll * N;
   const int P = across ? N : M, X = across ? M : N;
   const int64_t tiles = (P + 15) / 16, steps = (K + gt::BK - 1) / gt::BK;
   // chunks of a tile within 32-bit offsets, threads of the preparing kernel within a grid
   if (8 * steps * st::kChunk >= (1ll << 31) || tiles * steps >= (1ll << 24)) return plain;
   Plan p = best_plan(P, X, K, 1, true, kProductSplitCost);
-  if (p.us + 2.5 + 1e-3 * static_cast<double>(tiles * steps) >= plain.us) return plain;
+  if (p.us + 3.5 + 1e-3 * static_cast<double>(tiles * steps) >= plain.us) return plain;
   p.prepared = true;
   p.across = across;
   return p;
