@@ -49,7 +49,7 @@ Plan best_plan(int M, int N, int K, int batch, bool may_split, const TileCost &c
 // choice takes 7.69 ms, the better of the two each time 7.64, fp32 alone 9.81; the seven that 2.5 us took as well 148 us, fp32 146.
 Plan choose_plan(int M, int N, int K, int batch, bool may_split) {
   const Plan plain = best_plan(M, N, K, batch, may_split, kProductCost);
-  if (!may_split || K < 2 * gt::BK) return plain;
+  if (!may_split || K < 2 * gt::BK || plain.us < 6) return plain;   // (the prepared form is at best 0.55 of it and the 3.5 us)
   const bool across = N % 4 == 0 ? M > N : M > 4ll * N;
   const int P = across ? N : M, X = across ? M : N;
   const int64_t tiles = (P + 15) / 16, steps = (K + gt::BK - 1) / gt::BK;
@@ -62,15 +62,17 @@ Plan choose_plan(int M, int N, int K, int batch, bool may_split) {
   return p;
 }
 
-// the plans of the shapes this thread asked for last (working one out takes about 2 us of host time)
+// the plans of the shapes this thread asked for last (working one out takes 2-4 us of host time)
 Plan plan_product(int M, int N, int K, int batch, bool may_split) {
   struct Entry {
     int M, N, K, batch;
     bool may_split;
     Plan plan;
   };
-  static thread_local Entry known[64] = {};
-  Entry &e = known[(static_cast<unsigned>(M) * 31u + static_cast<unsigned>(N) * 7u + static_cast<unsigned>(K) + static_cast<unsigned>(batch) * 13u) % 64];
+  static thread_local Entry known[256] = {};
+  // (multiplied through: sums of small multiples put every shape of a net of power-of-two sizes into two places)
+  const unsigned mix = ((static_cast<unsigned>(M) * 31u + static_cast<unsigned>(N)) * 31u + static_cast<unsigned>(K)) * 31u + static_cast<unsigned>(batch);
+  Entry &e = known[(mix * 2654435769u) >> 24];
   if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.may_split != may_split)
     e = {M, N, K, batch, may_split, choose_plan(M, N, K, batch, may_split)};
   return e.plan;
