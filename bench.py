@@ -37,7 +37,6 @@ sys.path.insert(0, ROOT)
 
 PEAK_TFLOPS_FP32_MFMA = 157.3
 PEAK_TFLOPS_BF16_MFMA = 2500.0   # dense bf16 matrix peak
-PEAK_TFLOPS_SPLIT = PEAK_TFLOPS_BF16_MFMA / 6   # fp32 products taken as six bf16 ones
 PEAK_HBM_GBS = 8000.0
 # Kernel names (as rocprofv3 prints them) behind the operator classes that can be the step's largest
 # single kernel; their HBM bytes per launch are read from the counter summary under profiles/.
@@ -46,13 +45,13 @@ TRAFFIC_PROFILE_FUSED = os.path.join(ROOT, "profiles", "vgg16_b64_fused_bn_relu_
 TRAFFIC_PROFILE_SPLIT = os.path.join(ROOT, "profiles", "vgg16_b64_split_bf16_train_step_hbm_traffic.txt")          # --split-bf16
 TRAFFIC_PROFILE_FUSED_SPLIT = os.path.join(ROOT, "profiles", "vgg16_b64_fused_split_bf16_train_step_hbm_traffic.txt")
 TRAFFIC_KERNELS = {
-    "winograd_gemm": ("gemm_split_kernel<4, 4, 2, 2, true, false>",),
-    "winograd_filter_grad_gemm": ("gemm_both_kernel<4, 4, 2, 2, false, true>",),
+    "winograd_gemm": ("wino_gemm_kernel<128, 128>",),
+    "winograd_filter_grad_gemm": ("wino_grad_gemm_kernel<3>",),
     "winograd_gemm_64_rows": ("wino_gemm_kernel<64, 256>",),
     "winograd_fused": ("wino_fused_kernel<",),
     "winograd_filter_grad_fused": ("wino_fgrad_fused_kernel",),
-    "winograd_gemm_split_bf16": ("gemm_split_kernel<4, 4, 2, 2, true, false>",),
-    "winograd_filter_grad_gemm_split_bf16": ("gemm_both_kernel<4, 4, 2, 2, false, true>",),
+    "winograd_gemm_split_bf16": ("wino_gemm_split_kernel",),
+    "winograd_filter_grad_gemm_split_bf16": ("wino_grad_gemm_split_kernel<3>",),
 }
 
 
@@ -216,9 +215,9 @@ def main():
                          "symbols, let every convolution hand its output's statistics to the BatchNorm behind it and "
                          "update all parameters in one launch (symbols outside the reference's ABI)")
     ap.add_argument("--split-bf16", action="store_true",
-                    help="opt-in, outside the reference's ABI (TSplit_SplitBf16): layers with more than 64 channels on both sides on the "
-                         "three-kernel Winograd routine, whose GEMMs take their products as six bf16 terms of exact splits, and small matrix products "
-                         "split too")
+                    help="opt-in, outside the reference's ABI and outside the default path's fp32 matrix instructions: the "
+                         "Winograd GEMMs of layers with more than 64 channels on both sides take each fp32 product as six "
+                         "bf16 x bf16 products of the operands' exact three-term splits, accumulated in fp32")
     a = ap.parse_args()
     if a.gpus != 1:
         sys.exit("bench.py: this build is single-GPU by design (no collectives, no sharding); run with --gpus 1. "
@@ -272,13 +271,13 @@ def main():
         "metric": "train samples/s, fp32, 1 MI355X; conv MFMA util %; BN/relu HBM GB/s",
         "value": a.batch * a.steps / dt, "unit": "samples/s", "n_gpus": 1, "steps": a.steps, "warmup": a.warmup,
         "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": "f32 (products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)" if a.split_bf16 else "f32", "data": "synthetic",
-        "arithmetic": "f32 in memory and accumulation; the larger products as six bf16 x bf16 terms of exact operand splits, error below the f32 instruction's",
+        "dtype": "f32 (Winograd GEMM products of wide layers as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)"
+                 if a.split_bf16 else "f32", "data": "synthetic",
         "config": {"workload": "VGG-16 training step (fwd+bwd+momentum SGD), fp32 NCHW, batch %d, 3x224x224, "
                                "1000 classes, He init, %s%s" % (a.batch, "4 batch micro-tensors on the 4 largest conv layers"
                                                                 if split else "no micro-tensor split",
                                                                 (", BatchNorm+Relu pairs fused (with the max pooling behind them where one follows), BatchNorm statistics from the convolutions' epilogues, one optimizer launch" if a.fused else "")
-                                                                + (", wide layers on the three-kernel Winograd routine and small products split too" if a.split_bf16 else "")),
+                                                                + (", split-bf16 products in the wide layers' Winograd GEMMs" if a.split_bf16 else "")),
                    "global_batch": a.batch, "final_loss": loss},
     }
     if timer:
@@ -307,12 +306,11 @@ def main():
             if launches:
                 wino_exec_flop += flop
                 k[tag] = {"calls": launches, "ms_total": ms, "ms_avg": ms / launches, "work": flop,
-                          "work_per_call": flop / launches, "rate": flop / (ms * 1e-3) / 1e12, "unit": "flop",
-                          "peak": PEAK_TFLOPS_SPLIT if kind < 2 else PEAK_TFLOPS_FP32_MFMA}
+                          "work_per_call": flop / launches, "rate": flop / (ms * 1e-3) / 1e12, "unit": "flop"}
                 kernels[tag] = {"calls_per_step": launches / a.steps, "ms_per_step": ms / a.steps, "ms_avg": ms / launches,
-                                "achieved": k[tag]["rate"], "unit": "TFLOP/s", "frac": k[tag]["rate"] / k[tag]["peak"],
+                                "achieved": k[tag]["rate"], "unit": "TFLOP/s", "frac": k[tag]["rate"] / PEAK_TFLOPS_FP32_MFMA,
                                 "note": "one kernel inside the *_winograd calls above (its time is part of theirs); "
-                                        "executed FLOP" + ("; products as six bf16 terms, against a sixth of the bf16 peak" if kind < 2 else "")}
+                                        "executed FLOP"}
                 if kind == 5:
                     # forward / data gradient of the layers with 64 channels on one side as ONE kernel (transforms inside,
                     # the transformed tensors never leave the chip): its time is the whole call's, its bytes the activations'
@@ -394,8 +392,8 @@ def main():
             return 100.0 * flop / (ms * 1e-3) / 1e12 / PEAK_TFLOPS_FP32_MFMA if ms > 0 else None
         # executed: what the matrix pipe really multiplies (the Winograd calls count with their 36 GEMMs'
         # FLOP, the direct kernels with the algorithm's) over ALL conv time, transforms included
-        # (the wide layers' products run on the bf16 matrix instruction, six for one: counted as the fp32 product they stand for)
-        out["conv_mfma_util_executed_pct"] = pct(direct_flop + thin_flop + wino_exec_flop, conv_ms)
+        # (with split-bf16 products part of the work runs on the bf16 matrix instruction: no single peak applies)
+        out["conv_mfma_util_executed_pct"] = None if a.split_bf16 else pct(direct_flop + thin_flop + wino_exec_flop, conv_ms)
         # direct-equivalent: the direct algorithm's FLOP count of every layer over the same time; above 100
         # because the Winograd layers execute a quarter of it.  A throughput figure, not a utilisation
         out["conv_direct_equivalent_pct"] = pct(equivalent_flop, conv_ms)

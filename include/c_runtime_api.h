@@ -513,10 +513,9 @@ int TSplit_ConvTakesWinograd(int images, int in_channels, int out_channels, int 
  *      (not while the stream is being recorded into a graph), (2 + k) only the launches of kind k, so
  *      that a timed region carries the events of the one kernel it reports; (0) stops and forgets them.
  *      TSplit_WinogradGemmTimes waits for the launches of kind `which` (0: forward and data
- *      gradient on 128 x 128 tiles, 1: filter gradient, both in bf16 products of exact three-term splits
- *      where both sides have more than 64 channels, 2: forward and data gradient of layers that
- *      produce at most 64 channels, which run on 64 x 256 tiles, 3 / 4: those of 0 / 1
- *      while TSplit_SplitBf16 is on; 5: forward and data gradient of
+ *      gradient on 128 x 128 tiles, 1: filter gradient, 2: forward and data gradient of layers that
+ *      produce at most 64 channels, which run on 64 x 256 tiles, 3 / 4: forward and data gradient /
+ *      filter gradient with split-bf16 products, see TSplit_SplitBf16; 5: forward and data gradient of
  *      layers with at most 256 channels, which run as ONE kernel with the transforms inside, so that its
  *      milliseconds cover the whole call; 6: filter gradient of layers with at most 128 channels, one
  *      kernel with both transforms inside, followed by the filter's final 3x3 transform: one kernel per
@@ -529,15 +528,14 @@ int TSplit_WinogradGemmTiming(int on);
 int TSplit_WinogradGemmTimes(int which, double *launches, double *ms, double *flop);
 int TSplit_WinogradGemmBytes(int which, double *bytes);
 
-/* ---- Split-bf16 products also where they are not the default.  NO counterpart in the reference; off by default.
- *      Products, convolutions and the Winograd routine's GEMMs that are large enough split each fp32 operand
- *      exactly into three bf16 terms, a = a1 + a2 + a3, and take a product as the six bf16 x bf16 products a_i b_j
+/* ---- Split-bf16 products in the Winograd routine's GEMMs and in DLGpuMatrixMultiply.  NO counterpart in
+ *      the reference; opt-in, off by default (every product of the default path is an fp32 matrix
+ *      instruction).  With TSplit_SplitBf16(1, NULL) the GEMMs of 3x3 layers with more than 64 channels on
+ *      both sides and the matrix products whose depth is a multiple of 4 split each fp32 operand exactly
+ *      into three bf16 terms, a = a1 + a2 + a3, and take a product as the six bf16 x bf16 products a_i b_j
  *      with i + j <= 4, accumulated in fp32 by the bf16 matrix instruction; what is left out is below
- *      2^-23 of the product, the rounding of one fp32 multiplication, the measured error below the fp32
- *      instruction's, and values without such a split (infinities, NaN, above bf16's largest, below 2^-102) go to that
- *      instruction.  Operands and results stay fp32 in memory.  With TSplit_SplitBf16(1, NULL) smaller matrix products (depth
- *      a multiple of 4, operands below 2^127) are taken so too, and 3x3 layers with more than 64 channels on both sides go to the
- *      GEMMs of the three-kernel Winograd routine instead of the one-kernel form.  Affects calls issued afterwards, on every stream; `was` (may be NULL) receives the
+ *      2^-23 of the product, the rounding of one fp32 multiplication.  Operands and results stay fp32 in
+ *      memory.  Affects calls issued afterwards, on every stream; `was` (may be NULL) receives the
  *      previous setting.  The environment variable TSPLIT_SPLIT_BF16=1 turns it on from the start. ---- */
 int TSplit_SplitBf16(int on, int *was);
 

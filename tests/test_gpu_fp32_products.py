@@ -1,0 +1,81 @@
+"""With the split-bf16 switch off every multiplication is one of the fp32 matrix instruction.
+
+Bar: results with a single nonzero product are that product rounded once to fp32, to the bit: adding zeros changes nothing, and the
+product of two fp32 numbers is exact in float64.  Products of three-term bf16 splits leave out up to 2^-23 of it."""
+import numpy as np
+import pytest
+
+from oracle import ops as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def off():
+    from tsplit_amd import gpu_links as L
+    was = L.split_bf16(False)
+    yield L
+    L.split_bf16(was)
+
+
+def _one_per_row(rng, rows, cols):
+    """rows x cols with one nonzero value in each row."""
+    v = np.zeros((rows, cols), np.float32)
+    v[np.arange(rows), rng.randint(0, cols, rows)] = rng.normal(size=rows)
+    return v
+
+
+# M, N, K from a small product to large ones; fewer rows, fewer columns, about as many of both; ranges of the depth
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("shape", [(33, 65, 70), (515, 2047, 1031), (100, 4096, 2048), (4096, 100, 2045), (4098, 2100, 65), (2048, 2048, 512)])
+def test_products(shape, ta, tb, rng, off):
+    from tsplit_amd import ndarray as nd
+    ctx, (M, N, K) = nd.gpu(0), shape
+    for sparse_a in (True, False):
+        a = _one_per_row(rng, M, K) if sparse_a else rng.normal(size=(M, K)).astype(np.float32)
+        b = rng.normal(size=(K, N)).astype(np.float32) if sparse_a else np.ascontiguousarray(_one_per_row(rng, N, K).T)
+        ga, gb = (nd.array(np.ascontiguousarray(v.T) if t else v, ctx) for v, t in ((a, ta), (b, tb)))
+        c = nd.array(np.full((M, N), 7, np.float32), ctx)
+        off.matrix_multiply(ga, ta, gb, tb, c)
+        np.testing.assert_array_equal(c.asnumpy(), (a.astype(np.float64) @ b.astype(np.float64)).astype(np.float32))
+
+
+# N, C, H, W, O, kh, kw, ph, pw, s: channels in blocks, the filter's own order, one tap, pairs of phases, ragged
+@pytest.mark.parametrize("layer", [(3, 40, 13, 11, 72, 3, 3, 1, 1, 1), (4, 3, 21, 19, 33, 5, 5, 2, 2, 1), (2, 24, 17, 15, 130, 3, 3, 0, 0, 2),
+                                   (16, 256, 28, 28, 256, 1, 1, 0, 0, 1), (3, 40, 20, 21, 48, 1, 7, 0, 3, 1)])
+def test_convolutions(layer, rng, off, monkeypatch):
+    from tsplit_amd import ndarray as nd
+    monkeypatch.setenv("TSPLIT_CONV_WINOGRAD", "0")
+    ctx, (n, c, h, w, o, kh, kw, ph, pw, s) = nd.gpu(0), layer
+    ys = (n, o, (h + 2 * ph - kh) // s + 1, (w + 2 * pw - kw) // s + 1)
+    x, dy = rng.normal(size=(n, c, h, w)).astype(np.float32), rng.normal(size=ys).astype(np.float32)
+    one_of_depth = _one_per_row(rng, o, c * kh * kw).reshape(o, c, kh, kw)
+    one_of_outputs = np.ascontiguousarray(_one_per_row(rng, c, o * kh * kw).reshape(c, o, kh, kw).transpose(1, 0, 2, 3))
+    one_position = np.ascontiguousarray(_one_per_row(rng, o, n * ys[2] * ys[3]).reshape(o, n, ys[2], ys[3]).transpose(1, 0, 2, 3))
+    y, dx, dw = nd.empty(ys, ctx), nd.empty(x.shape, ctx), nd.empty((o, c, kh, kw), ctx)
+    off.CuDNN_conv2d(nd.array(x, ctx), nd.array(one_of_depth, ctx), y, ph, pw, s)
+    np.testing.assert_array_equal(y.asnumpy(), O.conv2d(x, one_of_depth, ph, pw, s).astype(np.float32), "forward")
+    off.CuDNN_conv2d_gradient_of_data(nd.array(one_of_outputs, ctx), nd.array(dy, ctx), dx, ph, pw, s)
+    np.testing.assert_array_equal(dx.asnumpy(), O.conv2d_grad_data(one_of_outputs, dy, x.shape, ph, pw, s).astype(np.float32), "data gradient")
+    off.CuDNN_conv2d_gradient_of_filter(nd.array(x, ctx), nd.array(one_position, ctx), dw, ph, pw, s)
+    np.testing.assert_array_equal(dw.asnumpy(), O.conv2d_grad_filter(x, one_position, dw.shape, ph, pw, s).astype(np.float32), "filter gradient")
+
+
+# the wide layers' GEMMs on planes that only the three-kernel form of the Winograd routine takes
+@pytest.mark.parametrize("case", [(3, 80, 30, 26, 144), (2, 288, 14, 14, 272)])
+def test_winograd_gemms_of_the_two_settings_differ(case, rng, off, monkeypatch):
+    """The switch chooses between two kernels: were both settings the same one, no bit would differ."""
+    from tsplit_amd import ndarray as nd
+    monkeypatch.setenv("TSPLIT_CONV_WINOGRAD", "1")
+    ctx, (n, c, h, w, o) = nd.gpu(0), case
+    x, f, dy = (rng.normal(size=s).astype(np.float32) for s in ((n, c, h, w), (o, c, 3, 3), (n, o, h, w)))
+    got = []
+    for on in (False, True):
+        off.split_bf16(on)
+        y, dx, dw = nd.empty(dy.shape, ctx), nd.empty(x.shape, ctx), nd.empty(f.shape, ctx)
+        off.CuDNN_conv2d(nd.array(x, ctx), nd.array(f, ctx), y, 1, 1, 1)
+        off.CuDNN_conv2d_gradient_of_data(nd.array(f, ctx), nd.array(dy, ctx), dx, 1, 1, 1)
+        off.CuDNN_conv2d_gradient_of_filter(nd.array(x, ctx), nd.array(dy, ctx), dw, 1, 1, 1)
+        got.append([v.asnumpy() for v in (y, dx, dw)])
+    for name, plain, split in zip(("forward", "data gradient", "filter gradient"), *got):
+        assert not np.array_equal(plain, split), name

@@ -1,9 +1,8 @@
-"""Products taken as bf16 products of three-term splits (csrc/split_tile.h): products with one operand prepared, convolutions and filter
-gradients, at ragged sizes and for values that have no split - infinities, NaN, numbers above bf16's largest and numbers so small that
-bf16 does not hold their parts, which a tile has to notice and multiply in fp32.
+"""Products, convolutions and filter gradients at ragged sizes and for values that have no split into three bf16 numbers - infinities, NaN, numbers
+above bf16's largest and numbers so small that bf16 does not hold their parts: with the split-bf16 switch off, as here, the fp32 instruction
+multiplies them like any other.
 
-Bar for ordinary values: the three-term splits are exact, the terms left out are below 2^-23 of a product, and a sum of K products is rounded
-less often than in fp32: within (K + 64) 2^-24 of the sum of the products' magnitudes, as for the fp32 instruction; and, as the mean over many results,
+Bar for ordinary values: within (K + 64) 2^-24 of the sum of the products' magnitudes; and, as the mean over many results,
 no further from 64 bits than fp32 sums in any order usually are (2^-24 sqrt(K) of the root of the squares' sum)."""
 import numpy as np
 import pytest
@@ -12,7 +11,7 @@ from oracle import ops as O
 
 pytestmark = pytest.mark.gpu
 
-# M, N, K of products large enough that one operand is prepared: rows or columns the fewer, ragged in every direction, depths that a step cuts
+# M, N, K: rows or columns the fewer, ragged in every direction, depths that a step cuts
 SHAPES = [(2048, 512, 512), (515, 2047, 1031), (2050, 516, 1001), (100, 4096, 4096), (4096, 100, 4093), (4099, 257, 130), (4098, 4100, 65)]
 
 
@@ -35,7 +34,7 @@ FLT_MAX = np.float32(3.4028235e38)
 
 
 def _special(a, rng, kind, where):
-    """Plants values of a kind into every 97th element or, "rows", makes some whole rows of them."""
+    """Plants values of a kind into every 9973rd element or, "rows", makes some whole rows of them."""
     at = np.zeros(a.shape, bool)
     if where == "rows":
         at[::37] = True
@@ -63,7 +62,7 @@ def _compare(got, want, tol):
 @pytest.mark.parametrize("prepared", [True, False])
 @pytest.mark.parametrize("kind,where", [("inf", "some"), ("nan", "some"), ("huge", "some"), ("small", "rows"), ("subnormal", "rows")])
 def test_products_of_values_without_a_split(kind, where, prepared, rng):
-    """In the operand that is prepared (the one with fewer rows) and in the one the waves split."""
+    """In the operand with fewer rows (`prepared`) and in the other one."""
     from tsplit_amd import gpu_links as L, ndarray as nd
     ctx, (M, N, K) = nd.gpu(0), (500, 2048, 520)
     a, b = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(N, K)).astype(np.float32)
@@ -82,7 +81,7 @@ def test_products_of_values_without_a_split(kind, where, prepared, rng):
 
 # N, C, H, W, O, kh, kw, ph, pw, s: blocks of channels and the filter's own order, 1 x 1, stride 2 in pairs of phases, few channels
 LAYERS = [(3, 40, 13, 11, 72, 3, 3, 1, 1, 1), (4, 3, 21, 19, 33, 5, 5, 2, 2, 1), (2, 24, 17, 15, 130, 3, 3, 0, 0, 2), (16, 512, 28, 28, 128, 1, 1, 0, 0, 1),
-          (3, 40, 20, 21, 48, 1, 7, 0, 3, 1), (6, 10, 50, 50, 375, 5, 5, 2, 2, 1)]   # the second and the last: few channels, forward without and with planes
+          (3, 40, 20, 21, 48, 1, 7, 0, 3, 1), (6, 10, 50, 50, 375, 5, 5, 2, 2, 1)]   # the second and the last: few channels
 
 
 @pytest.mark.parametrize("kind,where", [("inf", "some"), ("nan", "some"), ("huge", "some"), ("small", "rows"), ("subnormal", "rows")])
@@ -135,8 +134,8 @@ def test_convolutions_of_values_without_a_split(layer, kind, where, rng, monkeyp
 @pytest.mark.parametrize("scales", [(1.0, 1.0), (1e-36, 1e20), (1e20, 1e-36), (1e-41, 1e30), (1e35, 1e-3)])
 @pytest.mark.parametrize("layer", [(2, 144, 14, 18, 200), (3, 272, 7, 9, 130)])
 def test_winograd_gemms_hold_every_scale(layer, scales, rng, monkeypatch):
-    """Layers whose transformed tensors go through the prepared and the twice-split GEMMs (more than 64 channels on both sides, the
-    forms with both sides at most 256 switched to them by the ragged channel counts), with operands that have no split."""
+    """Forward and filter gradient of layers with more than 64 channels on both sides (their data gradients, whose summed channels are no
+    multiple of 16, take the direct kernels), with operands that have no split."""
     from tsplit_amd import gpu_links as L, ndarray as nd
     monkeypatch.setenv("TSPLIT_CONV_WINOGRAD", "1")
     ctx, (n, c, h, w, o) = nd.gpu(0), layer

@@ -1307,28 +1307,26 @@ inline bool winograd_shape(const ConvGeo &g) {
 }
 
 // wide enough for the 36 GEMMs to outweigh the transforms (64 channels on both sides: with tiles as
-// wide as the produced channels even the 64 -> 64 layer at 224 x 224 runs twice as fast as on the
+// wide as the produced channels even the 64 -> 64 layer at 224 x 224 runs a quarter faster than on the
 // direct kernels, forward and data gradient), little of the 4x4 tiling hanging over the plane's edge,
-// and enough tiles to fill the chip: positions that the tiling covers, with fewer than 96 channels on a side positions of the
-// plane (64 -> 64 at 14 x 14, 64 images: 27 us, direct 22)
-inline bool winograd_wide(const ConvGeo &g, int64_t enough) {
-  const int64_t covered = static_cast<int64_t>((g.H + 3) / 4) * ((g.W + 3) / 4) * 16, plane = static_cast<int64_t>(g.H) * g.W;
-  const int narrow = std::min(g.C, g.O);
-  return narrow >= 64 && covered * 3 <= plane * 4 && g.imgs * (narrow < 96 ? plane : covered) >= enough;
+// and enough tiles to fill the chip
+inline bool winograd_wide(const ConvGeo &g) {
+  const int64_t covered = static_cast<int64_t>((g.H + 3) / 4) * ((g.W + 3) / 4) * 16;
+  return std::min(g.C, g.O) >= 64 && covered * 3 <= static_cast<int64_t>(g.H) * g.W * 4 &&
+         static_cast<int64_t>(g.imgs) * covered >= 16 * 1024;
 }
 
 // forward and data gradient: the channels summed over are the GEMMs' K
 inline bool winograd_pays(const ConvGeo &g, int gathered) {
   const int forced = winograd_forced();
   if (!winograd_shape(g) || gathered % BK != 0 || forced == 0) return false;
-  return forced == 1 || winograd_wide(g, 16 * 1024);
+  return forced == 1 || winograd_wide(g);
 }
 
-// (64 channels on a side: 64 -> 128 at 32 x 32, 16 images 59 us, direct 34; at 112 x 112, 4 images 69 and 63, 8 images 68 and 109)
 inline bool winograd_filter_grad_pays(const ConvGeo &g) {
   const int forced = winograd_forced();
   if (!winograd_shape(g) || forced == 0) return false;
-  return forced == 1 || winograd_wide(g, std::min(g.C, g.O) < 96 ? 48 * 1024 : 16 * 1024);
+  return forced == 1 || winograd_wide(g);
 }
 
 // ------------------------------------------------------------------ statistics of the output

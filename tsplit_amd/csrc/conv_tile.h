@@ -1,22 +1,15 @@
-// Convolution forward and data gradient as implicit products on the tile kernel of split_tile.h (small layers whose filter can be
-// read where it lies on that of gemm_tile.h).
+// Convolution forward and data gradient as implicit products on the tile kernel of gemm_tile.h.
 //
 //   forward        y[img,o,p]  : M = O, N = imgs * oH * oW, depth (c, tap)   A = filter [O][depth]
-//   data gradient  dx[img,c,q] : M = C, N = imgs * H * W,   depth (o, tap)   A = filter [C][depth]
-//
-// A is prepared: re-laid in the order of the depth and split into three bf16 planes, in one kernel.  What bounds the products is what their
-// waves do beside them, splitting the columns, reading LDS and waiting for the gathers, at half to two thirds of the matrix pipe and, in the
-// largest layers, the clock that the chip's power allows (1.7-2.0 GHz).  Against the fp32 instruction, us, forward / data gradient: 3x3 of
-// 512 -> 512 at 28x28, 18 images 321 / 320 (563 / 562); 1x7 of 280 -> 452 at 25x25, 56 images 407 / 369 (599 / 560); 1x1 of 64 -> 256 at 56x56,
-// 64 images 80 / 54 (101 / 66); 7x7 stride 2 of 3 -> 64 at 224x224, data gradient 1951 (3099).
+//   data gradient  dx[img,c,q] : M = C, N = imgs * H * W,   depth (o, tap)   A = filter re-laid [C][depth]
 //
 // B is gathered: row k of the operand is one tap of one channel at the tile's columns, 64 columns a load of 4 bytes a lane
 // into LDS.  A lane's offset is fixed for the tile, what changes with k is wave-uniform and travels in the scalar offset; a
 // tap in the padding is an out-of-range offset, which LDS receives as zero.  The depth is ordered in blocks of 8 channels of
 // one tap, k = ((ch / 8) * taps + tap) * 8 + ch % 8 with channels padded to whole blocks: a wave's 8 rows of a 32-deep step
 // are then one block, and the choice between a lane's offset and the padding's is made once for all of them.  In the
-// filter's own order (ch, tap) it is made for every row, which costs vector instructions (17x17 images, 1x7 filters, 256 -> 256, with the
-// fp32 instruction: 128 us against 87 in blocks): only layers of few channels, where the padding would cost more, use
+// filter's own order (ch, tap) it is made for every row, which costs vector instructions the products pay for (17x17 images,
+// 1x7 filters, 256 -> 256: 128 us against 87 in blocks): only layers of few channels, where the padding would cost more, use
 // that order.  Where a layer has one tap, no padding and planes of whole 16-byte words, B is loaded in 16-byte words like a
 // dense operand.
 //
@@ -28,7 +21,6 @@
 
 #include "fastdiv.h"
 #include "gemm_tile.h"
-#include "split_tile.h"
 
 namespace tsplit {
 namespace ct {
@@ -48,15 +40,13 @@ struct Phase {
   int ph, pw;             // forward: padding.  Data gradient: the phase's own (see conv.hip)
   int bias;               // elements by which the gathered tensor's base is moved back so that no offset is negative
   int out_a0, out_b0;     // first output row / column of the phase
-  int w_at;               // where the phase's filter begins among the chunks
-  int tap_a, tap_b;       // the filter's tap that is the phase's first
+  int w_at;               // where the phase's filter begins in w
   int first_tile;         // tiles of the phases before it
   int kchunk;             // k range of one split (a multiple of 32)
 };
 
 struct Params {
   const float *src, *w;
-  const char *planes;   // the filter prepared for the products
   float *out;
   int64_t out_img_stride, z_stride;
   unsigned src_bytes;
@@ -67,46 +57,7 @@ struct Params {
   FastDiv tm, tiles;             // M tiles; tiles of all phases (of all pairs)
   int phases;
   float *stats;
-  int w_row, w_chan, w_width, w_s;   // distances of rows, channels and rows of taps in w; of a phase's taps
-  bool plain;                        // the depth in the order (channel, tap)
   Phase phase[kMaxPhases];
-};
-
-// The filter as the products see it: row (of M), k of a phase's depth, zeros outside and for the channels that pad the last block.
-struct FilterRows {
-  const float *w;
-  FastDiv taps, kw;
-  int M, K, chans, w_row, w_chan, w_width, w_s, tap_a, tap_b;
-  bool plain;
-  __host__ __device__ FilterRows(const Params &P, const Phase &F)
-      : w(P.w), taps(F.taps), kw(F.kw), M(P.M), K(F.K), chans(P.chans), w_row(P.w_row), w_chan(P.w_chan), w_width(P.w_width), w_s(P.w_s),
-        tap_a(F.tap_a), tap_b(F.tap_b), plain(P.plain) {}
-  __device__ __forceinline__ float at(int row, int k) const {
-    int ch, tap;
-    if (plain) {
-      ch = taps.div(k);
-      tap = k - ch * taps.d;
-    } else {
-      const int block = k >> 3, cb = taps.div(block);
-      tap = block - cb * taps.d;
-      ch = 8 * cb + (k & 7);
-    }
-    const int u = kw.div(tap), v = tap - u * kw.d;
-    return row < M && k < K && ch < chans ? w[row * w_row + ch * w_chan + (tap_a + w_s * u) * w_width + tap_b + w_s * v] : 0.f;
-  }
-  // values k to k + 3 of a row, k a multiple of 4; in blocks of channels they are of one tap
-  __device__ __forceinline__ void four(int row, int k, float (&v)[4]) const {
-    if (plain) {
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = at(row, k + j);
-      return;
-    }
-    const int block = k >> 3, cb = taps.div(block), tap = block - cb * taps.d, ch = 8 * cb + (k & 7), u = kw.div(tap);
-    const bool in = row < M && k < K;
-    const float *from = w + (in ? row * w_row + ch * w_chan + (tap_a + w_s * u) * w_width + tap_b + w_s * (tap - u * static_cast<int>(kw.d)) : 0);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = in && ch + j < chans ? from[j * w_chan] : 0.f;
-  }
 };
 
 // B, gathered.  BWD: element (k = (ch, u, v), position (r, c)) at [ch][r + ph - u][c + pw - v], else at
@@ -239,42 +190,22 @@ struct Pointwise {
 // How a pass reads B: words of a dense operand, one tap, up to 32 / 64 taps in blocks of 8 channels, up to 64 in the filter's order
 enum Gather { kWords, kOneTap, kBlocks32, kBlocks64, kTaps64 };
 
-// The tiles of tile_plan.h by product tiles and waves: of the kernel whose filter is prepared, and of the fp32 instruction's
-template <int TILE, bool PREPARED>
-struct Shape {
-  static constexpr int TM = TILE == 3 ? 2 : 4, TN = TILE == 0 ? 4 : 2, WM = TILE == 1 ? 1 : 2;
-};
-template <int TILE>
-struct Shape<TILE, false> {
-  static constexpr int TM = TILE == 0 || TILE == 2 ? 4 : 2, TN = TILE <= 1 ? 4 : 2, WM = 2;
-};
+// ACROSS: A is the filter in memory, [depth][M] (data gradient of one tap); else [M][depth]
+template <int TM, int TN, bool BWD, int GATHER, bool ACROSS>
+struct Pass {
+  static constexpr int BM = 32 * TM, BN = 32 * TN;
+  using BL = typename std::conditional<GATHER == kWords, Pointwise<BN, TN>,
+                                       Gathered<BN, TN, BWD, GATHER == kOneTap ? 0 : GATHER == kBlocks32 ? 32 : 64, GATHER != kTaps64>>::type;
+  using AL = typename std::conditional<ACROSS, gt::MnContig<BM, TM>, gt::KContig<BM, TM, false>>::type;
+  using C = gt::Core<TM, TN, 2, 2, AL, BL>;
 
-// PREPARED: the filter as planes (split_tile.h).  Else, for layers of one tap and forward ones in the filter's own order, the fp32 instruction and
-// the filter as it lies in memory, [M][depth] or (data gradient) [depth][M].
-template <int TILE, bool BWD, int GATHER, bool PREPARED>
-struct Pass : Shape<TILE, PREPARED> {
-  using S = Shape<TILE, PREPARED>;
-  static constexpr int WN = 4 / S::WM, BM = 16 * S::TM * S::WM, BN = 16 * S::TN * WN;
-  using BL = typename std::conditional<GATHER == kWords, Pointwise<BN, S::TN>,
-                                       Gathered<BN, S::TN, BWD, GATHER == kOneTap ? 0 : GATHER == kBlocks32 ? 32 : 64, GATHER != kTaps64>>::type;
-  using AL = typename std::conditional<BWD, gt::MnContig<BM, S::TM>, gt::KContig<BM, S::TM, false>>::type;
-  using C = typename std::conditional<PREPARED, st::Core<S::TM, S::TN, S::WM, WN, BL>, gt::Core<S::TM, S::TN, S::WM, WN, AL, BL>>::type;
-  static constexpr int kLdsFloats = C::kLdsFloats;
-
-  static __device__ __forceinline__ void run(const Params &P, const Phase &F, int m0, int n0, int z, float *lds, f32x4 (&acc)[S::TM][S::TN]) {
+  static __device__ __forceinline__ void run(const Params &P, const Phase &F, int m0, int n0, int z, float *lds, f32x4 (&acc)[TM][TN]) {
+    AL la;
     BL lb;
+    la.init(mg::DenseParams{P.w + F.w_at, ACROSS ? P.M : F.K, P.M, F.K}, m0);
     lb.init(P, F, n0);
-    const int kbegin = z * F.kchunk, kend = min(F.K, kbegin + F.kchunk);
-    if constexpr (PREPARED) {
-      typename C::AL la;
-      la.init(st::PlanesParams{P.planes + static_cast<int64_t>(F.w_at) * st::kChunk, (P.M + 15) / 16, (F.K + BK - 1) / BK}, m0);
-      if (!C::run(la, lb, kbegin, kend, reinterpret_cast<char *>(lds), acc))
-        C::exact(FilterRows(P, F), m0, lb, kbegin, kend, reinterpret_cast<char *>(lds), acc);
-    } else {
-      AL la;
-      la.init(mg::DenseParams{P.w, BWD ? P.M : F.K, P.M, F.K}, m0);
-      C::run(la, lb, kbegin, kend, lds, acc);
-    }
+    const int kbegin = z * F.kchunk;
+    C::run(la, lb, kbegin, min(F.K, kbegin + F.kchunk), lds, acc);
   }
 };
 
@@ -356,12 +287,11 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
 
 // STATS: each wave leaves the sums and sums of squares of its rows over its 16 TN columns, for column group
 // (first column) / (16 TN) at stats[(group * M + row) * 2].
-template <int TILE, bool BWD, int GATHER, bool PREPARED, bool STATS>
+template <int TM, int TN, bool BWD, int GATHER, bool ACROSS, bool STATS>
 __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, int total) {
-  using X = Pass<TILE, BWD, GATHER, PREPARED>;
+  using X = Pass<TM, TN, BWD, GATHER, ACROSS>;
   using C = typename X::C;
-  constexpr int TM = X::TM, TN = X::TN;
-  __shared__ __attribute__((aligned(1024))) float lds[X::kLdsFloats];
+  __shared__ __attribute__((aligned(1024))) float lds[C::kLdsFloats];
   int z, ip, tile_m, tile_n;
   if (!place(P, total, 1, z, ip, tile_m, tile_n)) return;
   const Phase &F = P.phase[ip];
@@ -374,7 +304,7 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
   const int img0 = F.plane.div(n0), plane_bytes = P.out_plane * 4;
   const __amdgpu_buffer_rsrc_t to =
       gt::output_buffer(P.out + z * P.z_stride + img0 * P.out_img_stride + static_cast<int64_t>(m) * P.out_plane, 0x7fffffffll);
-  if constexpr (BWD && (GATHER == kWords || GATHER == kOneTap))
+  if constexpr (BWD && ACROSS)
     if (P.out_s == 2) return spread<TM, TN>(P, F, acc, to, m, n, img0, C::lane_row(), [](int tm, int e) { return C::step_row(tm, e); });
   // where the lane's TN columns go: together if they lie in one image of a plane without gaps
   const unsigned at = static_cast<unsigned>(C::lane_row()) * plane_bytes;
@@ -419,6 +349,7 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
   else
     store(std::false_type{}, std::false_type{});
   if constexpr (STATS) {
+    static_assert(!ACROSS, "rows in order");
     // lane c of 16 (TM = 2: the pair c / 2) ends with row register c (tm = c / 4, e = c % 4) summed over the 16 lanes
     constexpr int R = 4 * TM;
     float sum[R], sq[R];
@@ -447,12 +378,11 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
 }
 
 // Data gradient of stride 2: phases 2 q and 2 q + 1 are the even and the odd columns of the same rows of positions.
-template <int TILE>
+template <int TM, int TN>
 __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_pair_kernel(Params P, int total) {
-  using X = Pass<TILE, true, kBlocks32, true>;
+  using X = Pass<TM, TN, true, kBlocks32, false>;
   using C = typename X::C;
-  constexpr int TM = X::TM, TN = X::TN;
-  __shared__ __attribute__((aligned(1024))) float lds[X::kLdsFloats];
+  __shared__ __attribute__((aligned(1024))) float lds[C::kLdsFloats];
   int z, ip, tile_m, tile_n;
   if (!place(P, total, 2, z, ip, tile_m, tile_n)) return;
   const Phase &F = P.phase[ip];
@@ -501,14 +431,38 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_pair_kernel(Params 
     }
 }
 
-// The filter's planes, every phase: a block a chunk
-static __global__ __launch_bounds__(64) void conv_planes_kernel(Params P, char *__restrict__ out) {
-  const int lane = threadIdx.x, chunk = blockIdx.x;
+// The filter in the order of the depth, for every phase: w[w_at + row * K + ((ch / 8) * taps + tap) * 8 + ch % 8], zeros for the
+// channels that pad the last block (or, `plain`, w[... + ch * taps + tap]).  Tap (u, v) of the phase is the filter's tap
+// (a + s u, b + s v); bwd: rows are C and channels O, else the other way.
+struct RelayPhase {
+  int w_at, K, a, b;
+  FastDiv taps, kw, k;
+};
+struct Relay {
+  const float *w;
+  float *out;
+  int rows, chans, w_row, w_chan, f_w, s, phases, total;
+  bool plain;
+  RelayPhase phase[kMaxPhases];
+};
+static __global__ __launch_bounds__(256) void conv_relay_kernel(Relay R) {
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= R.total) return;
   int ip = 0;
-  while (ip + 1 < P.phases && chunk >= P.phase[ip + 1].w_at) ++ip;
-  const Phase &F = P.phase[ip];
-  const int steps = (F.K + BK - 1) / BK, at = chunk - F.w_at, tile = at / steps;
-  st::put_planes(FilterRows(P, F), 16 * tile + (lane & 15), (at - tile * steps) * BK + 4 * (lane >> 4), out + static_cast<int64_t>(chunk) * st::kChunk, lane);
+  while (ip + 1 < R.phases && idx >= R.phase[ip + 1].w_at) ++ip;
+  const RelayPhase &F = R.phase[ip];
+  const int i = idx - F.w_at, row = F.k.div(i), k = i - row * F.K;
+  int ch, tap;
+  if (R.plain) {
+    ch = F.taps.div(k);
+    tap = k - ch * F.taps.d;
+  } else {
+    const int block = k >> 3, cb = F.taps.div(block);
+    tap = block - cb * F.taps.d;
+    ch = 8 * cb + (k & 7);
+  }
+  const int u = F.kw.div(tap), v = tap - u * F.kw.d;
+  R.out[idx] = ch < R.chans ? R.w[row * R.w_row + ch * R.w_chan + (F.a + R.s * u) * R.f_w + F.b + R.s * v] : 0.f;
 }
 
 }  // namespace ct

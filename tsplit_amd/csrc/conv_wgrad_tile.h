@@ -1,5 +1,4 @@
-// Convolution filter gradient as a product of two fp32 operands on the tile of gemm_tile.h, with bf16 products of split values
-// (split_tile.h) or, for some layers of one tap, the fp32 instruction: dw[o, (tap, c)] = sum over positions of
+// Convolution filter gradient as a product on the tile kernel of gemm_tile.h: dw[o, (tap, c)] = sum over positions of
 // dy[o, position] x[c, position shifted by the tap].
 //
 //   M = O, N = taps x C (a tap's channels in whole groups of 16, 4 or 2), depth = images x positions, an image's positions padded to
@@ -20,15 +19,16 @@
 // by value, positions outside the image as zeros.  Rows past the last channel hold values of the next image: they belong to
 // rows or columns of dw that do not exist.
 //
-// What bounds it is the splitting, which every wave does for all it multiplies (64 x 64 tiles split more than they multiply), and the
-// gathered loads, 4 bytes a lane.  Over 161 layers of several taps and 25 of one, the best tile and ranges each time: 10 985 and 1 253 us;
-// with the fp32 instruction 12 529 and 1 396.  3x3 of 512 -> 512 at 28x28, 18 images 425 us (570).
+// What bounds it is the matrix pipe where the tiles fill the chip (1x1 layers: 64 x 512 x 28 x 28 -> 128 in 62 us, 106 TFLOP/s) and
+// the gathered loads, 4 bytes a lane, elsewhere.  Against 16-deep steps whose operands went through vector registers: 1x1 layers of
+// ResNet-50 66, 62, 76, 76 us (were 90, 87, 90, 90), its first layer 259 (411), 1x7 of 256 -> 256 at 17x17 93 (96), 3x3 of 512 -> 512 at
+// 4x4 71 (79), 3x3 stride 2 of 96 -> 200 channels 17 (32); but 3x3 of 512 -> 512 at 28x28, 18 images, 570 (549), where the loads count
+// most.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include "fastdiv.h"
 #include "gemm_tile.h"
-#include "split_tile.h"
 
 namespace tsplit {
 namespace wt {
@@ -209,15 +209,13 @@ struct Taps {
   }
 };
 
-// G: channels of a group, the columns of one tap; 0: one tap, stride 1, no padding (the columns are the channels themselves).
-// SPLIT: bf16 products of split values (split_tile.h), else the fp32 instruction.
-template <int TM, int TN, int G, bool SPLIT>
+// G: channels of a group, the columns of one tap; 0: one tap, stride 1, no padding (the columns are the channels themselves)
+template <int TM, int TN, int G>
 __global__ __launch_bounds__(gt::kThreads, 2) void conv_wgrad_tile_kernel(Params P, mg::TileGrid tg) {
   constexpr int BM = 32 * TM, BN = 32 * TN, kGroup = G ? G : 16;
   using AL = Words<BM, TM>;
   using BL = typename std::conditional<G == 0, Words<BN, TN>, Taps<BN, TN, kGroup>>::type;
-  using F = gt::Core<TM, TN, 2, 2, AL, BL>;
-  using C = typename std::conditional<SPLIT, st::CoreBoth<TM, TN, 2, 2, AL, BL>, F>::type;
+  using C = gt::Core<TM, TN, 2, 2, AL, BL>;
   __shared__ __attribute__((aligned(1024))) float lds[C::kLdsFloats];
   int z, tile_m, tile_n;
   if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
@@ -225,22 +223,13 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_wgrad_tile_kernel(Params
   const int first_image = P.image.div(kbegin);
   AL la;
   BL lb;
-  auto begin = [&] {
-    la.init(P.dy, P.dy_bytes, P.image, P.plane, P.dy_img, m0, first_image, kbegin);
-    if constexpr (G == 0)
-      lb.init(P.x, P.x_bytes, P.image, P.plane, P.x_img, n0, first_image, kbegin);
-    else
-      lb.init(P, n0, first_image, kbegin);
-  };
-  begin();
+  la.init(P.dy, P.dy_bytes, P.image, P.plane, P.dy_img, m0, first_image, kbegin);
+  if constexpr (G == 0)
+    lb.init(P.x, P.x_bytes, P.image, P.plane, P.x_img, n0, first_image, kbegin);
+  else
+    lb.init(P, n0, first_image, kbegin);
   f32x4 acc[TM][TN];
-  if constexpr (!SPLIT) {
-    F::run(la, lb, kbegin, kend, lds, acc);
-  } else if (!C::run(la, lb, kbegin, kend, lds, acc)) {
-    __syncthreads();   // the verdict lies where the first step goes
-    begin();
-    F::run(la, lb, kbegin, kend, lds, acc);
-  }
+  C::run(la, lb, kbegin, kend, lds, acc);
 
   float *out = P.out + z * P.z_stride;
   const int lane = threadIdx.x & 63, m = m0 + C::wave_m0() + C::lane_row();

@@ -38,13 +38,13 @@ __global__ __launch_bounds__(256) void fold_tap_major_kernel(const float *__rest
   }
 }
 
-template <int G, bool SPLIT>
+template <int G>
 void launch_tile(const Params &P, int tile, const mg::TileGrid &tg, unsigned grid, hipStream_t st) {
   switch (tile) {
-    case 0: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 4, G, SPLIT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
-    case 1: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 4, G, SPLIT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
-    case 2: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 2, G, SPLIT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
-    default: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 2, G, SPLIT>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    case 0: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 4, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    case 1: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 4, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    case 2: hipLaunchKernelGGL((conv_wgrad_tile_kernel<4, 2, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
+    default: hipLaunchKernelGGL((conv_wgrad_tile_kernel<2, 2, G>), dim3(grid), dim3(gt::kThreads), 0, st, P, tg); break;
   }
 }
 
@@ -95,16 +95,7 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   P.n_groups = taps * static_cast<int>(P.groups.d);
   const int64_t cols = static_cast<int64_t>(group) * P.n_groups, values = static_cast<int64_t>(g.O) * P.cols;
   const int steps = (P.K + BK - 1) / BK;
-  // With several taps the split products are the faster on every tile.  With one, where the loads are cheap, they lose on 64 x 64 tiles with
-  // three or more of them on a CU, whose waves split more than they multiply (2.1 and 2.8 us a step, fp32 1.7 and 2.2).
-  auto planned = [&](const TileCost &cost) { return plan_tiles(g.O, &cols, &steps, 1, 1, 1024, static_cast<double>(values), cost); };
-  TilePlan plan = planned(point ? kFilterWordsSplitCost : kFilterTapsSplitCost);
-  bool split = true;
-  if (point) {
-    const TilePlan plain = planned(kFilterWordsCost);
-    split = plan.us < plain.us;
-    if (!split) plan = plain;
-  }
+  const TilePlan plan = plan_tiles(g.O, &cols, &steps, 1, 1, 1024, static_cast<double>(values), point ? kFilterWordsCost : kFilterTapsCost);
   const TileKind &k = kTiles[plan.tile];
   P.kchunk = range_depth(g, reach, plan.S);
   const int S = std::max(1, (P.K + P.kchunk - 1) / P.kchunk);
@@ -120,16 +111,14 @@ int conv_tile_bwd_filter(const float *x, const float *dy, float *dw, const ConvT
   }
   const mg::TileGrid tg{tm, tn, tm * tn * S};
   const unsigned grid = mg::grid_blocks(tm, tn, S);
-  if (point && !split)
-    launch_tile<0, false>(P, plan.tile, tg, grid, st);
-  else if (point)
-    launch_tile<0, true>(P, plan.tile, tg, grid, st);
+  if (point)
+    launch_tile<0>(P, plan.tile, tg, grid, st);
   else if (group == 16)
-    launch_tile<16, true>(P, plan.tile, tg, grid, st);
+    launch_tile<16>(P, plan.tile, tg, grid, st);
   else if (group == 4)
-    launch_tile<4, true>(P, plan.tile, tg, grid, st);
+    launch_tile<4>(P, plan.tile, tg, grid, st);
   else
-    launch_tile<2, true>(P, plan.tile, tg, grid, st);
+    launch_tile<2>(P, plan.tile, tg, grid, st);
   if (taps == 1 && S > 1 && S < 8)   // (four lanes share an output's ranges in the other)
     gt::launch_fold(P.out, dw, values, S, st);
   else if (!direct)

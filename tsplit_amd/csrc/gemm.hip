@@ -1,6 +1,5 @@
-// DLGpuMatrixMultiply and DLGpuBatchMatrixMultiply: row-major C = op(A) op(B) on the tile kernels of
-// split_tile.h (one operand prepared, bf16 products of split values) and, where a product is too small to
-// win back the preparing and for batches, of gemm_tile.h (the fp32 instruction).
+// DLGpuMatrixMultiply and DLGpuBatchMatrixMultiply: row-major C = op(A) op(B) on the fp32 MFMA
+// tile kernel of gemm_tile.h.
 //
 // The four transpose combinations only change which way each operand is staged (a transposed
 // operand is simply one whose other index is contiguous); nothing is ever transposed in memory.
@@ -15,7 +14,6 @@
 #include "gemm_tile.h"
 #include "mfma_gemm.h"
 #include "gemm_split.h"
-#include "split_tile.h"
 #include "tile_plan.h"
 
 namespace tsplit {
@@ -28,41 +26,19 @@ inline int64_t stored_rows(bool k_rows, int mn, int K) { return k_rows ? K : mn;
 
 struct Plan {
   int tile, S, kchunk;
-  double us;       // as the model has it
-  bool prepared;   // one operand prepared, bf16 products (split_tile.h)
-  bool across;     // ... the columns of C, else its rows
 };
 
-Plan best_plan(int M, int N, int K, int batch, bool may_split, const TileCost &cost) {
+Plan best_plan(int M, int N, int K, int batch, bool may_split) {
   const int64_t cols = N;
   const int steps = std::max(1, (K + gt::BK - 1) / gt::BK);
-  const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, cost);
-  Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK, t.us, false, false};
+  const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, kProductCost);
+  Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK};
   p.S = std::max(1, (K + p.kchunk - 1) / p.kchunk);
   if (p.S == 1) p.kchunk = K;
   return p;
 }
 
-// The operand with fewer rows is the one to prepare, unless the result then leaves in single words, which takes long with the columns
-// prepared (3930 x 3702 over 113: 58 us, fp32 44).  The preparing costs a launch, 3.5 us and 1 ns a chunk, and below two steps a product is
-// its stores (25088 x 4096 over 18: 110 us, fp32 88; over 64 139 and 153, over 66 160 and 191).  Else the model decides: over 276 products its
-// choice takes 7.69 ms, the better of the two each time 7.64, fp32 alone 9.81; the seven that 2.5 us took as well 148 us, fp32 146.
-Plan choose_plan(int M, int N, int K, int batch, bool may_split) {
-  const Plan plain = best_plan(M, N, K, batch, may_split, kProductCost);
-  if (!may_split || K < 2 * gt::BK || plain.us < 6) return plain;   // (the prepared form is at best 0.55 of it and the 3.5 us)
-  const bool across = N % 4 == 0 ? M > N : M > 4ll * N;
-  const int P = across ? N : M, X = across ? M : N;
-  const int64_t tiles = (P + 15) / 16, steps = (K + gt::BK - 1) / gt::BK;
-  // chunks of a tile within 32-bit offsets, threads of the preparing kernel within a grid
-  if (8 * steps * st::kChunk >= (1ll << 31) || tiles * steps >= (1ll << 24)) return plain;
-  Plan p = best_plan(P, X, K, 1, true, kProductSplitCost);
-  if (p.us + 3.5 + 1e-3 * static_cast<double>(tiles * steps) >= plain.us) return plain;
-  p.prepared = true;
-  p.across = across;
-  return p;
-}
-
-// the plans of the shapes this thread asked for last (working one out takes 2-4 us of host time)
+// the plans of the shapes this thread asked for last (working one out takes about 2 us of host time)
 Plan plan_product(int M, int N, int K, int batch, bool may_split) {
   struct Entry {
     int M, N, K, batch;
@@ -73,8 +49,7 @@ Plan plan_product(int M, int N, int K, int batch, bool may_split) {
   // (multiplied through: sums of small multiples put every shape of a net of power-of-two sizes into two places)
   const unsigned mix = ((static_cast<unsigned>(M) * 31u + static_cast<unsigned>(N)) * 31u + static_cast<unsigned>(K)) * 31u + static_cast<unsigned>(batch);
   Entry &e = known[(mix * 2654435769u) >> 24];
-  if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.may_split != may_split)
-    e = {M, N, K, batch, may_split, choose_plan(M, N, K, batch, may_split)};
+  if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.may_split != may_split) e = {M, N, K, batch, may_split, best_plan(M, N, K, batch, may_split)};
   return e.plan;
 }
 
@@ -100,53 +75,17 @@ void launch_planned(const float *A, int64_t lda, int64_t sa, const float *B, int
   }
 }
 
-// One operand prepared (split_tile.h).  The rows' operand is the one with fewer of them.
-template <int TM, int TN, int WM, int WN, bool XMN, bool ACROSS>
-void launch_split_tile(const st::PlanesParams &rows, const st::DenseRows &src, const DenseParams &xp, float *out, int64_t mn, bool wide, int P, int X,
-                       int K, const Plan &plan, hipStream_t s) {
-  const int tm = (P + 16 * TM * WM - 1) / (16 * TM * WM), tn = (X + 16 * TN * WN - 1) / (16 * TN * WN);
-  hipLaunchKernelGGL((st::gemm_split_kernel<TM, TN, WM, WN, XMN, ACROSS>), dim3(grid_blocks(tm, tn, plan.S)), dim3(gt::kThreads), 0, s, rows, src, xp,
-                     out, st::SplitStrides{0, 0, 0, mn}, wide, P, X, K, plan.kchunk, TileGrid{tm, tn, tm * tn * plan.S});
-}
-template <bool XMN, bool ACROSS>
-void launch_prepared(const st::DenseRows &src, const DenseParams &xp, char *planes, float *out, int P, int X, int K, const Plan &plan, hipStream_t s) {
-  const int steps = (K + gt::BK - 1) / gt::BK, tiles = (P + 15) / 16;
-  const int64_t mn = static_cast<int64_t>(P) * X;
-  hipLaunchKernelGGL(st::planes_kernel, dim3(tiles * steps), dim3(64), 0, s, src, 0, planes, FastDiv(steps));
-  const st::PlanesParams rows{planes, tiles, steps};
-  const bool wide = (ACROSS ? P : X) % 4 == 0 && aligned16(out);
-  switch (plan.tile) {
-    case 0: return launch_split_tile<4, 4, 2, 2, XMN, ACROSS>(rows, src, xp, out, mn, wide, P, X, K, plan, s);
-    case 1: return launch_split_tile<4, 2, 1, 4, XMN, ACROSS>(rows, src, xp, out, mn, wide, P, X, K, plan, s);
-    case 2: return launch_split_tile<4, 2, 2, 2, XMN, ACROSS>(rows, src, xp, out, mn, wide, P, X, K, plan, s);
-    default: return launch_split_tile<2, 2, 2, 2, XMN, ACROSS>(rows, src, xp, out, mn, wide, P, X, K, plan, s);
-  }
-}
-
 template <bool TA, bool TB>
-int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, Plan plan, hipStream_t s,
-                   int64_t *ws_elems) {
+int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws_elems) {
+  const Plan plan = plan_product(M, N, K, 1, true);
   const int64_t mn = static_cast<int64_t>(M) * N;
-  char *planes = nullptr;
-  if (plan.prepared) {
-    const size_t chunks = static_cast<size_t>(((plan.across ? N : M) + 15) / 16) * ((K + gt::BK - 1) / gt::BK);
-    planes = static_cast<char *>(scratch_get(s, 3, chunks * st::kChunk, true));
-    if (!planes) plan = best_plan(M, N, K, 1, true, kProductCost);   // no room for it: without
-  }
   float *out = C;
   if (plan.S > 1) {
     out = static_cast<float *>(scratch_get(s, 2, static_cast<size_t>(plan.S) * mn * 4));
     TS_REQUIRE(out, "DLGpuMatrixMultiply: no scratch memory for split-K");
     *ws_elems = plan.S * mn;
   }
-  if (plan.prepared) {
-    if (plan.across)
-      launch_prepared<TA, true>(st::dense_rows(B, TB ? ldb : 1, TB ? 1 : ldb, N, K), DenseParams{A, lda, M, K}, planes, out, N, M, K, plan, s);
-    else
-      launch_prepared<!TB, false>(st::dense_rows(A, TA ? 1 : lda, TA ? lda : 1, M, K), DenseParams{B, ldb, N, K}, planes, out, M, N, K, plan, s);
-  } else {
-    launch_planned<TA, TB>(A, lda, 0, B, ldb, 0, out, mn, 1, M, N, K, plan, s);
-  }
+  launch_planned<TA, TB>(A, lda, 0, B, ldb, 0, out, mn, 1, M, N, K, plan, s);
   if (plan.S > 1) gt::launch_fold(out, C, mn, plan.S, s);
   return 0;
 }
@@ -240,14 +179,10 @@ bool rows_reach(int N) { return 65ll * 4 * N < (1ll << 31); }
 template <bool TA, bool TB>
 int dispatch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws) {
   if (!near<TA, TB>(lda, ldb, M, N, K)) return dispatch_far<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
-  if (!rows_reach(N)) {
-    if (split_bf16_enabled() && K % 4 == 0 && K >= BK) return launch_gemm_split<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
-    return dispatch_far<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
-  }
-  const Plan plan = plan_product(M, N, K, 1, true);
-  // asked for split products where none are planned: K a multiple of 4 (a loaded word lies inside a row or outside it)
-  if (!plan.prepared && split_bf16_enabled() && K % 4 == 0 && K >= BK) return launch_gemm_split<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
-  return launch_product<TA, TB>(A, lda, B, ldb, C, M, N, K, plan, s, ws);
+  // split-bf16 products where asked for: K a multiple of 4 (a loaded word lies inside a row or outside it)
+  if (split_bf16_enabled() && K % 4 == 0 && K >= BK) return launch_gemm_split<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
+  if (!rows_reach(N)) return dispatch_far<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
+  return launch_product<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
 }
 
 template <bool TA, bool TB>

@@ -1,63 +1,18 @@
-// Row-major C = op(A) op(B) with split-bf16 products (opt-in, for products too small for split_tile.h): 128 x 128
+// Row-major C = op(A) op(B) with split-bf16 products (opt-in, see wino_gemm_split.h for the method): 128 x 128
 // tiles, 16 k values per step, split-K as in the fp32 engine.  The operands stay fp32 in memory; a loader
 // reads them as fp32, splits them in registers and leaves three bf16 planes per operand in LDS, laid out
 // plane[k / 8][index][k % 8] so that a lane's 8 consecutive k of one row or column are one 16-byte word.
-//
-// An fp32 number a is the exact sum a1 + a2 + a3 of three bf16 numbers: a1 = bf16(a) (round to nearest
-// even), a2 = bf16(a - a1), a3 = a - a1 - a2 (each difference is exact in fp32, and the last one has at
-// most 8 significant bits, so it is a bf16 number).  |a2| <= 2^-8 |a| and |a3| <= 2^-16 |a|.  A product
-// a b is then the sum of nine exact bf16 x bf16 products; the six with i + j <= 4 are kept:
-//     a1 b1 + (a1 b2 + a2 b1) + (a2 b2 + a1 b3 + a3 b1),
-// and what is left out, a2 b3 + a3 b2 + a3 b3, is at most 2^-23 |a b|: the size of the rounding of one
-// fp32 multiplication.  The bf16 matrix instruction (v_mfma_f32_32x32x16_bf16, fp32 accumulation) runs 16
-// times the multiplications per cycle of the fp32 one, so six of them cost 3/8 of the fp32 instruction's
-// time for the same product.  Not for operands above 2^127 (a1 would round to infinity).
 #pragma once
-#include "mfma_gemm.h"
+#include "wino_gemm_split.h"
 
 namespace tsplit {
 namespace mg {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// (x, y) -> packed bf16 pair of the leading terms; x and y are left holding the remainders
-__device__ __forceinline__ unsigned split_pair(float &x, float &y) {
-  const f32x2 v = {x, y};
-  const unsigned packed = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
-  x -= __uint_as_float(packed << 16);
-  y -= __uint_as_float(packed & 0xffff0000u);
-  return packed;
-}
-
-// eight fp32 values -> their three bf16 planes, 16 bytes each
-__device__ __forceinline__ void split8(const float (&in)[8], u32x4 (&out)[3]) {
-  float v[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = in[i];
-#pragma unroll
-  for (int s = 0; s < 3; ++s) {
-    out[s].x = split_pair(v[0], v[1]);
-    out[s].y = split_pair(v[2], v[3]);
-    out[s].z = split_pair(v[4], v[5]);
-    out[s].w = split_pair(v[6], v[7]);
-  }
-}
-
-// c + a b for one 32 x 32 x 16 step from the operands' three planes: the six products, smallest terms first
-__device__ __forceinline__ acc16 split_products(const bf16x8 (&a)[3], const bf16x8 (&b)[3], acc16 c) {
-  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[2], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[1], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1], b[0], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[1], c, 0, 0, 0);
-  c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0], b[0], c, 0, 0, 0);
-  return c;
-}
-
-constexpr int kSplitPlane = 2 * 128 * 8;             // bf16 elements of one plane of one operand (16 k x 128)
-constexpr int kSplitStage = 2 * 3 * kSplitPlane;     // both operands, three planes each
+using wg::bf16x8;
+using wg::kSplitPlane;
+using wg::kSplitStage;
+using wg::split8;
+using wg::split_products;
 
 // element (mn, k) at p[mn * ld + k]: a thread takes 8 consecutive k of one row as two 16-byte words, each of
 // which must lie wholly inside or outside the k range (K and the range bounds are multiples of 4)

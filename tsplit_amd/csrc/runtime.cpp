@@ -221,7 +221,7 @@ void *device_pool_alloc(int device_id, size_t bytes) {
   }
 }
 
-void *scratch_get(hipStream_t stream, int slot, size_t bytes, bool optional) {
+void *scratch_get(hipStream_t stream, int slot, size_t bytes) {
   std::lock_guard<std::mutex> lk(g_mu);
   ScratchBuf &b = g_scratch[ScratchKey{stream, slot}];
   hipStreamCaptureStatus recording = hipStreamCaptureStatusNone;
@@ -233,7 +233,6 @@ void *scratch_get(hipStream_t stream, int slot, size_t bytes, bool optional) {
   }
   if (b.p) {
     // growing is set-up, not part of a step: a recording cannot allocate on the way
-    if (in_recording && optional) return nullptr;
     if (in_recording) {
       std::fprintf(stderr, "[libc_runtime_api] scratch memory would have to grow while a step is being recorded; "
                            "run the step once before recording it\n");

@@ -1,4 +1,4 @@
-// Which tile of the tile kernels (gemm_tile.h, split_tile.h) a product runs on and into how many ranges its depth is cut: a small model of
+// Which tile of the tile kernel (gemm_tile.h) a product runs on and into how many ranges its depth is cut: a small model of
 // the chip, with figures measured on it.
 //
 // A CU takes its blocks in rounds of as many as are resident at once.  A 32-deep step of a round takes what it takes with that many
@@ -13,10 +13,6 @@
 // the same time however many blocks shared the CU, fitted to one count of ranges and with five 64 x 64 blocks resident everywhere, cost
 // 1.9, 2.9, 4.0, 2.2 and 3.3 %, at worst 40 (18 x 25088 x 4096 with the second operand transposed: 153 us on 64 x 128, 109 on 64 x 64;
 // 3x3 of 512 -> 512 at 7 x 7, data gradient: 181 us in 5 ranges, 156 in 6).
-//
-// The figures of split_tile.h's kernels come from 851 more launches in the same way; their choices cost 0.9 % (products), 0.5 (one tap), 0.6
-// (gathered), 1.1 (pairs), 0.1 and 1.1 (filter gradients in words and by tap) over the best; with the fp32 instruction's figures they
-// cost 5.9, 13, 5.6, 0, 11 and 14 % of all the launches' time.
 #pragma once
 #include <algorithm>
 #include <cstdint>
@@ -41,8 +37,7 @@ constexpr TileCost kProductCost = {{2, 3, 3, 5},
 constexpr TileCost kOneTapCost = {{2, 3, 3, 5},
                                   {{1.88, 3.76}, {1.41, 2.28, 2.84}, {0.89, 1.77, 2.84}, {0.48, 0.90, 1.25, 1.74, 2.46}},
                                   {4.2, 2.5, 2.6, 2.3}, 0.5, 11.8};
-// one operand gathered by tap, fp32 instruction (small forward layers of few channels; the pairs' and taps' figures below only serve the
-// test of this model, their kernels are gone): a load and a row of LDS for every 64 values instead of every 256
+// one operand gathered by tap: a load and a row of LDS for every 64 values instead of every 256
 constexpr TileCost kGatheredCost = {{2, 3, 3, 5},
                                     {{2.44, 4.63}, {1.34, 2.34, 3.57}, {1.44, 2.68, 3.27}, {0.82, 1.25, 1.77, 2.36, 3.07}},
                                     {1.9, 1.7, 0.7, 0.9}, 2.5, 8.1};
@@ -58,38 +53,15 @@ constexpr TileCost kFilterWordsCost = {{2, 3, 3, 4},
 constexpr TileCost kFilterTapsCost = {{2, 3, 3, 4},
                                       {{3.38, 4.57}, {1.44, 3.07, 3.68}, {1.35, 2.40, 3.34}, {0.85, 1.36, 2.04, 2.49}},
                                       {0.6, 0.5, 0, 0}, 2.0, 6.2};
-// the same two with the smaller operand prepared (split_tile.h)
-constexpr TileCost kProductSplitCost = {{2, 2, 2, 4},
-                                        {{1.78, 2.05}, {0.89, 1.26}, {0.92, 1.10}, {0.44, 0.79, 1.15, 1.61}},
-                                        {1.4, 1.4, 1.0, 0.7}, 2.8, 8.1};
-constexpr TileCost kOneTapSplitCost = {{2, 2, 2, 4},
-                                       {{1.32, 2.33}, {0.87, 1.29}, {1.06, 1.13}, {0.45, 0.90, 1.21, 1.42}},
-                                       {3.5, 2.5, 2.7, 2.1}, 1.8, 11.7};
-// filter prepared, the other operand gathered by tap: a load and a row of LDS for every 64 values instead of every 256
-constexpr TileCost kGatheredSplitCost = {{2, 2, 2, 4},
-                                         {{1.47, 1.94}, {1.06, 1.52}, {0.85, 1.22}, {0.60, 0.83, 1.35, 1.63}},
-                                         {4.1, 3.5, 2.4, 1.9}, 2.4, 7.6};
-// the same in pairs of phases (data gradients of stride 2)
-constexpr TileCost kPairsSplitCost = {{2, 2, 2, 4},
-                                      {{2.49, 3.03}, {1.18, 1.65}, {1.34, 1.63}, {0.60, 0.86, 1.13, 2.04}},
-                                      {5.0, 2.2, 1.9, 1.4}, 0.5, 4.6};
-// filter gradients, both operands split by the waves
-constexpr TileCost kFilterWordsSplitCost = {{2, 3, 3, 4},
-                                            {{2.11, 2.91}, {1.45, 1.88, 3.26}, {1.47, 1.86, 3.46}, {0.63, 1.07, 2.12, 2.76}},
-                                            {0.9, 0.1, 0, 0}, 8.7, 8.6};
-constexpr TileCost kFilterTapsSplitCost = {{2, 3, 3, 4},
-                                           {{2.22, 3.17}, {1.25, 2.07, 2.88}, {1.24, 2.06, 2.80}, {0.74, 1.19, 1.76, 2.28}},
-                                           {1.1, 0.7, 0, 0}, 0, 7.7};
 struct TilePlan {
   int tile, S;
-  double us;
 };
 
 // A launch of `parts` products of M rows each (the phases of a strided data gradient; 1 otherwise), every one `batch` times:
 // part i has cols[i] columns and a depth of steps[i] x 32.  max_split 1: the depth stays whole.
 inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int parts, int64_t batch, int max_split, double out_values,
                            const TileCost &cost) {
-  TilePlan best{0, 1, 0};
+  TilePlan best{0, 1};
   double least = 1e300;
   int deepest = 1;
   for (int i = 0; i < parts; ++i) deepest = std::max(deepest, steps[i]);
@@ -113,7 +85,7 @@ inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int
       if (S > 1) us += cost.fold + (2 * S + 1) * out_values * 4 / (cost.fold_tb * 1e6);
       if (us < least) {
         least = us;
-        best = {t, S, us};
+        best = {t, S};
       }
     };
     const int most = tiles > 1024 ? 1 : std::min(max_split, deepest);

@@ -1,8 +1,7 @@
-// The GEMMs of the Winograd routine's narrow layers, M[xi] (rows x cols) = U[xi] (rows x depth) V[xi] (depth x cols) for up to 64 rows,
-// on the fp32 MFMA tile engine of mfma_gemm.h: U is depth-contiguous, V and M are column-contiguous.  (Wider layers run on the tile kernels of
-// split_tile.h.)
+// The 36 GEMMs of the Winograd routine, M[xi] (rows x cols) = U[xi] (rows x depth) V[xi] (depth x cols),
+// on the fp32 MFMA tile engine of mfma_gemm.h: U is depth-contiguous, V and M are column-contiguous.
 //
-// Their depth is the layer's channel count (64 ... 512: 4 ... 32 k-steps per tile), far less
+// Their depth is the layer's channel count (64 ... 512: 4 ... 32 k-steps per 128x128 tile), far less
 // than in the direct convolutions, and they write as many bytes as they read, so what happens around a
 // tile's k-loop weighs more: with one tile per block, a block holds its slot on the CU until its 64 KB
 // of stores are acknowledged, and the kernel ran at the speed of "multiply, then write" (a version that
@@ -32,11 +31,16 @@ struct Problem {
 // that ends after its one tile holds its slot until the last store is acknowledged.)  The stores are
 // marked non-temporal: M is read next by another kernel, after the whole of it has been written.
 // Summation order is that of the one-tile-per-block engine: the results are the same bits.
-// Tiles are 64 x 256 (1 x 4 waves, so that no wave idles on rows that do not exist; 44 KB of LDS, three blocks).
-constexpr int kGemmBlocksPerCu = 3;
+// Tiles are 128 x 128 (2 x 2 waves; four resident blocks per compute unit: registers and 4 x 40 KB of LDS
+// allow exactly four) or, for layers that produce at most 64 channels, 64 x 256 (1 x 4 waves, so that no
+// wave idles on rows that do not exist; 44 KB of LDS, three blocks).
 template <int BM, int BN>
-static __global__ __launch_bounds__(kThreads, kGemmBlocksPerCu) void wino_gemm_kernel(Problem p, int total) {
-  static_assert(BM == 64 && BN == 256, "each of the 4 waves owns a 64x64 sub-tile");
+constexpr int gemm_blocks_per_cu() {
+  return BM == 128 ? 4 : 3;
+}
+template <int BM, int BN>
+static __global__ __launch_bounds__(kThreads, (gemm_blocks_per_cu<BM, BN>())) void wino_gemm_kernel(Problem p, int total) {
+  static_assert((BM == 128 && BN == 128) || (BM == 64 && BN == 256), "each of the 4 waves owns a 64x64 sub-tile");
   constexpr int WN = BN / 64;
   using ALoader = KContigBufLoader<BM>;
   using BLoader = MnContigBufLoader<BN>;
@@ -344,13 +348,144 @@ static __global__ __launch_bounds__(kThreads, 3) void wino_grad_gemm_narrow_kern
   }
 }
 
-// One resident round of blocks on `cus` compute units, never more blocks than tiles.
-inline void launch(Problem p, hipStream_t st, int cus) {
-  p.tm = (p.rows + 63) / 64;
-  p.tn = (p.ld + 255) / 256;
+// ---------------------------------------------------------------- filter-gradient GEMMs, 128 x 128 tiles
+// Same product and output layout as above.  The unit of work is one tile of one (range, xi) pair; the
+// grid is NB resident blocks on every compute unit and block L (in the XCD-aware order) takes units
+// L, L + G, L + 2G, ...: every block gets the same number of equal units when the host chooses the number
+// of ranges so that the units fill a whole number of rounds, and the blocks of one XCD work at any time
+// on the tiles of the same few (range, xi) pairs, which read the same rows of Y and V through that XCD's
+// L2.  (With one tile per block, a launch of 576 or 864 blocks left a quarter of the matrix pipes idle
+// in its last round, and a launch cut finer paid a prologue and a drained pipeline per block.)  As in the
+// forward kernel, the next unit's first loads are issued before the finished unit's stores.  The LDS
+// request is padded so that exactly NB blocks fit a compute unit: the dispatcher then cannot stack the
+// grid unevenly.
+template <int NB>
+static __global__ __launch_bounds__(kThreads, NB) void wino_grad_gemm_kernel(GradProblem p, int units) {
+  using Loader = KContigBufLoader<128>;
+  using Lds = typename Loader::Lds;
+  constexpr int kStage = 2 * Lds::kFloats;
+  constexpr int kFit = (160 * 1024 / (NB + 1)) / 4 + 64;   // more than an (NB+1)-th of the LDS
+  constexpr int kLds = 2 * kStage > kFit ? 2 * kStage : kFit;
+  __shared__ __attribute__((aligned(16))) float lds[kLds];
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int wm0 = (wave >> 1) * 64, wn0 = (wave & 1) * 64;
+  const int per_group = p.tm * p.tn;
+  const int G = gridDim.x;
+  int u = (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3);
+  if (u >= units) return;
+
+  int z, m0, n0, kbegin, kend;
+  Loader la, lb;
+  auto start = [&](int unit) {
+    z = unit / per_group;
+    const int tile = unit - z * per_group;
+    const int tile_n = tile / p.tm;
+    m0 = (tile - tile_n * p.tm) * 128;
+    n0 = tile_n * 128;
+    const int range = z / kXi, xi = z - range * kXi;
+    kbegin = range * p.kchunk;
+    kend = min(p.ld, kbegin + p.kchunk);
+    typename Loader::Params ap{p.Y + static_cast<int64_t>(xi) * p.rows * p.ld, p.ld, p.rows, p.ld};
+    typename Loader::Params bp{p.V + static_cast<int64_t>(xi) * p.cols * p.ld, p.ld, p.cols, p.ld};
+    la.init(ap, m0, tid);
+    lb.init(bp, n0, tid);
+    la.load(kbegin, kend);
+    lb.load(kbegin, kend);
+  };
+  start(u);
+
+  for (;;) {
+    acc16 acc[2][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    // the last k-step of the previous unit ended with a barrier: stage 0 is free
+    la.store(lds, tid);
+    lb.store(lds + Lds::kFloats, tid);
+    __syncthreads();
+
+    const bool live = m0 + wm0 < p.rows && n0 + wn0 < p.cols;
+    int stage = 0;
+    for (int k0 = kbegin; k0 < kend; k0 += BK) {
+      const bool more = k0 + BK < kend;
+      if (more) {
+        la.load(k0 + BK, kend);
+        lb.load(k0 + BK, kend);
+      }
+      if (live) {
+        const float *sa = lds + stage * kStage, *sb = sa + Lds::kFloats;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          float fa[2][4], fb[2][4];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            Lds::frag(sa, wm0 + 32 * i, j, lane, fa[i]);
+            Lds::frag(sb, wn0 + 32 * i, j, lane, fb[i]);
+          }
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int mi = 0; mi < 2; ++mi)
+#pragma unroll
+              for (int ni = 0; ni < 2; ++ni)
+                acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[mi][e], fb[ni][e], acc[mi][ni], 0, 0, 0);
+        }
+      }
+      if (more) {
+        float *sa = lds + (stage ^ 1) * kStage;
+        la.store(sa, tid);
+        lb.store(sa + Lds::kFloats, tid);
+      }
+      __syncthreads();
+      stage ^= 1;
+    }
+
+    float *__restrict__ o = p.out + static_cast<int64_t>(z) * p.rows * p.cols;
+    const int om0 = m0 + wm0, on0 = n0 + wn0;
+    u += G;
+    const bool again = u < units;
+    if (again) start(u);
+    if (live) {
+#pragma unroll
+      for (int ni = 0; ni < 2; ++ni) {
+        const int n = on0 + 32 * ni + (lane & 31);
+        if (n >= p.cols) continue;
+#pragma unroll
+        for (int mi = 0; mi < 2; ++mi) {
+          const int mb = om0 + 32 * mi + 4 * (lane >> 5);
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            const int m = mb + 8 * (e >> 2) + (e & 3);
+            if (m < p.rows) o[static_cast<int64_t>(m) * p.cols + n] = acc[mi][ni][e];
+          }
+        }
+      }
+    }
+    if (!again) break;
+  }
+}
+
+// One resident round of blocks on `cus` compute units (with four per unit the 128 x 128 kernel ran 3 %
+// faster over the launches of a VGG-16 step than with three), never more blocks than tiles.
+template <int BM, int BN>
+inline void launch_tiles(Problem p, hipStream_t st, int cus) {
+  p.tm = (p.rows + BM - 1) / BM;
+  p.tn = (p.ld + BN - 1) / BN;
   const int total = p.tm * p.tn * kXi;
-  const int grid = std::min(cus * kGemmBlocksPerCu / 8 * 8, (total + 7) / 8 * 8);
-  hipLaunchKernelGGL((wino_gemm_kernel<64, 256>), dim3(grid), dim3(kThreads), 0, st, p, total);
+  int grid = cus * gemm_blocks_per_cu<BM, BN>() / 8 * 8;
+  if (grid > (total + 7) / 8 * 8) grid = (total + 7) / 8 * 8;
+  if (grid < 8) grid = 8;
+  hipLaunchKernelGGL((wino_gemm_kernel<BM, BN>), dim3(grid), dim3(kThreads), 0, st, p, total);
+}
+inline void launch(const Problem &p, hipStream_t st, int cus) {
+  if (p.rows <= 64)
+    launch_tiles<64, 256>(p, st, cus);
+  else
+    launch_tiles<128, 128>(p, st, cus);
 }
 
 }  // namespace wg

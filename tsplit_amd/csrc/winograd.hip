@@ -28,8 +28,7 @@
 #include "common.h"
 #include "mfma_gemm.h"
 #include "reduce.h"
-#include "split_tile.h"
-#include "wino_gemm.h"
+#include "wino_gemm_split.h"
 
 namespace tsplit {
 using namespace mg;
@@ -481,22 +480,24 @@ inline int compute_units() {
   return n;
 }
 
-// How the filter-gradient GEMMs of one run are cut: tile shape and depth per range.  Narrow layers (64 produced or gathered channels) take
-// 64-wide fp32 tiles whose idle waves share the depth, with as many ranges as give three blocks per compute unit.  The
-// others run on 128 x 128 tiles of split products (split_tile.h), two on a compute unit: the number of ranges is chosen so that the blocks
-// (tiles x ranges x 36) fill one, two or three rounds of them as fully as possible, fewer rounds winning unless more
-// rounds fill at least 7 % better; a range keeps at least 12 x 16 of the depth.
+// How the filter-gradient GEMMs of one run are cut: tile shape, depth per range, and (128 x 128 tiles) the
+// persistent grid.  Narrow layers (64 produced or gathered channels) take 64-wide tiles whose idle waves
+// share the depth, one tile per block, with as many ranges as give three blocks per compute unit.  The
+// others run on the persistent kernel: the number of ranges is chosen so that the units (tiles x ranges x
+// 36) fill one, two or three rounds of the grid as fully as possible, fewer rounds winning unless more
+// rounds fill at least 7 % better; a range keeps at least 12 k-steps.
 struct GradPlan {
   int tile_m, tile_n;   // block tile
   int tm, tn;           // tiles
   int kchunk;           // depth per range
+  int grid;             // persistent grid (128 x 128 tiles), else 0
 };
-constexpr int kNarrowBlocksPerCu = 3, kWideBlocksPerCu = 2;
+constexpr int kGradBlocksPerCu = 3;
 
 inline GradPlan plan_grad_gemm(int O, int C, int ld, int cus) {
   GradPlan g{};
+  const int slots = cus * kGradBlocksPerCu / 8 * 8;
   if (O <= 64 || C <= 64) {
-    const int slots = cus * kNarrowBlocksPerCu / 8 * 8;
     g.tile_m = O <= 64 ? 64 : 128;
     g.tile_n = (g.tile_m == 128 || C <= 64) ? 64 : 128;
     g.tm = (O + g.tile_m - 1) / g.tile_m;
@@ -505,9 +506,9 @@ inline GradPlan plan_grad_gemm(int O, int C, int ld, int cus) {
     int ranges = std::max(1, (slots + per / 2) / per);
     ranges = std::min(ranges, std::max(1, ld / 1024));
     g.kchunk = ((ld + ranges - 1) / ranges + 63) / 64 * 64;
+    g.grid = 0;
     return g;
   }
-  const int slots = cus * kWideBlocksPerCu / 8 * 8;
   g.tile_m = g.tile_n = 128;
   g.tm = (O + 127) / 128;
   g.tn = (C + 127) / 128;
@@ -525,22 +526,24 @@ inline GradPlan plan_grad_gemm(int O, int C, int ld, int cus) {
     }
   }
   g.kchunk = ((ld + best_ranges - 1) / best_ranges + BK - 1) / BK * BK;
+  g.grid = slots;
   return g;
 }
 
 // `here` ranges of p.kchunk cover p.ld; partial sum z = range * 36 + xi goes to p.out + z * rows * cols
-inline void launch_grad_gemm(const GradPlan &g, wg::GradProblem p, int here, hipStream_t st) {
+inline void launch_grad_gemm(const GradPlan &g, wg::GradProblem p, int here, hipStream_t st, bool split) {
   p.tm = g.tm;
   p.tn = g.tn;
   const int units = g.tm * g.tn * kXi * here;
-  const TileGrid tg{g.tm, g.tn, units};
-  if (g.tile_m == 128 && g.tile_n == 128) {
-    hipLaunchKernelGGL((st::gemm_both_kernel<4, 4, 2, 2, false, true>), dim3(grid_blocks(g.tm, g.tn, kXi * here)), dim3(gt::kThreads), 0, st,
-                       DenseParams{p.Y, p.ld, p.rows, p.ld}, DenseParams{p.V, p.ld, p.cols, p.ld}, p.out,
-                       gt::Strides{static_cast<int64_t>(p.rows) * p.ld, static_cast<int64_t>(p.cols) * p.ld, static_cast<int64_t>(p.rows) * p.cols}, kXi,
-                       p.cols % 4 == 0, p.rows, p.cols, p.ld, p.kchunk, tg);
+  if (g.grid > 0) {
+    const int grid = std::min(g.grid, (units + 7) / 8 * 8);
+    if (split)
+      hipLaunchKernelGGL((wg::wino_grad_gemm_split_kernel<kGradBlocksPerCu>), dim3(grid), dim3(kThreads), 0, st, p, units);
+    else
+      hipLaunchKernelGGL((wg::wino_grad_gemm_kernel<kGradBlocksPerCu>), dim3(grid), dim3(kThreads), 0, st, p, units);
     return;
   }
+  const TileGrid tg{g.tm, g.tn, units};
   const dim3 grid(grid_blocks(g.tm, g.tn, kXi * here));
   if (g.tile_m == 64 && g.tile_n == 64)
     hipLaunchKernelGGL((wg::wino_grad_gemm_narrow_kernel<64, 64>), grid, dim3(kThreads), 0, st, p, tg);
@@ -572,7 +575,7 @@ inline int run_images(int imgs, int per_img, int chans_a, int chans_b) {
 }  // namespace
 
 // Opt-in: the Winograd GEMMs of layers with more than 64 channels on both sides and the matrix products take
-// their products in split bf16 (split_tile.h, gemm_split.h).  -1 until asked: the environment variable
+// their products in split bf16 (wino_gemm_split.h, gemm_split.h).  -1 until asked: the environment variable
 // TSPLIT_SPLIT_BF16 then gives the first value.
 std::atomic<int> g_split_bf16{-1};
 bool split_bf16_enabled() {
@@ -588,9 +591,8 @@ bool split_bf16_enabled() {
 // Which layers take the one-kernel form: up to 256 channels on either side (in bands of 64 produced channels and
 // chunks of 16 gathered ones).  Measured per 16- or 64-image call against the three-kernel routine: 64 -> 64 at
 // 224 x 224 forward 467 -> 251 us, 128 -> 128 at 112 x 112 284 -> 232, 128 -> 256 at 56 x 56 486 -> 382, 256 -> 256
-// at 56 x 56 778 -> 708 (against the split products that the three-kernel routine takes now 680 and 610); beyond that its GEMM, which runs at
-// 190 TFLOP/s against 93 here, outweighs the transforms it pays for.
-// TSPLIT_WINOGRAD_FUSED=0 switches the form off, =2 lifts the limit.
+// at 56 x 56 778 -> 708; beyond that the three-kernel routine's GEMM, which runs at 120 TFLOP/s against 90 here,
+// outweighs the transforms it pays for.  TSPLIT_WINOGRAD_FUSED=0 switches the form off, =2 lifts the limit.
 namespace {
 // 0: not this layer; otherwise the value of TSPLIT_WINOGRAD_FUSED (1 unless set)
 inline int fused_form(int gathered, int produced) {
@@ -654,13 +656,7 @@ int conv_winograd_3x3(const float *x, const float *w, float *y, int imgs, int ga
   const int run = run_images(imgs, per_img, gathered, produced);
   TS_REQUIRE(run > 0, "conv (Winograd): one image's tiles do not fit 32-bit offsets");
   const int ld_max = (run * per_img + 3) / 4 * 4;
-  // The GEMMs of layers that produce more than 64 channels take bf16 products of the prepared filter (split_tile.h); for 64 and fewer they are
-  // bound by V and M and stay on the fp32 kernel.
-  const bool prepared = produced > 64;
-  const int steps = (gathered + st::BK - 1) / st::BK, row_tiles = (produced + 15) / 16;
-  const size_t u_bytes = static_cast<size_t>(kXi) * produced * gathered * 4, plane_bytes = static_cast<size_t>(row_tiles) * steps * st::kChunk;
-  float *U = static_cast<float *>(scratch_get(st, 3, u_bytes + (prepared ? kXi * plane_bytes : 0)));
-  char *planes = reinterpret_cast<char *>(U) + u_bytes;
+  float *U = static_cast<float *>(scratch_get(st, 3, static_cast<size_t>(kXi) * produced * gathered * 4));
   float *VM = static_cast<float *>(scratch_get(st, 2, static_cast<size_t>(kXi) * (gathered + produced) * ld_max * 4));
   TS_REQUIRE(U && VM, "conv (Winograd): no scratch memory");
   float *V = VM, *M = VM + static_cast<int64_t>(kXi) * gathered * ld_max;
@@ -691,21 +687,13 @@ int conv_winograd_3x3(const float *x, const float *w, float *y, int imgs, int ga
       // every operand read once, the result written once
       const double flop = 2.0 * kXi * produced * static_cast<double>(gi.ld) * gathered;
       const double bytes = 4.0 * kXi * (static_cast<double>(produced) * gathered + static_cast<double>(gathered + produced) * gi.ld);
-      if (prepared && first == 0)
-        hipLaunchKernelGGL(st::planes_kernel, dim3(row_tiles * steps, kXi), dim3(64), 0, st, st::dense_rows(U, gathered, 1, produced, gathered),
-                           static_cast<int64_t>(produced) * gathered, planes, FastDiv(steps));
-      const bool asked = prepared && (gathered & 7) == 0 && split_bf16_enabled();
-      GemmTiming timed(st, asked ? 3 : prepared ? 0 : 2, flop, bytes);
-      if (prepared) {
-        const int tm = (produced + 127) / 128, tn = (gi.ld + 127) / 128;
-        hipLaunchKernelGGL((st::gemm_split_kernel<4, 4, 2, 2, true, false>), dim3(grid_blocks(tm, tn, kXi)), dim3(gt::kThreads), 0, st,
-                           st::PlanesParams{planes, row_tiles, steps}, st::dense_rows(U, gathered, 1, produced, gathered), DenseParams{V, gi.ld, gi.ld, gathered},
-                           M, st::SplitStrides{static_cast<int64_t>(plane_bytes), static_cast<int64_t>(produced) * gathered,
-                           static_cast<int64_t>(gathered) * gi.ld, static_cast<int64_t>(produced) * gi.ld}, true, produced, gi.ld, gathered, gathered,
-                           TileGrid{tm, tn, tm * tn * kXi});
-      } else {
-        wg::launch(wg::Problem{U, V, M, produced, gathered, gi.ld, 0, 0}, st, compute_units());
-      }
+      const bool split = produced > 64 && (gathered & 7) == 0 && split_bf16_enabled();
+      GemmTiming timed(st, split ? 3 : produced <= 64 ? 2 : 0, flop, bytes);
+      const wg::Problem gemm{U, V, M, produced, gathered, gi.ld, 0, 0};
+      if (split)
+        wg::launch_split(gemm, st, compute_units());
+      else
+        wg::launch(gemm, st, compute_units());
     }
     const dim3 grid_out((go.tiles + 255) / 256, produced);
     float *yr = y + static_cast<int64_t>(first) * produced * H * W;
@@ -790,11 +778,11 @@ int conv_winograd_3x3_filter_grad(const float *x, const float *dy, float *dw, in
       hipLaunchKernelGGL((wino_grad_pair_kernel<false, false>), grid_xy, dim3(256), 0, st, xr, V, gx, dyr, Y, gy);
     const int here = (gx.ld + kchunk - 1) / kchunk;
     {
-      const bool asked = plan.tile_m == 128 && plan.tile_n == 128 && split_bf16_enabled();
-      GemmTiming timed(st, asked ? 4 : 1, 2.0 * kXi * O * static_cast<double>(gx.ld) * C,
+      const bool split = plan.grid > 0 && split_bf16_enabled();
+      GemmTiming timed(st, split ? 4 : 1, 2.0 * kXi * O * static_cast<double>(gx.ld) * C,
                        4.0 * kXi * (static_cast<double>(O) * C * here + static_cast<double>(O + C) * gx.ld));
       launch_grad_gemm(plan, wg::GradProblem{Y, V, part + static_cast<int64_t>(parts) * kXi * oc, O, C, gx.ld, kchunk, 0, 0},
-                       here, st);
+                       here, st, split);
     }
     parts += here;
   }

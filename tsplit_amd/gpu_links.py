@@ -440,8 +440,8 @@ def winograd_gemm_timing(on, kind=None):
 
 
 def split_bf16(on):
-    """Switches split-bf16 products on or off also where they are not the default (small matrix products; layers that take the one-kernel
-    Winograd form); returns the previous setting."""
+    """Switches the split-bf16 products of the Winograd routine's GEMMs on or off (off by default); returns
+    the previous setting."""
     was = ctypes.c_int()
     check_call(_LIB.TSplit_SplitBf16(int(bool(on)), ctypes.byref(was)))
     return bool(was.value)
@@ -450,8 +450,8 @@ def split_bf16(on):
 def winograd_gemm_times(filter_gradient=False, kind=None):
     """-> (launches, total ms, total executed FLOP, total algorithmic bytes) of the timed GEMM launches of
     kind 0 (forward / data gradient on 128 x 128 tiles), 1 (filter gradient), 2 (forward / data gradient
-    of layers that produce at most 64 channels, on 64 x 256 tiles), 3 / 4 (those of 0 / 1 while split_bf16 is
-    on), 5 (forward / data gradient as one kernel), 6 (filter gradient as
+    of layers that produce at most 64 channels, on 64 x 256 tiles), 3 / 4 (forward and data gradient /
+    filter gradient with split-bf16 products), 5 (forward / data gradient as one kernel), 6 (filter gradient as
     one kernel)."""
     which = int(bool(filter_gradient)) if kind is None else int(kind)
     n, ms, flop, nbytes = ctypes.c_double(), ctypes.c_double(), ctypes.c_double(), ctypes.c_double()

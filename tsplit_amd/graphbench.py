@@ -3,7 +3,8 @@ sizes of the reference's benchmark configurations, on one MI355X through the C A
 
     python -m tsplit_amd.graphbench --net resnet50|resnet101|inception_v4|transformer|lstm|mlp|vgg19 [--steps 5] [--warmup 2] [--record] [--split-bf16]
 
---split-bf16 takes split-bf16 products also where they are not the default (TSplit_SplitBf16).  --record issues the step once into a HIP graph after the warm-up and times replays of that graph
+--split-bf16 turns on the opt-in split-bf16 products of the matrix products and the Winograd GEMMs
+(TSplit_SplitBf16).  --record issues the step once into a HIP graph after the warm-up and times replays of that graph
 (one host call per step) instead of Python issuing every operator again.
 
 Prints one JSON object: samples/s, ms/step, final loss, operator calls per step, and - from a second pass
@@ -287,8 +288,8 @@ def layer_list(a, ctx):
     print(json.dumps({"net": a.net, "workload": desc, "samples_per_s": n * steps / dt,
                       "ms_per_step": dt / steps * 1e3, "steps": steps, "warmup": a.warmup, "final_loss": t.loss_value(),
                       "recorded": bool(a.record),
-                      "dtype": "f32 (products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)" if a.split_bf16 else "f32",
-                      "arithmetic": "the larger products as six bf16 x bf16 terms of exact operand splits, fp32 accumulation", "data": "synthetic"}))
+                      "dtype": "f32 (matrix products and Winograd GEMMs as six bf16 x bf16 terms of exact operand splits, fp32 accumulation)"
+                      if a.split_bf16 else "f32", "data": "synthetic"}))
 
 
 if __name__ == "__main__":

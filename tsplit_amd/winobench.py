@@ -7,9 +7,9 @@ Shapes are those of the benchmark step (batch 64; the 224x224 and 112x112 layers
 images).  A call is timed over `iters` back-to-back launches between two HIP events after two untimed
 ones; the GEMM inside a Winograd call by the library's own event pairs (TSplit_WinogradGemmTiming).
 "direct-equivalent" rates count the direct algorithm's FLOP, of which the routine executes a quarter;
-GEMM rates count executed FLOP (2 * 36 * rows * tiles * depth) against the 157.3 TFLOP/s fp32 matrix peak; GEMMs of layers with more than
-64 channels on both sides take their products as six bf16 x bf16 terms, and their rate is the fp32-equivalent one (the same FLOP count).
-With --split-bf16 (TSplit_SplitBf16) those layers never run as one kernel.
+GEMM rates count executed FLOP (2 * 36 * rows * tiles * depth) against the 157.3 TFLOP/s fp32 matrix peak.
+With --split-bf16 the GEMMs of layers with more than 64 channels on both sides take their products as six
+bf16 x bf16 terms (TSplit_SplitBf16); their rate is then the fp32-equivalent one (the same FLOP count).
 Layers with 64 channels on one side run forward and data gradient as one kernel (transforms inside): its "GEMM" time
 is the whole call's.
 Prints one JSON object per layer and pass and a final table.
@@ -87,7 +87,9 @@ def main():
             r["winograd_us"], r["direct_tflops_direct_equivalent"], r["winograd_tflops_direct_equivalent"], r["gemm_us"],
             r["gemm_tflops_executed"]))
     print("(* rate of the direct algorithm's FLOP count)")
-    print("(GEMMs of layers with more than 64 channels on both sides take split-bf16 products: GEMM TF is the fp32-equivalent rate)")
+    if a.split_bf16:
+        print("(split-bf16 products in the GEMMs of layers with more than 64 channels on both sides: GEMM TF is the "
+              "fp32-equivalent rate)")
 
 
 if __name__ == "__main__":
