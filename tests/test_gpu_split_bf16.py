@@ -3,8 +3,8 @@ through the C ABI.
 
 Bars: with the switch on, the three convolutions of wide 3x3 layers meet the float64 oracle within the
 convolution tolerance (2e-3 max relative error, and below 1e-4 as the fp32 path does), their error against
-the oracle is no larger than 1.5 times the fp32 path's on the same inputs (the six bf16 products leave out
-less than the rounding of an fp32 multiplication), layers the switch does not cover give the same bits as
+the oracle is no larger than 1.5 times the fp32 path's on the same inputs (dense ones, for which the split
+products' sums are rounded less often), layers the switch does not cover give the same bits as
 before, and a network with such layers still tracks the oracle's training run."""
 import numpy as np
 import pytest
