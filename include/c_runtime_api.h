@@ -14,6 +14,8 @@
  *  - a DLStreamHandle of NULL means the default stream; all operator calls are
  *    asynchronous on their stream unless a non-NULL ProfilerHandle is given, in
  *    which case the call blocks and fills the Profiler (time in ms, sizes in MiB);
+ *  - one host thread at a time calls on a stream: a call may be several launches that
+ *    hand data on in the stream's scratch memory (streams share none of it);
  *  - return 0 on success, -1 on failure (a message goes to stderr).
  */
 #ifndef TSPLIT_AMD_C_RUNTIME_API_H_

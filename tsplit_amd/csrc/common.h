@@ -88,7 +88,8 @@ inline float mib(int64_t elems) { return static_cast<float>(elems) * 4.0f / (102
 
 // Grow-only device scratch, one buffer per (stream, slot), kept until the process ends.
 // Kernels launched on one stream are ordered, so a buffer may be reused by the next op on
-// that stream without waiting; ops on different streams never share one.
+// that stream without waiting; ops on different streams never share one.  One host thread at a time
+// issues an op on a stream: its launches must not mix with another op's.
 void *scratch_get(hipStream_t stream, int slot, size_t bytes);
 
 // Forgets the table of arrays TSplit_OptimizerUpdateMulti keeps for a stream (elementwise.hip);
