@@ -477,6 +477,40 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
                                          DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                                          DLStreamHandle stream_handle, ProfilerHandle p);
 
+/* ---- Matrix products with the operators behind them in the same launch (outside the reference's ABI).
+ *      TSplit_MatrixMultiplyAdd: C = op(A) op(B), + bias[column] where given, + addend where given (an array of
+ *      C's size; it may be C), and, where given, relu = max(C, 0).  An array of more than two axes is taken as a matrix
+ *      of its last axis' columns.  Each step is rounded as the operators
+ *      DLGpuMatrixMultiply, DLGpuBroadcastTo + DLGpuMatrixElementwiseAdd and DLGpuRelu round it: the same bits.
+ *      TSplit_HeadsMatrixMultiply: for every n and head, C = alpha * op(A) op(B), + mask_value in the columns where
+ *      mask (of n x columns values) is 0, then `fill` in the columns right of the row where causal != 0, then
+ *      + addend (laid out as C, not C).  A, B and C are each [n, heads, rows, columns], or [n, rows, heads *
+ *      columns] with a head's columns side by side: heads are neither split off nor merged by a transpose.
+ *      The reference's graph spells these out node by node (examples/transformer.py:56-171). ---- */
+int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
+                             const DLArrayHandle bias, const DLArrayHandle addend, DLArrayHandle matC,
+                             DLArrayHandle relu, DLStreamHandle stream);
+int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
+                               DLArrayHandle matC, int heads, float alpha, const DLArrayHandle mask,
+                               float mask_value, int causal, float fill, const DLArrayHandle addend,
+                               DLStreamHandle stream);
+/* ---- Softmax cross-entropy with labels that are one class index a row (a float, as the reference's OneHot takes it),
+ *      smoothed: label[j] = on * (j == id) + off (outside the reference's ABI; examples/transformer.py:184-186 builds
+ *      the label array).  Otherwise DLGpuSoftmaxCrossEntropy and its gradient. ---- */
+int TSplit_SoftmaxCrossEntropyIds(const DLArrayHandle logits, const DLArrayHandle ids, float on, float off,
+                                  DLArrayHandle output, DLStreamHandle stream);
+int TSplit_SoftmaxCrossEntropyIds_Gradient(const DLArrayHandle logits, const DLArrayHandle ids, float on, float off,
+                                           const DLArrayHandle adjoint, DLArrayHandle output, DLStreamHandle stream);
+/* ---- output = scale * table[id] + (id != 0 ? positions : 0), positions of the output's size, and the table's gradient,
+ *      added to what table_grad holds where add_to != 0 (outside the reference's ABI; examples/transformer.py:189-232 node by node). ---- */
+int TSplit_EmbeddingAdd(const DLArrayHandle table, const DLArrayHandle ids, float scale, const DLArrayHandle positions,
+                        DLArrayHandle output, DLStreamHandle stream);
+int TSplit_EmbeddingAdd_Gradient(const DLArrayHandle output_grad, const DLArrayHandle ids, float scale, int add_to,
+                                 DLArrayHandle table_grad, DLStreamHandle stream);
+/* ---- A view of `input` under another shape of as many values (outside the reference's ABI): the new struct's data
+ *      pointer is input's, so it is released like a micro-tensor view (data set to NULL, then DLArrayFree). ---- */
+int TSplit_ArrayView(const DLArrayHandle input, const int64_t *shape, int ndim, DLArrayHandle *view);
+
 /* ---- Optimizer update of a whole model in one launch.  NO counterpart in the reference, whose
  *      optimizer issues one SGDOptimizerUpdate / MomentumOptimizerUpdate per parameter
  *      (python/athena/optimizer.py:95-176): dozens of launches, most of them on BatchNorm vectors

@@ -75,6 +75,37 @@ void launch_planned(const float *A, int64_t lda, int64_t sa, const float *B, int
   }
 }
 
+// the same tiles with something behind the products (S = 1)
+template <int TM, int TN, bool TA, bool TB>
+void launch_epilogue_tile(const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch, int M,
+                          int N, int K, const gt::Epilogue &ep, hipStream_t s) {
+  using T = gt::Tile<TM, TN, 2, 2, TA, TB>;
+  const int tm = (M + T::BM - 1) / T::BM, tn = (N + T::BN - 1) / T::BN;
+  const bool wide = N % 4 == 0 && ldc % 4 == 0 && zs.co % 4 == 0 && zs.ci % 4 == 0 && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu);
+  hipLaunchKernelGGL((gt::gemm_epilogue_kernel<TM, TN, TA, TB>), dim3(grid_blocks(tm, tn, batch)), dim3(gt::kThreads), 0, s, DenseParams{A, lda, M, K},
+                     DenseParams{B, ldb, N, K}, out, ldc, zs, ep, wide, M, N, K, TileGrid{tm, tn, tm * tn * batch});
+}
+
+template <bool TA, bool TB>
+void launch_epilogue(int tile, const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch,
+                     int M, int N, int K, const gt::Epilogue &ep, hipStream_t s) {
+  switch (tile) {
+    case 0: return launch_epilogue_tile<4, 4, TA, TB>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, s);
+    case 1: return launch_epilogue_tile<2, 4, TA, TB>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, s);
+    case 2: return launch_epilogue_tile<4, 2, TA, TB>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, s);
+    default: return launch_epilogue_tile<2, 2, TA, TB>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, s);
+  }
+}
+
+// the results of S ranges (or of one) summed, with what follows
+int launch_epilogue_fold(const float *part, float *out, int64_t mn, int N, int S, const gt::Epilogue &ep, hipStream_t s) {
+  if (N % 4 == 0 && aligned16(part) && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu))
+    hipLaunchKernelGGL(gt::fold_epilogue_kernel<4>, dim3(static_cast<unsigned>((mn / 4 + 255) / 256)), dim3(256), 0, s, part, out, mn, N, S, ep);
+  else
+    hipLaunchKernelGGL(gt::fold_epilogue_kernel<1>, dim3(static_cast<unsigned>((mn + 255) / 256)), dim3(256), 0, s, part, out, mn, N, S, ep);
+  return 0;
+}
+
 template <bool TA, bool TB>
 int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws_elems) {
   const Plan plan = plan_product(M, N, K, 1, true);
@@ -185,6 +216,32 @@ int dispatch_product(const float *A, int64_t lda, const float *B, int64_t ldb, f
   return launch_product<TA, TB>(A, lda, B, ldb, C, M, N, K, s, ws);
 }
 
+// A product with something behind it: on the tile kernel in one launch, or, where K is cut into ranges, in the launch that adds them up.
+// Operands that other kernels take (beyond 32-bit offsets, split-bf16) are multiplied there and the rest follows by a pass over the result.
+template <bool TA, bool TB>
+int dispatch_epilogue(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, const gt::Epilogue &ep, hipStream_t s) {
+  const int64_t mn = static_cast<int64_t>(M) * N;
+  if (near<TA, TB>(lda, ldb, M, N, K) && rows_reach(N) && !(split_bf16_enabled() && K % 4 == 0 && K >= BK)) {
+    const Plan plan = plan_product(M, N, K, 1, true);
+    if (plan.S == 1) {
+      launch_epilogue<TA, TB>(plan.tile, A, lda, B, ldb, C, N, gt::BatchOf{1, 0, 0, 0, 0, 0, 0}, 1, M, N, K, ep, s);
+      return 0;
+    }
+    float *part = static_cast<float *>(scratch_get(s, 2, static_cast<size_t>(plan.S) * mn * 4));
+    TS_REQUIRE(part, "TSplit_MatrixMultiplyAdd: no scratch memory for split-K");
+    launch_planned<TA, TB>(A, lda, 0, B, ldb, 0, part, mn, 1, M, N, K, plan, s);
+    return launch_epilogue_fold(part, C, mn, N, plan.S, ep, s);
+  }
+  int64_t ws = 0;
+  float *product = C;
+  if (ep.add == C) {   // read by the pass behind the product
+    product = static_cast<float *>(scratch_get(s, 3, static_cast<size_t>(mn) * 4));
+    TS_REQUIRE(product, "TSplit_MatrixMultiplyAdd: no scratch memory for the product");
+  }
+  if (const int rc = dispatch_product<TA, TB>(A, lda, B, ldb, product, M, N, K, s, &ws)) return rc;
+  return launch_epilogue_fold(product, C, mn, N, 1, ep, s);
+}
+
 template <bool TA, bool TB>
 int dispatch_batched(const float *A, int64_t lda, int64_t sa, const float *B, int64_t ldb, int64_t sb, float *C,
                      int batch, int M, int N, int K, hipStream_t s) {
@@ -200,10 +257,113 @@ int dispatch_batched(const float *A, int64_t lda, int64_t sa, const float *B, in
   return 0;
 }
 
+// an array as a matrix of its last axis' columns
+void rows_by_cols(const DLArray *a, int64_t &rows, int64_t &cols) {
+  rows = 1;
+  for (int d = 0; d + 1 < a->ndim; ++d) rows *= a->shape[d];
+  cols = a->shape[a->ndim - 1];
+}
+
+// One operand or result of a product over heads: [n, heads, rows, cols], or [n, rows, heads * cols] with a head's columns side by side
+struct HeadArray {
+  float *p;
+  int64_t n, rows, cols, ld, outer, inner;
+};
+bool head_array(const DLArray *a, int heads, HeadArray &h) {
+  const int64_t *s = a->shape;
+  if (a->ndim == 4 && s[1] == heads)
+    h = {static_cast<float *>(a->data), s[0], s[2], s[3], s[3], s[1] * s[2] * s[3], s[2] * s[3]};
+  else if (a->ndim == 3 && s[2] % heads == 0)
+    h = {static_cast<float *>(a->data), s[0], s[1], s[2] / heads, s[2], s[1] * s[2], s[2] / heads};
+  else
+    return false;
+  return true;
+}
+
+template <bool TA, bool TB>
+int dispatch_heads(const HeadArray &a, const HeadArray &b, const HeadArray &c, int heads, int M, int N, int K, const gt::Epilogue &ep, hipStream_t s) {
+  TS_REQUIRE((near<TA, TB>(a.ld, b.ld, M, N, K) && 65ll * 4 * c.ld < (1ll << 31)),
+             "TSplit_HeadsMatrixMultiply: a matrix reaches beyond 32-bit byte offsets");
+  const int batch = static_cast<int>(c.n) * heads;
+  const Plan plan = plan_product(M, N, K, batch, false);
+  launch_epilogue<TA, TB>(plan.tile, a.p, a.ld, b.p, b.ld, c.p, c.ld, gt::BatchOf{heads, a.outer, a.inner, b.outer, b.inner, c.outer, c.inner}, batch,
+                          M, N, K, ep, s);
+  return 0;
+}
+
 }  // namespace
 }  // namespace tsplit
 
 using namespace tsplit;
+
+extern "C" int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
+                                        const DLArrayHandle bias, const DLArrayHandle addend, DLArrayHandle matC, DLArrayHandle relu,
+                                        DLStreamHandle stream_handle) {
+  const char *who = "TSplit_MatrixMultiplyAdd";
+  TS_REQUIRE(matA && matB && matC, "%s: NULL array", who);
+  TS_REQUIRE(matA->ndim >= 2 && matB->ndim >= 2 && matC->ndim >= 2, "%s: arrays of two axes or more only", who);
+  int64_t a_rows, lda, b_rows, ldb, M, N;
+  rows_by_cols(matA, a_rows, lda);
+  rows_by_cols(matB, b_rows, ldb);
+  rows_by_cols(matC, M, N);
+  const int64_t K = transposeA ? a_rows : lda;
+  TS_REQUIRE((transposeA ? lda : a_rows) == M && (transposeB ? b_rows : ldb) == N && (transposeB ? ldb : b_rows) == K, "%s: shapes do not conform",
+             who);
+  TS_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) - 64, "%s: dimension too large", who);
+  TS_REQUIRE(!bias || numel(bias) == N, "%s: the bias has %lld values for %lld columns", who, (long long)(bias ? numel(bias) : 0), (long long)N);
+  TS_REQUIRE(!addend || numel(addend) == M * N, "%s: the addend is of the result's size", who);
+  TS_REQUIRE(!relu || (numel(relu) == M * N && relu->data != matC->data), "%s: Relu's result is another array of the result's size", who);
+  hipStream_t s = stream_of(stream_handle);
+  ProfileScope ps(nullptr, s, 0, 0, 0);
+  int rc = 0;
+  if (M > 0 && N > 0) {
+    const float *A = static_cast<const float *>(matA->data), *B = static_cast<const float *>(matB->data);
+    float *C = static_cast<float *>(matC->data);
+    const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+    const gt::Epilogue ep{1.f, bias ? static_cast<const float *>(bias->data) : nullptr, nullptr, 0.f, 0, 0.f,
+                          addend ? static_cast<const float *>(addend->data) : nullptr, relu ? static_cast<float *>(relu->data) : nullptr};
+    if (!transposeA && !transposeB) rc = dispatch_epilogue<false, false>(A, lda, B, ldb, C, m, n, k, ep, s);
+    if (!transposeA && transposeB) rc = dispatch_epilogue<false, true>(A, lda, B, ldb, C, m, n, k, ep, s);
+    if (transposeA && !transposeB) rc = dispatch_epilogue<true, false>(A, lda, B, ldb, C, m, n, k, ep, s);
+    if (transposeA && transposeB) rc = dispatch_epilogue<true, true>(A, lda, B, ldb, C, m, n, k, ep, s);
+  }
+  if (rc) return rc;
+  return ps.finish();
+}
+
+extern "C" int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB, DLArrayHandle matC,
+                                          int heads, float alpha, const DLArrayHandle mask, float mask_value, int causal, float fill,
+                                          const DLArrayHandle addend, DLStreamHandle stream_handle) {
+  const char *who = "TSplit_HeadsMatrixMultiply";
+  TS_REQUIRE(matA && matB && matC, "%s: NULL array", who);
+  HeadArray a, b, c;
+  TS_REQUIRE(heads > 0 && head_array(matA, heads, a) && head_array(matB, heads, b) && head_array(matC, heads, c),
+             "%s: arrays are [n, heads, rows, columns] or [n, rows, heads * columns]", who);
+  const int64_t M = c.rows, N = c.cols, K = transposeA ? a.rows : a.cols;
+  TS_REQUIRE(a.n == c.n && b.n == c.n && (transposeA ? a.cols : a.rows) == M && (transposeB ? b.rows : b.cols) == N &&
+                 (transposeB ? b.cols : b.rows) == K,
+             "%s: shapes do not conform", who);
+  TS_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) - 64, "%s: dimension too large", who);
+  TS_REQUIRE((M + 63) / 64 * ((N + 63) / 64) < (1ll << 31) / heads && c.n <= ((1ll << 31) - 9) / heads / ((M + 63) / 64 * ((N + 63) / 64) + 1),
+             "%s: too many tiles", who);
+  TS_REQUIRE(!mask || numel(mask) == c.n * N, "%s: the mask has a value for every column of every n", who);
+  TS_REQUIRE(!addend || (addend->ndim == matC->ndim && numel(addend) == numel(matC) && addend->data != matC->data),
+             "%s: the addend is another array of the result's layout", who);
+  hipStream_t s = stream_of(stream_handle);
+  ProfileScope ps(nullptr, s, 0, 0, 0);
+  int rc = 0;
+  if (M > 0 && N > 0 && c.n > 0) {
+    const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+    const gt::Epilogue ep{alpha, nullptr, mask ? static_cast<const float *>(mask->data) : nullptr, mask_value, causal, fill,
+                          addend ? static_cast<const float *>(addend->data) : nullptr, nullptr};
+    if (!transposeA && !transposeB) rc = dispatch_heads<false, false>(a, b, c, heads, m, n, k, ep, s);
+    if (!transposeA && transposeB) rc = dispatch_heads<false, true>(a, b, c, heads, m, n, k, ep, s);
+    if (transposeA && !transposeB) rc = dispatch_heads<true, false>(a, b, c, heads, m, n, k, ep, s);
+    if (transposeA && transposeB) rc = dispatch_heads<true, true>(a, b, c, heads, m, n, k, ep, s);
+  }
+  if (rc) return rc;
+  return ps.finish();
+}
 
 extern "C" int DLGpuMatrixMultiply(const DLArrayHandle matA, bool transposeA, const DLArrayHandle matB,
                                    bool transposeB, DLArrayHandle matC, DLStreamHandle stream_handle,

@@ -80,7 +80,8 @@ struct KContig {
     lane = threadIdx.x & 63;
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rows_left = P.mn_total - mn0;
-    rsrc = raw_buffer(P.p + static_cast<int64_t>(mn0) * P.ld, static_cast<int64_t>(rows_left) * P.ld * 4);
+    // (rows that are part of longer ones end with their own last value)
+    rsrc = raw_buffer(P.p + static_cast<int64_t>(mn0) * P.ld, (static_cast<int64_t>(rows_left - 1) * P.ld + P.k_total) * 4);
     const int slot0 = wave * kLoads * 8 + (lane >> 3);
     const unsigned row_bytes = static_cast<unsigned>(P.ld) * 4u;
     if constexpr (PERM) {
@@ -152,7 +153,7 @@ struct MnContig {
     const int lane = threadIdx.x & 63;
     wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     row_bytes = static_cast<int>(P.ld) * 4;
-    rsrc = raw_buffer(P.p, static_cast<int64_t>(P.k_total) * P.ld * 4);
+    rsrc = raw_buffer(P.p, (static_cast<int64_t>(P.k_total - 1) * P.ld + P.mn_total) * 4);
     const int col = mn0 + 4 * (lane % kWords);
     voff = col < P.mn_total ? (static_cast<unsigned>(lane / kWords) * static_cast<unsigned>(P.ld) + static_cast<unsigned>(col)) * 4u : kOobOffset;
   }
@@ -314,6 +315,143 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(mg::DenseParams 
   bp.p += z * zs.b;
   const int kbegin = kchunk < K ? z * kchunk : 0;
   T::run(ap, bp, out + z * zs.c, N, wide, M, N, tile_m * T::BM, tile_n * T::BN, kbegin, min(K, kbegin + kchunk), lds);
+}
+
+// ---- products whose result is worked on before it is stored
+// What follows the sum of products, in this order and with a rounding each, as the operators behind a product would do it:
+// v = alpha * sum; + bias[column]; + mask_value where mask[column] is 0; fill where the column lies right of the row; + add; stored, and
+// max(v, 0) stored as well.  Each of these as an operator of its own reads and writes the whole result again: scores of 32 x 8 x 256 x
+// 256 (67 MB) took 29 us as a product and 175 with a scale, a mask and a causal selection behind it, a projection of 8192 x 512 over 512
+// 36 and 64 us with its bias and a residual.
+struct Epilogue {
+  float alpha;
+  const float *bias;     // of N; null: none
+  const float *mask;     // of N, for the outer batch index; null: none
+  float mask_value;
+  int causal;
+  float fill;
+  const float *add;      // laid out as the result, which it may be (a lane reads a value before it writes it); null: none
+  float *relu;           // likewise; null: not stored
+  __device__ __forceinline__ float at(float v, int m, int n, float b, bool masked) const {
+    v *= alpha;
+    if (bias) v += b;
+    if (mask) v += masked ? mask_value : 0.f;
+    if (causal && n > m) v = fill;
+    return v;
+  }
+};
+// Batch z is (z / inner, z % inner); an operand's matrices lie `o` apart by the first index and `i` by the second (heads that share the rows
+// of one array lie a head's width apart).
+struct BatchOf {
+  int inner;
+  int64_t ao, ai, bo, bi, co, ci;
+};
+
+template <int TM, int TN, bool TA, bool TB>
+__global__ __launch_bounds__(kThreads, 2) void gemm_epilogue_kernel(mg::DenseParams ap, mg::DenseParams bp, float *out, int64_t ldc,
+                                                                    BatchOf zs, Epilogue ep, bool wide, int M, int N, int K, mg::TileGrid tg) {
+  using T = Tile<TM, TN, 2, 2, TA, TB>;
+  using C = typename T::C;
+  __shared__ __attribute__((aligned(1024))) float lds[C::kLdsFloats];
+  int z, tile_m, tile_n;
+  if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
+  const int zo = z / zs.inner, zi = z - zo * zs.inner;
+  ap.p += zo * zs.ao + zi * zs.ai;
+  bp.p += zo * zs.bo + zi * zs.bi;
+  const int64_t c_at = zo * zs.co + zi * zs.ci;
+  const int m0 = tile_m * T::BM, n0 = tile_n * T::BN;
+  typename T::AL la;
+  typename T::BL lb;
+  la.init(ap, m0);
+  lb.init(bp, n0);
+  f32x4 acc[TM][TN];
+  C::run(la, lb, 0, K, lds, acc);
+  const int m = m0 + C::wave_m0(), n = n0 + C::wave_n0() + TN * (threadIdx.x & 15);
+  if (m >= M) return;
+  // rows past the last one are out of range; a row's columns past N go nowhere
+  const int64_t from = c_at + static_cast<int64_t>(m) * ldc, bytes = (static_cast<int64_t>(M - m - 1) * ldc + N) * 4;
+  const __amdgpu_buffer_rsrc_t to = output_buffer(out + from, bytes);
+  const __amdgpu_buffer_rsrc_t add = output_buffer(const_cast<float *>(ep.add ? ep.add + from : out + from), bytes);
+  const __amdgpu_buffer_rsrc_t relu = output_buffer(ep.relu ? ep.relu + from : out + from, bytes);
+  const int row_bytes = static_cast<int>(ldc) * 4, row0 = m + C::lane_row();
+  const unsigned at = (static_cast<unsigned>(C::lane_row()) * static_cast<unsigned>(ldc) + static_cast<unsigned>(n)) * 4u;
+  unsigned off[TN];
+  float b[TN];
+  bool masked[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    off[j] = n + j < N ? at + 4u * j : kOobOffset;
+    b[j] = ep.bias && n + j < N ? ep.bias[n + j] : 0.f;
+    masked[j] = ep.mask && n + j < N && ep.mask[static_cast<int64_t>(zo) * N + n + j] == 0.f;
+  }
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int step = C::step_row(tm, e), soff = step * row_bytes;
+      float v[TN];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) v[j] = ep.at(acc[tm][j][e], row0 + step, n + j, b[j], masked[j]);
+      if (wide) {   // N and ldc are multiples of 4: a word lies inside its row or behind it
+        if (ep.add) {
+          if constexpr (TN == 4) {
+            const mg::u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(add, off[0] + soff, 0, 0);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) v[j] += __uint_as_float(r[j]);
+          } else {
+            const u32x2 r = __builtin_amdgcn_raw_buffer_load_b64(add, off[0] + soff, 0, 0);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) v[j] += __uint_as_float(r[j]);
+          }
+        }
+        store_words<TN>(to, off[0], soff, v);
+        if (ep.relu) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) v[j] = fmaxf(v[j], 0.f);
+          store_words<TN>(relu, off[0], soff, v);
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          if (ep.add) v[j] += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(add, off[j] + soff, 0, 0));
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), to, off[j] + soff, 0, 0);
+          if (ep.relu) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(fmaxf(v[j], 0.f)), relu, off[j] + soff, 0, 0);
+        }
+      }
+    }
+}
+
+// out[i] = what follows the sum over the S ranges' results (a bias, an addend, Relu's second result), VEC values a thread
+template <int VEC>
+static __global__ __launch_bounds__(256) void fold_epilogue_kernel(const float *part, float *out, int64_t n, int N, int S,
+                                                                   Epilogue ep) {
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * VEC;
+  if (i >= n) return;
+  typedef float vec __attribute__((ext_vector_type(VEC)));
+  auto read = [](const float *p) { return *reinterpret_cast<const vec *>(p); };
+  vec s = read(part + i);
+  int z = 1;
+  for (; z + 4 <= S; z += 4) {
+    const vec a = read(part + z * n + i), b = read(part + (z + 1) * n + i), c = read(part + (z + 2) * n + i), d = read(part + (z + 3) * n + i);
+    s += a;
+    s += b;
+    s += c;
+    s += d;
+  }
+  for (; z < S; ++z) s += read(part + z * n + i);
+  s *= ep.alpha;
+  const int col = static_cast<int>(i % N);
+  if (ep.bias) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) s[j] += ep.bias[col + j];
+  }
+  if (ep.add) s += read(ep.add + i);
+  *reinterpret_cast<vec *>(out + i) = s;
+  if (ep.relu) {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) s[j] = fmaxf(s[j], 0.f);
+    *reinterpret_cast<vec *>(ep.relu + i) = s;
+  }
 }
 
 // out[i] = sum_z part[z * n + i], z ascending, four values a thread (n a multiple of 4)

@@ -693,4 +693,18 @@ int DLArraySliceForMicroTensor(DLArrayHandle input, DLArrayHandle *output, int t
   return 0;
 }
 
+int TSplit_ArrayView(const DLArrayHandle input, const int64_t *shape, int ndim, DLArrayHandle *view) {
+  TS_REQUIRE(input && shape && view && ndim >= 1, "TSplit_ArrayView: bad argument");
+  int64_t n = 1;
+  for (int i = 0; i < ndim; ++i) {
+    TS_REQUIRE(shape[i] >= 0, "TSplit_ArrayView: negative dimension");
+    n *= shape[i];
+  }
+  TS_REQUIRE(n == numel(input), "TSplit_ArrayView: %lld values seen as %lld", (long long)numel(input), (long long)n);
+  DLArray *v = new_array(shape, ndim, input->ctx);
+  v->data = input->data;
+  *view = v;
+  return 0;
+}
+
 }  // extern "C"

@@ -27,7 +27,8 @@ __all__ = [
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
     "batch_norm_relu", "batch_norm_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
-    "optimizer_update_multi",
+    "optimizer_update_multi", "matrix_multiply_add", "heads_matrix_multiply",
+    "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "CuDNN_Dropout", "CuDNN_Dropout_gradient", "CuSparse_Csrmv", "CuSparse_Csrmm",
 ]
 
@@ -88,6 +89,22 @@ def matrix_multiply(matA, transA, matB, transB, matC, stream=None, profiler=None
                                         ctypes.c_bool(bool(transB)), _h(matC), _s(stream), _p(profiler)))
 
 
+def matrix_multiply_add(matA, transA, matB, transB, matC, bias=None, addend=None, relu=None, stream=None):
+    """matC = op(matA) op(matB) + bias + addend, relu = max(matC, 0), each where given: the bits of matrix_multiply,
+    broadcast_to and matrix_elementwise_add, and relu (no counterpart in the reference's gpu_links)."""
+    check_call(_LIB.TSplit_MatrixMultiplyAdd(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(bias) if bias else None,
+                                             _h(addend) if addend else None, _h(matC), _h(relu) if relu else None, _s(stream)))
+
+
+def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0,
+                          addend=None, stream=None):
+    """For every sample and head matC = alpha * op(matA) op(matB), + mask_value in columns where mask is 0, `fill` right of the
+    diagonal with `causal`, + addend.  Arrays are [n, heads, rows, columns] or [n, rows, heads * columns]."""
+    check_call(_LIB.TSplit_HeadsMatrixMultiply(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(matC), int(heads),
+                                               ctypes.c_float(alpha), _h(mask) if mask else None, ctypes.c_float(mask_value),
+                                               int(bool(causal)), ctypes.c_float(fill), _h(addend) if addend else None, _s(stream)))
+
+
 # ---- Softmax / CE (gpu_links/SoftmaxLink.py, SoftmaxCrossEntropyLink.py:8,17) ----
 def softmax(in_arr, out_arr, stream=None, profiler=None):
     check_call(_LIB.DLGpuSoftmax(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
@@ -106,6 +123,25 @@ def softmax_cross_entropy_no_alloc(in_arr_a, in_arr_b, out_arr, stream=None):
 def softmax_cross_entropy_gradient(in_arr_a, in_arr_b, in_arr_c, out_arr, stream=None, profiler=None):
     check_call(_LIB.DLGpuSoftmaxCrossEntropy_Gradient(_h(in_arr_a), _h(in_arr_b), _h(in_arr_c), _h(out_arr),
                                                       _s(stream), _p(profiler)))
+
+
+def softmax_cross_entropy_ids(logits, ids, on, off, out_arr, stream=None):
+    """softmax_cross_entropy with labels on * one_hot(ids) + off that are never written."""
+    check_call(_LIB.TSplit_SoftmaxCrossEntropyIds(_h(logits), _h(ids), ctypes.c_float(on), ctypes.c_float(off), _h(out_arr), _s(stream)))
+
+
+def softmax_cross_entropy_ids_gradient(logits, ids, on, off, adjoint, out_arr, stream=None):
+    check_call(_LIB.TSplit_SoftmaxCrossEntropyIds_Gradient(_h(logits), _h(ids), ctypes.c_float(on), ctypes.c_float(off), _h(adjoint),
+                                                           _h(out_arr), _s(stream)))
+
+
+def embedding_add(table, ids, scale, positions, out_arr, stream=None):
+    """scale * table[id] + (id != 0 ? positions : 0)."""
+    check_call(_LIB.TSplit_EmbeddingAdd(_h(table), _h(ids), ctypes.c_float(scale), _h(positions), _h(out_arr), _s(stream)))
+
+
+def embedding_add_gradient(out_grad, ids, scale, table_grad, add_to=False, stream=None):
+    check_call(_LIB.TSplit_EmbeddingAdd_Gradient(_h(out_grad), _h(ids), ctypes.c_float(scale), int(bool(add_to)), _h(table_grad), _s(stream)))
 
 
 # ---- Conv2d (gpu_links/CudnnConv2d.py:8,21,33; gpu_links/Conv2dLink.py:8,24,35) ----

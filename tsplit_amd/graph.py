@@ -20,11 +20,12 @@ from . import ndarray
 class Var(object):
     """A value on the tape: backend array, shape, accumulated gradient; `node` is the index of the
     operator call that produced it on its tape (-1 for parameters, inputs and constants)."""
-    __slots__ = ["value", "shape", "grad", "needs_grad", "name", "node"]
+    __slots__ = ["value", "shape", "grad", "needs_grad", "name", "node", "own"]
 
     def __init__(self, value, shape, needs_grad, name=None):
         self.value, self.shape, self.grad, self.needs_grad, self.name = value, tuple(shape), None, needs_grad, name
         self.node = -1
+        self.own = False     # during a reverse sweep: `grad` is an array of this value alone, so more may be added in place
 
 
 class Node(object):
@@ -37,6 +38,17 @@ class Node(object):
         # for operators that are cheap to run again (one to three passes over HBM): a closure that
         # computes the output once more from the inputs' current values, with the same bits
         self.redo = redo
+
+
+class _Shape(object):
+    """Stands for a value on a backend that computes nothing: the operand's shape."""
+
+    def __init__(self, shape):
+        self.shape = shape
+
+
+def _shaped(value, shape):
+    return _Shape(shape) if value is None else value
 
 
 SELF = object()      # in a `saved` list: the operator's own output
@@ -87,6 +99,10 @@ class GpuBackend(object):
         self.L.array_reshape(x, out, self.stream)
         return out
 
+    def view(self, x, shape):
+        """x under another shape, without a copy."""
+        return ndarray.view(x, shape)
+
     # ---- contractions
     def conv2d(self, x, w, xs, ws, ph, pw, s):
         y = self.empty((xs[0], ws[0], conv_out(xs[2], ws[2], ph, s), conv_out(xs[3], ws[3], pw, s)))
@@ -111,6 +127,20 @@ class GpuBackend(object):
     def batch_matmul(self, a, ta, b, tb, out_shape):
         c = self.empty(out_shape)
         self.L.batch_matrix_multiply(a, ta, b, tb, c, self.stream)
+        return c
+
+    def matmul_add(self, a, ta, b, tb, out_shape, bias=None, addend=None, relu=False, out=None):
+        """-> (op(a) op(b) + bias + addend, its Relu or None) in one call; arrays of more axes are matrices of the last one's columns.
+        out: the array to write (it may be the addend), or None for a new one."""
+        c = self.empty(out_shape) if out is None else out
+        r = self.empty(out_shape) if relu else None
+        self.L.matrix_multiply_add(a, ta, b, tb, c, bias, addend, r, self.stream)
+        return c, r
+
+    def heads_matmul(self, a, ta, b, tb, out_shape, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0, addend=None):
+        """Products per sample and head (gpu_links.heads_matrix_multiply)."""
+        c = self.empty(out_shape)
+        self.L.heads_matrix_multiply(a, ta, b, tb, c, heads, alpha, mask, mask_value, causal, fill, addend, self.stream)
         return c
 
     # ---- normalisation, activations, pooling
@@ -170,6 +200,10 @@ class GpuBackend(object):
         c = self.empty(shape)
         self.L.matrix_elementwise_add(a, b, c, self.stream)
         return c
+
+    def add_to(self, a, b):
+        """a += b."""
+        self.L.matrix_elementwise_add(a, b, a, self.stream)
 
     def mul_const(self, a, c, shape):
         out = self.empty(shape)
@@ -261,6 +295,17 @@ class GpuBackend(object):
         self.L.embedding_lookup_gradient(dy, ids, g, self.stream)
         return g
 
+    def embedding_add(self, table, ids, scale, positions, out_shape):
+        out = self.empty(out_shape)
+        self.L.embedding_add(table, ids, scale, positions, out, self.stream)
+        return out
+
+    def embedding_add_grad(self, dy, ids, scale, table_shape, add_to=None):
+        """The gradient of the table, or that added to the array `add_to`."""
+        g = self.empty(table_shape) if add_to is None else add_to
+        self.L.embedding_add_gradient(dy, ids, scale, g, add_to is not None, self.stream)
+        return g
+
     def zeros(self, shape):
         out = self.empty(shape)
         self.L.array_set(out, 0.0, self.stream)
@@ -277,6 +322,18 @@ class GpuBackend(object):
         self.L.array_set(one, float(seed), self.stream)
         g = self.empty(shape)
         self.L.softmax_cross_entropy_gradient(logits, labels, one, g, self.stream)
+        return g
+
+    def softmax_ce_ids(self, logits, ids, on, off):
+        loss = self.empty((1,))
+        self.L.softmax_cross_entropy_ids(logits, ids, on, off, loss, self.stream)
+        return loss
+
+    def softmax_ce_ids_grad(self, logits, ids, on, off, shape, seed=1.0):
+        one = self.empty((1,))
+        self.L.array_set(one, float(seed), self.stream)
+        g = self.empty(shape)
+        self.L.softmax_cross_entropy_ids_gradient(logits, ids, on, off, one, g, self.stream)
         return g
 
     def sgd(self, p, g, lr):
@@ -305,6 +362,11 @@ class Tape(object):
     def __init__(self, backend):
         self.b = backend
         self._nodes = []     # every operator call, in order (Node)
+        self._readers = []   # per operator call: how many inputs of later calls its output is
+        self._ready = {}     # operator call -> the Relu of its output, where its launch has left that too
+        self._leaves = []    # leaves whose gradient arrays are this sweep's
+        self._scores = {}    # head_scores call -> (scale, causal)
+        self._scaled = set() # head_scores calls whose gradient has arrived with scale and selection applied
         self._log = None     # with a list here, every operator call is appended as (name, args, kwargs)
 
     def _call(self, fn, args, kwargs):
@@ -328,6 +390,10 @@ class Tape(object):
         node = Node(v, backward if v.needs_grad else None, inputs, saved if v.needs_grad else (), len(self._nodes), redo)
         v.node = node.index
         self._nodes.append(node)
+        self._readers.append(0)
+        for i in inputs:
+            if i.node >= 0:
+                self._readers[i.node] += 1
         self._after_forward(node)
         return v
 
@@ -341,10 +407,91 @@ class Tape(object):
     def _after_backward(self, node):
         pass
 
-    def _acc(self, var, g):
+    def _acc(self, var, g, fresh=False):
+        """Adds g to var's gradient.  fresh: g is an array that nothing else holds."""
         if not var.needs_grad:
             return
-        var.grad = g if var.grad is None else self.b.add(var.grad, g, var.shape)
+        if var.grad is None:
+            var.grad = g
+            self._owns(var, fresh)
+        elif var.own:
+            self.b.add_to(var.grad, g)
+        else:
+            var.grad = self.b.add(var.grad, g, var.shape)
+            self._owns(var, True)
+
+    def _owns(self, var, fresh):
+        var.own = fresh and self._can("add_to")
+        if var.own and var.node < 0:
+            self._leaves.append(var)      # a leaf's gradient is the caller's once the sweep ends
+
+    # ---- products with something behind them: one call where the backend has it, else the operators one by one
+    def _can(self, name):
+        return hasattr(type(self.b), name)
+
+    def _seen_as(self, value, shape):
+        """An operator's output (or a gradient) under another shape: a view where the backend has views."""
+        return (self.b.view if self._can("view") else self.b.reshape)(value, shape)
+
+    def _product(self, a, a_shape, ta, b, b_shape, tb, out_shape, bias=None, addend=None, relu=False):
+        """-> (op(a) op(b) + bias + addend, its Relu or None); arrays of more than two axes are matrices of the last one's columns."""
+        if self._can("matmul_add"):
+            return self.b.matmul_add(a, ta, b, tb, out_shape, bias, addend, relu)
+        flat = [_shaped(self.b.reshape(v, sh) if v is not None and sh != whole else v, sh)
+                for v, whole, sh in ((v, sh, (_prod(sh[:-1]), sh[-1])) for v, sh in ((a, a_shape), (b, b_shape)))]
+        rows = (_prod(out_shape[:-1]), out_shape[-1])
+        y = self.b.matmul(flat[0], ta, flat[1], tb, rows)
+        if bias is not None:
+            y = self.b.add(y, self.b.broadcast_to(bias, rows), rows)
+        if len(out_shape) > 2:
+            y = self.b.reshape(y, out_shape)
+        if addend is not None:
+            y = self.b.add(y, addend, out_shape)
+        return y, self.b.relu(y, out_shape) if relu else None
+
+    def _acc_product(self, var, a, a_shape, ta, b, b_shape, tb):
+        """Adds op(a) op(b) to var's gradient."""
+        if not var.needs_grad:
+            return
+        if var.own:
+            self.b.matmul_add(a, ta, b, tb, var.shape, addend=var.grad, out=var.grad)
+        else:
+            var.grad = self._product(a, a_shape, ta, b, b_shape, tb, var.shape, addend=var.grad)[0]
+            self._owns(var, True)
+
+    def _heads_product(self, a, a_shape, ta, b, b_shape, tb, out_shape, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False,
+                       fill=0.0, addend=None):
+        """For every sample and head alpha * op(a) op(b), + mask_value where mask (a value a column) is 0, `fill` right of the
+        diagonal with causal, + addend.  A shape of three axes holds the heads' columns side by side in its rows."""
+        # (a matrix one launch cannot address goes the long way: 2^31 bytes, and 128 rows of it)
+        reach = all(_prod(sh[1:]) < (1 << 29) and sh[-1] < (1 << 22) for sh in (a_shape, b_shape, out_shape))
+        if self._can("heads_matmul") and reach:
+            return self.b.heads_matmul(a, ta, b, tb, out_shape, heads, alpha, mask, mask_value, causal, fill, addend)
+
+        def split(v, sh):
+            if len(sh) == 4:
+                return v, sh
+            v = self.b.reshape(v, (sh[0], sh[1], heads, sh[2] // heads))
+            sh = (sh[0], heads, sh[1], sh[2] // heads)
+            return self.b.transpose(v, [0, 2, 1, 3], sh), sh
+
+        def side(v, sh):
+            return _shaped(*split(v, sh))
+        n = out_shape[0]
+        four = out_shape if len(out_shape) == 4 else (n, heads, out_shape[1], out_shape[2] // heads)
+        y = self.b.batch_matmul(side(a, a_shape), ta, side(b, b_shape), tb, four)
+        if alpha != 1.0:
+            y = self.b.mul_const(y, alpha, four)
+        if mask is not None:
+            cols = (n, four[3])
+            m = self.b.where(mask, self.b.zeros(cols), self.b.add_const(self.b.zeros(cols), mask_value, cols), cols)
+            y = self.b.add(y, self.b.broadcast_shape(self.b.reshape(m, (n, 1, 1, four[3])), four), four)
+        if causal:
+            tril = self.b.broadcast_shape(self.b.from_numpy(np.tril(np.ones(four[2:], np.float32))), four)
+            y = self.b.where(tril, y, self.b.add_const(self.b.zeros(four), fill, four), four)
+        if len(out_shape) == 3:
+            y = self.b.reshape(self.b.transpose(y, [0, 2, 1, 3], (n, four[2], heads, four[3])), out_shape)
+        return y if addend is None else self.b.add(y, addend, out_shape)
 
     # ---- operators (reference gradient rules cited)
     @_op
@@ -355,9 +502,9 @@ class Tape(object):
 
         def back(g):
             if w.needs_grad:
-                self._acc(w, self.b.conv2d_grad_filter(x.value, g, w.shape, ph, pw, stride))
+                self._acc(w, self.b.conv2d_grad_filter(x.value, g, w.shape, ph, pw, stride), fresh=True)
             if x.needs_grad:
-                self._acc(x, self.b.conv2d_grad_data(w.value, g, x.shape, ph, pw, stride))
+                self._acc(x, self.b.conv2d_grad_data(w.value, g, x.shape, ph, pw, stride), fresh=True)
         return self._out(y, ys, [x, w], back, saved=[x, w])
 
     @_op
@@ -406,7 +553,8 @@ class Tape(object):
         """gpu_ops/Relu.py:51,117."""
         def fwd():
             return self.b.relu(x.value, x.shape)
-        return self._out(fwd(), x.shape, [x], lambda g: self._acc(x, self.b.relu_grad(x.value, g, x.shape)), redo=fwd)
+        y = self._ready.pop(x.node, None)
+        return self._out(fwd() if y is None else y, x.shape, [x], lambda g: self._acc(x, self.b.relu_grad(x.value, g, x.shape)), redo=fwd)
 
     @_op
     def max_pool(self, x, k, pad, stride):
@@ -504,15 +652,17 @@ class Tape(object):
 
     @_op
     def reshape(self, a, shape):
-        """gpu_ops/Reshape.py:42 (compute: a copy), :61 (gradient: reshaped back)."""
+        """gpu_ops/Reshape.py:42 (compute: a copy there), :61 (gradient: reshaped back)."""
         shape = list(shape)
         if -1 in shape:
             known = _prod([s for s in shape if s != -1])
             shape[shape.index(-1)] = _prod(a.shape) // known
         shape = tuple(shape)
+        # operators' outputs and gradients are written once, so another shape of one is a view of it; parameters and inputs are
+        # the caller's to write again, so they are copied
         def fwd():
-            return self.b.reshape(a.value, shape)
-        return self._out(fwd(), shape, [a], lambda g: self._acc(a, self.b.reshape(g, a.shape)), saved=[], redo=fwd)
+            return self._seen_as(a.value, shape) if a.node >= 0 else self.b.reshape(a.value, shape)
+        return self._out(fwd(), shape, [a], lambda g: self._acc(a, self._seen_as(g, a.shape)), saved=[], redo=fwd)
 
     @_op
     def concat(self, a, b, axis):
@@ -539,19 +689,95 @@ class Tape(object):
         y = self.b.matmul(a.value, trans_a, b.value, trans_b, (m, n))
 
         def back(g):
-            if a.needs_grad:
-                if not trans_a:
-                    ga = self.b.matmul(g, False, b.value, not trans_b, a.shape)
-                else:
-                    ga = self.b.matmul(b.value, trans_b, g, True, a.shape)
-                self._acc(a, ga)
-            if b.needs_grad:
-                if not trans_b:
-                    gb = self.b.matmul(a.value, not trans_a, g, False, b.shape)
-                else:
-                    gb = self.b.matmul(g, True, a.value, trans_a, b.shape)
-                self._acc(b, gb)
+            gs = (m, n)
+            if not trans_a:
+                self._acc_product(a, g, gs, False, b.value, b.shape, not trans_b)
+            else:
+                self._acc_product(a, b.value, b.shape, trans_b, g, gs, True)
+            if not trans_b:
+                self._acc_product(b, a.value, a.shape, not trans_a, g, gs, False)
+            else:
+                self._acc_product(b, g, gs, True, a.value, a.shape, trans_a)
         return self._out(y, (m, n), [a, b], back)
+
+    # whether a launch may leave a later operator's output as well (not on a tape that accounts for every value where it is made)
+    _ahead = True
+
+    @_op
+    def dense(self, x, w, bias=None, residual=None, relu_follows=False):
+        """x [..., fan_in] w [fan_in, fan_out] + bias + residual as one node; the reference's graph has MatrixMult, Broadcast and
+        AddElewise nodes (examples/transformer.py:56-69, :174-181).  relu_follows: relu() of the output comes next, and the launch may
+        leave that too."""
+        ys = tuple(x.shape[:-1]) + (w.shape[1],)
+        relu = relu_follows and self._ahead and self._can("matmul_add")
+        y, r = self._product(x.value, x.shape, False, w.value, w.shape, False, ys, bias.value if bias is not None else None,
+                             residual.value if residual is not None else None, relu)
+
+        def back(g):
+            if residual is not None:
+                self._acc(residual, g)
+            self._acc_product(w, x.value, x.shape, True, g, ys, False)
+            if bias is not None and bias.needs_grad:
+                rows = self._seen_as(g, (_prod(ys[:-1]), ys[-1])) if len(ys) > 2 else g
+                self._acc(bias, self.b.reduce_sum_axis_zero(rows, bias.shape), fresh=True)
+            self._acc_product(x, g, ys, False, w.value, w.shape, True)
+        out = self._out(y, ys, [v for v in (x, w, bias, residual) if v is not None], back, saved=[x, w])
+        if r is not None:
+            self._ready[out.node] = r
+        return out
+
+    @_op
+    def head_scores(self, q, k, heads, scale, mask_ids=None, mask_value=0.0, causal=False):
+        """Attention scores [N, heads, tq, tk] of projections [N, t, heads * dh] whose heads lie side by side: scale * q k', mask_value
+        added in the columns of padding (ids of 0), mask_value in place of what lies in the future.  The reference's graph spells
+        this out (examples/transformer.py:93-160: reshape, transpose, BatchMatrixMultiply, MultiplyConst, Where, Broadcast, Add)."""
+        n, tq, tk = q.shape[0], q.shape[1], k.shape[1]
+        ys = (n, heads, tq, tk)
+        y = self._heads_product(q.value, q.shape, False, k.value, k.shape, True, ys, heads, scale,
+                                mask_ids.value if mask_ids is not None else None, mask_value, causal, mask_value)
+        out = None
+
+        def back(g):
+            if out.node in self._scaled:
+                self._scaled.discard(out.node)
+            else:
+                if causal:
+                    tril = self.b.broadcast_shape(self.b.from_numpy(np.tril(np.ones((tq, tk), np.float32))), ys)
+                    g = self.b.where(tril, g, self.b.zeros(ys), ys)
+                g = self.b.mul_const(g, scale, ys)
+            for var, ta, other in ((q, False, k), (k, True, q)):
+                if var.needs_grad:
+                    var.grad = self._heads_product(g, ys, ta, other.value, other.shape, False, var.shape, heads, addend=var.grad)
+                    self._owns(var, True)
+        out = self._out(y, ys, [v for v in (q, k, mask_ids) if v is not None], back, saved=[q, k])
+        if out.node >= 0:
+            self._scores[out.node] = (scale, causal)
+        return out
+
+    @_op
+    def head_context(self, scores, v, heads, residual=None):
+        """scores [N, heads, tq, tk] times v [N, tk, heads * dh], the heads side by side again: [N, tq, heads * dh], + residual
+        (examples/transformer.py:161-171)."""
+        ys = (v.shape[0], scores.shape[2], v.shape[2])
+        y = self._heads_product(scores.value, scores.shape, False, v.value, v.shape, False, ys, heads,
+                                addend=residual.value if residual is not None else None)
+
+        def back(g):
+            if residual is not None:
+                self._acc(residual, g)
+            if v.needs_grad:
+                v.grad = self._heads_product(scores.value, scores.shape, True, g, ys, False, v.shape, heads, addend=v.grad)
+                self._owns(v, True)
+            if scores.needs_grad:
+                # scores that go nowhere else take their scale and their selection behind this product
+                alone = scores.node in self._scores and self._readers[scores.node] == 1 and scores.grad is None
+                scale, causal = self._scores[scores.node] if alone else (1.0, False)
+                scores.grad = self._heads_product(g, ys, False, v.value, v.shape, True, scores.shape, heads, scale, causal=causal,
+                                                  addend=scores.grad)
+                self._owns(scores, True)
+                if alone:
+                    self._scaled.add(scores.node)
+        return self._out(y, ys, [u for u in (scores, v, residual) if u is not None], back, saved=[scores, v])
 
     @_op
     def batch_matmul(self, a, b, trans_a=False, trans_b=False):
@@ -651,21 +877,57 @@ class Tape(object):
                          saved=[ids])
 
     @_op
-    def softmax_ce(self, logits, labels, weight=1.0):
+    def embedding_add(self, table, ids, scale, positions):
+        """scale * table[id] + positions, those left out where the id is 0 (examples/transformer.py:189-232 node by node)."""
+        ys = tuple(ids.shape) + (table.shape[1],)
+        fused = self._can("embedding_add")
+        if fused:
+            y = self.b.embedding_add(table.value, ids.value, scale, positions.value, ys)
+        else:
+            cond = self.b.broadcast_shape(self.b.reshape(ids.value, tuple(ids.shape) + (1,)), ys)
+            y = self.b.add(self.b.mul_const(self.b.embedding(table.value, ids.value, ys), scale, ys),
+                           self.b.where(cond, positions.value, self.b.zeros(ys), ys), ys)
+
+        def back(g):
+            if fused and table.own:
+                self.b.embedding_add_grad(g, ids.value, scale, table.shape, table.grad)
+            elif fused:
+                self._acc(table, self.b.embedding_add_grad(g, ids.value, scale, table.shape), fresh=True)
+            else:
+                self._acc(table, self.b.embedding_grad(self.b.mul_const(g, scale, ys), ids.value, table.shape))
+        return self._out(y, ys, [table, ids, positions], back, saved=[ids])
+
+    @_op
+    def softmax_ce(self, logits, labels, weight=1.0, smoothing=None):
         """gpu_ops/SoftmaxCrossEntropy.py:46-67 (compute), :73 and :134-135 (gradient) with an adjoint of one.
         `weight` scales the loss and, through the gradient operator's adjoint argument, its gradient: the
-        share of a batch micro-tensor in the mean over the whole batch."""
+        share of a batch micro-tensor in the mean over the whole batch.  With `smoothing` the labels are one class
+        index a row (smoothed_softmax_ce)."""
         assert len(logits.shape) == 2
-        loss = self.b.softmax_ce(logits.value, labels.value)
+        if smoothing is None:
+            forward, gradient, lab = self.b.softmax_ce, self.b.softmax_ce_grad, lambda: (labels.value,)
+        else:
+            on, off = 1.0 - smoothing, smoothing / logits.shape[1]
+            forward, gradient, lab = self.b.softmax_ce_ids, self.b.softmax_ce_ids_grad, lambda: (labels.value, on, off)
+        loss = forward(logits.value, *lab())
         if weight != 1.0:
             loss = self.b.mul_const(loss, weight, (1,))
 
         def back(g):
             if weight != 1.0:
-                self._acc(logits, self.b.softmax_ce_grad(logits.value, labels.value, logits.shape, weight))
+                self._acc(logits, gradient(logits.value, *lab(), logits.shape, weight))
             else:
-                self._acc(logits, self.b.softmax_ce_grad(logits.value, labels.value, logits.shape))
+                self._acc(logits, gradient(logits.value, *lab(), logits.shape))
         return self._out(loss, (1,), [logits, labels], back, saved=[logits, labels])
+
+    def smoothed_softmax_ce(self, logits, ids, smoothing):
+        """The loss for labels (1 - smoothing) * one-hot(ids) + smoothing / classes (examples/transformer.py:184-186).  The label
+        array is written, by the reference's three nodes, only where a planner accounts for it or the backend has no other loss."""
+        if self._ahead and self._can("softmax_ce_ids"):
+            return self.softmax_ce(logits, ids, smoothing=smoothing)
+        classes = logits.shape[1]
+        labels = self.shift(self.scale(self.one_hot(ids, classes), 1.0 - smoothing), smoothing / classes)
+        return self.softmax_ce(logits, labels)
 
     # ---- reverse sweep
     def backward(self, loss):
@@ -679,9 +941,17 @@ class Tape(object):
             if node.back is not None and v.grad is not None:
                 node.back(v.grad)
                 if v is not loss:
-                    v.grad = None      # interior gradients are dropped as soon as they are consumed
+                    v.grad, v.own = None, False      # interior gradients are dropped as soon as they are consumed
             self._after_backward(node)
-        self._nodes = []
+        self._release_leaves()
+        self._nodes, self._readers = [], []
+        self._ready, self._scores, self._scaled = {}, {}, set()
+
+
+    def _release_leaves(self):
+        for v in self._leaves:
+            v.own = False
+        self._leaves = []
 
 
 # ---------------------------------------------------------------- batch micro-tensors on the tape
@@ -715,6 +985,8 @@ class _PieceTape(Tape):
     t; `drop_after_backward[j]`: values whose last backward reader is operator j) and tells its owner after
     every operator."""
 
+    _ahead = False
+
     def __init__(self, backend, owner, drop_after_forward=None, drop_after_backward=None):
         Tape.__init__(self, backend)
         self._owner = owner
@@ -729,6 +1001,9 @@ class _PieceTape(Tape):
         for m in self._drop_b.get(node.index, ()):
             self._nodes[m].out.value = None
         self._owner._inside_piece()
+
+    def _release_leaves(self):
+        pass                 # the next piece adds to the same arrays
 
 
 def _last_readers(nodes):
@@ -774,6 +1049,8 @@ class MicroTape(Tape):
     On the outer tape the stretch is ONE operator whose output is the loss and whose backward
     operators have already run.  Nothing in the stretch may couple the samples of a batch
     (COUPLES_SAMPLES); the batch must divide by `pieces`."""
+
+    _ahead = False
 
     def __init__(self, backend, split_from=None, pieces=1, piece_calls=None, total_calls=None):
         Tape.__init__(self, backend)
@@ -857,7 +1134,9 @@ class MicroTape(Tape):
                         outside[id(actual)] = [actual, follows, None]
                         outside_vars.append(actual)
                     value = b.piece(actual.value, k, i) if follows else actual.value
-                    wrapped[id(actual)] = Var(value, traced.shape, actual.needs_grad, actual.name)
+                    wrapped[id(actual)] = w = Var(value, traced.shape, actual.needs_grad, actual.name)
+                    if not follows:
+                        w.grad, w.own = actual.grad, actual.own      # a parameter's pieces add to one array
                 return wrapped[id(actual)]
 
             for n, (name, args, kwargs, _) in enumerate(self._put_off):
@@ -881,7 +1160,8 @@ class MicroTape(Tape):
                         whole = outside[key][2] = b.empty(actual.shape)
                     b.assign(b.piece(whole, k, i), w.grad)
                 else:
-                    self._acc(actual, w.grad)           # a parameter: summed over the pieces
+                    actual.grad = w.grad                # a parameter: summed over the pieces
+                    self._owns(actual, w.own)
                 w.grad = None
             del piece_tape, env, wrapped, piece_loss
         for v in outside_vars:

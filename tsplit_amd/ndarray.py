@@ -312,6 +312,14 @@ def slice_for_micro_tensor(input_tensor, index, total_number, dimension="batch")
     return NDArray(h, auto_deleted=False, owner=input_tensor, is_view=True)
 
 
+def view(array, shape):
+    """`array` under another shape of as many values: no copy, the view keeps the array alive."""
+    cshape = c_array(ctypes.c_int64, tuple(int(s) for s in shape))
+    h = DLArrayHandle()
+    check_call(_LIB.TSplit_ArrayView(array.handle, cshape, ctypes.c_int(len(cshape)), ctypes.byref(h)))
+    return NDArray(h, auto_deleted=False, owner=array, is_view=True)
+
+
 def split_shape(input_shape, total_number=0, dimension="batch"):
     assert total_number > 0
     d = 0 if dimension == "batch" else 1

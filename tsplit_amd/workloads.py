@@ -239,57 +239,32 @@ class TransformerConfig(object):
         self.pos_amplitude = pos_amplitude
 
 
-def _dense(t, b, x, fan_in, fan_out, relu=False):
+def _dense(t, b, x, fan_in, fan_out, relu=False, residual=None):
     """examples/transformer.py:56-69."""
     name = b.unique("dense")
-    y = t.matmul(x, b.get(name + "_weight", (fan_in, fan_out), np.sqrt(1.0 / fan_in)))
-    y = t.add_bias(y, b.get(name + "_bias", (fan_out,), "zero"))
+    w = b.get(name + "_weight", (fan_in, fan_out), np.sqrt(1.0 / fan_in))
+    y = t.dense(x, w, b.get(name + "_bias", (fan_out,), "zero"), residual, relu)
     return t.relu(y) if relu else y
-
-
-def _const_full(t, b, value, shape):
-    one = b.constant(("scalar", float(value)), lambda: np.full((1,), value, np.float32))
-    return t.broadcast_like(one, shape)
 
 
 def _attention(t, b, cfg, queries, keys, values, mask_ids, causal):
     """examples/transformer.py:93-171: projections, head split, scaled scores, padding mask
     added, causal mask selected, scores x values (no softmax), head merge, residual."""
-    N, h, d = cfg.batch, cfg.heads, cfg.d_model
-    dh = d // h
-    tq, tk = queries.shape[1], keys.shape[1]
-
-    def heads(x2d, length):
-        return t.transpose(t.reshape(x2d, (N, length, h, dh)), (0, 2, 1, 3))
-
-    q = heads(_dense(t, b, t.reshape(queries, (-1, d)), d, d), tq)
-    k = heads(_dense(t, b, t.reshape(keys, (-1, d)), d, d), tk)
-    v = heads(_dense(t, b, t.reshape(values, (-1, d)), d, d), tk)
-    scores = t.scale(t.batch_matmul(q, k, trans_b=True), 1.0 / np.sqrt(float(dh)))     # [N,h,tq,tk]
-    if mask_ids is not None:
-        zeros = _const_full(t, b, 0.0, mask_ids.shape)
-        adder = _const_full(t, b, cfg.mask_value, mask_ids.shape)
-        m = t.where(mask_ids, zeros, adder)                                             # [N,tk]
-        m = t.reshape(m, (N, 1, 1, tk))
-        scores = t.add(scores, t.broadcast_like(m, scores.shape))
-    if causal:
-        tril = b.constant(("tril", tq, tk), lambda: np.tril(np.ones((tq, tk), np.float32)))
-        future = t.broadcast_like(tril, scores.shape)
-        scores = t.where(future, scores, _const_full(t, b, cfg.mask_value, scores.shape))
-    ctx = t.batch_matmul(scores, v)                                                     # [N,h,tq,dh]
-    out = t.reshape(t.transpose(ctx, (0, 2, 1, 3)), (N, tq, d))
-    return t.add(out, queries)
+    d, dh = cfg.d_model, cfg.d_model // cfg.heads
+    q = _dense(t, b, queries, d, d)
+    k = _dense(t, b, keys, d, d)
+    v = _dense(t, b, values, d, d)
+    scores = t.head_scores(q, k, cfg.heads, 1.0 / np.sqrt(float(dh)), mask_ids, cfg.mask_value, causal)     # [N,h,tq,tk]
+    return t.head_context(scores, v, cfg.heads, queries)                                                    # [N,tq,d]
 
 
 def _ffn(t, b, cfg, x):
     """examples/transformer.py:174-181."""
-    y = _dense(t, b, t.reshape(x, (-1, cfg.d_model)), cfg.d_model, cfg.d_ff, relu=True)
-    y = _dense(t, b, y, cfg.d_ff, cfg.d_model)
-    return t.add(t.reshape(y, x.shape), x)
+    return _dense(t, b, _dense(t, b, x, cfg.d_model, cfg.d_ff, relu=True), cfg.d_ff, cfg.d_model, residual=x)
 
 
 def _positions(t, b, ids, length, d, amplitude):
-    """examples/transformer.py:189-212: sinusoids, zeroed where the token id is 0."""
+    """examples/transformer.py:189-212: sinusoids (left out where the token id is 0 when they are added)."""
     n = ids.shape[0]
 
     def table():
@@ -297,10 +272,7 @@ def _positions(t, b, ids, length, d, amplitude):
         pos[:, 0::2] = np.sin(pos[:, 0::2])
         pos[:, 1::2] = np.cos(pos[:, 1::2])
         return np.tile((amplitude * pos[None]).astype(np.float32), (n, 1, 1))
-    enc = b.constant(("pos", n, length, d, float(amplitude)), table)
-    zeros = b.constant(("zeros", n, length, d), lambda: np.zeros((n, length, d), np.float32))
-    cond = t.broadcast_like(t.reshape(ids, (n, length, 1)), (n, length, d))
-    return t.where(cond, enc, zeros)
+    return b.constant(("pos", n, length, d, float(amplitude)), table)
 
 
 def transformer(t, b, cfg, xs, ys_in, ys_out):
@@ -312,8 +284,7 @@ def transformer(t, b, cfg, xs, ys_in, ys_out):
     table = b.get("embedding_table", (cfg.vocab, d), cfg.embed_std)
 
     def embed(ids, length):
-        e = t.scale(t.embedding(table, ids), d ** 0.5)
-        return t.add(e, _positions(t, b, ids, length, d, cfg.pos_amplitude))
+        return t.embedding_add(table, ids, d ** 0.5, _positions(t, b, ids, length, d, cfg.pos_amplitude))
 
     enc = embed(xs, cfg.len1)
     for _ in range(cfg.blocks):
@@ -324,9 +295,7 @@ def transformer(t, b, cfg, xs, ys_in, ys_out):
         dec = _attention(t, b, cfg, dec, enc, enc, xs, False)
         dec = _ffn(t, b, cfg, dec)
     logits = t.matmul(t.reshape(dec, (-1, d)), table, trans_b=True)                      # [N*len2, vocab]
-    onehot = t.one_hot(t.reshape(ys_out, (-1,)), cfg.vocab)
-    labels = t.shift(t.scale(onehot, 1.0 - cfg.smoothing), cfg.smoothing / cfg.vocab)   # :184-186
-    return t.softmax_ce(logits, labels), logits
+    return t.smoothed_softmax_ce(logits, t.reshape(ys_out, (-1,)), cfg.smoothing), logits
 
 
 # ------------------------------------------------------------------ LSTM
