@@ -501,6 +501,20 @@ int TSplit_SoftmaxCrossEntropyIds(const DLArrayHandle logits, const DLArrayHandl
                                   DLArrayHandle output, DLStreamHandle stream);
 int TSplit_SoftmaxCrossEntropyIds_Gradient(const DLArrayHandle logits, const DLArrayHandle ids, float on, float off,
                                            const DLArrayHandle adjoint, DLArrayHandle output, DLStreamHandle stream);
+/* ---- A sequence of LSTM cells (outside the reference's ABI; examples/LSTM.py:21-90 node by node).  x [n, steps * frame]; params:
+ *      W [frame, units], U [units, units] and b [units] of the forget, input, output and candidate gates in turn; `initial`: the one
+ *      value that h and c start from; last [n, units]: h after the last step.  With depth and units_padded of TSplit_LstmSizes,
+ *      rows [n, steps, depth], packed [4 * units_padded * (depth + units_padded)], gates [n, steps, 4, units_padded] and cells
+ *      [n, steps, units] are what the gradient reads again, all on 16 bytes.  The gradient writes all twelve parameters' gradients
+ *      into dparams, in the order of params; dgates is scratch of the size of gates. ---- */
+int TSplit_LstmSizes(int frame, int units, int *depth, int *units_padded);
+int TSplit_Lstm(const DLArrayHandle x, const DLArrayHandle *params, const DLArrayHandle initial, int steps,
+                DLArrayHandle rows, DLArrayHandle packed, DLArrayHandle gates, DLArrayHandle cells, DLArrayHandle last,
+                DLStreamHandle stream);
+int TSplit_LstmGradient(const DLArrayHandle dlast, const DLArrayHandle x, const DLArrayHandle *params,
+                        const DLArrayHandle initial, int steps, const DLArrayHandle rows, const DLArrayHandle packed,
+                        const DLArrayHandle gates, const DLArrayHandle cells, DLArrayHandle dgates,
+                        DLArrayHandle *dparams, DLStreamHandle stream);
 /* ---- output = scale * table[id] + (id != 0 ? positions : 0), positions of the output's size, and the table's gradient,
  *      added to what table_grad holds where add_to != 0 (outside the reference's ABI; examples/transformer.py:189-232 node by node). ---- */
 int TSplit_EmbeddingAdd(const DLArrayHandle table, const DLArrayHandle ids, float scale, const DLArrayHandle positions,

@@ -13,6 +13,7 @@
 #include <mutex>
 #include <vector>
 
+#include "activations.h"
 #include "common.h"
 
 namespace tsplit {
@@ -180,11 +181,11 @@ struct RsqrtOp {  // correctly rounded quotient rather than the approximate rsqr
 };
 struct TanhOp {
   static constexpr int N = 2, LOAD = 2, STORE = 1;
-  __device__ void apply(float (&v)[2]) const { v[0] = tanhf(v[1]); }
+  __device__ void apply(float (&v)[2]) const { v[0] = tanh_of(v[1]); }
 };
-struct SigmoidOp {   // 1/(1+1/exp(x)) (src/ops/Sigmoid.cu:6); saturates to 0 and 1 without NaN
+struct SigmoidOp {
   static constexpr int N = 2, LOAD = 2, STORE = 1;
-  __device__ void apply(float (&v)[2]) const { v[0] = 1.f / (1.f + expf(-v[1])); }
+  __device__ void apply(float (&v)[2]) const { v[0] = sigmoid_of(v[1]); }
 };
 struct WhereOp {     // out = cond != 0 ? a : b ; arrays: out, cond, a, b
   static constexpr int N = 4, LOAD = 14, STORE = 1;

@@ -8,7 +8,7 @@ here (the reference's wrappers ignore them).
 import ctypes
 
 from . import ndarray as _nd
-from ._base import _LIB, check_call
+from ._base import _LIB, c_array, check_call
 
 __all__ = [
     "array_set", "matrix_elementwise_add", "matrix_elementwise_add_by_const",
@@ -29,6 +29,7 @@ __all__ = [
     "batch_norm_relu", "batch_norm_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
     "optimizer_update_multi", "matrix_multiply_add", "heads_matrix_multiply",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
+    "lstm_sizes", "lstm", "lstm_gradient",
     "CuDNN_Dropout", "CuDNN_Dropout_gradient", "CuSparse_Csrmv", "CuSparse_Csrmm",
 ]
 
@@ -103,6 +104,29 @@ def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, ma
     check_call(_LIB.TSplit_HeadsMatrixMultiply(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(matC), int(heads),
                                                ctypes.c_float(alpha), _h(mask) if mask else None, ctypes.c_float(mask_value),
                                                int(bool(causal)), ctypes.c_float(fill), _h(addend) if addend else None, _s(stream)))
+
+
+def lstm_sizes(frame, units):
+    """-> (depth, units_padded) of the arrays lstm() leaves for its gradient."""
+    depth, padded = ctypes.c_int(), ctypes.c_int()
+    check_call(_LIB.TSplit_LstmSizes(int(frame), int(units), ctypes.byref(depth), ctypes.byref(padded)))
+    return depth.value, padded.value
+
+
+def _handles(arrays):
+    return c_array(_nd.DLArrayHandle, [_h(a) for a in arrays])
+
+
+def lstm(x, params, initial, steps, rows, packed, gates, cells, last, stream=None):
+    """A sequence of LSTM cells; params: W, U, b of the forget, input, output and candidate gates (no counterpart in the reference's
+    gpu_links; sizes of the arrays it leaves: include/c_runtime_api.h)."""
+    check_call(_LIB.TSplit_Lstm(_h(x), _handles(params), _h(initial), int(steps), _h(rows), _h(packed), _h(gates), _h(cells), _h(last), _s(stream)))
+
+
+def lstm_gradient(dlast, x, params, initial, steps, rows, packed, gates, cells, dgates, dparams, stream=None):
+    """The gradients of lstm()'s twelve parameters from that of its last state."""
+    check_call(_LIB.TSplit_LstmGradient(_h(dlast), _h(x), _handles(params), _h(initial), int(steps), _h(rows), _h(packed), _h(gates), _h(cells),
+                                        _h(dgates), _handles(dparams), _s(stream)))
 
 
 # ---- Softmax / CE (gpu_links/SoftmaxLink.py, SoftmaxCrossEntropyLink.py:8,17) ----

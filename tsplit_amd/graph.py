@@ -306,6 +306,21 @@ class GpuBackend(object):
         self.L.embedding_add_gradient(dy, ids, scale, g, add_to is not None, self.stream)
         return g
 
+    def lstm(self, x, params, initial, steps):
+        """-> (last state [n, units], what lstm_grad reads again)."""
+        n, units = x.shape[0], params[1].shape[0]
+        depth, padded = self.L.lstm_sizes(x.shape[1] // steps, units)
+        saved = [self.empty(s) for s in ((n, steps, depth), (4 * padded * (depth + padded),), (n, steps, 4, padded), (n, steps, units))]
+        last = self.empty((n, units))
+        self.L.lstm(x, params, initial, steps, *saved, last, self.stream)
+        return last, saved
+
+    def lstm_grad(self, dlast, x, params, initial, steps, saved):
+        """-> the gradients of `params`."""
+        grads = [self.empty(p.shape) for p in params]
+        self.L.lstm_gradient(dlast, x, params, initial, steps, *saved, self.empty(saved[2].shape), grads, self.stream)
+        return grads
+
     def zeros(self, shape):
         out = self.empty(shape)
         self.L.array_set(out, 0.0, self.stream)
@@ -778,6 +793,25 @@ class Tape(object):
                 if alone:
                     self._scaled.add(scores.node)
         return self._out(y, ys, [u for u in (scores, v, residual) if u is not None], back, saved=[scores, v])
+
+    def takes_cells(self, x, initial, steps, units):
+        """Whether lstm_cells() is there for these operands: the data get no gradient, every value of x is a frame's, and the sizes
+        are those TSplit_Lstm addresses."""
+        return (self._ahead and self._can("lstm") and not x.needs_grad and not initial.needs_grad and initial.shape == (1,)
+                and len(x.shape) == 2 and 0 < x.shape[0] < 1 << 20 and x.shape[1] % steps == 0 and x.shape[1] // steps < 1 << 24
+                and x.shape[0] * steps < (1 << 31) - 64 and units < 1 << 20 and (x.shape[0] // 16 + 1) * (units // 16 + 1) < 1 << 30)
+
+    @_op
+    def lstm_cells(self, x, params, initial, steps):
+        """The last hidden state of `steps` LSTM cells on the frames of x, from a state of one value everywhere; params: W, U and b of
+        the forget, input, output and candidate gates.  The reference's graph spells out every cell (examples/LSTM.py:52-84)."""
+        values = [p.value for p in params]
+        y, saved = self.b.lstm(x.value, values, initial.value, steps)
+
+        def back(g):
+            for p, gp in zip(params, self.b.lstm_grad(g, x.value, values, initial.value, steps, saved)):
+                self._acc(p, gp, fresh=True)
+        return self._out(y, (x.shape[0], params[1].shape[0]), [x] + list(params) + [initial], back)
 
     @_op
     def batch_matmul(self, a, b, trans_a=False, trans_b=False):

@@ -320,8 +320,11 @@ def lstm(t, b, x, labels, dim_input=28, dim_hidden=128, classes=10, steps=28, st
         z = t.add(z, t.broadcast_like(bias, z.shape))
         return act(z)
 
+    at_once = x.shape[1] == steps * dim_input and t.takes_cells(x, initial, steps, dim_hidden)
     c = h = None
-    for i in range(steps):
+    if at_once:
+        h = t.lstm_cells(x, [v for g in gates.values() for v in g], initial, steps)
+    for i in range(0 if at_once else steps):
         frame = t.slice(x, (0, i * dim_input), (-1, dim_input))
         if i == 0:
             c = t.broadcast_like(initial, (n, dim_hidden))
@@ -332,8 +335,7 @@ def lstm(t, b, x, labels, dim_input=28, dim_hidden=128, classes=10, steps=28, st
         cand = gate("tanh", frame, h, t.tanh)
         c = t.add(t.mul(c, f), t.mul(ig, cand))
         h = t.mul(t.tanh(c), o)
-    logits = t.matmul(h, out_w)
-    logits = t.add(logits, t.broadcast_like(out_b, logits.shape))
+    logits = t.dense(h, out_w, out_b)
     return t.softmax_ce(logits, labels), logits
 
 
