@@ -1,5 +1,5 @@
 """The sequence of LSTM cells in one call (TSplit_Lstm, TSplit_LstmGradient) against the cells operator by operator in float64:
-sizes around the 16 x 16 tiles, one step, one unit, frames of one value.  Bound: a gradient is a sum of n * steps terms, each
+sizes around the 16 x 16 tiles and the 64 and 128 units whose weights stay in registers, one step, one unit, frames of one value.  Bound: a gradient is a sum of n * steps terms, each
 behind at most `steps` cells whose gates are sums of h + d + 1 products; every sum of m terms in fp32 is within
 m 2^-24 of its terms' magnitudes, and random signs leave about its square root: 2e-6 of the largest value leaves a factor of four
 over the largest seen."""
@@ -37,7 +37,7 @@ def _oracle(x, params, initial, steps, dlast):
     return h, grads
 
 
-@pytest.mark.parametrize("n,steps,d,units", [(1, 1, 1, 1), (16, 3, 15, 16), (17, 4, 7, 33), (3, 28, 28, 128), (33, 5, 64, 257), (130, 6, 3, 100)])
+@pytest.mark.parametrize("n,steps,d,units", [(1, 1, 1, 1), (16, 3, 15, 16), (17, 4, 7, 33), (3, 28, 28, 128), (33, 5, 64, 257), (130, 6, 3, 100), (5, 2, 9, 64), (20, 3, 5, 129)])
 def test_cells_against_float64(n, steps, d, units):
     from tsplit_amd import graph, ndarray
     rng = np.random.default_rng(n * 1000 + units)
