@@ -482,8 +482,10 @@ inline int compute_units() {
 
 // How the filter-gradient GEMMs of one run are cut: tile shape, depth per range, and (128 x 128 tiles) the
 // persistent grid.  Narrow layers (64 produced or gathered channels) take 64-wide tiles whose idle waves
-// share the depth, one tile per block, with as many ranges as give three blocks per compute unit.  The
-// others run on the persistent kernel: the number of ranges is chosen so that the units (tiles x ranges x
+// share the depth, one tile per block, with as many ranges as give three blocks per compute unit, of at least
+// 12 k-steps each (at least 1024 deep, a layer of 1024 tiles ran as 36 blocks; whole call, at least 1024 / 512 /
+// 192 / 128 deep: 64 -> 128 at 32 x 32, 16 images 59 / 41 / 31 / 31 us, 64 -> 96 at 35 x 35, 32 images 75 / 47 / 45 / 42,
+// 64 -> 64 at 56 x 56, 16 images 46 / 37 / 37 / 39).  The others run on the persistent kernel: the number of ranges is chosen so that the units (tiles x ranges x
 // 36) fill one, two or three rounds of the grid as fully as possible, fewer rounds winning unless more
 // rounds fill at least 7 % better; a range keeps at least 12 k-steps.
 struct GradPlan {
@@ -504,7 +506,7 @@ inline GradPlan plan_grad_gemm(int O, int C, int ld, int cus) {
     g.tn = (C + g.tile_n - 1) / g.tile_n;
     const int per = kXi * g.tm * g.tn;
     int ranges = std::max(1, (slots + per / 2) / per);
-    ranges = std::min(ranges, std::max(1, ld / 1024));
+    ranges = std::min(ranges, std::max(1, ld / (12 * BK)));
     g.kchunk = ((ld + ranges - 1) / ranges + 63) / 64 * 64;
     g.grid = 0;
     return g;
