@@ -479,17 +479,18 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
 
 /* ---- Matrix products with the operators behind them in the same launch (outside the reference's ABI).
  *      TSplit_MatrixMultiplyAdd: C = op(A) op(B), + bias[column] where given, + addend where given (an array of
- *      C's size; it may be C), and, where given, relu = max(C, 0).  An array of more than two axes is taken as a matrix
- *      of its last axis' columns.  Each step is rounded as the operators
- *      DLGpuMatrixMultiply, DLGpuBroadcastTo + DLGpuMatrixElementwiseAdd and DLGpuRelu round it: the same bits.
+ *      C's size; it may be C), and, where given, relu = max(C, 0).  With `gate`, the input of a Relu of C's size, C is
+ *      taken through that Relu's gradient: relu = that where relu is given, otherwise C itself.  An array of more than two
+ *      axes is taken as a matrix of its last axis' columns.  Each step is rounded as the operators DLGpuMatrixMultiply,
+ *      DLGpuBroadcastTo + DLGpuMatrixElementwiseAdd, DLGpuRelu and DLGpuReluGradient round it: the same bits.
  *      TSplit_HeadsMatrixMultiply: for every n and head, C = alpha * op(A) op(B), + mask_value in the columns where
  *      mask (of n x columns values) is 0, then `fill` in the columns right of the row where causal != 0, then
  *      + addend (laid out as C, not C).  A, B and C are each [n, heads, rows, columns], or [n, rows, heads *
  *      columns] with a head's columns side by side: heads are neither split off nor merged by a transpose.
  *      The reference's graph spells these out node by node (examples/transformer.py:56-171). ---- */
 int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
-                             const DLArrayHandle bias, const DLArrayHandle addend, DLArrayHandle matC,
-                             DLArrayHandle relu, DLStreamHandle stream);
+                             const DLArrayHandle bias, const DLArrayHandle addend, const DLArrayHandle gate,
+                             DLArrayHandle matC, DLArrayHandle relu, DLStreamHandle stream);
 int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
                                DLArrayHandle matC, int heads, float alpha, const DLArrayHandle mask,
                                float mask_value, int causal, float fill, const DLArrayHandle addend,

@@ -40,6 +40,17 @@ def test_product_with_bias_addend_and_relu(shape, ta, tb, rng):
         np.testing.assert_array_equal(c.asnumpy(), want)
         if with_relu:
             np.testing.assert_array_equal(r.asnumpy(), np.maximum(want, 0))
+    x = rng.normal(size=(M, N)).astype(np.float32)        # a Relu's input: zeros of both signs and NaN among it
+    x.ravel()[::5], x.ravel()[1::7], x.ravel()[2::11] = 0.0, -0.0, np.nan
+    gx, c, r, grad = _dev(x)[0], _full((M, N)), _full((M, N)), _full((M, N))
+    L.matrix_multiply_add(ga, ta, gb, tb, c, addend=gadd, relu=r, gate=gx)
+    L.relu_gradient(gx, c, grad)
+    np.testing.assert_array_equal(c.asnumpy(), product + add)
+    np.testing.assert_array_equal(r.asnumpy(), grad.asnumpy())
+    L.matrix_multiply_add(ga, ta, gb, tb, c, addend=gadd, gate=gx)
+    np.testing.assert_array_equal(c.asnumpy(), grad.asnumpy())
+    with pytest.raises(RuntimeError):
+        L.matrix_multiply_add(ga, ta, gb, tb, c, gate=c)
     acc = _dev(add)[0]                                    # added to in place
     L.matrix_multiply_add(ga, ta, gb, tb, acc, addend=acc)
     np.testing.assert_array_equal(acc.asnumpy(), product + add)

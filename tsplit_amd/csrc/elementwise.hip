@@ -152,11 +152,7 @@ struct ReluOp {
 };
 struct ReluGradOp {   // out = (sign(x)+1)*0.5*dy ; arrays: out, x, dy
   static constexpr int N = 3, LOAD = 6, STORE = 1;
-  __device__ void apply(float (&v)[3]) const {
-    const float x = v[1];
-    const float sgn = x > 0.f ? 1.f : (x < 0.f ? -1.f : x);   // keeps +-0 and NaN like np.sign
-    v[0] = (sgn + 1.f) * 0.5f * v[2];
-  }
+  __device__ void apply(float (&v)[3]) const { v[0] = relu_grad_of(v[1], v[2]); }
 };
 struct DivOp {    // out = a / b
   static constexpr int N = 3, LOAD = 6, STORE = 1;

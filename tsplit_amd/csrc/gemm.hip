@@ -81,7 +81,7 @@ void launch_epilogue_tile(const float *A, int64_t lda, const float *B, int64_t l
                           int N, int K, const gt::Epilogue &ep, hipStream_t s) {
   using T = gt::Tile<TM, TN, 2, 2, TA, TB>;
   const int tm = (M + T::BM - 1) / T::BM, tn = (N + T::BN - 1) / T::BN;
-  const bool wide = N % 4 == 0 && ldc % 4 == 0 && zs.co % 4 == 0 && zs.ci % 4 == 0 && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu);
+  const bool wide = N % 4 == 0 && ldc % 4 == 0 && zs.co % 4 == 0 && zs.ci % 4 == 0 && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu) && aligned16(ep.gate);
   hipLaunchKernelGGL((gt::gemm_epilogue_kernel<TM, TN, TA, TB>), dim3(grid_blocks(tm, tn, batch)), dim3(gt::kThreads), 0, s, DenseParams{A, lda, M, K},
                      DenseParams{B, ldb, N, K}, out, ldc, zs, ep, wide, M, N, K, TileGrid{tm, tn, tm * tn * batch});
 }
@@ -99,7 +99,7 @@ void launch_epilogue(int tile, const float *A, int64_t lda, const float *B, int6
 
 // the results of S ranges (or of one) summed, with what follows
 int launch_epilogue_fold(const float *part, float *out, int64_t mn, int N, int S, const gt::Epilogue &ep, hipStream_t s) {
-  if (N % 4 == 0 && aligned16(part) && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu))
+  if (N % 4 == 0 && aligned16(part) && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu) && aligned16(ep.gate))
     hipLaunchKernelGGL(gt::fold_epilogue_kernel<4>, dim3(static_cast<unsigned>((mn / 4 + 255) / 256)), dim3(256), 0, s, part, out, mn, N, S, ep);
   else
     hipLaunchKernelGGL(gt::fold_epilogue_kernel<1>, dim3(static_cast<unsigned>((mn + 255) / 256)), dim3(256), 0, s, part, out, mn, N, S, ep);
@@ -297,8 +297,8 @@ int dispatch_heads(const HeadArray &a, const HeadArray &b, const HeadArray &c, i
 using namespace tsplit;
 
 extern "C" int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
-                                        const DLArrayHandle bias, const DLArrayHandle addend, DLArrayHandle matC, DLArrayHandle relu,
-                                        DLStreamHandle stream_handle) {
+                                        const DLArrayHandle bias, const DLArrayHandle addend, const DLArrayHandle gate, DLArrayHandle matC,
+                                        DLArrayHandle relu, DLStreamHandle stream_handle) {
   const char *who = "TSplit_MatrixMultiplyAdd";
   TS_REQUIRE(matA && matB && matC, "%s: NULL array", who);
   TS_REQUIRE(matA->ndim >= 2 && matB->ndim >= 2 && matC->ndim >= 2, "%s: arrays of two axes or more only", who);
@@ -313,6 +313,8 @@ extern "C" int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA
   TS_REQUIRE(!bias || numel(bias) == N, "%s: the bias has %lld values for %lld columns", who, (long long)(bias ? numel(bias) : 0), (long long)N);
   TS_REQUIRE(!addend || numel(addend) == M * N, "%s: the addend is of the result's size", who);
   TS_REQUIRE(!relu || (numel(relu) == M * N && relu->data != matC->data), "%s: Relu's result is another array of the result's size", who);
+  TS_REQUIRE(!gate || (numel(gate) == M * N && gate->data != matC->data && (!relu || gate->data != relu->data)),
+             "%s: the gate is another array of the result's size", who);
   hipStream_t s = stream_of(stream_handle);
   ProfileScope ps(nullptr, s, 0, 0, 0);
   int rc = 0;
@@ -321,7 +323,8 @@ extern "C" int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA
     float *C = static_cast<float *>(matC->data);
     const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
     const gt::Epilogue ep{1.f, bias ? static_cast<const float *>(bias->data) : nullptr, nullptr, 0.f, 0, 0.f,
-                          addend ? static_cast<const float *>(addend->data) : nullptr, relu ? static_cast<float *>(relu->data) : nullptr};
+                          addend ? static_cast<const float *>(addend->data) : nullptr, relu ? static_cast<float *>(relu->data) : nullptr,
+                          gate ? static_cast<const float *>(gate->data) : nullptr};
     if (!transposeA && !transposeB) rc = dispatch_epilogue<false, false>(A, lda, B, ldb, C, m, n, k, ep, s);
     if (!transposeA && transposeB) rc = dispatch_epilogue<false, true>(A, lda, B, ldb, C, m, n, k, ep, s);
     if (transposeA && !transposeB) rc = dispatch_epilogue<true, false>(A, lda, B, ldb, C, m, n, k, ep, s);
@@ -355,7 +358,7 @@ extern "C" int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transpos
   if (M > 0 && N > 0 && c.n > 0) {
     const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
     const gt::Epilogue ep{alpha, nullptr, mask ? static_cast<const float *>(mask->data) : nullptr, mask_value, causal, fill,
-                          addend ? static_cast<const float *>(addend->data) : nullptr, nullptr};
+                          addend ? static_cast<const float *>(addend->data) : nullptr, nullptr, nullptr};
     if (!transposeA && !transposeB) rc = dispatch_heads<false, false>(a, b, c, heads, m, n, k, ep, s);
     if (!transposeA && transposeB) rc = dispatch_heads<false, true>(a, b, c, heads, m, n, k, ep, s);
     if (transposeA && !transposeB) rc = dispatch_heads<true, false>(a, b, c, heads, m, n, k, ep, s);

@@ -18,6 +18,7 @@
 
 #include <cstdint>
 
+#include "activations.h"
 #include "mfma_gemm.h"
 
 namespace tsplit {
@@ -198,6 +199,18 @@ __device__ __forceinline__ void store_words(__amdgpu_buffer_rsrc_t to, unsigned 
   else
     __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(v[0]), __float_as_uint(v[1])}, to, voff, 0, 0);
 }
+template <int T>
+__device__ __forceinline__ void load_words(__amdgpu_buffer_rsrc_t from, unsigned voff, int step, float (&v)[T]) {
+  if constexpr (T == 4) {
+    const mg::u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(from, voff + step, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = __uint_as_float(r[j]);
+  } else {
+    const u32x2 r = __builtin_amdgcn_raw_buffer_load_b64(from, voff + step, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) v[j] = __uint_as_float(r[j]);
+  }
+}
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t output_buffer(float *p, int64_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(p, 0, static_cast<int>(bytes < 0x7fffffffll ? bytes : 0x7fffffffll), mg::kBufFlags);
 }
@@ -320,7 +333,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(mg::DenseParams 
 // ---- products whose result is worked on before it is stored
 // What follows the sum of products, in this order and with a rounding each, as the operators behind a product would do it:
 // v = alpha * sum; + bias[column]; + mask_value where mask[column] is 0; fill where the column lies right of the row; + add; stored, and
-// max(v, 0) stored as well.  Each of these as an operator of its own reads and writes the whole result again: scores of 32 x 8 x 256 x
+// max(v, 0) stored as well; or the result, as the gradient behind a Relu, taken through it: as a second array or in place of the result.
+// Each of these as an operator of its own reads and writes the whole result again: scores of 32 x 8 x 256 x
 // 256 (67 MB) took 29 us as a product and 175 with a scale, a mask and a causal selection behind it, a projection of 8192 x 512 over 512
 // 36 and 64 us with its bias and a residual.
 struct Epilogue {
@@ -332,6 +346,9 @@ struct Epilogue {
   float fill;
   const float *add;      // laid out as the result, which it may be (a lane reads a value before it writes it); null: none
   float *relu;           // likewise; null: not stored
+  const float *gate;     // the input of the Relu that the result is taken through, laid out as the result and no array written; null: none
+  // the second value of v: Relu, or its gradient where it let x through
+  __device__ __forceinline__ float second(float v, float x) const { return gate ? relu_grad_of(x, v) : fmaxf(v, 0.f); }
   __device__ __forceinline__ float at(float v, int m, int n, float b, bool masked) const {
     v *= alpha;
     if (bias) v += b;
@@ -373,6 +390,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_epilogue_kernel(mg::DensePar
   const __amdgpu_buffer_rsrc_t to = output_buffer(out + from, bytes);
   const __amdgpu_buffer_rsrc_t add = output_buffer(const_cast<float *>(ep.add ? ep.add + from : out + from), bytes);
   const __amdgpu_buffer_rsrc_t relu = output_buffer(ep.relu ? ep.relu + from : out + from, bytes);
+  const __amdgpu_buffer_rsrc_t gate = output_buffer(const_cast<float *>(ep.gate ? ep.gate + from : out + from), bytes);
+  const bool first = !ep.gate || ep.relu, second = ep.gate || ep.relu;   // which of the two values leave
   const int row_bytes = static_cast<int>(ldc) * 4, row0 = m + C::lane_row();
   const unsigned at = (static_cast<unsigned>(C::lane_row()) * static_cast<unsigned>(ldc) + static_cast<unsigned>(n)) * 4u;
   unsigned off[TN];
@@ -394,28 +413,28 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_epilogue_kernel(mg::DensePar
       for (int j = 0; j < TN; ++j) v[j] = ep.at(acc[tm][j][e], row0 + step, n + j, b[j], masked[j]);
       if (wide) {   // N and ldc are multiples of 4: a word lies inside its row or behind it
         if (ep.add) {
-          if constexpr (TN == 4) {
-            const mg::u32x4 r = __builtin_amdgcn_raw_buffer_load_b128(add, off[0] + soff, 0, 0);
+          float r[TN];
+          load_words<TN>(add, off[0], soff, r);
 #pragma unroll
-            for (int j = 0; j < TN; ++j) v[j] += __uint_as_float(r[j]);
-          } else {
-            const u32x2 r = __builtin_amdgcn_raw_buffer_load_b64(add, off[0] + soff, 0, 0);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) v[j] += __uint_as_float(r[j]);
-          }
+          for (int j = 0; j < TN; ++j) v[j] += r[j];
         }
-        store_words<TN>(to, off[0], soff, v);
-        if (ep.relu) {
+        if (first) store_words<TN>(to, off[0], soff, v);
+        if (second) {
+          float x[TN] = {};
+          if (ep.gate) load_words<TN>(gate, off[0], soff, x);
 #pragma unroll
-          for (int j = 0; j < TN; ++j) v[j] = fmaxf(v[j], 0.f);
+          for (int j = 0; j < TN; ++j) v[j] = ep.second(v[j], x[j]);
           store_words<TN>(relu, off[0], soff, v);
         }
       } else {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           if (ep.add) v[j] += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(add, off[j] + soff, 0, 0));
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), to, off[j] + soff, 0, 0);
-          if (ep.relu) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(fmaxf(v[j], 0.f)), relu, off[j] + soff, 0, 0);
+          if (first) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), to, off[j] + soff, 0, 0);
+          if (second) {
+            const float x = ep.gate ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(gate, off[j] + soff, 0, 0)) : 0.f;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ep.second(v[j], x)), relu, off[j] + soff, 0, 0);
+          }
         }
       }
     }
@@ -446,11 +465,13 @@ static __global__ __launch_bounds__(256) void fold_epilogue_kernel(const float *
     for (int j = 0; j < VEC; ++j) s[j] += ep.bias[col + j];
   }
   if (ep.add) s += read(ep.add + i);
-  *reinterpret_cast<vec *>(out + i) = s;
-  if (ep.relu) {
+  if (!ep.gate || ep.relu) *reinterpret_cast<vec *>(out + i) = s;
+  if (ep.gate || ep.relu) {
+    vec x = s;
+    if (ep.gate) x = read(ep.gate + i);
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) s[j] = fmaxf(s[j], 0.f);
-    *reinterpret_cast<vec *>(ep.relu + i) = s;
+    for (int j = 0; j < VEC; ++j) s[j] = ep.second(s[j], x[j]);
+    *reinterpret_cast<vec *>((ep.relu ? ep.relu : out) + i) = s;
   }
 }
 

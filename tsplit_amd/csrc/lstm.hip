@@ -428,7 +428,7 @@ extern "C" int TSplit_Lstm(const DLArrayHandle x, const DLArrayHandle *params, c
   if (flat) {
     int64_t ashape[2] = {static_cast<int64_t>(z.n) * steps, z.d}, bshape[2] = {z.d, wide}, cshape[2] = {static_cast<int64_t>(z.n) * steps, wide};
     DLArray A{x->data, x->ctx, 2, ashape}, B{fwd, x->ctx, 2, bshape}, bias{fwd + z.d * wide, x->ctx, 1, bshape + 1}, C{gates->data, x->ctx, 2, cshape};
-    if (const int rc = TSplit_MatrixMultiplyAdd(&A, 0, &B, 0, &bias, nullptr, &C, nullptr, stream_handle)) return rc;
+    if (const int rc = TSplit_MatrixMultiplyAdd(&A, 0, &B, 0, &bias, nullptr, nullptr, &C, nullptr, stream_handle)) return rc;
     hipLaunchKernelGGL((z.h <= 64 ? resident_kernel<64> : resident_kernel<128>), dim3((z.n + kSamples - 1) / kSamples), dim3(kResident), 0, s, z, q,
                        fp(gates), fp(rows), fp(cells), fp(initial), fp(last));
     return ps.finish();

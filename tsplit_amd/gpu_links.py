@@ -90,11 +90,13 @@ def matrix_multiply(matA, transA, matB, transB, matC, stream=None, profiler=None
                                         ctypes.c_bool(bool(transB)), _h(matC), _s(stream), _p(profiler)))
 
 
-def matrix_multiply_add(matA, transA, matB, transB, matC, bias=None, addend=None, relu=None, stream=None):
+def matrix_multiply_add(matA, transA, matB, transB, matC, bias=None, addend=None, relu=None, stream=None, gate=None):
     """matC = op(matA) op(matB) + bias + addend, relu = max(matC, 0), each where given: the bits of matrix_multiply,
-    broadcast_to and matrix_elementwise_add, and relu (no counterpart in the reference's gpu_links)."""
+    broadcast_to and matrix_elementwise_add, and relu (no counterpart in the reference's gpu_links).  With `gate`, a Relu's input,
+    that Relu's gradient of the result: in relu where it is given, else in matC."""
     check_call(_LIB.TSplit_MatrixMultiplyAdd(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(bias) if bias else None,
-                                             _h(addend) if addend else None, _h(matC), _h(relu) if relu else None, _s(stream)))
+                                             _h(addend) if addend else None, _h(gate) if gate else None, _h(matC),
+                                             _h(relu) if relu else None, _s(stream)))
 
 
 def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0,

@@ -129,12 +129,13 @@ class GpuBackend(object):
         self.L.batch_matrix_multiply(a, ta, b, tb, c, self.stream)
         return c
 
-    def matmul_add(self, a, ta, b, tb, out_shape, bias=None, addend=None, relu=False, out=None):
+    def matmul_add(self, a, ta, b, tb, out_shape, bias=None, addend=None, relu=False, out=None, gate=None):
         """-> (op(a) op(b) + bias + addend, its Relu or None) in one call; arrays of more axes are matrices of the last one's columns.
-        out: the array to write (it may be the addend), or None for a new one."""
+        out: the array to write (it may be the addend), or None for a new one.  gate: the input of a Relu that the result, its
+        gradient, is taken through."""
         c = self.empty(out_shape) if out is None else out
         r = self.empty(out_shape) if relu else None
-        self.L.matrix_multiply_add(a, ta, b, tb, c, bias, addend, r, self.stream)
+        self.L.matrix_multiply_add(a, ta, b, tb, c, bias, addend, r, self.stream, gate)
         return c, r
 
     def heads_matmul(self, a, ta, b, tb, out_shape, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0, addend=None):
@@ -382,6 +383,8 @@ class Tape(object):
         self._leaves = []    # leaves whose gradient arrays are this sweep's
         self._scores = {}    # head_scores call -> (scale, causal)
         self._scaled = set() # head_scores calls whose gradient has arrived with scale and selection applied
+        self._gates = {}     # relu call -> its input
+        self._gated = set()  # relu calls whose gradient has arrived taken through them
         self._log = None     # with a list here, every operator call is appended as (name, args, kwargs)
 
     def _call(self, fn, args, kwargs):
@@ -468,7 +471,12 @@ class Tape(object):
         """Adds op(a) op(b) to var's gradient."""
         if not var.needs_grad:
             return
-        if var.own:
+        if var.node in self._gates and self._readers[var.node] == 1 and var.grad is None:
+            # a Relu's output that goes nowhere else: its gradient behind the product that makes it
+            var.grad = self.b.matmul_add(a, ta, b, tb, var.shape, gate=self._gates[var.node].value)[0]
+            self._owns(var, True)
+            self._gated.add(var.node)
+        elif var.own:
             self.b.matmul_add(a, ta, b, tb, var.shape, addend=var.grad, out=var.grad)
         else:
             var.grad = self._product(a, a_shape, ta, b, b_shape, tb, var.shape, addend=var.grad)[0]
@@ -569,7 +577,17 @@ class Tape(object):
         def fwd():
             return self.b.relu(x.value, x.shape)
         y = self._ready.pop(x.node, None)
-        return self._out(fwd() if y is None else y, x.shape, [x], lambda g: self._acc(x, self.b.relu_grad(x.value, g, x.shape)), redo=fwd)
+        out = None
+
+        def back(g):
+            if out.node in self._gated:
+                self._acc(x, g, fresh=True)
+            else:
+                self._acc(x, self.b.relu_grad(x.value, g, x.shape))
+        out = self._out(fwd() if y is None else y, x.shape, [x], back, redo=fwd)
+        if out.node >= 0 and self._ahead and self._can("matmul_add"):
+            self._gates[out.node] = x
+        return out
 
     @_op
     def max_pool(self, x, k, pad, stride):
@@ -979,7 +997,7 @@ class Tape(object):
             self._after_backward(node)
         self._release_leaves()
         self._nodes, self._readers = [], []
-        self._ready, self._scores, self._scaled = {}, {}, set()
+        self._ready, self._scores, self._scaled, self._gates, self._gated = {}, {}, set(), {}, set()
 
 
     def _release_leaves(self):

@@ -20,6 +20,8 @@ Layer spec entries:
     ("conv", name, Cin, Cout, k, pad, stride) | ("bn", name, C) | ("relu",) |
     ("maxpool", k, pad, stride) | ("flatten",) | ("fc", name, n_in, n_out)
 """
+import math
+
 import numpy as np
 
 from . import gpu_links as L
@@ -133,6 +135,12 @@ class Trainer(object):
         # activation in front of the pooling is never written (filled in below, where the shapes are known)
         self.fused_pool = set()
         want_pool = bool(fuse_max_pool and fuse_bn_relu)
+        # Relu layers behind a linear layer, whose output leaves in the product's call, and in front of one, whose gradient does
+        # (the same bits in the same arrays)
+        kinds = [l[0] for l in self.spec]
+        self.relu_of_fc = {li for li in range(1, len(kinds)) if kinds[li] == "relu" and kinds[li - 1] == "fc"}
+        self.relu_before_fc = {li for li in range(1, len(kinds) - 1)
+                               if kinds[li] == "relu" and kinds[li + 1] == "fc" and li - 1 not in self.fused}
         # with conv_bn_stats a ("conv", ...) layer directly followed by ("bn", ...) hands the BatchNorm its
         # batch statistics (one row of sums per micro-tensor; symbols outside the reference's ABI), so
         # the BatchNorm reads the convolution's output once instead of twice
@@ -192,20 +200,20 @@ class Trainer(object):
                 self.acts[li].split_tensor(self.split[li])
                 self.dacts[li].split_tensor(self.split[li])
 
-    def _run(self, tag, work, unit, fn, *args, moved=None):
+    def _run(self, tag, work, unit, fn, *args, moved=None, **more):
         """Issue one operator call on the compute stream; `work` is its algorithmic FLOP or
         byte count (each distinct input read once, each output written once); `moved` gives the
         byte count of a call whose work is counted in FLOP but which sits near the ridge."""
         if self.timer is None:
-            fn(*args, self.stream)
+            fn(*args, self.stream, **more)
         else:
             self.timer.begin(self.stream)
-            fn(*args, self.stream)
+            fn(*args, self.stream, **more)
             self.timer.end(self.stream, tag, work, unit, moved)
 
     @staticmethod
     def _n(shape):
-        return int(np.prod(shape))
+        return math.prod(shape)
 
     @staticmethod
     def _rows(rows):
@@ -214,7 +222,7 @@ class Trainer(object):
 
     # ---------------------------------------------------------------- forward
     def forward(self, x, labels):
-        n = self._n
+        n, shapes = self._n, self.shapes
         self.acts[0] = x
         if 0 in self.split:
             x.split_tensor(self.split[0])
@@ -243,7 +251,7 @@ class Trainer(object):
                 sm, sv = self.saved[li]
                 pooled = self.acts[li + 3]
                 from_stats = li - 1 in self.stats_of
-                self._run("bn_relu_pool_fwd_from_stats" if from_stats else "bn_relu_pool_fwd", 4.0 * (n(a.shape) + n(pooled.shape)),
+                self._run("bn_relu_pool_fwd_from_stats" if from_stats else "bn_relu_pool_fwd", 4.0 * (n(shapes[li]) + n(pooled.shape)),
                           "byte", L.batch_norm_relu_max_pool, a, self.params[name + "_scale"], self.params[name + "_bias"],
                           pooled, sm, sv, self.eps, self.stats_of[li - 1] if from_stats else None,
                           self.split.get(li - 1, 1) if from_stats else 0)
@@ -251,7 +259,7 @@ class Trainer(object):
                 name = layer[1]
                 sm, sv = self.saved[li]
                 fused = li in self.fused
-                self._run("bn_relu_fwd_from_stats" if fused else "bn_fwd_from_stats", 8.0 * n(a.shape), "byte",
+                self._run("bn_relu_fwd_from_stats" if fused else "bn_fwd_from_stats", 8.0 * n(shapes[li]), "byte",
                           L.batch_norm_from_stats, a, self.stats_of[li - 1], self.split.get(li - 1, 1),
                           self.params[name + "_scale"], self.params[name + "_bias"],
                           self.acts[li + 2] if fused else out, sm, sv, self.eps, fused)
@@ -259,38 +267,40 @@ class Trainer(object):
                 name = layer[1]
                 sm, sv = self.saved[li]
                 # writes the Relu layer's output directly
-                self._run("bn_relu_fwd", 8.0 * n(a.shape), "byte", L.batch_norm_relu, a, self.params[name + "_scale"],
+                self._run("bn_relu_fwd", 8.0 * n(shapes[li]), "byte", L.batch_norm_relu, a, self.params[name + "_scale"],
                           self.params[name + "_bias"], self.acts[li + 2], sm, sv, self.eps)
             elif kind == "bn":
                 name = layer[1]
                 sm, sv = self.saved[li]
-                self._run("bn_fwd", 8.0 * n(a.shape), "byte", L.CuDNN_Batch_Normalization, a,
+                self._run("bn_fwd", 8.0 * n(shapes[li]), "byte", L.CuDNN_Batch_Normalization, a,
                           self.params[name + "_scale"], self.params[name + "_bias"], out, sm, sv, 0.99, self.eps)
-            elif kind == "relu" and li - 1 in self.fused:
+            elif kind == "relu" and (li - 1 in self.fused or li in self.relu_of_fc):
                 pass
             elif kind == "relu":
-                self._run("relu_fwd", 8.0 * n(a.shape), "byte", L.relu, a, out)
+                self._run("relu_fwd", 8.0 * n(shapes[li]), "byte", L.relu, a, out)
             elif kind == "maxpool" and li - 2 in self.fused_pool:
                 pass
             elif kind == "maxpool":
                 _, k, pad, stride = layer
-                self._run("maxpool_fwd", 4.0 * (n(a.shape) + n(out.shape)), "byte", L.CuDNN_max_pooling2d, a, k, k, out,
+                self._run("maxpool_fwd", 4.0 * (n(shapes[li]) + n(shapes[li + 1])), "byte", L.CuDNN_max_pooling2d, a, k, k, out,
                           pad, stride)
             elif kind == "flatten":
-                self._run("reshape", 8.0 * n(a.shape), "byte", L.array_reshape, a, out)
+                self._run("reshape", 8.0 * n(shapes[li]), "byte", L.array_reshape, a, out)
             elif kind == "fc":
                 _, name, n_in, n_out = layer
-                self._run("matmul_" + self._rows(a.shape[0]), 2.0 * a.shape[0] * n_in * n_out, "flop",
-                          L.matrix_multiply, a, False, self.params[name + "_weight"], False, out,
-                          moved=4.0 * (a.shape[0] * n_in + n_in * n_out + a.shape[0] * n_out))
-        self._run("softmax_ce_fwd", 8.0 * n(self.acts[-1].shape), "byte", L.softmax_cross_entropy, self.acts[-1],
+                call, args = L.matrix_multiply, (a, False, self.params[name + "_weight"], False, out)
+                if li + 1 in self.relu_of_fc:        # the Relu behind it leaves in the same call
+                    call, args = L.matrix_multiply_add, args + (None, None, self.acts[li + 2])
+                self._run("matmul_" + self._rows(shapes[li][0]), 2.0 * shapes[li][0] * n_in * n_out, "flop", call, *args,
+                          moved=4.0 * (shapes[li][0] * n_in + n_in * n_out + shapes[li][0] * n_out))
+        self._run("softmax_ce_fwd", 8.0 * n(shapes[-1]), "byte", L.softmax_cross_entropy, self.acts[-1],
                   labels, self.loss)
         return self.loss
 
     # ---------------------------------------------------------------- backward
     def backward(self, labels):
-        n = self._n
-        self._run("softmax_ce_bwd", 12.0 * n(self.acts[-1].shape), "byte", L.softmax_cross_entropy_gradient,
+        n, shapes = self._n, self.shapes
+        self._run("softmax_ce_bwd", 12.0 * n(shapes[-1]), "byte", L.softmax_cross_entropy_gradient,
                   self.acts[-1], labels, self.ones, self.dacts[-1])
         for li in range(len(self.spec) - 1, -1, -1):
             layer = self.spec[li]
@@ -330,44 +340,46 @@ class Trainer(object):
                 name = layer[1]
                 sm, sv = self.saved[li]
                 gp = self.dacts[li + 3]      # the gradient behind the pooling
-                self._run("bn_relu_pool_bwd", 4.0 * (2 * n(a.shape) + n(gp.shape)), "byte", L.batch_norm_relu_max_pool_gradient,
+                self._run("bn_relu_pool_bwd", 4.0 * (2 * n(shapes[li]) + n(gp.shape)), "byte", L.batch_norm_relu_max_pool_gradient,
                           gp, a, self.params[name + "_scale"], self.params[name + "_bias"], g_in,
                           self.grads[name + "_scale"], self.grads[name + "_bias"], sm, sv, self.eps)
             elif kind == "bn" and li in self.fused:
                 name = layer[1]
                 sm, sv = self.saved[li]
                 # consumes the gradient behind the Relu layer
-                self._run("bn_relu_bwd", 12.0 * n(a.shape), "byte", L.batch_norm_relu_gradient, self.dacts[li + 2], a,
+                self._run("bn_relu_bwd", 12.0 * n(shapes[li]), "byte", L.batch_norm_relu_gradient, self.dacts[li + 2], a,
                           self.params[name + "_scale"], self.params[name + "_bias"], g_in,
                           self.grads[name + "_scale"], self.grads[name + "_bias"], sm, sv, self.eps)
             elif kind == "bn":
                 name = layer[1]
                 sm, sv = self.saved[li]
-                self._run("bn_bwd", 12.0 * n(a.shape), "byte", L.CuDNN_Batch_Normalization_gradient, g_out, a,
+                self._run("bn_bwd", 12.0 * n(shapes[li]), "byte", L.CuDNN_Batch_Normalization_gradient, g_out, a,
                           self.params[name + "_scale"], g_in, self.grads[name + "_scale"],
                           self.grads[name + "_bias"], sm, sv, self.eps)
-            elif kind == "relu" and li - 1 in self.fused:
+            elif kind == "relu" and (li - 1 in self.fused or li in self.relu_before_fc):
                 pass
             elif kind == "relu":
-                self._run("relu_bwd", 12.0 * n(a.shape), "byte", L.relu_gradient, a, g_out, g_in)
+                self._run("relu_bwd", 12.0 * n(shapes[li]), "byte", L.relu_gradient, a, g_out, g_in)
             elif kind == "maxpool" and li - 2 in self.fused_pool:
                 pass
             elif kind == "maxpool":
                 _, k, pad, stride = layer
-                self._run("maxpool_bwd", 4.0 * (2 * n(a.shape) + n(g_out.shape)), "byte",
+                self._run("maxpool_bwd", 4.0 * (2 * n(shapes[li]) + n(shapes[li + 1])), "byte",
                           L.CuDNN_max_pooling2d_gradient, self.acts[li + 1], g_out, a, k, k, g_in, pad, stride)
             elif kind == "flatten":
-                self._run("reshape", 8.0 * n(a.shape), "byte", L.array_reshape, g_out, g_in)
+                self._run("reshape", 8.0 * n(shapes[li]), "byte", L.array_reshape, g_out, g_in)
             elif kind == "fc":
                 _, name, n_in, n_out = layer
                 w = self.params[name + "_weight"]
-                m = a.shape[0]
+                m = shapes[li][0]
                 moved = 4.0 * (m * n_in + n_in * n_out + m * n_out)
                 self._run("matmul_" + self._rows(n_in), 2.0 * m * n_in * n_out, "flop", L.matrix_multiply, a, True,
                           g_out, False, self.grads[name + "_weight"], moved=moved)
                 if not first:
-                    self._run("matmul_" + self._rows(m), 2.0 * m * n_in * n_out, "flop", L.matrix_multiply, g_out,
-                              False, w, True, g_in, moved=moved)
+                    call, args, more = L.matrix_multiply, (g_out, False, w, True, g_in), {}
+                    if li - 1 in self.relu_before_fc:        # that Relu's gradient leaves in the same call
+                        call, args, more = L.matrix_multiply_add, args + (None, None, self.dacts[li - 1]), {"gate": self.acts[li - 1]}
+                    self._run("matmul_" + self._rows(m), 2.0 * m * n_in * n_out, "flop", call, *args, moved=moved, **more)
 
     # ---------------------------------------------------------------- update
     def update(self):
