@@ -414,7 +414,9 @@ int CuSparse_DLGpuCsrmm(const DLArrayHandle data_handle, const DLArrayHandle row
  *      behind the Relu; it is gated with the reference's Relu derivative (sign(z)+1)/2 of
  *      z = BN(input_X), rebuilt from input_X, bn_scale, bn_bias and the saved statistics of the
  *      fused forward call, then the BatchNorm gradient is taken.  Results equal the two-call
- *      sequence (same float expressions). ---- */
+ *      sequence (same float expressions): to rounding with save arrays of C floats, to the bit
+ *      (the gradient's where that call has no saved arrays) with save arrays of 2 C floats on
+ *      8 bytes, which then hold C doubles each. ---- */
 int TSplit_BatchNormRelu(const DLArrayHandle input_X, const DLArrayHandle bn_scale,
                          const DLArrayHandle bn_bias, DLArrayHandle output_Y, float eps,
                          DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,

@@ -172,3 +172,32 @@ def test_training_with_the_fused_stage_ends_tracks_oracle(stats):
     assert rel <= 1e-3, (rel, losses, ref_losses)
     for k in params:
         assert_close(t.params[k].asnumpy(), ref_params[k], 2e-3, k)
+
+
+# one-pass channels of every size class, split channels in words and without, planes in memory order; a value at BatchNorm's zero
+@pytest.mark.parametrize("shape", [(2, 3, 4, 4), (8, 5, 16, 16), (4, 7, 56, 56), (3, 6, 35, 33), (64, 4, 56, 56), (16, 65, 112, 112)])
+def test_pair_with_double_statistics_has_the_bits_of_the_two_calls(shape, rng):
+    """BatchNorm + Relu in one call with statistics saved as doubles: output and gradients bit for bit those of the two calls."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    ctx = nd.gpu(0)
+    n, c, h, w = shape
+    x = rng.normal(size=shape).astype(np.float32) + np.float32(3)
+    x[0, 0, 0, 0] = x[:, 0].mean()
+    gx, gdy = nd.array(x, ctx), nd.array(rng.normal(size=shape).astype(np.float32), ctx)
+    gamma, beta = nd.array(rng.normal(size=(1, c, 1, 1)), ctx), nd.array(0.1 * rng.normal(size=(1, c, 1, 1)), ctx)
+    bn, y, pair, g, dx0, dx1 = [nd.empty(shape, ctx) for _ in range(6)]
+    dg0, db0, dg1, db1 = [nd.empty((1, c, 1, 1), ctx) for _ in range(4)]
+    L.CuDNN_Batch_Normalization(gx, gamma, beta, bn, None, None, 0.99, 0.01)
+    L.relu(bn, y)
+    L.relu_gradient(bn, gdy, g)
+    L.CuDNN_Batch_Normalization_gradient(g, gx, gamma, dx0, dg0, db0, None, None, 0.01)
+    mean, istd = nd.empty((c, 2), ctx), nd.empty((c, 2), ctx)
+    L.batch_norm_relu(gx, gamma, beta, pair, mean, istd, 0.01)
+    L.batch_norm_relu_gradient(gdy, gx, gamma, beta, dx1, dg1, db1, mean, istd, 0.01)
+    np.testing.assert_array_equal(pair.asnumpy(), y.asnumpy())
+    ref = x.astype(np.float64).mean((0, 2, 3))
+    np.testing.assert_allclose(mean.asnumpy().view(np.float64).ravel(), ref, rtol=2e-7)
+    for a, b in ((dx0, dx1), (dg0, dg1), (db0, db1)):
+        np.testing.assert_array_equal(a.asnumpy(), b.asnumpy())
+    with pytest.raises(RuntimeError):
+        L.batch_norm_relu(gx, gamma, beta, pair, mean, nd.empty((c,), ctx), 0.01)

@@ -58,27 +58,28 @@ __device__ __forceinline__ int64_t word_addr(const Geo &g, uint32_t i, int c) {
   return (static_cast<int64_t>(n) * g.C + c) * g.wpp + j;
 }
 
+// (fused multiply-adds are spelled out: left to the compiler, two forms of a kernel round the same sum differently)
 __device__ __forceinline__ void acc2(const f32x4 &v, float &s, float &q) {
   s += (v.x + v.y) + (v.z + v.w);
-  q += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+  q += fmaf(v.x, v.x, v.y * v.y) + fmaf(v.z, v.z, v.w * v.w);
 }
 __device__ __forceinline__ void acc2(const float &v, float &s, float &q) {
   s += v;
-  q += v * v;
+  q = fmaf(v, v, q);
 }
 __device__ __forceinline__ void acc_dot(const f32x4 &a, const f32x4 &b, float &s, float &d) {
   s += (a.x + a.y) + (a.z + a.w);
-  d += (a.x * b.x + a.y * b.y) + (a.z * b.z + a.w * b.w);
+  d += fmaf(a.x, b.x, a.y * b.y) + fmaf(a.z, b.z, a.w * b.w);
 }
 __device__ __forceinline__ void acc_dot(const float &a, const float &b, float &s, float &d) {
   s += a;
-  d += a * b;
+  d = fmaf(a, b, d);
 }
+__device__ __forceinline__ float axpb(const float &x, float a, float b) { return fmaf(a, x, b); }
 __device__ __forceinline__ f32x4 axpb(const f32x4 &x, float a, float b) {
-  const f32x4 r = {a * x.x + b, a * x.y + b, a * x.z + b, a * x.w + b};
+  const f32x4 r = {fmaf(a, x.x, b), fmaf(a, x.y, b), fmaf(a, x.z, b), fmaf(a, x.w, b)};
   return r;
 }
-__device__ __forceinline__ float axpb(const float &x, float a, float b) { return a * x + b; }
 // Relu and its reference gradient factor (sign(z)+1)/2 (0.5 at z == 0)
 __device__ __forceinline__ float relu1(float z) { return fmaxf(z, 0.f); }
 __device__ __forceinline__ f32x4 relu_w(const f32x4 &z) {
@@ -88,21 +89,15 @@ __device__ __forceinline__ f32x4 relu_w(const f32x4 &z) {
 __device__ __forceinline__ float relu_w(const float &z) { return relu1(z); }
 __device__ __forceinline__ float gate1(float z) { return z > 0.f ? 1.f : (z < 0.f ? 0.f : 0.5f); }
 // dy * relu'(a*x + b)
+__device__ __forceinline__ float gated(const float &dy, const float &x, float a, float b) { return dy * gate1(axpb(x, a, b)); }
 __device__ __forceinline__ f32x4 gated(const f32x4 &dy, const f32x4 &x, float a, float b) {
-  const f32x4 r = {dy.x * gate1(a * x.x + b), dy.y * gate1(a * x.y + b), dy.z * gate1(a * x.z + b),
-                   dy.w * gate1(a * x.w + b)};
+  const f32x4 r = {gated(dy.x, x.x, a, b), gated(dy.y, x.y, a, b), gated(dy.z, x.z, a, b), gated(dy.w, x.w, a, b)};
   return r;
 }
-__device__ __forceinline__ float gated(const float &dy, const float &x, float a, float b) {
-  return dy * gate1(a * x + b);
-}
+__device__ __forceinline__ float lin2(const float &dy, const float &x, float k1, float k2, float k3) { return fmaf(k2, x, k1 * dy) + k3; }
 __device__ __forceinline__ f32x4 lin2(const f32x4 &dy, const f32x4 &x, float k1, float k2, float k3) {
-  const f32x4 r = {k1 * dy.x + k2 * x.x + k3, k1 * dy.y + k2 * x.y + k3, k1 * dy.z + k2 * x.z + k3,
-                   k1 * dy.w + k2 * x.w + k3};
+  const f32x4 r = {lin2(dy.x, x.x, k1, k2, k3), lin2(dy.y, x.y, k1, k2, k3), lin2(dy.z, x.z, k1, k2, k3), lin2(dy.w, x.w, k1, k2, k3)};
   return r;
-}
-__device__ __forceinline__ float lin2(const float &dy, const float &x, float k1, float k2, float k3) {
-  return k1 * dy + k2 * x + k3;
 }
 
 // partial layout: [C][S][NQ] doubles
@@ -153,12 +148,26 @@ __global__ __launch_bounds__(kThreads) void bn_stats_kernel(const float *__restr
 // thread, fixed tree: deterministic) into the coefficients of y = a*x + b, coef[2c] and coef[2c + 1],
 // and the saved statistics.  One block per channel, so that the streaming pass behind it starts with
 // two loads instead of a reduction in every block.
+// Saved statistics: one float a channel, or (wide, the fused forms only) one double in the place of two floats.  From floats the
+// fused backward pass cannot rebuild the a and b of an unfused forward pass, so the fused forward pass then takes rounded statistics too;
+// from doubles it can, and the fused pair has the bits of BatchNorm and Relu one by one; its gradient then forms the statistics of
+// dx from x again, as the unfused gradient without saved arrays does, and has its bits too.
+__device__ __forceinline__ double saved_stat(const float *p, int c, bool wide) {
+  return wide ? reinterpret_cast<const double *>(p)[c] : static_cast<double>(p[c]);
+}
+__device__ __forceinline__ void save_stat(float *p, int c, bool wide, double v) {
+  if (wide)
+    reinterpret_cast<double *>(p)[c] = v;
+  else
+    p[c] = static_cast<float>(v);
+}
+
 template <bool RELU>
 __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restrict__ part, int S, int64_t part_c,
                                                            int64_t part_k, const float *__restrict__ gamma,
                                                            const float *__restrict__ beta, float eps, double inv_m,
                                                            float *__restrict__ coef, float *__restrict__ save_mean,
-                                                           float *__restrict__ save_istd) {
+                                                           float *__restrict__ save_istd, bool wide) {
   __shared__ double sm[kWaves];
   const int c = blockIdx.x;
   double s = 0.0, q = 0.0;
@@ -176,7 +185,7 @@ __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restr
     if (var < 0.0) var = 0.0;
     double istd = 1.0 / sqrt(var + static_cast<double>(eps));
     double mean_used = mean;
-    if (RELU) {
+    if (RELU && !wide) {
       // the fused backward pass rebuilds a and b from the saved float statistics and must see
       // the same sign of a*x + b: derive the coefficients from the rounded values here too
       mean_used = static_cast<double>(static_cast<float>(mean));
@@ -185,8 +194,8 @@ __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restr
     const double a = static_cast<double>(gamma[c]) * istd;
     coef[2 * c] = static_cast<float>(a);
     coef[2 * c + 1] = static_cast<float>(static_cast<double>(beta[c]) - mean_used * a);
-    if (save_mean) save_mean[c] = static_cast<float>(mean);
-    if (save_istd) save_istd[c] = static_cast<float>(istd);
+    if (save_mean) save_stat(save_mean, c, wide, mean);
+    if (save_istd) save_stat(save_istd, c, wide, istd);
   }
 }
 
@@ -251,16 +260,16 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
                                                                  const float *__restrict__ gamma,
                                                                  const float *__restrict__ beta,
                                                                  const float *__restrict__ save_mean,
-                                                                 const float *__restrict__ save_istd) {
+                                                                 const float *__restrict__ save_istd, bool wide) {
   using W = typename Word<VEC>::T;
   __shared__ double sm[4 * kWaves];
   const int c = blockIdx.y, s = blockIdx.x;
   float ga = 0.f, gb = 0.f;
   if (RELU) {
     // the same float expressions as the forward pass, so that the sign of a*x + b is the same
-    const double a = static_cast<double>(gamma[c]) * static_cast<double>(save_istd[c]);
+    const double a = static_cast<double>(gamma[c]) * saved_stat(save_istd, c, wide);
     ga = static_cast<float>(a);
-    gb = static_cast<float>(static_cast<double>(beta[c]) - static_cast<double>(save_mean[c]) * a);
+    gb = static_cast<float>(static_cast<double>(beta[c]) - saved_stat(save_mean, c, wide) * a);
   }
   const uint32_t begin = s * g.chunk;
   const uint32_t end = min(begin + g.chunk, g.words);
@@ -320,7 +329,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_coef_kernel(const double *__r
                                                                const float *__restrict__ gamma,
                                                                const float *__restrict__ beta, float eps, double inv_m,
                                                                const float *__restrict__ save_mean,
-                                                               const float *__restrict__ save_istd,
+                                                               const float *__restrict__ save_istd, bool wide,
                                                                float *__restrict__ coef, float *__restrict__ dgamma,
                                                                float *__restrict__ dbeta) {
   __shared__ double sm[kWaves];
@@ -341,9 +350,9 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_coef_kernel(const double *__r
   }
   if (threadIdx.x == 0) {
     double mean, istd;
-    if (save_mean && save_istd) {
-      mean = static_cast<double>(save_mean[c]);
-      istd = static_cast<double>(save_istd[c]);
+    if (save_mean && save_istd && !wide) {
+      mean = save_mean[c];
+      istd = save_istd[c];
     } else {
       mean = sx * inv_m;
       double var = sq * inv_m - mean * mean;
@@ -360,8 +369,9 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_coef_kernel(const double *__r
     o[1] = static_cast<float>(k2);
     o[2] = static_cast<float>(k3);
     if (RELU) {
-      o[3] = static_cast<float>(k1);   // a = gamma * istd
-      o[4] = static_cast<float>(static_cast<double>(beta[c]) - mean * k1);
+      const double a = static_cast<double>(gamma[c]) * saved_stat(save_istd, c, wide);   // (k1 where not wide)
+      o[3] = static_cast<float>(a);
+      o[4] = static_cast<float>(static_cast<double>(beta[c]) - saved_stat(save_mean, c, wide) * a);
     }
     if (dgamma) dgamma[c] = static_cast<float>(dscale);
     if (dbeta) dbeta[c] = static_cast<float>(dbias);
@@ -426,7 +436,7 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
                                                                   const float *__restrict__ beta, FastDiv hw, int C,
                                                                   uint32_t m, float eps, double inv_m,
                                                                   float *__restrict__ save_mean,
-                                                                  float *__restrict__ save_istd) {
+                                                                  float *__restrict__ save_istd, bool wide) {
   __shared__ double sm[kWaves];
   __shared__ float coef[2];
   const int c = blockIdx.x;
@@ -456,15 +466,15 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
   if (threadIdx.x == 0) {
     double istd = 1.0 / sqrt(var + static_cast<double>(eps));
     double mean_used = mean;
-    if (RELU) {      // as in bn_apply_kernel: coefficients from the rounded statistics the backward pass will read
+    if (RELU && !wide) {      // as in bn_coef_kernel: coefficients from the rounded statistics the backward pass will read
       mean_used = static_cast<double>(static_cast<float>(mean));
       istd = static_cast<double>(static_cast<float>(istd));
     }
     const double a = static_cast<double>(gamma[c]) * istd;
     coef[0] = static_cast<float>(a);
     coef[1] = static_cast<float>(static_cast<double>(beta[c]) - mean_used * a);
-    if (save_mean) save_mean[c] = static_cast<float>(mean);
-    if (save_istd) save_istd[c] = static_cast<float>(istd);
+    if (save_mean) save_stat(save_mean, c, wide, mean);
+    if (save_istd) save_stat(save_istd, c, wide, istd);
   }
   __syncthreads();
   const float a = coef[0], b = coef[1];
@@ -472,7 +482,7 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
   for (int r = 0; r < R; ++r) {
     const uint32_t e = r * kThreads + threadIdx.x;
     if (e < m) {
-      const float z = a * v[r] + b;
+      const float z = axpb(v[r], a, b);
       __builtin_nontemporal_store(RELU ? relu1(z) : z, y + chan_addr(hw, e, c, C));
     }
   }
@@ -484,16 +494,16 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
                                                                   const float *__restrict__ beta, FastDiv hw, int C,
                                                                   uint32_t m, float eps, double inv_m,
                                                                   const float *__restrict__ save_mean,
-                                                                  const float *__restrict__ save_istd,
+                                                                  const float *__restrict__ save_istd, bool wide,
                                                                   float *__restrict__ dgamma, float *__restrict__ dbeta) {
   __shared__ double sm[kWaves];
   __shared__ float coef[3];
   const int c = blockIdx.x;
   float ga = 0.f, gb = 0.f;
   if (RELU) {
-    const double a = static_cast<double>(gamma[c]) * static_cast<double>(save_istd[c]);
+    const double a = static_cast<double>(gamma[c]) * saved_stat(save_istd, c, wide);
     ga = static_cast<float>(a);
-    gb = static_cast<float>(static_cast<double>(beta[c]) - static_cast<double>(save_mean[c]) * a);
+    gb = static_cast<float>(static_cast<double>(beta[c]) - saved_stat(save_mean, c, wide) * a);
   }
   float xv[R], dv[R];
   float sdy = 0.f, sdx = 0.f, sx = 0.f, sq = 0.f;
@@ -518,8 +528,8 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
   if (threadIdx.x == 0) {
     double mean, istd;
     if (!STATS) {
-      mean = static_cast<double>(save_mean[c]);
-      istd = static_cast<double>(save_istd[c]);
+      mean = save_mean[c];
+      istd = save_istd[c];
     } else {
       mean = r2 * inv_m;
       double var = r3 * inv_m - mean * mean;
@@ -844,6 +854,14 @@ int TSplit_BatchNormLookBehind(long long *calls_served, int *notes_live) {
   return 0;
 }
 
+// whether the fused forms' saved statistics are doubles (arrays of 2 C floats on 8 bytes)
+static bool wide_stats(const DLArray *a, int64_t C) { return a && C > 0 && numel(a) == 2 * C; }
+static bool stats_fit(const DLArray *mean, const DLArray *istd, int64_t C, bool relu) {
+  const auto on8 = [](const DLArray *a) { return (reinterpret_cast<uintptr_t>(a->data) & 7) == 0; };
+  if (relu && mean && istd && wide_stats(mean, C) && wide_stats(istd, C)) return on8(mean) && on8(istd);
+  return (!mean || numel(mean) == C) && (!istd || numel(istd) == C);
+}
+
 // coefficients from the partial sums (pair k of channel c at part[(c * part_c + k * part_k) * 2]), then
 // the streaming pass y = a*x + b (+ Relu)
 static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t part_k, float *coef, const Plan &ap,
@@ -853,12 +871,13 @@ static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t par
   const double inv_m = 1.0 / static_cast<double>(ap.m);
   float *sm = save_mean_arr ? mf(save_mean_arr) : nullptr;
   float *sv = save_var_arr ? mf(save_var_arr) : nullptr;
+  const bool wide = relu && wide_stats(save_mean_arr, C);
   if (relu)
     hipLaunchKernelGGL(bn_coef_kernel<true>, dim3(C), dim3(kThreads), 0, s, part, S, part_c, part_k, cf(scale), cf(bias),
-                       eps, inv_m, coef, sm, sv);
+                       eps, inv_m, coef, sm, sv, wide);
   else
     hipLaunchKernelGGL(bn_coef_kernel<false>, dim3(C), dim3(kThreads), 0, s, part, S, part_c, part_k, cf(scale), cf(bias),
-                       eps, inv_m, coef, sm, sv);
+                       eps, inv_m, coef, sm, sv, false);
   PlaneGeo pg;
   unsigned blocks = 0;
   if (plane_major_ok(ap, x, pg, blocks)) {
@@ -895,8 +914,7 @@ static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, c
   TS_REQUIRE(numel(input_X) == numel(output_Y), "%s: input/output sizes differ", who);
   const int64_t C = input_X->shape[1];
   TS_REQUIRE(numel(bn_scale) == C && numel(bn_bias) == C, "%s: scale/bias must hold C=%lld elements", who, (long long)C);
-  TS_REQUIRE(!save_mean_arr || numel(save_mean_arr) == C, "%s: save_mean must hold C elements", who);
-  TS_REQUIRE(!save_var_arr || numel(save_var_arr) == C, "%s: save_var must hold C elements", who);
+  TS_REQUIRE(stats_fit(save_mean_arr, save_var_arr, C, relu), "%s: save_mean and save_var must hold C elements each", who);
   TS_REQUIRE(!relu || (save_mean_arr && save_var_arr), "%s: the fused form needs both save arrays", who);
   // sums a convolution left for exactly this tensor on this stream (common.h): looked up before
   // stream_of() ends all notes, since this call writes too
@@ -929,7 +947,7 @@ static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, c
 #define BN_FWD1(R, RL)                                                                                              \
   hipLaunchKernelGGL((bn_fwd_onepass_kernel<R, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,         \
                      cf(input_X), mf(output_Y), cf(bn_scale), cf(bn_bias), FastDiv(hw), static_cast<int>(C), m, eps, \
-                     1.0 / static_cast<double>(m), sm1, sv1)
+                     1.0 / static_cast<double>(m), sm1, sv1, relu && wide_stats(save_mean_arr, C))
 #define BN_FWD1_R(RL)   \
   do {                  \
     if (per <= 16)      \
@@ -1028,8 +1046,8 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
   TS_REQUIRE(!gradient_bn_scale || numel(gradient_bn_scale) == C, "%s: dscale must hold C elements", who);
   TS_REQUIRE(!gradient_bn_bias || numel(gradient_bn_bias) == C, "%s: dbias must hold C elements", who);
   const bool saved = save_mean_arr && save_var_arr;
-  TS_REQUIRE(!saved || (numel(save_mean_arr) == C && numel(save_var_arr) == C),
-             "%s: saved statistics must hold C elements", who);
+  TS_REQUIRE(!saved || stats_fit(save_mean_arr, save_var_arr, C, relu), "%s: saved statistics must hold C elements", who);
+  const bool wide = relu && wide_stats(save_mean_arr, C);
   TS_REQUIRE(!relu || (saved && bn_bias && numel(bn_bias) == C),
              "%s: the fused form needs the bias and the statistics saved by the fused forward call", who);
   hipStream_t s = stream_of(stream_handle);
@@ -1046,7 +1064,7 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
 #define BN_BWD1(R, ST, RL)                                                                                          \
   hipLaunchKernelGGL((bn_bwd_onepass_kernel<R, ST, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,     \
                      cf(gradient_Y), cf(input_X), mf(gradient_X), cf(bn_scale), bias1, FastDiv(hw),                 \
-                     static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, sv1, dg1, db1)
+                     static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, sv1, wide, dg1, db1)
 #define BN_BWD1_R(ST, RL)   \
   do {                      \
     if (per <= 16)          \
@@ -1056,7 +1074,9 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
     else                    \
       BN_BWD1(64, ST, RL);  \
   } while (0)
-    if (relu)
+    if (wide)
+      BN_BWD1_R(true, true);
+    else if (relu)
       BN_BWD1_R(false, true);
     else if (saved)
       BN_BWD1_R(false, false);
@@ -1092,9 +1112,9 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
 #define BN_BWD(V, ST, R)                                                                                            \
   do {                                                                                                              \
     hipLaunchKernelGGL((bn_bwd_reduce_kernel<V, ST, R>), gr, dim3(kThreads), 0, s, cf(gradient_Y), cf(input_X),     \
-                       part, rd.g, rd.S, cf(bn_scale), bias, sm, sv);                                               \
+                       part, rd.g, rd.S, cf(bn_scale), bias, sm, sv, wide);                                               \
     hipLaunchKernelGGL((bn_bwd_coef_kernel<R>), dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(part),  \
-                       rd.S, cf(bn_scale), bias, eps, inv_m, sm, sv, coef, dg, db);                                 \
+                       rd.S, cf(bn_scale), bias, eps, inv_m, sm, sv, wide, coef, dg, db);                                 \
     if (V == 4 && plane_major)                                                                                      \
       hipLaunchKernelGGL((bn_bwd_dx_plane_kernel<R>), dim3(blocks), dim3(kThreads), 0, s, dyw, xw, dxw,             \
                          static_cast<const float *>(coef), pg);                                                     \
@@ -1103,14 +1123,18 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
                          mf(gradient_X), static_cast<const float *>(coef), dxp.g);                                  \
   } while (0)
   if (rd.vec == 4) {
-    if (relu)
+    if (wide)
+      BN_BWD(4, true, true);
+    else if (relu)
       BN_BWD(4, false, true);
     else if (saved)
       BN_BWD(4, false, false);
     else
       BN_BWD(4, true, false);
   } else {
-    if (relu)
+    if (wide)
+      BN_BWD(1, true, true);
+    else if (relu)
       BN_BWD(1, false, true);
     else if (saved)
       BN_BWD(1, false, false);
@@ -1172,7 +1196,7 @@ static int bn_relu_pool_forward(const char *who, const DLArrayHandle input_X, co
     TS_REQUIRE(coef, "%s: no scratch memory", who);
     hipLaunchKernelGGL(bn_coef_kernel<true>, dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(stats->data), slots,
                        static_cast<int64_t>(1), C, cf(bn_scale), cf(bn_bias), eps, inv_m, coef, mf(save_mean_arr),
-                       mf(save_var_arr));
+                       mf(save_var_arr), false);
   } else {
     Plan st;
     TS_REQUIRE(make_plan(input_X, aligned16(input_X->data), kStatsWords, 16384, st), "%s: unsupported shape", who);
@@ -1187,7 +1211,7 @@ static int bn_relu_pool_forward(const char *who, const DLArrayHandle input_X, co
       hipLaunchKernelGGL(bn_stats_kernel<1>, gs, dim3(kThreads), 0, s, cf(input_X), part, st.g, st.S);
     hipLaunchKernelGGL(bn_coef_kernel<true>, dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(part), st.S,
                        static_cast<int64_t>(st.S), static_cast<int64_t>(1), cf(bn_scale), cf(bn_bias), eps, inv_m, coef,
-                       mf(save_mean_arr), mf(save_var_arr));
+                       mf(save_mean_arr), mf(save_var_arr), false);
   }
   const unsigned blocks = (pg.words + kThreads - 1) / kThreads;
   if (vecw == 4)
@@ -1274,7 +1298,7 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
                        cf(save_mean_arr), cf(save_var_arr));                                                         \
     hipLaunchKernelGGL(bn_bwd_coef_kernel<true>, dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(part),  \
                        static_cast<int>(S), cf(bn_scale), cf(bn_bias), eps, inv_m, cf(save_mean_arr),                \
-                       cf(save_var_arr), coef, dg, db);                                                              \
+                       cf(save_var_arr), false, coef, dg, db);                                                              \
     hipLaunchKernelGGL(bn_pool_bwd_dx_kernel<V>, dim3(blocks), dim3(kThreads), 0, s, cf(gradient_Y), cf(input_X),    \
                        mf(gradient_X), static_cast<const float *>(coef), pg);                                        \
   } while (0)

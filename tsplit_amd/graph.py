@@ -68,6 +68,7 @@ def conv_out(size, k, pad, stride):
 class GpuBackend(object):
     """Primitives on device arrays, one `gpu_links` call each (plus the output allocation)."""
 
+    fuses_pairs = True   # bn_relu is bn and relu, bit for bit
     L = L        # the links module; a subclass that only counts memory puts a stand-in here
 
     def __init__(self, ctx=None, stream=None):
@@ -157,7 +158,8 @@ class GpuBackend(object):
 
     def bn_relu(self, x, gamma, beta, xs, eps):
         """-> (relu(bn(x)), saved mean, saved inverse deviation): one call, the BatchNorm output is never written."""
-        y, mean, istd = self.empty(xs), self.empty((1, xs[1], 1, 1)), self.empty((1, xs[1], 1, 1))
+        # (statistics as doubles: the pair then has the bits of bn and relu)
+        y, mean, istd = self.empty(xs), self.empty((xs[1], 2)), self.empty((xs[1], 2))
         self.L.batch_norm_relu(x, gamma, beta, y, mean, istd, eps, stream=self.stream)
         return y, mean, istd
 
@@ -566,8 +568,10 @@ class Tape(object):
         return self._out(fwd(), x.shape, [x, gamma, beta], back, saved=[x, gamma, beta], redo=fwd)
 
     def bn_then_relu(self, x, gamma, beta, eps=0.01):
-        """The pair as the reference's graph has it (two nodes), or as one node when the tape was asked to fuse."""
-        if self.fuse_bn_relu:
+        """The pair as the reference's graph has it (two nodes), or as one node: when the tape was asked to fuse, and on the device
+        on a tape that accounts for no value, where nothing can read the BatchNorm's output (the same values from two passes of
+        five less going forward, three of eight less going back)."""
+        if self.fuse_bn_relu or (self._ahead and getattr(type(self.b), "fuses_pairs", False)):
             return self.batch_norm_relu(x, gamma, beta, eps)
         return self.relu(self.batch_norm(x, gamma, beta, eps))
 
