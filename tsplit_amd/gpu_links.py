@@ -34,8 +34,8 @@ __all__ = [
 ]
 
 
-def _h(arr):
-    assert isinstance(arr, _nd.NDArray)
+def _h(arr, _NDArray=_nd.NDArray):
+    assert isinstance(arr, _NDArray)
     return arr.handle
 
 

@@ -93,7 +93,7 @@ class GpuBackend(object):
         return x.asnumpy()
 
     def empty(self, shape):
-        return ndarray.empty(tuple(int(s) for s in shape), self.ctx)
+        return ndarray.empty(shape, self.ctx)
 
     def reshape(self, x, shape):
         out = self.empty(shape)

@@ -42,6 +42,32 @@ class DLArray(ctypes.Structure):
 DLArrayHandle = ctypes.POINTER(DLArray)
 
 
+def _prototype(name, *argtypes):
+    """A function of the library with its argument types, for the calls that are made for every array (a function object of its
+    own: looked up as an attribute it would be shared)."""
+    fn = _LIB[name]
+    fn.argtypes = argtypes
+    return fn
+
+
+_int64_p, _handle_p = ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(DLArrayHandle)
+_alloc = _prototype("DLArrayAlloc", _int64_p, ctypes.c_int64, DLContext, _handle_p, ctypes.c_int)
+_free = _prototype("DLArrayFree", DLArrayHandle, ctypes.c_int)
+_array_view = _prototype("TSplit_ArrayView", DLArrayHandle, _int64_p, ctypes.c_int, _handle_p)
+_shapes = {}     # shape -> the same as a C array, which the library copies
+
+
+def _c_shape(shape):
+    try:
+        return _shapes[shape]
+    except (KeyError, TypeError):       # new, or no tuple
+        shape = tuple(int(s) for s in shape)
+        if len(_shapes) >= 4096:
+            _shapes.clear()
+        c = _shapes[shape] = c_array(ctypes.c_int64, shape)
+        return c
+
+
 def cpu(dev_id=0):
     return DLContext(dev_id, 1)
 
@@ -73,19 +99,19 @@ class NDArray(object):
         self._is_view = is_view
         self._keeper = current_keeper()     # set while a step is being recorded into a graph
 
-    def __del__(self):
+    def __del__(self, _free=_free):
         h = getattr(self, "handle", None)
-        if not h:
+        if not h or MEMORY_MANAGE_RULE is None:      # (None: the interpreter is going down)
             return
         if self._is_view:
             # a view owns its struct and shape but not its data
             h.contents.data = None
-            _LIB.DLArrayFree(h, ctypes.c_int(MEMORY_MANAGE_RULE))
+            _free(h, MEMORY_MANAGE_RULE)
         elif self.auto_deleted:
             # an array born inside a recorded step outlives this object: the graph replays into it
-            keeper = getattr(self, "_keeper", None)
+            keeper = self._keeper
             if keeper is None or h.contents.ctx.device_type != 2 or not keeper.take(h, MEMORY_MANAGE_RULE):
-                _LIB.DLArrayFree(h, ctypes.c_int(MEMORY_MANAGE_RULE))
+                _free(h, MEMORY_MANAGE_RULE)
         self.handle = None
 
     # ---- events used by swapping executors (created lazily) ----
@@ -138,7 +164,7 @@ class NDArray(object):
     @property
     def shape(self):
         c = self.handle.contents
-        return tuple(c.shape[i] for i in range(c.ndim))
+        return tuple(c.shape[:c.ndim])
 
     @property
     def ctx(self):
@@ -226,10 +252,9 @@ def array(arr, ctx, stream_handle=None, event_handle=None):
 
 
 def empty(shape, ctx=cpu(0)):
-    cshape = c_array(ctypes.c_int64, tuple(int(s) for s in shape))
+    cshape = _c_shape(shape)
     handle = DLArrayHandle()
-    check_call(_LIB.DLArrayAlloc(cshape, ctypes.c_int64(len(cshape)), ctx, ctypes.byref(handle),
-                                 ctypes.c_int(MEMORY_MANAGE_RULE)))
+    check_call(_alloc(cshape, len(cshape), ctx, ctypes.byref(handle), MEMORY_MANAGE_RULE))
     return NDArray(handle)
 
 
@@ -314,9 +339,9 @@ def slice_for_micro_tensor(input_tensor, index, total_number, dimension="batch")
 
 def view(array, shape):
     """`array` under another shape of as many values: no copy, the view keeps the array alive."""
-    cshape = c_array(ctypes.c_int64, tuple(int(s) for s in shape))
+    cshape = _c_shape(shape)
     h = DLArrayHandle()
-    check_call(_LIB.TSplit_ArrayView(array.handle, cshape, ctypes.c_int(len(cshape)), ctypes.byref(h)))
+    check_call(_array_view(array.handle, cshape, len(cshape), ctypes.byref(h)))
     return NDArray(h, auto_deleted=False, owner=array, is_view=True)
 
 
