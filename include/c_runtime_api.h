@@ -428,6 +428,20 @@ int TSplit_BatchNormRelu_gradient(const DLArrayHandle gradient_Y, const DLArrayH
                                   DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                                   DLStreamHandle stream_handle, ProfilerHandle p);
 
+/* ---- CuDNN_DLGpuBatch_Normalization and DLGpuRelu of its output as one call each way that writes everything the
+ *      two write, with their bits (outside the reference's ABI).  `pair` (2 C floats) carries the pair's coefficients
+ *      from the forward call to the gradient; gradient_R is the gradient behind the Relu, gradient_Y receives the one
+ *      between the two.  The save arrays (C floats) may be NULL, as for the two calls. ---- */
+int TSplit_BatchNormThenRelu(const DLArrayHandle input_X, const DLArrayHandle bn_scale, const DLArrayHandle bn_bias,
+                             DLArrayHandle output_Y, DLArrayHandle relu_R, DLArrayHandle pair, float eps,
+                             DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr, DLStreamHandle stream_handle,
+                             ProfilerHandle p);
+int TSplit_BatchNormThenRelu_gradient(const DLArrayHandle gradient_R, const DLArrayHandle input_X,
+                                      const DLArrayHandle bn_scale, const DLArrayHandle pair, DLArrayHandle gradient_Y,
+                                      DLArrayHandle gradient_X, DLArrayHandle gradient_bn_scale,
+                                      DLArrayHandle gradient_bn_bias, float eps, DLArrayHandle save_mean_arr,
+                                      DLArrayHandle save_var_arr, DLStreamHandle stream_handle, ProfilerHandle p);
+
 /* ---- Convolution that hands its output's batch statistics to the BatchNorm behind it.  NO counterpart
  *      in the reference, where the BatchNorm call (src/ops/CudnnBn.cu:12-210) reads the convolution's
  *      output (src/ops/CudnnConv2d.cu:6-206) once more to get them; for hosts that know a BatchNorm

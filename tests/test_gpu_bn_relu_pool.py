@@ -175,7 +175,7 @@ def test_training_with_the_fused_stage_ends_tracks_oracle(stats):
 
 
 # one-pass channels of every size class, split channels in words and without, planes in memory order; a value at BatchNorm's zero
-@pytest.mark.parametrize("shape", [(2, 3, 4, 4), (8, 5, 16, 16), (4, 7, 56, 56), (3, 6, 35, 33), (64, 4, 56, 56), (16, 65, 112, 112)])
+@pytest.mark.parametrize("shape", [(2, 3, 4, 4), (8, 5, 16, 16), (4, 7, 56, 56), (3, 6, 35, 33), (5, 3, 45, 43), (64, 4, 56, 56), (16, 65, 112, 112)])
 def test_pair_with_double_statistics_has_the_bits_of_the_two_calls(shape, rng):
     """BatchNorm + Relu in one call with statistics saved as doubles: output and gradients bit for bit those of the two calls."""
     from tsplit_amd import gpu_links as L, ndarray as nd
@@ -201,3 +201,18 @@ def test_pair_with_double_statistics_has_the_bits_of_the_two_calls(shape, rng):
         np.testing.assert_array_equal(a.asnumpy(), b.asnumpy())
     with pytest.raises(RuntimeError):
         L.batch_norm_relu(gx, gamma, beta, pair, mean, nd.empty((c,), ctx), 0.01)
+    # one call that writes what the two calls write, with saved statistics and without
+    sm0, sv0, sm1, sv1 = [nd.empty((1, c, 1, 1), ctx) for _ in range(4)]
+    L.CuDNN_Batch_Normalization(gx, gamma, beta, bn, sm0, sv0, 0.99, 0.01)
+    ab, bn1, y1, g1 = nd.empty((c, 2), ctx), nd.empty(shape, ctx), nd.empty(shape, ctx), nd.empty(shape, ctx)
+    for saved in (False, True):
+        s0, s1 = ((sm0, sv0), (sm1, sv1)) if saved else ((None, None), (None, None))
+        L.batch_norm_then_relu(gx, gamma, beta, bn1, y1, ab, *s1, 0.01)
+        L.CuDNN_Batch_Normalization_gradient(g, gx, gamma, dx0, dg0, db0, *s0, 0.01)
+        L.batch_norm_then_relu_gradient(gdy, gx, gamma, ab, g1, dx1, dg1, db1, *s1, 0.01)
+        for a, b in ((bn, bn1), (y, y1), (g, g1), (dx0, dx1), (dg0, dg1), (db0, db1)) + (((sm0, sm1), (sv0, sv1)) if saved else ()):
+            np.testing.assert_array_equal(a.asnumpy(), b.asnumpy())
+    with pytest.raises(RuntimeError):
+        L.batch_norm_then_relu(gx, gamma, beta, bn1, bn1, ab)
+    with pytest.raises(RuntimeError):
+        L.batch_norm_then_relu_gradient(gdy, gx, gamma, ab, dx1, dx1, dg1, db1)

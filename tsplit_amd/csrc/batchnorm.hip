@@ -18,6 +18,7 @@
 // Small channels (N*H*W <= 16384: 14x14 and smaller planes at batch 64, 17x17 at batch 32) take
 // one-pass kernels instead: one block per channel keeps the channel's values in registers, so
 // x (and dy) are read once - the algorithmic 8 and 12 B/elem - in one launch per direction.
+#include "activations.h"
 #include "common.h"
 #include "fastdiv.h"
 #include "reduce.h"
@@ -92,6 +93,12 @@ __device__ __forceinline__ float gate1(float z) { return z > 0.f ? 1.f : (z < 0.
 __device__ __forceinline__ float gated(const float &dy, const float &x, float a, float b) { return dy * gate1(axpb(x, a, b)); }
 __device__ __forceinline__ f32x4 gated(const f32x4 &dy, const f32x4 &x, float a, float b) {
   const f32x4 r = {gated(dy.x, x.x, a, b), gated(dy.y, x.y, a, b), gated(dy.z, x.z, a, b), gated(dy.w, x.w, a, b)};
+  return r;
+}
+// the same as Relu's gradient operator has it, NaN included
+__device__ __forceinline__ float gated_op(const float &dy, const float &x, float a, float b) { return relu_grad_of(axpb(x, a, b), dy); }
+__device__ __forceinline__ f32x4 gated_op(const f32x4 &dy, const f32x4 &x, float a, float b) {
+  const f32x4 r = {gated_op(dy.x, x.x, a, b), gated_op(dy.y, x.y, a, b), gated_op(dy.z, x.z, a, b), gated_op(dy.w, x.w, a, b)};
   return r;
 }
 __device__ __forceinline__ float lin2(const float &dy, const float &x, float k1, float k2, float k3) { return fmaf(k2, x, k1 * dy) + k3; }
@@ -201,8 +208,10 @@ __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restr
 
 // y = a*x + b (then Relu) over a (split, channel) grid: for planes too short for the plane-major kernel
 // and for arrays without 16-byte words
-template <int VEC, bool RELU>
-__global__ __launch_bounds__(kThreads) void bn_apply_kernel(const float *__restrict__ x, float *__restrict__ y,
+// kFused: y is Relu's result, the BatchNorm's own never leaves.  kBoth: y is the BatchNorm's, r Relu's of it.
+enum Pair { kAlone, kFused, kBoth };
+template <int VEC, int RELU>
+__global__ __launch_bounds__(kThreads) void bn_apply_kernel(const float *__restrict__ x, float *__restrict__ y, float *__restrict__ r,
                                                             const float *__restrict__ coef, Geo g) {
   using W = typename Word<VEC>::T;
   const int c = blockIdx.y;
@@ -216,13 +225,19 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(const float *__restr
   for (; i + kThreads < end; i += 2 * kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c), a1 = word_addr<VEC>(g, i + kThreads, c);
     const W v0 = __builtin_nontemporal_load(xw + a0), v1 = __builtin_nontemporal_load(xw + a1);
-    __builtin_nontemporal_store(RELU ? relu_w(axpb(v0, a, b)) : axpb(v0, a, b), yw + a0);
-    __builtin_nontemporal_store(RELU ? relu_w(axpb(v1, a, b)) : axpb(v1, a, b), yw + a1);
+    const W z0 = axpb(v0, a, b), z1 = axpb(v1, a, b);
+    __builtin_nontemporal_store(RELU == kFused ? relu_w(z0) : z0, yw + a0);
+    __builtin_nontemporal_store(RELU == kFused ? relu_w(z1) : z1, yw + a1);
+    if (RELU == kBoth) {
+      __builtin_nontemporal_store(relu_w(z0), reinterpret_cast<W *>(r) + a0);
+      __builtin_nontemporal_store(relu_w(z1), reinterpret_cast<W *>(r) + a1);
+    }
   }
   for (; i < end; i += kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c);
     const W z = axpb(__builtin_nontemporal_load(xw + a0), a, b);
-    __builtin_nontemporal_store(RELU ? relu_w(z) : z, yw + a0);
+    __builtin_nontemporal_store(RELU == kFused ? relu_w(z) : z, yw + a0);
+    if (RELU == kBoth) __builtin_nontemporal_store(relu_w(z), reinterpret_cast<W *>(r) + a0);
   }
 }
 
@@ -239,33 +254,37 @@ __device__ __forceinline__ uint32_t word_channel(const PlaneGeo &g, uint32_t i) 
   const uint32_t plane = g.wpp.div(i);
   return plane - g.chans.div(plane) * g.chans.d;
 }
-template <bool RELU>
-__global__ __launch_bounds__(kThreads) void bn_apply_plane_kernel(const f32x4 *__restrict__ x, f32x4 *__restrict__ y,
+template <int RELU>
+__global__ __launch_bounds__(kThreads) void bn_apply_plane_kernel(const f32x4 *__restrict__ x, f32x4 *__restrict__ y, f32x4 *__restrict__ r,
                                                                   const float *__restrict__ coef, PlaneGeo g) {
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= g.words) return;
   const uint32_t c = word_channel(g, i);
   const float a = coef[2 * c], b = coef[2 * c + 1];
   const f32x4 z = axpb(__builtin_nontemporal_load(x + i), a, b);
-  __builtin_nontemporal_store(RELU ? relu_w(z) : z, y + i);
+  __builtin_nontemporal_store(RELU == kFused ? relu_w(z) : z, y + i);
+  if (RELU == kBoth) __builtin_nontemporal_store(relu_w(z), r + i);
 }
 
 // partials per block: sum dy, sum dy*x, sum x, sum x^2
 // RELU: dy is the gradient behind a fused Relu; it is gated with relu'(a*x + b), a and b rebuilt
 // from the saved statistics (gamma, beta, save_mean, save_istd must be given).
-template <int VEC, bool STATS, bool RELU>
+// kBoth: dy is the gradient behind a Relu whose a and b lie in `pair`; the gradient of its input goes to dg.
+template <int VEC, bool STATS, int RELU>
 __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__restrict__ dy,
                                                                  const float *__restrict__ x,
                                                                  double *__restrict__ part, Geo g, int S,
                                                                  const float *__restrict__ gamma,
                                                                  const float *__restrict__ beta,
                                                                  const float *__restrict__ save_mean,
-                                                                 const float *__restrict__ save_istd, bool wide) {
+                                                                 const float *__restrict__ save_istd, bool wide,
+                                                                 const float *__restrict__ pair, float *__restrict__ dg) {
   using W = typename Word<VEC>::T;
   __shared__ double sm[4 * kWaves];
   const int c = blockIdx.y, s = blockIdx.x;
   float ga = 0.f, gb = 0.f;
-  if (RELU) {
+  if (RELU == kBoth) ga = pair[2 * c], gb = pair[2 * c + 1];
+  if (RELU == kFused) {
     // the same float expressions as the forward pass, so that the sign of a*x + b is the same
     const double a = static_cast<double>(gamma[c]) * saved_stat(save_istd, c, wide);
     ga = static_cast<float>(a);
@@ -287,7 +306,11 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
     }
 #pragma unroll
     for (int u = 0; u < kReadAhead; ++u) {
-      if (RELU) dv[u] = gated(dv[u], xv[u], ga, gb);
+      if (RELU == kFused) dv[u] = gated(dv[u], xv[u], ga, gb);
+      if (RELU == kBoth) {
+        dv[u] = gated_op(dv[u], xv[u], ga, gb);
+        reinterpret_cast<W *>(dg)[word_addr<VEC>(g, i + u * kThreads, c)] = dv[u];
+      }
       acc_dot(dv[u], xv[u], sdy, sdx);
       if (STATS) acc2(xv[u], sx, sq);
     }
@@ -295,7 +318,8 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
   for (; i < end; i += kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c);
     W x0 = xw[a0], d0 = dw[a0];
-    if (RELU) d0 = gated(d0, x0, ga, gb);
+    if (RELU == kFused) d0 = gated(d0, x0, ga, gb);
+    if (RELU == kBoth) reinterpret_cast<W *>(dg)[a0] = d0 = gated_op(d0, x0, ga, gb);
     acc_dot(d0, x0, sdy, sdx);
     if (STATS) acc2(x0, sx, sq);
   }
@@ -430,13 +454,14 @@ __device__ __forceinline__ int64_t chan_addr(const FastDiv &hw, uint32_t e, int 
 }
 
 // R: values per thread (compile-time bound of the register arrays)
-template <int R, bool RELU>
+template <int R, int RELU>
 __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *__restrict__ x, float *__restrict__ y,
                                                                   const float *__restrict__ gamma,
                                                                   const float *__restrict__ beta, FastDiv hw, int C,
                                                                   uint32_t m, float eps, double inv_m,
                                                                   float *__restrict__ save_mean,
-                                                                  float *__restrict__ save_istd, bool wide) {
+                                                                  float *__restrict__ save_istd, bool wide,
+                                                                  float *__restrict__ rl, float *__restrict__ pair) {
   __shared__ double sm[kWaves];
   __shared__ float coef[2];
   const int c = blockIdx.x;
@@ -466,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
   if (threadIdx.x == 0) {
     double istd = 1.0 / sqrt(var + static_cast<double>(eps));
     double mean_used = mean;
-    if (RELU && !wide) {      // as in bn_coef_kernel: coefficients from the rounded statistics the backward pass will read
+    if (RELU == kFused && !wide) {      // as in bn_coef_kernel: coefficients from the rounded statistics the backward pass will read
       mean_used = static_cast<double>(static_cast<float>(mean));
       istd = static_cast<double>(static_cast<float>(istd));
     }
@@ -478,29 +503,33 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
   }
   __syncthreads();
   const float a = coef[0], b = coef[1];
+  if (RELU == kBoth && threadIdx.x < 2) pair[2 * c + threadIdx.x] = coef[threadIdx.x];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const uint32_t e = r * kThreads + threadIdx.x;
     if (e < m) {
       const float z = axpb(v[r], a, b);
-      __builtin_nontemporal_store(RELU ? relu1(z) : z, y + chan_addr(hw, e, c, C));
+      __builtin_nontemporal_store(RELU == kFused ? relu1(z) : z, y + chan_addr(hw, e, c, C));
+      if (RELU == kBoth) __builtin_nontemporal_store(relu1(z), rl + chan_addr(hw, e, c, C));
     }
   }
 }
 
-template <int R, bool STATS, bool RELU>
+template <int R, bool STATS, int RELU>
 __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *__restrict__ dy, const float *__restrict__ x,
                                                                   float *__restrict__ dx, const float *__restrict__ gamma,
                                                                   const float *__restrict__ beta, FastDiv hw, int C,
                                                                   uint32_t m, float eps, double inv_m,
                                                                   const float *__restrict__ save_mean,
                                                                   const float *__restrict__ save_istd, bool wide,
-                                                                  float *__restrict__ dgamma, float *__restrict__ dbeta) {
+                                                                  float *__restrict__ dgamma, float *__restrict__ dbeta,
+                                                                  const float *__restrict__ pair, float *__restrict__ dg) {
   __shared__ double sm[kWaves];
   __shared__ float coef[3];
   const int c = blockIdx.x;
   float ga = 0.f, gb = 0.f;
-  if (RELU) {
+  if (RELU == kBoth) ga = pair[2 * c], gb = pair[2 * c + 1];
+  if (RELU == kFused) {
     const double a = static_cast<double>(gamma[c]) * saved_stat(save_istd, c, wide);
     ga = static_cast<float>(a);
     gb = static_cast<float>(static_cast<double>(beta[c]) - saved_stat(save_mean, c, wide) * a);
@@ -514,7 +543,12 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     const int64_t at = ok ? chan_addr(hw, e, c, C) : 0;
     xv[r] = ok ? __builtin_nontemporal_load(x + at) : 0.f;
     dv[r] = ok ? __builtin_nontemporal_load(dy + at) : 0.f;
-    if (RELU) dv[r] = gated(dv[r], xv[r], ga, gb);
+  }
+  if (RELU == kBoth) __builtin_amdgcn_sched_barrier(0);   // (with its selects the compiler waits for every load by itself: 43 us for 17)
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (RELU == kFused) dv[r] = gated(dv[r], xv[r], ga, gb);
+    if (RELU == kBoth) dv[r] = r * kThreads + threadIdx.x < m ? gated_op(dv[r], xv[r], ga, gb) : 0.f;
     acc_dot(dv[r], xv[r], sdy, sdx);
     if (STATS) acc2(xv[r], sx, sq);
   }
@@ -552,7 +586,10 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const uint32_t e = r * kThreads + threadIdx.x;
-    if (e < m) __builtin_nontemporal_store(lin2(dv[r], xv[r], k1, k2, k3), dx + chan_addr(hw, e, c, C));
+    if (e < m) {
+      if (RELU == kBoth) __builtin_nontemporal_store(dv[r], dg + chan_addr(hw, e, c, C));
+      __builtin_nontemporal_store(lin2(dv[r], xv[r], k1, k2, k3), dx + chan_addr(hw, e, c, C));
+    }
   }
 }
 
@@ -621,6 +658,17 @@ inline bool plane_major_ok(const Plan &pl, const DLArray *x, PlaneGeo &pg, unsig
   pg.words = static_cast<uint32_t>(words);
   blocks = static_cast<unsigned>((words + kThreads - 1) / kThreads);
   return true;
+}
+
+// dg = dy taken through Relu at a x + b (`pair`: a, b of every channel), in the order of memory
+template <int VEC>
+__global__ __launch_bounds__(kThreads) void bn_gate_kernel(const float *__restrict__ dy, const float *__restrict__ x,
+                                                           const float *__restrict__ pair, float *__restrict__ dg, PlaneGeo g) {
+  using W = typename Word<VEC>::T;
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= g.words) return;
+  const uint32_t c = word_channel(g, i);
+  reinterpret_cast<W *>(dg)[i] = gated_op(reinterpret_cast<const W *>(dy)[i], reinterpret_cast<const W *>(x)[i], pair[2 * c], pair[2 * c + 1]);
 }
 
 // ---------------------------------------------------------------- BatchNorm + Relu + 2x2 / stride 2 max pooling
@@ -865,14 +913,14 @@ static bool stats_fit(const DLArray *mean, const DLArray *istd, int64_t C, bool 
 // coefficients from the partial sums (pair k of channel c at part[(c * part_c + k * part_k) * 2]), then
 // the streaming pass y = a*x + b (+ Relu)
 static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t part_k, float *coef, const Plan &ap,
-                          bool relu, const DLArray *x, const DLArray *scale, const DLArray *bias, DLArray *y,
+                          int relu, float *r, const DLArray *x, const DLArray *scale, const DLArray *bias, DLArray *y,
                           float eps, DLArray *save_mean_arr, DLArray *save_var_arr, hipStream_t s) {
   const unsigned C = static_cast<unsigned>(x->shape[1]);
   const double inv_m = 1.0 / static_cast<double>(ap.m);
   float *sm = save_mean_arr ? mf(save_mean_arr) : nullptr;
   float *sv = save_var_arr ? mf(save_var_arr) : nullptr;
-  const bool wide = relu && wide_stats(save_mean_arr, C);
-  if (relu)
+  const bool wide = relu == kFused && wide_stats(save_mean_arr, C);
+  if (relu == kFused)
     hipLaunchKernelGGL(bn_coef_kernel<true>, dim3(C), dim3(kThreads), 0, s, part, S, part_c, part_k, cf(scale), cf(bias),
                        eps, inv_m, coef, sm, sv, wide);
   else
@@ -882,40 +930,37 @@ static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t par
   unsigned blocks = 0;
   if (plane_major_ok(ap, x, pg, blocks)) {
     const f32x4 *xw = reinterpret_cast<const f32x4 *>(x->data);
-    f32x4 *yw = reinterpret_cast<f32x4 *>(y->data);
-    if (relu)
-      hipLaunchKernelGGL(bn_apply_plane_kernel<true>, dim3(blocks), dim3(kThreads), 0, s, xw, yw, coef, pg);
-    else
-      hipLaunchKernelGGL(bn_apply_plane_kernel<false>, dim3(blocks), dim3(kThreads), 0, s, xw, yw, coef, pg);
+    f32x4 *yw = reinterpret_cast<f32x4 *>(y->data), *rw = reinterpret_cast<f32x4 *>(r);
+    const auto kernel = relu == kBoth ? bn_apply_plane_kernel<kBoth> : relu == kFused ? bn_apply_plane_kernel<kFused> : bn_apply_plane_kernel<kAlone>;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, xw, yw, rw, coef, pg);
     return;
   }
   const dim3 ga(ap.S, C);
-#define BN_APPLY(V, R) \
-  hipLaunchKernelGGL((bn_apply_kernel<V, R>), ga, dim3(kThreads), 0, s, cf(x), mf(y), static_cast<const float *>(coef), ap.g)
-  if (ap.vec == 4) {
-    if (relu)
-      BN_APPLY(4, true);
-    else
-      BN_APPLY(4, false);
-  } else {
-    if (relu)
-      BN_APPLY(1, true);
-    else
-      BN_APPLY(1, false);
-  }
+#define BN_APPLY(V)                                                                                                                        \
+  hipLaunchKernelGGL((relu == kBoth ? bn_apply_kernel<V, kBoth> : relu == kFused ? bn_apply_kernel<V, kFused> : bn_apply_kernel<V, kAlone>), \
+                     ga, dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), ap.g)
+  if (ap.vec == 4)
+    BN_APPLY(4);
+  else
+    BN_APPLY(1);
 #undef BN_APPLY
 }
 
-static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, const DLArrayHandle bn_scale,
+static int bn_forward(const char *who, int relu, const DLArrayHandle input_X, const DLArrayHandle bn_scale,
                       const DLArrayHandle bn_bias, DLArrayHandle output_Y, float eps, DLArrayHandle save_mean_arr,
-                      DLArrayHandle save_var_arr, DLStreamHandle stream_handle, ProfilerHandle p) {
+                      DLArrayHandle save_var_arr, DLStreamHandle stream_handle, ProfilerHandle p, DLArrayHandle relu_R = nullptr,
+                      DLArrayHandle pair_arr = nullptr) {
   TS_REQUIRE(input_X && bn_scale && bn_bias && output_Y, "%s: NULL array", who);
   TS_REQUIRE(input_X->ndim == 4 && output_Y->ndim == 4, "%s: input and output must be 4-D NCHW", who);
   TS_REQUIRE(numel(input_X) == numel(output_Y), "%s: input/output sizes differ", who);
   const int64_t C = input_X->shape[1];
   TS_REQUIRE(numel(bn_scale) == C && numel(bn_bias) == C, "%s: scale/bias must hold C=%lld elements", who, (long long)C);
-  TS_REQUIRE(stats_fit(save_mean_arr, save_var_arr, C, relu), "%s: save_mean and save_var must hold C elements each", who);
-  TS_REQUIRE(!relu || (save_mean_arr && save_var_arr), "%s: the fused form needs both save arrays", who);
+  TS_REQUIRE(relu != kBoth || (relu_R && pair_arr && numel(relu_R) == numel(input_X) && numel(pair_arr) == 2 * C &&
+                               relu_R->data != output_Y->data && relu_R->data != input_X->data),
+             "%s: Relu's result is another array of the input's size, the pair's coefficients take 2 C elements", who);
+  float *const r = relu == kBoth ? mf(relu_R) : nullptr, *const pair = relu == kBoth ? mf(pair_arr) : nullptr;
+  TS_REQUIRE(stats_fit(save_mean_arr, save_var_arr, C, relu == kFused), "%s: save_mean and save_var must hold C elements each", who);
+  TS_REQUIRE(relu != kFused || (save_mean_arr && save_var_arr), "%s: the fused form needs both save arrays", who);
   // sums a convolution left for exactly this tensor on this stream (common.h): looked up before
   // stream_of() ends all notes, since this call writes too
   const double *note_sums = nullptr;
@@ -928,12 +973,12 @@ static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, c
     // the later convolutions that reuse the sums' memory are ordered behind this call on its stream
     g_bn_from_notes.fetch_add(1, std::memory_order_relaxed);
     ProfileScope psn(p, s, numel(input_X) + 2 * C, numel(output_Y), 0);
-    const bool aln = aligned16(input_X->data) && aligned16(output_Y->data);
+    const bool aln = aligned16(input_X->data) && aligned16(output_Y->data) && aligned16(r);
     Plan apn;
     TS_REQUIRE(make_plan(input_X, aln, 4 * kThreads, 1 << 22, apn), "%s: unsupported shape", who);
-    float *coefn = static_cast<float *>(scratch_get(s, 1, static_cast<size_t>(C) * 2 * sizeof(float)));
+    float *coefn = pair ? pair : static_cast<float *>(scratch_get(s, 1, static_cast<size_t>(C) * 2 * sizeof(float)));
     TS_REQUIRE(coefn, "%s: no scratch memory", who);
-    bn_apply_from(note_sums, note_slots, 1, C, coefn, apn, relu, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr,
+    bn_apply_from(note_sums, note_slots, 1, C, coefn, apn, relu, r, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr,
                   save_var_arr, s);
     return psn.finish();
   }
@@ -947,7 +992,7 @@ static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, c
 #define BN_FWD1(R, RL)                                                                                              \
   hipLaunchKernelGGL((bn_fwd_onepass_kernel<R, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,         \
                      cf(input_X), mf(output_Y), cf(bn_scale), cf(bn_bias), FastDiv(hw), static_cast<int>(C), m, eps, \
-                     1.0 / static_cast<double>(m), sm1, sv1, relu && wide_stats(save_mean_arr, C))
+                     1.0 / static_cast<double>(m), sm1, sv1, relu == kFused && wide_stats(save_mean_arr, C), r, pair)
 #define BN_FWD1_R(RL)   \
   do {                  \
     if (per <= 16)      \
@@ -957,15 +1002,17 @@ static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, c
     else                \
       BN_FWD1(64, RL);  \
   } while (0)
-    if (relu)
-      BN_FWD1_R(true);
+    if (relu == kBoth)
+      BN_FWD1_R(kBoth);
+    else if (relu == kFused)
+      BN_FWD1_R(kFused);
     else
-      BN_FWD1_R(false);
+      BN_FWD1_R(kAlone);
 #undef BN_FWD1_R
 #undef BN_FWD1
     return ps1.finish();
   }
-  const bool al = aligned16(input_X->data) && aligned16(output_Y->data);
+  const bool al = aligned16(input_X->data) && aligned16(output_Y->data) && aligned16(r);
   Plan st, ap;
   TS_REQUIRE(make_plan(input_X, al, kStatsWords, 16384, st), "%s: unsupported shape", who);
   TS_REQUIRE(make_plan(input_X, al, 4 * kThreads, 1 << 22, ap), "%s: unsupported shape", who);
@@ -973,14 +1020,14 @@ static int bn_forward(const char *who, bool relu, const DLArrayHandle input_X, c
   const size_t part_bytes = static_cast<size_t>(C) * st.S * 2 * sizeof(double);
   double *part = static_cast<double *>(scratch_get(s, 1, part_bytes + static_cast<size_t>(C) * 2 * sizeof(float)));
   TS_REQUIRE(part, "%s: no scratch memory", who);
-  float *coef = reinterpret_cast<float *>(part + static_cast<size_t>(C) * st.S * 2);
+  float *coef = pair ? pair : reinterpret_cast<float *>(part + static_cast<size_t>(C) * st.S * 2);
   ProfileScope ps(p, s, numel(input_X) + 2 * C, numel(output_Y), C * st.S * 4);
   const dim3 gs(st.S, static_cast<unsigned>(C));
   if (st.vec == 4)
     hipLaunchKernelGGL(bn_stats_kernel<4>, gs, dim3(kThreads), 0, s, cf(input_X), part, st.g, st.S);
   else
     hipLaunchKernelGGL(bn_stats_kernel<1>, gs, dim3(kThreads), 0, s, cf(input_X), part, st.g, st.S);
-  bn_apply_from(part, st.S, static_cast<int64_t>(st.S), 1, coef, ap, relu, input_X, bn_scale, bn_bias, output_Y, eps,
+  bn_apply_from(part, st.S, static_cast<int64_t>(st.S), 1, coef, ap, relu, r, input_X, bn_scale, bn_bias, output_Y, eps,
                 save_mean_arr, save_var_arr, s);
   return ps.finish();
 }
@@ -990,14 +1037,14 @@ int CuDNN_DLGpuBatch_Normalization(const DLArrayHandle input_X, const DLArrayHan
                                    DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                                    DLStreamHandle stream_handle, ProfilerHandle p) {
   (void)momentum;
-  return bn_forward("BatchNorm", false, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr, save_var_arr,
+  return bn_forward("BatchNorm", kAlone, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr, save_var_arr,
                     stream_handle, p);
 }
 
 int TSplit_BatchNormRelu(const DLArrayHandle input_X, const DLArrayHandle bn_scale, const DLArrayHandle bn_bias,
                          DLArrayHandle output_Y, float eps, DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                          DLStreamHandle stream_handle, ProfilerHandle p) {
-  return bn_forward("TSplit_BatchNormRelu", true, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr,
+  return bn_forward("TSplit_BatchNormRelu", kFused, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr,
                     save_var_arr, stream_handle, p);
 }
 
@@ -1028,16 +1075,16 @@ int TSplit_BatchNormFromStats(const DLArrayHandle input_X, const DLArrayHandle s
   TS_REQUIRE(make_plan(input_X, al, 4 * kThreads, 1 << 22, ap), "%s: unsupported shape", who);
   float *coef = static_cast<float *>(scratch_get(s, 1, static_cast<size_t>(C) * 2 * sizeof(float)));
   TS_REQUIRE(coef, "%s: no scratch memory", who);
-  bn_apply_from(static_cast<const double *>(stats->data), slots, 1, C, coef, ap, relu != 0, input_X, bn_scale, bn_bias,
+  bn_apply_from(static_cast<const double *>(stats->data), slots, 1, C, coef, ap, relu != 0 ? kFused : kAlone, nullptr, input_X, bn_scale, bn_bias,
                 output_Y, eps, save_mean_arr, save_var_arr, s);
   return ps.finish();
 }
 
-static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_Y, const DLArrayHandle input_X,
+static int bn_backward(const char *who, int relu, const DLArrayHandle gradient_Y, const DLArrayHandle input_X,
                        const DLArrayHandle bn_scale, const DLArrayHandle bn_bias, DLArrayHandle gradient_X,
                        DLArrayHandle gradient_bn_scale, DLArrayHandle gradient_bn_bias, float eps,
                        DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr, DLStreamHandle stream_handle,
-                       ProfilerHandle p) {
+                       ProfilerHandle p, const DLArrayHandle pair_arr = nullptr, DLArrayHandle gradient_R = nullptr) {
   TS_REQUIRE(gradient_Y && input_X && bn_scale && gradient_X, "%s: NULL array", who);
   TS_REQUIRE(input_X->ndim == 4, "%s: input must be 4-D NCHW", who);
   TS_REQUIRE(numel(input_X) == numel(gradient_Y) && numel(input_X) == numel(gradient_X), "%s: x, dy, dx sizes differ", who);
@@ -1046,9 +1093,15 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
   TS_REQUIRE(!gradient_bn_scale || numel(gradient_bn_scale) == C, "%s: dscale must hold C elements", who);
   TS_REQUIRE(!gradient_bn_bias || numel(gradient_bn_bias) == C, "%s: dbias must hold C elements", who);
   const bool saved = save_mean_arr && save_var_arr;
-  TS_REQUIRE(!saved || stats_fit(save_mean_arr, save_var_arr, C, relu), "%s: saved statistics must hold C elements", who);
-  const bool wide = relu && wide_stats(save_mean_arr, C);
-  TS_REQUIRE(!relu || (saved && bn_bias && numel(bn_bias) == C),
+  TS_REQUIRE(!saved || stats_fit(save_mean_arr, save_var_arr, C, relu == kFused), "%s: saved statistics must hold C elements", who);
+  TS_REQUIRE(relu != kBoth || (pair_arr && gradient_R && numel(pair_arr) == 2 * C && numel(gradient_R) == numel(input_X) &&
+                               gradient_R->data != input_X->data && gradient_R->data != gradient_X->data &&
+                               gradient_R->data != gradient_Y->data),
+             "%s: the gradient of Relu's input is another array of the input's size, the pair's coefficients are of 2 C elements", who);
+  const bool wide = relu == kFused && wide_stats(save_mean_arr, C);
+  const float *const pair = relu == kBoth ? cf(pair_arr) : nullptr;
+  float *const dr = relu == kBoth ? mf(gradient_R) : nullptr;
+  TS_REQUIRE(relu != kFused || (saved && bn_bias && numel(bn_bias) == C),
              "%s: the fused form needs the bias and the statistics saved by the fused forward call", who);
   hipStream_t s = stream_of(stream_handle);
   if (one_pass_ok(input_X)) {
@@ -1061,10 +1114,24 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
     float *dg1 = gradient_bn_scale ? mf(gradient_bn_scale) : nullptr;
     float *db1 = gradient_bn_bias ? mf(gradient_bn_bias) : nullptr;
     const int per = static_cast<int>((m + kThreads - 1) / kThreads);
+    const float *dy1 = cf(gradient_Y);
+    if (relu == kBoth && per > 16) {
+      // a block a channel writes two arrays of this size no faster than one after the other, a launch over all of them does (128
+      // channels of 16 K values: one launch 34 us, 17 + 5 as two; 512 of 4 K or less 7 and 6 + 4)
+      PlaneGeo pg;
+      const bool words = hw % 4 == 0 && aligned16(dy1) && aligned16(input_X->data) && aligned16(dr);
+      pg.wpp = FastDiv(words ? hw / 4 : hw);
+      pg.chans = FastDiv(static_cast<uint32_t>(C));
+      pg.words = static_cast<uint32_t>(numel(input_X) / (words ? 4 : 1));
+      hipLaunchKernelGGL((words ? bn_gate_kernel<4> : bn_gate_kernel<1>), dim3((pg.words + kThreads - 1) / kThreads), dim3(kThreads), 0, s, dy1,
+                         cf(input_X), pair, dr, pg);
+      dy1 = dr;
+      relu = kAlone;
+    }
 #define BN_BWD1(R, ST, RL)                                                                                          \
   hipLaunchKernelGGL((bn_bwd_onepass_kernel<R, ST, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,     \
-                     cf(gradient_Y), cf(input_X), mf(gradient_X), cf(bn_scale), bias1, FastDiv(hw),                 \
-                     static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, sv1, wide, dg1, db1)
+                     dy1, cf(input_X), mf(gradient_X), cf(bn_scale), bias1, FastDiv(hw),                 \
+                     static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, sv1, wide, dg1, db1, pair, dr)
 #define BN_BWD1_R(ST, RL)   \
   do {                      \
     if (per <= 16)          \
@@ -1074,19 +1141,23 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
     else                    \
       BN_BWD1(64, ST, RL);  \
   } while (0)
-    if (wide)
-      BN_BWD1_R(true, true);
+    if (relu == kBoth && saved)
+      BN_BWD1(16, false, kBoth);
+    else if (relu == kBoth)
+      BN_BWD1(16, true, kBoth);
+    else if (wide)
+      BN_BWD1_R(true, kFused);
     else if (relu)
-      BN_BWD1_R(false, true);
+      BN_BWD1_R(false, kFused);
     else if (saved)
-      BN_BWD1_R(false, false);
+      BN_BWD1_R(false, kAlone);
     else
-      BN_BWD1_R(true, false);
+      BN_BWD1_R(true, kAlone);
 #undef BN_BWD1_R
 #undef BN_BWD1
     return ps1.finish();
   }
-  const bool al = aligned16(input_X->data) && aligned16(gradient_Y->data) && aligned16(gradient_X->data);
+  const bool al = aligned16(input_X->data) && aligned16(gradient_Y->data) && aligned16(gradient_X->data) && aligned16(dr);
   Plan rd, dxp;
   TS_REQUIRE(make_plan(input_X, al, kStatsWords, 16384, rd), "%s: unsupported shape", who);
   TS_REQUIRE(make_plan(input_X, al, 4 * kThreads, 1 << 22, dxp), "%s: unsupported shape", who);
@@ -1107,39 +1178,47 @@ static int bn_backward(const char *who, bool relu, const DLArrayHandle gradient_
   PlaneGeo pg;
   unsigned blocks = 0;
   const bool plane_major = plane_major_ok(dxp, input_X, pg, blocks);
-  const f32x4 *xw = reinterpret_cast<const f32x4 *>(input_X->data), *dyw = reinterpret_cast<const f32x4 *>(gradient_Y->data);
+  const f32x4 *xw = reinterpret_cast<const f32x4 *>(input_X->data), *dyw = reinterpret_cast<const f32x4 *>(dr ? dr : cf(gradient_Y));
   f32x4 *dxw = reinterpret_cast<f32x4 *>(gradient_X->data);
 #define BN_BWD(V, ST, R)                                                                                            \
   do {                                                                                                              \
     hipLaunchKernelGGL((bn_bwd_reduce_kernel<V, ST, R>), gr, dim3(kThreads), 0, s, cf(gradient_Y), cf(input_X),     \
-                       part, rd.g, rd.S, cf(bn_scale), bias, sm, sv, wide);                                               \
-    hipLaunchKernelGGL((bn_bwd_coef_kernel<R>), dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(part),  \
+                       part, rd.g, rd.S, cf(bn_scale), bias, sm, sv, wide, pair, dr);                                               \
+    hipLaunchKernelGGL((bn_bwd_coef_kernel<R == kFused>), dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(part),  \
                        rd.S, cf(bn_scale), bias, eps, inv_m, sm, sv, wide, coef, dg, db);                                 \
     if (V == 4 && plane_major)                                                                                      \
-      hipLaunchKernelGGL((bn_bwd_dx_plane_kernel<R>), dim3(blocks), dim3(kThreads), 0, s, dyw, xw, dxw,             \
+      hipLaunchKernelGGL((bn_bwd_dx_plane_kernel<R == kFused>), dim3(blocks), dim3(kThreads), 0, s, dyw, xw, dxw,             \
                          static_cast<const float *>(coef), pg);                                                     \
     else                                                                                                            \
-      hipLaunchKernelGGL((bn_bwd_dx_kernel<V, R>), gd, dim3(kThreads), 0, s, cf(gradient_Y), cf(input_X),           \
+      hipLaunchKernelGGL((bn_bwd_dx_kernel<V, R == kFused>), gd, dim3(kThreads), 0, s, dr ? dr : cf(gradient_Y), cf(input_X),           \
                          mf(gradient_X), static_cast<const float *>(coef), dxp.g);                                  \
   } while (0)
   if (rd.vec == 4) {
-    if (wide)
-      BN_BWD(4, true, true);
+    if (relu == kBoth && saved)
+      BN_BWD(4, false, kBoth);
+    else if (relu == kBoth)
+      BN_BWD(4, true, kBoth);
+    else if (wide)
+      BN_BWD(4, true, kFused);
     else if (relu)
-      BN_BWD(4, false, true);
+      BN_BWD(4, false, kFused);
     else if (saved)
-      BN_BWD(4, false, false);
+      BN_BWD(4, false, kAlone);
     else
-      BN_BWD(4, true, false);
+      BN_BWD(4, true, kAlone);
   } else {
-    if (wide)
-      BN_BWD(1, true, true);
+    if (relu == kBoth && saved)
+      BN_BWD(1, false, kBoth);
+    else if (relu == kBoth)
+      BN_BWD(1, true, kBoth);
+    else if (wide)
+      BN_BWD(1, true, kFused);
     else if (relu)
-      BN_BWD(1, false, true);
+      BN_BWD(1, false, kFused);
     else if (saved)
-      BN_BWD(1, false, false);
+      BN_BWD(1, false, kAlone);
     else
-      BN_BWD(1, true, false);
+      BN_BWD(1, true, kAlone);
   }
 #undef BN_BWD
   return ps.finish();
@@ -1150,7 +1229,7 @@ int CuDNN_DLGpuBatch_Normalization_gradient(const DLArrayHandle gradient_Y, cons
                                             DLArrayHandle gradient_bn_scale, DLArrayHandle gradient_bn_bias,
                                             float eps, DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                                             DLStreamHandle stream_handle, ProfilerHandle p) {
-  return bn_backward("BatchNorm gradient", false, gradient_Y, input_X, bn_scale, nullptr, gradient_X, gradient_bn_scale,
+  return bn_backward("BatchNorm gradient", kAlone, gradient_Y, input_X, bn_scale, nullptr, gradient_X, gradient_bn_scale,
                      gradient_bn_bias, eps, save_mean_arr, save_var_arr, stream_handle, p);
 }
 
@@ -1159,8 +1238,25 @@ int TSplit_BatchNormRelu_gradient(const DLArrayHandle gradient_Y, const DLArrayH
                                   DLArrayHandle gradient_bn_scale, DLArrayHandle gradient_bn_bias, float eps,
                                   DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                                   DLStreamHandle stream_handle, ProfilerHandle p) {
-  return bn_backward("TSplit_BatchNormRelu_gradient", true, gradient_Y, input_X, bn_scale, bn_bias, gradient_X,
+  return bn_backward("TSplit_BatchNormRelu_gradient", kFused, gradient_Y, input_X, bn_scale, bn_bias, gradient_X,
                      gradient_bn_scale, gradient_bn_bias, eps, save_mean_arr, save_var_arr, stream_handle, p);
+}
+
+// CuDNN_DLGpuBatch_Normalization and DLGpuRelu of its output, and their gradients, as one call each way that writes what the two write:
+// the forward pass reads the BatchNorm's output no more, the gradient's sums are taken while Relu's gradient is written.
+int TSplit_BatchNormThenRelu(const DLArrayHandle input_X, const DLArrayHandle bn_scale, const DLArrayHandle bn_bias, DLArrayHandle output_Y,
+                             DLArrayHandle relu_R, DLArrayHandle pair, float eps, DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
+                             DLStreamHandle stream_handle, ProfilerHandle p) {
+  return bn_forward("TSplit_BatchNormThenRelu", kBoth, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr, save_var_arr, stream_handle, p,
+                    relu_R, pair);
+}
+
+int TSplit_BatchNormThenRelu_gradient(const DLArrayHandle gradient_R, const DLArrayHandle input_X, const DLArrayHandle bn_scale,
+                                      const DLArrayHandle pair, DLArrayHandle gradient_Y, DLArrayHandle gradient_X, DLArrayHandle gradient_bn_scale,
+                                      DLArrayHandle gradient_bn_bias, float eps, DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
+                                      DLStreamHandle stream_handle, ProfilerHandle p) {
+  return bn_backward("TSplit_BatchNormThenRelu_gradient", kBoth, gradient_R, input_X, bn_scale, nullptr, gradient_X, gradient_bn_scale,
+                     gradient_bn_bias, eps, save_mean_arr, save_var_arr, stream_handle, p, pair, gradient_Y);
 }
 
 // ---- BatchNorm + Relu + 2x2 / stride 2 max pooling as one call each way (outside the reference's ABI) ----

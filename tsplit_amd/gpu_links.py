@@ -26,7 +26,7 @@ __all__ = [
     "matrix_transpose", "batch_matrix_multiply", "one_hot", "where", "embedding_lookup",
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
-    "batch_norm_relu", "batch_norm_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
+    "batch_norm_relu", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
     "optimizer_update_multi", "matrix_multiply_add", "heads_matrix_multiply",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "lstm_sizes", "lstm", "lstm_gradient",
@@ -527,6 +527,24 @@ def batch_norm_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_
                     profiler=None):
     check_call(_LIB.TSplit_BatchNormRelu(_h(in_arr), _h(bn_scale_arr), _h(bn_bias_arr), _h(out_arr),
                                          ctypes.c_float(eps), _h(save_mean), _h(save_var), _s(stream), _p(profiler)))
+
+
+def batch_norm_then_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, relu_arr, pair, save_mean=None, save_var=None, eps=0.01, stream=None,
+                         profiler=None):
+    """out_arr = BatchNorm, relu_arr = Relu of it: CuDNN_Batch_Normalization and relu in one call, with their bits; `pair` (2 C
+    values) is what the gradient reads again."""
+    check_call(_LIB.TSplit_BatchNormThenRelu(_h(in_arr), _h(bn_scale_arr), _h(bn_bias_arr), _h(out_arr), _h(relu_arr), _h(pair),
+                                             ctypes.c_float(eps), _h(save_mean) if save_mean else None, _h(save_var) if save_var else None,
+                                             _s(stream), _p(profiler)))
+
+
+def batch_norm_then_relu_gradient(in_gradient, in_arr, in_bn_scale, pair, out_gradient_y, out_gradient_x, out_gradient_bn_scale,
+                                  out_gradient_bn_bias, saved_mean=None, saved_var=None, eps=0.01, stream=None, profiler=None):
+    """relu_gradient and CuDNN_Batch_Normalization_gradient in one call, with their bits; out_gradient_y: between the two."""
+    check_call(_LIB.TSplit_BatchNormThenRelu_gradient(
+        _h(in_gradient), _h(in_arr), _h(in_bn_scale), _h(pair), _h(out_gradient_y), _h(out_gradient_x), _h(out_gradient_bn_scale),
+        _h(out_gradient_bn_bias), ctypes.c_float(eps), _h(saved_mean) if saved_mean else None, _h(saved_var) if saved_var else None,
+        _s(stream), _p(profiler)))
 
 
 def batch_norm_relu_max_pool(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var, eps=0.01, stats=None, slots=0,

@@ -140,7 +140,10 @@ class Trainer(object):
         kinds = [l[0] for l in self.spec]
         self.relu_of_fc = {li for li in range(1, len(kinds)) if kinds[li] == "relu" and kinds[li - 1] == "fc"}
         self.relu_before_fc = {li for li in range(1, len(kinds) - 1)
-                               if kinds[li] == "relu" and kinds[li + 1] == "fc" and li - 1 not in self.fused}
+                               if kinds[li] == "relu" and kinds[li + 1] == "fc" and kinds[li - 1] != "bn"}
+        # otherwise the pair is one call each way that writes both layers' arrays, with the bits of the two calls
+        self.pairs = {li: None for li, l in enumerate(self.spec[:-1])
+                      if l[0] == "bn" and self.spec[li + 1][0] == "relu" and li not in self.fused and not conv_bn_stats}
         # with conv_bn_stats a ("conv", ...) layer directly followed by ("bn", ...) hands the BatchNorm its
         # batch statistics (one row of sums per micro-tensor; symbols outside the reference's ABI), so
         # the BatchNorm reads the convolution's output once instead of twice
@@ -183,6 +186,8 @@ class Trainer(object):
             if layer[0] == "bn":
                 c = layer[2]
                 self.saved[li] = (ndarray.empty((1, c, 1, 1), self.ctx), ndarray.empty((1, c, 1, 1), self.ctx))
+                if li in self.pairs:
+                    self.pairs[li] = ndarray.empty((c, 2), self.ctx)
             if layer[0] == "conv" and li in self.split:
                 self.acts[-1].split_tensor(self.split[li])
                 self.dacts[-1].split_tensor(self.split[li])
@@ -269,12 +274,17 @@ class Trainer(object):
                 # writes the Relu layer's output directly
                 self._run("bn_relu_fwd", 8.0 * n(shapes[li]), "byte", L.batch_norm_relu, a, self.params[name + "_scale"],
                           self.params[name + "_bias"], self.acts[li + 2], sm, sv, self.eps)
+            elif kind == "bn" and li in self.pairs:
+                name = layer[1]
+                sm, sv = self.saved[li]
+                self._run("bn_then_relu_fwd", 12.0 * n(shapes[li]), "byte", L.batch_norm_then_relu, a, self.params[name + "_scale"],
+                          self.params[name + "_bias"], out, self.acts[li + 2], self.pairs[li], sm, sv, self.eps)
             elif kind == "bn":
                 name = layer[1]
                 sm, sv = self.saved[li]
                 self._run("bn_fwd", 8.0 * n(shapes[li]), "byte", L.CuDNN_Batch_Normalization, a,
                           self.params[name + "_scale"], self.params[name + "_bias"], out, sm, sv, 0.99, self.eps)
-            elif kind == "relu" and (li - 1 in self.fused or li in self.relu_of_fc):
+            elif kind == "relu" and (li - 1 in self.fused or li - 1 in self.pairs or li in self.relu_of_fc):
                 pass
             elif kind == "relu":
                 self._run("relu_fwd", 8.0 * n(shapes[li]), "byte", L.relu, a, out)
@@ -350,13 +360,20 @@ class Trainer(object):
                 self._run("bn_relu_bwd", 12.0 * n(shapes[li]), "byte", L.batch_norm_relu_gradient, self.dacts[li + 2], a,
                           self.params[name + "_scale"], self.params[name + "_bias"], g_in,
                           self.grads[name + "_scale"], self.grads[name + "_bias"], sm, sv, self.eps)
+            elif kind == "bn" and li in self.pairs:
+                name = layer[1]
+                sm, sv = self.saved[li]
+                # consumes the gradient behind the Relu layer, writes the one in front of it too
+                self._run("bn_then_relu_bwd", 16.0 * n(shapes[li]), "byte", L.batch_norm_then_relu_gradient, self.dacts[li + 2], a,
+                          self.params[name + "_scale"], self.pairs[li], g_out, g_in, self.grads[name + "_scale"],
+                          self.grads[name + "_bias"], sm, sv, self.eps)
             elif kind == "bn":
                 name = layer[1]
                 sm, sv = self.saved[li]
                 self._run("bn_bwd", 12.0 * n(shapes[li]), "byte", L.CuDNN_Batch_Normalization_gradient, g_out, a,
                           self.params[name + "_scale"], g_in, self.grads[name + "_scale"],
                           self.grads[name + "_bias"], sm, sv, self.eps)
-            elif kind == "relu" and (li - 1 in self.fused or li in self.relu_before_fc):
+            elif kind == "relu" and (li - 1 in self.fused or li - 1 in self.pairs or li in self.relu_before_fc):
                 pass
             elif kind == "relu":
                 self._run("relu_bwd", 12.0 * n(shapes[li]), "byte", L.relu_gradient, a, g_out, g_in)
