@@ -507,6 +507,10 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
 int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
                              const DLArrayHandle bias, const DLArrayHandle addend, const DLArrayHandle gate,
                              DLArrayHandle matC, DLArrayHandle relu, DLStreamHandle stream);
+/* C [M, N] = A' B and sums [N] = the sums of B's columns, A and B of K rows (the last axis' columns): a linear layer's parameter
+ * gradients.  C has the bits of DLGpuMatrixMultiply. */
+int TSplit_MatrixMultiplySums(const DLArrayHandle matA, const DLArrayHandle matB, DLArrayHandle matC, DLArrayHandle sums,
+                              DLStreamHandle stream);
 int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
                                DLArrayHandle matC, int heads, float alpha, const DLArrayHandle mask,
                                float mask_value, int causal, float fill, const DLArrayHandle addend,

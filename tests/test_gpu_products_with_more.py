@@ -56,6 +56,36 @@ def test_product_with_bias_addend_and_relu(shape, ta, tb, rng):
     np.testing.assert_array_equal(acc.asnumpy(), product + add)
 
 
+# tiles' edges, one range and many, depths off the steps, columns that are no words, one column; operands of three axes; split-bf16
+@pytest.mark.parametrize("shape", [(1, 1, 1), (64, 64, 32), (65, 130, 33), (33, 35, 5000), (512, 512, 8192), (256, 1024, 250), (130, 66, 2047), (784, 10, 100)])
+def test_product_with_column_sums(shape, rng):
+    """Bar of the sums: every value passes at most 40 roundings of partial sums (pairs in a step, eight steps, 64 groups of steps as a tree
+    of ranges), each below 2^-24 of the sum of magnitudes."""
+    from tsplit_amd import gpu_links as L
+    M, N, K = shape
+    a, b = rng.normal(size=(K, M)).astype(np.float32), (rng.normal(size=(K, N)) + 0.5).astype(np.float32)
+    ga, gb = _dev(a, b)
+    plain = _full((M, N))
+    L.matrix_multiply(ga, True, gb, False, plain)
+    for split in (False, True):
+        c, sums = _full((M, N)), _full((N,))
+        was = L.split_bf16(split)
+        try:
+            L.matrix_multiply_sums(ga, gb, c, sums)
+        finally:
+            L.split_bf16(was)
+        if not split:
+            np.testing.assert_array_equal(c.asnumpy(), plain.asnumpy())
+        assert np.all(np.abs(sums.asnumpy() - b.astype(np.float64).sum(0)) <= 40 * EPS * np.abs(b.astype(np.float64)).sum(0))
+    if K % 2 == 0:
+        from tsplit_amd import ndarray as nd
+        c, sums = _full((M, N)), _full((N,))
+        L.matrix_multiply_sums(nd.view(ga, (2, K // 2, M)), nd.view(gb, (2, K // 2, N)), c, sums)
+        np.testing.assert_array_equal(c.asnumpy(), plain.asnumpy())
+    with pytest.raises(RuntimeError):
+        L.matrix_multiply_sums(ga, gb, plain, _full((N + 1,)))
+
+
 def test_product_with_more_split_bf16_and_arrays_of_more_axes(rng):
     from tsplit_amd import gpu_links as L
     x, w, add = rng.normal(size=(3, 7, 40)).astype(np.float32), rng.normal(size=(40, 36)).astype(np.float32), rng.normal(size=(3, 7, 36)).astype(np.float32)

@@ -121,6 +121,40 @@ int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, flo
   return 0;
 }
 
+// C = A^T B and the column sums of B, where the tile kernel takes the product: false elsewhere
+template <int TM, int TN>
+void launch_sums_tile(const float *A, int64_t lda, const float *B, int64_t ldb, float *out, float *sums, int64_t zs, int M, int N, int K,
+                      const Plan &plan, hipStream_t s) {
+  using T = gt::Tile<TM, TN, 2, 2, true, false>;
+  const int tm = (M + T::BM - 1) / T::BM, tn = (N + T::BN - 1) / T::BN;
+  const bool wide = N % 4 == 0 && zs % 4 == 0 && aligned16(out);
+  hipLaunchKernelGGL((gt::gemm_sums_kernel<TM, TN>), dim3(grid_blocks(tm, tn, plan.S)), dim3(gt::kThreads), 0, s, DenseParams{A, lda, M, K},
+                     DenseParams{B, ldb, N, K}, out, sums, zs, wide, M, N, K, plan.kchunk, TileGrid{tm, tn, tm * tn * plan.S});
+}
+int launch_sums(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, float *sums, int M, int N, int K, hipStream_t s) {
+  const Plan plan = plan_product(M, N, K, 1, true);
+  const int64_t mn = static_cast<int64_t>(M) * N, n = mn + N;
+  float *out = C, *to = sums;
+  if (plan.S > 1) {
+    out = static_cast<float *>(scratch_get(s, 2, static_cast<size_t>(plan.S) * n * 4));
+    TS_REQUIRE(out, "TSplit_MatrixMultiplySums: no scratch memory for split-K");
+    to = out + mn;
+  }
+  const int64_t zs = plan.S > 1 ? n : 0;
+  switch (plan.tile) {
+    case 0: launch_sums_tile<4, 4>(A, lda, B, ldb, out, to, zs, M, N, K, plan, s); break;
+    case 1: launch_sums_tile<2, 4>(A, lda, B, ldb, out, to, zs, M, N, K, plan, s); break;
+    case 2: launch_sums_tile<4, 2>(A, lda, B, ldb, out, to, zs, M, N, K, plan, s); break;
+    default: launch_sums_tile<2, 2>(A, lda, B, ldb, out, to, zs, M, N, K, plan, s); break;
+  }
+  if (plan.S > 1) {
+    const int vec = N % 4 == 0 && aligned16(C) && aligned16(sums) ? 4 : 1;
+    hipLaunchKernelGGL((vec == 4 ? gt::fold_two_kernel<4> : gt::fold_two_kernel<1>), dim3(static_cast<unsigned>((n / vec + 255) / 256)), dim3(256), 0, s,
+                       out, C, sums, mn, n, plan.S);
+  }
+  return 0;
+}
+
 // operands or rows of the result beyond 32-bit offsets: the loaders with 64-bit addresses
 template <int BM, int BN, bool TA, bool TB>
 struct Far {
@@ -331,6 +365,33 @@ extern "C" int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA
     if (transposeA && transposeB) rc = dispatch_epilogue<true, true>(A, lda, B, ldb, C, m, n, k, ep, s);
   }
   if (rc) return rc;
+  return ps.finish();
+}
+
+extern "C" int TSplit_MatrixMultiplySums(const DLArrayHandle matA, const DLArrayHandle matB, DLArrayHandle matC, DLArrayHandle sums,
+                                         DLStreamHandle stream_handle) {
+  const char *who = "TSplit_MatrixMultiplySums";
+  TS_REQUIRE(matA && matB && matC && sums, "%s: NULL array", who);
+  TS_REQUIRE(matA->ndim >= 2 && matB->ndim >= 2 && matC->ndim == 2, "%s: operands of two axes or more, a result of two", who);
+  int64_t K, lda, b_rows, ldb;
+  rows_by_cols(matA, K, lda);
+  rows_by_cols(matB, b_rows, ldb);
+  const int64_t M = matC->shape[0], N = matC->shape[1];
+  TS_REQUIRE(K == b_rows && lda == M && ldb == N && numel(sums) == N, "%s: shapes do not conform", who);
+  TS_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) - 64, "%s: dimension too large", who);
+  const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+  const bool here = M > 0 && N > 0 && K > 0 && near<true, false>(lda, ldb, m, n, k) && rows_reach(n) && !(split_bf16_enabled() && K % 4 == 0 && K >= BK);
+  if (!here) {   // the product's other kernels, and the sums by themselves
+    int64_t ashape[2] = {K, M}, bshape[2] = {K, N};
+    DLArray A{matA->data, matA->ctx, 2, ashape}, B{matB->data, matB->ctx, 2, bshape};
+    if (const int rc = DLGpuMatrixMultiply(&A, true, &B, false, matC, stream_handle, nullptr)) return rc;
+    return DLGpuReduceSumAxisZero(&B, sums, stream_handle, nullptr);
+  }
+  hipStream_t s = stream_of(stream_handle);
+  ProfileScope ps(nullptr, s, 0, 0, 0);
+  if (const int rc = launch_sums(static_cast<const float *>(matA->data), lda, static_cast<const float *>(matB->data), ldb,
+                                 static_cast<float *>(matC->data), static_cast<float *>(sums->data), m, n, k, s))
+    return rc;
   return ps.finish();
 }
 

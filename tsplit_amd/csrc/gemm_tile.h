@@ -230,14 +230,34 @@ struct Core {
   static __device__ __forceinline__ constexpr int step_row(int tm, int e) { return AL::kDealt ? TM * e + tm : 16 * tm + e; }
 
   static __device__ __forceinline__ void run(AL &la, BL &lb, int kbegin, int kend, float *lds, f32x4 (&acc)[TM][TN]) {
+    float none[TN];
+    run<false>(la, lb, kbegin, kend, lds, acc, false, none);
+  }
+  // SUMS, where `on`: col[t] is also the sum over the range of what this lane supplies of B's column of tile t (of lane group g the
+  // k = 4 g + i of every half).  Eight of a step are added pairwise, eight steps one by one, then those: no longer a chain of
+  // roundings than a reduction in slices has.
+  template <bool SUMS>
+  static __device__ __forceinline__ void run(AL &la, BL &lb, int kbegin, int kend, float *lds, f32x4 (&acc)[TM][TN], bool on, float (&col)[TN]) {
     const int lane = threadIdx.x & 63, wm0 = wave_m0(), wn0 = wave_n0();
     const unsigned lds_at = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) float *)lds));
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float some[TN];
+    if constexpr (SUMS) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) col[j] = some[j] = 0.f;
+    }
     if (kbegin >= kend) return;
     float a0[TM][4], b0[TN][4], a1[TM][4], b1[TN][4];
+    auto add = [&](const float (&b)[TN][4]) {
+      if constexpr (SUMS)
+        if (on) {
+#pragma unroll
+          for (int j = 0; j < TN; ++j) some[j] += (b[j][0] + b[j][1]) + (b[j][2] + b[j][3]);
+        }
+    };
     la.load(kbegin, kend, lds_at);
     lb.load(kbegin, kend, lds_at + AL::kFloats * 4);
     int stage = 0;
@@ -257,15 +277,32 @@ struct Core {
       AL::frag(sa, wm0, 0, lane, a0);
       BL::frag(sb, wn0, 0, lane, b0);
       __builtin_amdgcn_sched_barrier(0);
-      if (k0 != kbegin) products<TM, TN>(a1, b1, acc);
+      if (k0 != kbegin) {
+        products<TM, TN>(a1, b1, acc);
+        add(b1);
+        if constexpr (SUMS)
+          if (((k0 - kbegin) & (8 * BK - 1)) == 0) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+              col[j] += some[j];
+              some[j] = 0.f;
+            }
+          }
+      }
       __builtin_amdgcn_sched_barrier(0);
       AL::frag(sa, wm0, 1, lane, a1);
       BL::frag(sb, wn0, 1, lane, b1);
       __builtin_amdgcn_sched_barrier(0);
       products<TM, TN>(a0, b0, acc);
+      add(b0);
       __builtin_amdgcn_sched_barrier(0);
     }
     products<TM, TN>(a1, b1, acc);
+    add(b1);
+    if constexpr (SUMS) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) col[j] += some[j];
+    }
   }
 };
 
@@ -277,14 +314,31 @@ struct Tile {
   using BL = typename std::conditional<TB, KContig<BN, TN, true>, MnContig<BN, TN>>::type;
   using C = Core<TM, TN, WM, WN, AL, BL>;
 
+  // SUMS: the tiles of the first row also leave the sums of B's columns over the range
+  template <bool SUMS = false>
   static __device__ __forceinline__ void run(const mg::DenseParams &ap, const mg::DenseParams &bp, float *__restrict__ o, int64_t ldc,
-                                             bool wide, int M, int N, int m0, int n0, int kbegin, int kend, float *lds) {
+                                             bool wide, int M, int N, int m0, int n0, int kbegin, int kend, float *lds, float *__restrict__ sums = nullptr) {
     AL la;
     BL lb;
     la.init(ap, m0);
     lb.init(bp, n0);
     f32x4 acc[TM][TN];
-    C::run(la, lb, kbegin, kend, lds, acc);
+    if constexpr (SUMS) {
+      float col[TN];
+      const bool on = m0 == 0 && C::wave_m0() == 0;   // two waves have all columns between them
+      C::template run<true>(la, lb, kbegin, kend, lds, acc, on, col);
+      if (on) {
+        const int lane = threadIdx.x & 63, c = n0 + C::wave_n0() + TN * (lane & 15);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          col[j] += __shfl_xor(col[j], 16, 64);
+          col[j] += __shfl_xor(col[j], 32, 64);
+          if (lane < 16 && c + j < N) sums[c + j] = col[j];
+        }
+      }
+    } else {
+      C::run(la, lb, kbegin, kend, lds, acc);
+    }
     // the wave's rows to the end of C: rows past it are out of range
     const int m = m0 + C::wave_m0(), n = n0 + C::wave_n0() + TN * (threadIdx.x & 15);
     if (m >= M) return;
@@ -328,6 +382,40 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_tile_kernel(mg::DenseParams 
   bp.p += z * zs.b;
   const int kbegin = kchunk < K ? z * kchunk : 0;
   T::run(ap, bp, out + z * zs.c, N, wide, M, N, tile_m * T::BM, tile_n * T::BN, kbegin, min(K, kbegin + kchunk), lds);
+}
+
+// C = A^T B and the sums of B's columns (a linear layer's two parameter gradients from its input and the gradient of its output): the
+// blocks of the first row of tiles have every column of B in their registers on the way.  As a reduction of its own the sums take two
+// launches, 10.5 us for 8192 x 512 where the product takes 35.  Column sums of range z go to sums + z * zs.
+template <int TM, int TN>
+__global__ __launch_bounds__(kThreads, 2) void gemm_sums_kernel(mg::DenseParams ap, mg::DenseParams bp, float *__restrict__ out, float *__restrict__ sums,
+                                                                int64_t zs, bool wide, int M, int N, int K, int kchunk, mg::TileGrid tg) {
+  using T = Tile<TM, TN, 2, 2, true, false>;
+  __shared__ __attribute__((aligned(1024))) float lds[T::C::kLdsFloats];
+  int z, tile_m, tile_n;
+  if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
+  T::template run<true>(ap, bp, out + z * zs, N, wide, M, N, tile_m * T::BM, tile_n * T::BN, z * kchunk, min(K, (z + 1) * kchunk), lds, sums + z * zs);
+}
+
+// The ranges of both added: first[i] for i < split, second[i - split] behind that, of `n` values a range (split and n multiples of VEC)
+template <int VEC>
+static __global__ __launch_bounds__(256) void fold_two_kernel(const float *__restrict__ part, float *__restrict__ first, float *__restrict__ second,
+                                                              int64_t split, int64_t n, int S) {
+  typedef float vec __attribute__((ext_vector_type(VEC)));
+  const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * VEC;
+  if (i >= n) return;
+  auto read = [&](int z) { return *reinterpret_cast<const vec *>(part + z * n + i); };
+  vec s = read(0);
+  int z = 1;
+  for (; z + 4 <= S; z += 4) {
+    const vec a = read(z), b = read(z + 1), c = read(z + 2), d = read(z + 3);
+    s += a;
+    s += b;
+    s += c;
+    s += d;
+  }
+  for (; z < S; ++z) s += read(z);
+  *reinterpret_cast<vec *>(i < split ? first + i : second + (i - split)) = s;
 }
 
 // ---- products whose result is worked on before it is stored

@@ -27,7 +27,7 @@ __all__ = [
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
     "batch_norm_relu", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
-    "optimizer_update_multi", "matrix_multiply_add", "heads_matrix_multiply",
+    "optimizer_update_multi", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "lstm_sizes", "lstm", "lstm_gradient",
     "CuDNN_Dropout", "CuDNN_Dropout_gradient", "CuSparse_Csrmv", "CuSparse_Csrmm",
@@ -97,6 +97,11 @@ def matrix_multiply_add(matA, transA, matB, transB, matC, bias=None, addend=None
     check_call(_LIB.TSplit_MatrixMultiplyAdd(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(bias) if bias else None,
                                              _h(addend) if addend else None, _h(gate) if gate else None, _h(matC),
                                              _h(relu) if relu else None, _s(stream)))
+
+
+def matrix_multiply_sums(matA, matB, matC, sums, stream=None):
+    """matC = matA' matB (the bits of matrix_multiply), sums = the sums of matB's columns (no counterpart in the reference's gpu_links)."""
+    check_call(_LIB.TSplit_MatrixMultiplySums(_h(matA), _h(matB), _h(matC), _h(sums), _s(stream)))
 
 
 def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0,

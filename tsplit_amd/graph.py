@@ -139,6 +139,12 @@ class GpuBackend(object):
         self.L.matrix_multiply_add(a, ta, b, tb, c, bias, addend, r, self.stream, gate)
         return c, r
 
+    def matmul_sums(self, a, b, out_shape, sums_shape):
+        """-> (a' b, the sums of b's columns); arrays of more axes are matrices of the last one's columns."""
+        c, sums = self.empty(out_shape), self.empty(sums_shape)
+        self.L.matrix_multiply_sums(a, b, c, sums, self.stream)
+        return c, sums
+
     def heads_matmul(self, a, ta, b, tb, out_shape, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0, addend=None):
         """Products per sample and head (gpu_links.heads_matrix_multiply)."""
         c = self.empty(out_shape)
@@ -753,8 +759,14 @@ class Tape(object):
         def back(g):
             if residual is not None:
                 self._acc(residual, g)
-            self._acc_product(w, x.value, x.shape, True, g, ys, False)
-            if bias is not None and bias.needs_grad:
+            both = bias is not None and bias.needs_grad and w.needs_grad and bias.grad is None and w.grad is None and self._can("matmul_sums")
+            if both:
+                w.grad, bias.grad = self.b.matmul_sums(x.value, g, w.shape, bias.shape)
+                self._owns(w, True)
+                self._owns(bias, True)
+            else:
+                self._acc_product(w, x.value, x.shape, True, g, ys, False)
+            if bias is not None and bias.needs_grad and not both:
                 rows = self._seen_as(g, (_prod(ys[:-1]), ys[-1])) if len(ys) > 2 else g
                 self._acc(bias, self.b.reduce_sum_axis_zero(rows, bias.shape), fresh=True)
             self._acc_product(x, g, ys, False, w.value, w.shape, True)
