@@ -465,5 +465,32 @@ static __global__ __launch_bounds__(256) void conv_relay_kernel(Relay R) {
   R.out[idx] = ch < R.chans ? R.w[row * R.w_row + ch * R.w_chan + (F.a + R.s * u) * R.f_w + F.b + R.s * v] : 0.f;
 }
 
+// The same for a filter of one phase with all its taps, kTurnRows rows x kTurnChans channels a block, through LDS: `along` the rows of the
+// output, memory holds a row's channels (forward) or a channel's rows (data gradient) side by side, and runs of either are read, and
+// written, whole.  One thread a value fetched every value by itself: 512 x 512 x 9 behind other
+// layers 14.5 us, 1.3 TB/s (five such layers both ways: 2.117 -> 2.092 ms a step).
+constexpr int kRelayRows = 8, kRelayChans = 32;
+static __global__ __launch_bounds__(256) void conv_relay_tiles_kernel(const float *__restrict__ w, float *__restrict__ out, int rows, int chans, int padded,
+                                                                      FastDiv taps, int64_t w_row, int64_t w_chan, FastDiv tiles) {
+  extern __shared__ float lds[];   // [row][channel][tap], a channel to spare a row
+  const int n_taps = taps.d, pitch = (kRelayChans + 1) * n_taps;
+  const uint32_t tr = tiles.div(blockIdx.x);
+  const int r0 = tr * kRelayRows, c0 = (blockIdx.x - tr * tiles.d) * kRelayChans;
+  const bool across = w_row < w_chan;   // a channel's rows lie side by side
+  for (int e = threadIdx.x; e < kRelayRows * kRelayChans * n_taps; e += 256) {
+    const int i = taps.div(e), tap = e - i * n_taps;
+    const int r = across ? i % kRelayRows : i / kRelayChans, c = across ? i / kRelayRows : i % kRelayChans;
+    lds[r * pitch + c * n_taps + tap] = r0 + r < rows && c0 + c < chans ? w[(r0 + r) * w_row + (c0 + c) * w_chan + tap] : 0.f;
+  }
+  __syncthreads();
+  const int here = min(kRelayChans, padded - c0) * n_taps;   // values of a row, side by side in the output
+  for (int e = threadIdx.x; e < kRelayRows * kRelayChans * n_taps; e += 256) {
+    const int i = taps.div(e >> 3), tap = (e >> 3) - i * n_taps;   // i: block of 8 channels, of row i / 4
+    const int r = i / (kRelayChans / 8), b = i % (kRelayChans / 8), at = (b * n_taps + tap) * 8 + (e & 7);
+    if (r0 + r < rows && at < here)
+      out[(static_cast<int64_t>(r0 + r) * padded + c0) * n_taps + at] = lds[r * pitch + (8 * b + (e & 7)) * n_taps + tap];
+  }
+}
+
 }  // namespace ct
 }  // namespace tsplit

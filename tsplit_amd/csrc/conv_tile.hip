@@ -117,6 +117,9 @@ inline int padded(int chans) { return (chans + 7) / 8 * 8; }
 // blocks of 8 channels, unless padding the last one adds more depth than the filter's own order costs
 inline bool in_blocks(int chans) { return padded(chans) * 3 <= chans * 4; }
 
+// filters re-laid in tiles (below that a launch of either takes what any launch takes: 590 K values 5.7 us by single values, the call 2 us
+// longer in tiles)
+constexpr int kRelayTilesFrom = 1 << 20;
 // the re-laid filter of P's phases (their K and w_at are set), in scratch
 int relay(Params &P, const float *w, int rows, int chans, int w_row, int w_chan, int f_w, int s, const int (*first_tap)[2], bool plain,
           hipStream_t st) {
@@ -139,7 +142,15 @@ int relay(Params &P, const float *w, int rows, int chans, int w_row, int w_chan,
   }
   R.out = static_cast<float *>(scratch_get(st, 3, static_cast<size_t>(std::max(4, R.total)) * sizeof(float)));
   TS_REQUIRE(R.out, "conv: no scratch memory for the re-laid filter");
-  if (R.total > 0) hipLaunchKernelGGL(conv_relay_kernel, dim3((R.total + 255) / 256), dim3(256), 0, st, R);
+  const int taps = static_cast<int>(P.phase[0].taps.d);
+  if (P.phases == 1 && s == 1 && !plain && static_cast<int>(P.phase[0].kw.d) == f_w && taps <= 25 && R.total >= kRelayTilesFrom) {
+    const int all = (chans + 7) / 8 * 8, tiles = (all + kRelayChans - 1) / kRelayChans;
+    hipLaunchKernelGGL(conv_relay_tiles_kernel, dim3((rows + kRelayRows - 1) / kRelayRows * tiles), dim3(256),
+                       kRelayRows * (kRelayChans + 1) * taps * sizeof(float), st, w, R.out, rows, chans, all, P.phase[0].taps, w_row, w_chan,
+                       FastDiv(tiles));
+  } else if (R.total > 0) {
+    hipLaunchKernelGGL(conv_relay_kernel, dim3((R.total + 255) / 256), dim3(256), 0, st, R);
+  }
   P.w = R.out;
   return 0;
 }

@@ -38,6 +38,32 @@ __global__ __launch_bounds__(256) void fold_tap_major_kernel(const float *__rest
   }
 }
 
+// The same sums of few ranges, kFoldChans channels of one output channel a block: the taps of a channel come together in LDS, so that dw is
+// written in whole lines: filter gradients of 512 -> 512, 64 images of 4 x 4 72 -> 66 us, of 2 x 2 40 -> 32; from a million values on (590 K: 61.1
+// and 61.6, 173 K 17.5 and 22.1).
+constexpr int kFoldChans = 64;
+__global__ __launch_bounds__(256) void fold_tap_major_tiles_kernel(const float *__restrict__ part, float *__restrict__ dw, int C, FastDiv tiles, int kHW,
+                                                                   int64_t stride, int S) {
+  extern __shared__ float lds[];   // [channel][tap]
+  const uint32_t o = tiles.div(blockIdx.x);
+  const int c0 = (blockIdx.x - o * tiles.d) * kFoldChans, here = min(kFoldChans, C - c0);
+  const float *from = part + static_cast<int64_t>(o) * kHW * C + c0;
+  const int c = threadIdx.x & (kFoldChans - 1);
+  for (int tap = threadIdx.x / kFoldChans; tap < kHW; tap += 256 / kFoldChans) {
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    if (c < here)
+      for (int z = 0; z < S; z += 4)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (z + i < S) acc[i] += from[(z + i) * stride + static_cast<int64_t>(tap) * C + c];
+    lds[c * kHW + tap] = ((acc[0] + acc[1]) + acc[2]) + acc[3];
+  }
+  __syncthreads();
+  float *to = dw + (static_cast<int64_t>(o) * C + c0) * kHW;
+  for (int e = threadIdx.x; e < here * kHW; e += 256) to[e] = lds[e];
+}
+constexpr int64_t kFoldTilesFrom = 1 << 20;
+
 template <int G>
 void launch_tile(const Params &P, int tile, const mg::TileGrid &tg, unsigned grid, hipStream_t st) {
   switch (tile) {
@@ -60,7 +86,13 @@ int group_size(int chans) {
 }  // namespace
 
 void conv_fold_tap_major(const float *part, float *dw, int O, int C, int taps, int S, hipStream_t st) {
-  const int64_t mn = static_cast<int64_t>(O) * C * taps;
+  const int64_t mn = static_cast<int64_t>(O) * C * taps, tiles = (C + kFoldChans - 1) / kFoldChans;
+  // (a range's result written as a lane's four accumulators from zero adds up to the same bits)
+  if (mn >= kFoldTilesFrom && C >= 32 && S <= 16 && taps <= 64 && tiles * O < (1ll << 31)) {
+    hipLaunchKernelGGL(fold_tap_major_tiles_kernel, dim3(static_cast<unsigned>(tiles * O)), dim3(256), kFoldChans * taps * sizeof(float), st, part, dw, C,
+                       FastDiv(static_cast<uint32_t>(tiles)), taps, mn, S);
+    return;
+  }
   hipLaunchKernelGGL(fold_tap_major_kernel, dim3(static_cast<unsigned>((mn + 63) / 64)), dim3(256), 0, st, part, dw, O, C, taps, mn, S);
 }
 
