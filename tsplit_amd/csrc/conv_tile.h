@@ -65,6 +65,7 @@ struct Params {
 // depth in blocks of 8 channels of one tap, else (ch, tap).
 template <int BN, int T, bool BWD, int TAPS, bool BLOCKS>
 struct Gathered {
+  static constexpr bool kDense = false;
   static constexpr int kFloats = BK * BN, H = BN / 64;
   using Mask = typename std::conditional<(TAPS > 32), uint64_t, uint32_t>::type;
   unsigned voff[H];
@@ -151,6 +152,7 @@ struct Gathered {
 // B of a layer with one tap, no padding, stride 1 and planes of whole 16-byte words: four columns of one image are one word.
 template <int BN, int T>
 struct Pointwise {
+  static constexpr bool kDense = false;
   static constexpr int kFloats = BK * BN;
   static constexpr int kLoads = BN / 32, kWords = BN / 4, kRows = 64 / kWords;
   unsigned voff;

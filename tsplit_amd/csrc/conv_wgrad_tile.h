@@ -63,7 +63,7 @@ __device__ __forceinline__ i32x4 from_image(const float *p, int64_t bytes, int i
 // q ^ (r / 2 % 4): a product tile's 16 rows then start on 16 different bank groups.
 template <int MN, int T>
 struct Words {
-  static constexpr bool kDealt = false;
+  static constexpr bool kDense = false, kDealt = false;
   static constexpr int kGroup = 272, kLoads = MN / 32, kFloats = MN / 8 * kGroup;
   i32x4 rsrc;
   FastDiv image;
@@ -127,6 +127,7 @@ struct Words {
 // BN columns of x, in groups of G channels of one tap, 4 bytes a lane.  LDS: two rows of a load in 64 floats and 4 to spare.
 template <int BN, int T, int G>
 struct Taps {
+  static constexpr bool kDense = false;
   static constexpr int kPair = 68, kGroups = BN / 4 / G, kFloats = BN / 2 * kPair;   // a wave's groups
   i32x4 rsrc;
   FastDiv image, width;

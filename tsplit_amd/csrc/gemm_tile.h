@@ -71,6 +71,7 @@ __device__ __forceinline__ void lds_ready() {
 // holds matrix row (s % 16) * T + s / 16, so that tile t's lane c supplies index T c + t.
 template <int MN, int T, bool PERM>
 struct KContig {
+  static constexpr bool kDense = true;
   static constexpr bool kDealt = PERM;   // tile t's lane r supplies index T r + t, not 16 t + r
   static constexpr int kFloats = MN * BK;
   static constexpr int kLoads = MN / 32;   // a wave's loads a step, 8 rows each
@@ -141,7 +142,7 @@ struct KContig {
 // row's first values: they belong to rows or columns of C that do not exist.
 template <int MN, int T>
 struct MnContig {
-  static constexpr bool kDealt = true;
+  static constexpr bool kDense = true, kDealt = true;
   static constexpr int kFloats = BK * MN;
   static constexpr int kLoads = MN / 32;
   static constexpr int kWords = MN / 4;            // 16-byte words of a row
@@ -297,7 +298,9 @@ struct Core {
       add(b0);
       __builtin_amdgcn_sched_barrier(0);
     }
-    products<TM, TN>(a1, b1, acc);
+    // (a depth whose last half step is all zeros: 100 x 4096' x 4096 46 -> 43 us; convolutions' depths are cut and padded otherwise, and gained
+    // nothing)
+    if (!BL::kDense || ((kend - kbegin - 1) & (BK - 1)) >= BK / 2) products<TM, TN>(a1, b1, acc);
     add(b1);
     if constexpr (SUMS) {
 #pragma unroll
