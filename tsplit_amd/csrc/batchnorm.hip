@@ -201,8 +201,8 @@ __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restr
     const double a = static_cast<double>(gamma[c]) * istd;
     coef[2 * c] = static_cast<float>(a);
     coef[2 * c + 1] = static_cast<float>(static_cast<double>(beta[c]) - mean_used * a);
-    if (save_mean) save_stat(save_mean, c, wide, mean);
-    if (save_istd) save_stat(save_istd, c, wide, istd);
+    if (save_mean) save_stat(save_mean, c, RELU && wide, mean);
+    if (save_istd) save_stat(save_istd, c, RELU && wide, istd);
   }
 }
 
@@ -374,7 +374,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_coef_kernel(const double *__r
   }
   if (threadIdx.x == 0) {
     double mean, istd;
-    if (save_mean && save_istd && !wide) {
+    if (save_mean && save_istd && !(RELU && wide)) {
       mean = save_mean[c];
       istd = save_istd[c];
     } else {
@@ -498,8 +498,8 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
     const double a = static_cast<double>(gamma[c]) * istd;
     coef[0] = static_cast<float>(a);
     coef[1] = static_cast<float>(static_cast<double>(beta[c]) - mean_used * a);
-    if (save_mean) save_stat(save_mean, c, wide, mean);
-    if (save_istd) save_stat(save_istd, c, wide, istd);
+    if (save_mean) save_stat(save_mean, c, RELU == kFused && wide, mean);
+    if (save_istd) save_stat(save_istd, c, RELU == kFused && wide, istd);
   }
   __syncthreads();
   const float a = coef[0], b = coef[1];
@@ -543,14 +543,21 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     const int64_t at = ok ? chan_addr(hw, e, c, C) : 0;
     xv[r] = ok ? __builtin_nontemporal_load(x + at) : 0.f;
     dv[r] = ok ? __builtin_nontemporal_load(dy + at) : 0.f;
+    if constexpr (RELU != kBoth) {
+      if (RELU == kFused) dv[r] = gated(dv[r], xv[r], ga, gb);
+      acc_dot(dv[r], xv[r], sdy, sdx);
+      if (STATS) acc2(xv[r], sx, sq);
+    }
   }
-  if (RELU == kBoth) __builtin_amdgcn_sched_barrier(0);   // (with its selects the compiler waits for every load by itself: 43 us for 17)
+  if constexpr (RELU == kBoth) {
+    // (with its selects the compiler waits for every load by itself unless all are asked for first: 43 us for 17)
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (RELU == kFused) dv[r] = gated(dv[r], xv[r], ga, gb);
-    if (RELU == kBoth) dv[r] = r * kThreads + threadIdx.x < m ? gated_op(dv[r], xv[r], ga, gb) : 0.f;
-    acc_dot(dv[r], xv[r], sdy, sdx);
-    if (STATS) acc2(xv[r], sx, sq);
+    for (int r = 0; r < R; ++r) {
+      dv[r] = r * kThreads + threadIdx.x < m ? gated_op(dv[r], xv[r], ga, gb) : 0.f;
+      acc_dot(dv[r], xv[r], sdy, sdx);
+      if (STATS) acc2(xv[r], sx, sq);
+    }
   }
   const double r0 = block_sum<double, kWaves>(static_cast<double>(sdy), sm);
   const double r1 = block_sum<double, kWaves>(static_cast<double>(sdx), sm);

@@ -832,7 +832,7 @@ class Tape(object):
         """Whether lstm_cells() is there for these operands: the data get no gradient, every value of x is a frame's, and the sizes
         are those TSplit_Lstm addresses."""
         return (self._ahead and self._can("lstm") and not x.needs_grad and not initial.needs_grad and initial.shape == (1,)
-                and len(x.shape) == 2 and 0 < x.shape[0] < 1 << 20 and x.shape[1] % steps == 0 and x.shape[1] // steps < 1 << 24
+                and len(x.shape) == 2 and 0 < x.shape[0] < 1 << 20 and x.shape[1] % steps == 0 and 0 < x.shape[1] // steps < 1 << 24
                 and x.shape[0] * steps < (1 << 31) - 64 and units < 1 << 20 and (x.shape[0] // 16 + 1) * (units // 16 + 1) < 1 << 30)
 
     @_op
