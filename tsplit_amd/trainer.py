@@ -10,6 +10,9 @@ executor.py:160-196), filter gradients issued before data gradients (executor.py
 the data gradient of the first layer never evaluated, then one optimizer call per parameter
 (python/athena/optimizer.py:95-176).
 
+Pairs of layers that the library has one call for (BatchNorm and the Relu behind it, a linear layer and the Relu behind or
+in front of it) are that call; it writes the arrays of both nodes with the bits of the two calls.
+
 The TSplit part: `split={layer_index: pieces}` runs that conv layer (forward, both
 backward passes) on `pieces` zero-copy batch micro-tensors (DLArraySliceForMicroTensor);
 per-piece filter gradients are summed with DLGpuMatrixElementwiseAdd.  BatchNorm always
