@@ -542,6 +542,10 @@ int TSplit_EmbeddingAdd(const DLArrayHandle table, const DLArrayHandle ids, floa
                         DLArrayHandle output, DLStreamHandle stream);
 int TSplit_EmbeddingAdd_Gradient(const DLArrayHandle output_grad, const DLArrayHandle ids, float scale, int add_to,
                                  DLArrayHandle table_grad, DLStreamHandle stream);
+/* ---- 1 to 8 parts joined along an axis in one launch, and the parts of a whole (outside the reference's ABI; DLGpuConcat and
+ *      DLGpuConcat_gradient take two). ---- */
+int TSplit_Join(const DLArrayHandle *parts, int count, DLArrayHandle whole, int axis, DLStreamHandle stream);
+int TSplit_Part(const DLArrayHandle whole, DLArrayHandle *parts, int count, int axis, DLStreamHandle stream);
 /* ---- A view of `input` under another shape of as many values (outside the reference's ABI): the new struct's data
  *      pointer is input's, so it is released like a micro-tensor view (data set to NULL, then DLArrayFree). ---- */
 int TSplit_ArrayView(const DLArrayHandle input, const int64_t *shape, int ndim, DLArrayHandle *view);

@@ -29,7 +29,7 @@ __all__ = [
     "batch_norm_relu", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
     "optimizer_update_multi", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
-    "lstm_sizes", "lstm", "lstm_gradient",
+    "join", "part", "lstm_sizes", "lstm", "lstm_gradient",
     "CuDNN_Dropout", "CuDNN_Dropout_gradient", "CuSparse_Csrmv", "CuSparse_Csrmm",
 ]
 
@@ -111,6 +111,16 @@ def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, ma
     check_call(_LIB.TSplit_HeadsMatrixMultiply(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(matC), int(heads),
                                                ctypes.c_float(alpha), _h(mask) if mask else None, ctypes.c_float(mask_value),
                                                int(bool(causal)), ctypes.c_float(fill), _h(addend) if addend else None, _s(stream)))
+
+
+def join(parts, whole, axis, stream=None):
+    """whole = the parts (1 to 8) one behind the other along `axis` (no counterpart in the reference's gpu_links)."""
+    check_call(_LIB.TSplit_Join(_handles(parts), len(parts), _h(whole), int(axis), _s(stream)))
+
+
+def part(whole, parts, axis, stream=None):
+    """The parts (1 to 8) of `whole` along `axis`."""
+    check_call(_LIB.TSplit_Part(_h(whole), _handles(parts), len(parts), int(axis), _s(stream)))
 
 
 def lstm_sizes(frame, units):

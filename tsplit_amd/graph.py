@@ -279,6 +279,16 @@ class GpuBackend(object):
         self.L.concat_gradient(dout, g, axis, idx, self.stream)
         return g
 
+    def join(self, parts, out_shape, axis):
+        out = self.empty(out_shape)
+        self.L.join(parts, out, axis, self.stream)
+        return out
+
+    def part(self, whole, shapes, axis):
+        out = [self.empty(s) for s in shapes]
+        self.L.part(whole, out, axis, self.stream)
+        return out
+
     def transpose(self, x, perm, out_shape):
         out = self.empty(out_shape)
         self.L.matrix_transpose(x, out, perm, self.stream)
@@ -723,6 +733,32 @@ class Tape(object):
             if b.needs_grad:
                 self._acc(b, self.b.concat_grad(g, b.shape, axis, 1))
         return self._out(y, shape, [a, b], back, saved=[], redo=fwd)
+
+    def concat_all(self, parts, axis):
+        """The parts one behind the other: one node where the backend joins any number, else chained concats of two
+        (examples/imagenet_inceptionv4.py concatenates in pairs)."""
+        if 2 < len(parts) <= 8 and self._ahead and self._can("join"):
+            return self.join(parts, axis)
+        x = parts[0]
+        for p in parts[1:]:
+            x = self.concat(x, p, axis)
+        return x
+
+    @_op
+    def join(self, parts, axis):
+        """The parts one behind the other along `axis`; the gradient is cut up again."""
+        shape = list(parts[0].shape)
+        shape[axis] = sum(p.shape[axis] for p in parts)
+        shape = tuple(shape)
+
+        def fwd():
+            return self.b.join([p.value for p in parts], shape, axis)
+
+        def back(g):
+            for p, gp in zip(parts, self.b.part(g, [p.shape for p in parts], axis)):
+                if p.needs_grad:
+                    self._acc(p, gp, fresh=True)
+        return self._out(fwd(), shape, list(parts), back, saved=[], redo=fwd)
 
     @_op
     def matmul(self, a, b, trans_a=False, trans_b=False):

@@ -167,10 +167,7 @@ def _conv_bn(t, b, x, cout, kh, kw, stride=1, same=True, eps=0.01):
 
 
 def _cat(t, parts):
-    x = parts[0]
-    for p in parts[1:]:
-        x = t.concat(x, p, 1)
-    return x
+    return t.concat_all(parts, 1)
 
 
 def inception_v4(t, b, x, labels, n_a=4, n_b=7, n_c=3, div=1, classes=1000, eps=0.01):
