@@ -1,0 +1,55 @@
+"""BatchNorm's results to the bit, in both directions.
+
+Behind many Relu layers a last bit of one BatchNorm call decides on which side of zero single values fall, and a network's gradients
+move by 1e-3: so which product of a sum is rounded by itself and which is fused, in which order, belongs to a call's results.  The digests
+are those of the calls' results on an MI355X, recorded from the plain calls while the compiler still chose the fused products; every later
+form of the kernels has to give the same."""
+import zlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# one-pass kernels of 16, 32 and 64 values a thread; ranges of 16-byte words, with read-ahead loops and remainders; ranges without words
+SHAPES = [(2, 3, 5, 5), (16, 4, 14, 14), (32, 4, 15, 15), (32, 6, 17, 17), (16, 3, 32, 32), (8, 4, 112, 112), (16, 3, 71, 71)]
+GOLDEN = {
+    (2, 3, 5, 5): (1803107568, 3230562865, 1183227773, 1171934599),
+    (16, 4, 14, 14): (3954799238, 3671639413, 239292508, 3001953959),
+    (32, 4, 15, 15): (2466055982, 49538025, 2270622261, 3741949911),
+    (32, 6, 17, 17): (204916229, 279849675, 1670038264, 1180378973),
+    (16, 3, 32, 32): (2237242307, 4129929770, 1863065929, 1882697053),
+    (8, 4, 112, 112): (613838288, 2268043695, 4016568529, 2412863682),
+    (16, 3, 71, 71): (2639025669, 1539595629, 2947938412, 1927376946),
+}
+
+
+def digests(shape):
+    """(forward, gradient from saved statistics, gradient without, the fused pair's gradient from saved statistics)"""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    ctx = nd.gpu(0)
+    rng = np.random.RandomState(sum(shape))
+    c = shape[1]
+    x, dy = [nd.array(rng.normal(size=shape).astype(np.float32), ctx) for _ in range(2)]
+    gamma, beta = [nd.array(rng.normal(size=(1, c, 1, 1)).astype(np.float32), ctx) for _ in range(2)]
+    y, dx = nd.empty(shape, ctx), nd.empty(shape, ctx)
+    mean, istd, dg, db = [nd.empty((1, c, 1, 1), ctx) for _ in range(4)]
+
+    def digest(*arrays):
+        crc = 0
+        for a in arrays:
+            crc = zlib.crc32(np.ascontiguousarray(a.asnumpy()).tobytes(), crc)
+        return crc
+    L.CuDNN_Batch_Normalization(x, gamma, beta, y, mean, istd, 0.99, 0.01)
+    out = [digest(y, mean, istd)]
+    for saved in ((mean, istd), (None, None)):
+        L.CuDNN_Batch_Normalization_gradient(dy, x, gamma, dx, dg, db, *saved, 0.01)
+        out.append(digest(dx, dg, db))
+    L.batch_norm_relu(x, gamma, beta, y, mean, istd, 0.01)
+    L.batch_norm_relu_gradient(dy, x, gamma, beta, dx, dg, db, mean, istd, 0.01)
+    return tuple(out + [digest(y, mean, istd, dx, dg, db)])
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_results_keep_their_bits(shape):
+    assert digests(shape) == GOLDEN[shape]

@@ -59,7 +59,9 @@ __device__ __forceinline__ int64_t word_addr(const Geo &g, uint32_t i, int c) {
   return (static_cast<int64_t>(n) * g.C + c) * g.wpp + j;
 }
 
-// (fused multiply-adds are spelled out: left to the compiler, two forms of a kernel round the same sum differently)
+// Fused multiply-adds are spelled out: left to the compiler, two forms of a kernel round the same sum differently.  Which product
+// of a sum of two is rounded by itself is part of a call's result: the forms below are what every call has always given, and BatchNorm
+// behind many Relu layers turns another last bit into 1e-3 of a gradient.
 __device__ __forceinline__ void acc2(const f32x4 &v, float &s, float &q) {
   s += (v.x + v.y) + (v.z + v.w);
   q += fmaf(v.x, v.x, v.y * v.y) + fmaf(v.z, v.z, v.w * v.w);
@@ -68,10 +70,13 @@ __device__ __forceinline__ void acc2(const float &v, float &s, float &q) {
   s += v;
   q = fmaf(v, v, q);
 }
+// LAST: of the second pair the last product is the fused one (the read-ahead loop of TSplit_BatchNormRelu_gradient with saved floats)
+template <bool LAST = false>
 __device__ __forceinline__ void acc_dot(const f32x4 &a, const f32x4 &b, float &s, float &d) {
   s += (a.x + a.y) + (a.z + a.w);
-  d += fmaf(a.x, b.x, a.y * b.y) + fmaf(a.z, b.z, a.w * b.w);
+  d += fmaf(a.x, b.x, a.y * b.y) + (LAST ? fmaf(a.w, b.w, a.z * b.z) : fmaf(a.z, b.z, a.w * b.w));
 }
+template <bool LAST = false>
 __device__ __forceinline__ void acc_dot(const float &a, const float &b, float &s, float &d) {
   s += a;
   d = fmaf(a, b, d);
@@ -101,11 +106,13 @@ __device__ __forceinline__ f32x4 gated_op(const f32x4 &dy, const f32x4 &x, float
   const f32x4 r = {gated_op(dy.x, x.x, a, b), gated_op(dy.y, x.y, a, b), gated_op(dy.z, x.z, a, b), gated_op(dy.w, x.w, a, b)};
   return r;
 }
+// k1 dy + k2 x + k3; in the one-pass kernels the other product is the fused one
 __device__ __forceinline__ float lin2(const float &dy, const float &x, float k1, float k2, float k3) { return fmaf(k2, x, k1 * dy) + k3; }
 __device__ __forceinline__ f32x4 lin2(const f32x4 &dy, const f32x4 &x, float k1, float k2, float k3) {
   const f32x4 r = {lin2(dy.x, x.x, k1, k2, k3), lin2(dy.y, x.y, k1, k2, k3), lin2(dy.z, x.z, k1, k2, k3), lin2(dy.w, x.w, k1, k2, k3)};
   return r;
 }
+__device__ __forceinline__ float lin2_onepass(float dy, float x, float k1, float k2, float k3) { return fmaf(k1, dy, k2 * x) + k3; }
 
 // partial layout: [C][S][NQ] doubles
 template <int VEC>
@@ -280,6 +287,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
                                                                  const float *__restrict__ save_istd, bool wide,
                                                                  const float *__restrict__ pair, float *__restrict__ dg) {
   using W = typename Word<VEC>::T;
+  constexpr bool kLast = RELU == kFused && !STATS;
   __shared__ double sm[4 * kWaves];
   const int c = blockIdx.y, s = blockIdx.x;
   float ga = 0.f, gb = 0.f;
@@ -311,7 +319,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
         dv[u] = gated_op(dv[u], xv[u], ga, gb);
         reinterpret_cast<W *>(dg)[word_addr<VEC>(g, i + u * kThreads, c)] = dv[u];
       }
-      acc_dot(dv[u], xv[u], sdy, sdx);
+      acc_dot<kLast>(dv[u], xv[u], sdy, sdx);
       if (STATS) acc2(xv[u], sx, sq);
     }
   }
@@ -453,6 +461,13 @@ __device__ __forceinline__ int64_t chan_addr(const FastDiv &hw, uint32_t e, int 
   return (static_cast<int64_t>(n) * C + c) * hw.d + (e - n * hw.d);
 }
 
+// v[r] into a channel's sums: of the first two squares the first is the fused one
+template <int R>
+__device__ __forceinline__ void squares_onepass(const float (&v)[R], int r, float &s, float &q) {
+  s += v[r];
+  if (r > 0) q = fmaf(v[r == 1 ? 0 : r], v[r == 1 ? 0 : r], r == 1 ? v[1] * v[1] : q);
+}
+
 // R: values per thread (compile-time bound of the register arrays)
 template <int R, int RELU>
 __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *__restrict__ x, float *__restrict__ y,
@@ -546,7 +561,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     if constexpr (RELU != kBoth) {
       if (RELU == kFused) dv[r] = gated(dv[r], xv[r], ga, gb);
       acc_dot(dv[r], xv[r], sdy, sdx);
-      if (STATS) acc2(xv[r], sx, sq);
+      if (STATS) squares_onepass(xv, r, sx, sq);
     }
   }
   if constexpr (RELU == kBoth) {
@@ -556,7 +571,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     for (int r = 0; r < R; ++r) {
       dv[r] = r * kThreads + threadIdx.x < m ? gated_op(dv[r], xv[r], ga, gb) : 0.f;
       acc_dot(dv[r], xv[r], sdy, sdx);
-      if (STATS) acc2(xv[r], sx, sq);
+      if (STATS) squares_onepass(xv, r, sx, sq);
     }
   }
   const double r0 = block_sum<double, kWaves>(static_cast<double>(sdy), sm);
@@ -595,7 +610,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     const uint32_t e = r * kThreads + threadIdx.x;
     if (e < m) {
       if (RELU == kBoth) __builtin_nontemporal_store(dv[r], dg + chan_addr(hw, e, c, C));
-      __builtin_nontemporal_store(lin2(dv[r], xv[r], k1, k2, k3), dx + chan_addr(hw, e, c, C));
+      __builtin_nontemporal_store(lin2_onepass(dv[r], xv[r], k1, k2, k3), dx + chan_addr(hw, e, c, C));
     }
   }
 }
