@@ -348,6 +348,111 @@ static __global__ __launch_bounds__(kThreads, 3) void wino_grad_gemm_narrow_kern
   }
 }
 
+// The same sums to the bit on tiles of 32 x 64 (KG = 2) or 32 x 32 (KG = 4), for launches of few blocks: a wave holds one 32 x 32 tile
+// of its k-group, so the chains that one wave above runs four of side by side, four waves run.  What bounds a launch here is that chain,
+// kchunk / KG values at 32 cycles each (1024 deep, KG = 2: 6.8 us), so it is only kept fed: kAhead chunks of 64 are in flight in
+// registers (a chunk is 512 or 1024 cycles of products, a trip to memory about 2000), two LDS stages, a barrier a chunk.
+template <int KG>
+static __global__ __launch_bounds__(kThreads, 2) void wino_grad_gemm_fine_kernel(GradProblem p, TileGrid tg) {
+  constexpr int SUB = 4 / KG;                  // 32 x 32 tiles of the block
+  constexpr int TM = 32, TN = 32 * SUB;
+  constexpr int CH = BK * KG, D = 64;          // the groups' turn, the depth of a chunk in LDS
+  constexpr int STRIDE = D + 4, kStage = (TM + TN) * STRIDE;
+  constexpr int RPP = kThreads / 16, P = (TM + TN) / RPP;   // rows a pass, passes (the first two load Y's rows)
+  constexpr int kAhead = KG;
+  static_assert(kAhead % 2 == 0 && TM / RPP == 2, "stage and pass of a chunk are known at compile time");
+  __shared__ __attribute__((aligned(16))) float lds[2 * kStage];
+
+  int z, tile_m, tile_n;
+  if (!block_tile(tg, z, tile_m, tile_n)) return;
+  const int range = z / kXi, xi = z - range * kXi;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int sub = wave % SUB, g = wave / SUB;
+  const int m0 = tile_m * TM, n0 = tile_n * TN, wn0 = 32 * sub;
+  const int kbegin = range * p.kchunk, kend = min(p.ld, kbegin + p.kchunk);
+
+  const int quad = tid % 16, prow = tid / 16;
+  const int arows = min(TM, p.rows - m0), brows = min(TN, p.cols - n0);
+  const __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.Y + (static_cast<int64_t>(xi) * p.rows + m0) * p.ld), 0,
+                                        static_cast<int>(static_cast<int64_t>(arows) * p.ld * 4), kBufFlags);
+  const __amdgpu_buffer_rsrc_t rb =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.V + (static_cast<int64_t>(xi) * p.cols + n0) * p.ld), 0,
+                                        static_cast<int>(static_cast<int64_t>(brows) * p.ld * 4), kBufFlags);
+  unsigned voff[P];
+#pragma unroll
+  for (int s = 0; s < P; ++s) {
+    const int row = prow + RPP * (s < 2 ? s : s - 2);
+    voff[s] = row < (s < 2 ? arows : brows) ? (static_cast<unsigned>(row) * static_cast<unsigned>(p.ld) + 4u * quad) * 4u : kOobOffset;
+  }
+  u32x4 held[kAhead][P];
+  auto load = [&](u32x4 (&to)[P], int k0) {
+    const bool in = k0 + 4 * quad < kend;   // (a word lies wholly inside the range or outside)
+#pragma unroll
+    for (int s = 0; s < P; ++s) to[s] = __builtin_amdgcn_raw_buffer_load_b128(s < 2 ? ra : rb, in ? voff[s] : kOobOffset, k0 * 4, 0);
+  };
+  acc16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+#pragma unroll
+  for (int a = 0; a < kAhead; ++a) {
+    load(held[a], kbegin + D * a);
+    __builtin_amdgcn_sched_barrier(0);   // (in this order, or the loop waits for all of them)
+  }
+  const bool live = m0 < p.rows && n0 + wn0 < p.cols;
+  auto chunk = [&](int a, int k0) {
+    // (every wave has multiplied this stage's last chunk: it has passed the barrier of the one between)
+    float *stage = lds + (a & 1) * kStage;
+#pragma unroll
+    for (int s = 0; s < P; ++s) *reinterpret_cast<u32x4 *>(stage + (prow + RPP * s) * STRIDE + 4 * quad) = held[a][s];
+    load(held[a], k0 + kAhead * D);
+    __syncthreads();
+    if (!live) return;
+    const float *pa = stage + (lane & 31) * STRIDE + BK * g + 4 * (lane >> 5), *pb = pa + (TM + wn0) * STRIDE;
+#pragma unroll
+    for (int c = 0; c < D; c += CH)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float4 qa = *reinterpret_cast<const float4 *>(pa + c + 8 * j), qb = *reinterpret_cast<const float4 *>(pb + c + 8 * j);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qa.x, qb.x, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qa.y, qb.y, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qa.z, qb.z, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(qa.w, qb.w, acc, 0, 0, 0);
+      }
+  };
+  // (whole turns in the loop: a way back from the middle of one would wait for every load in flight)
+  int k0 = kbegin;
+  for (; k0 + (kAhead - 1) * D < kend; k0 += kAhead * D)
+#pragma unroll
+    for (int a = 0; a < kAhead; ++a) chunk(a, k0 + a * D);
+#pragma unroll
+  for (int a = 0; a < kAhead - 1; ++a)
+    if (k0 + a * D < kend) chunk(a, k0 + a * D);
+  __syncthreads();
+  // the k-groups' sum in the order of the kernel above
+#pragma unroll
+  for (int half = KG / 2; half >= 1; half /= 2) {
+    if (g >= half && g < 2 * half) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) lds[(((g - half) * SUB + sub) * 16 + e) * 64 + lane] = acc[e];
+    }
+    __syncthreads();
+    if (g < half) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[e] += lds[((g * SUB + sub) * 16 + e) * 64 + lane];
+    }
+    __syncthreads();
+  }
+  const int n = n0 + wn0 + (lane & 31);
+  if (g != 0 || n >= p.cols) return;
+  float *__restrict__ o = p.out + static_cast<int64_t>(z) * p.rows * p.cols + n;
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    const int m = m0 + 4 * (lane >> 5) + 8 * (e >> 2) + (e & 3);
+    if (m < p.rows) o[static_cast<int64_t>(m) * p.cols] = acc[e];
+  }
+}
+
 // ---------------------------------------------------------------- filter-gradient GEMMs, 128 x 128 tiles
 // Same product and output layout as above.  The unit of work is one tile of one (range, xi) pair; the
 // grid is NB resident blocks on every compute unit and block L (in the XCD-aware order) takes units

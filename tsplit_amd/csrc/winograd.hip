@@ -482,10 +482,12 @@ inline int compute_units() {
 
 // How the filter-gradient GEMMs of one run are cut: tile shape, depth per range, and (128 x 128 tiles) the
 // persistent grid.  Narrow layers (64 produced or gathered channels) take 64-wide tiles whose idle waves
-// share the depth, one tile per block, with as many ranges as give three blocks per compute unit, of at least
-// 12 k-steps each (at least 1024 deep, a layer of 1024 tiles ran as 36 blocks; whole call, at least 1024 / 512 /
-// 192 / 128 deep: 64 -> 128 at 32 x 32, 16 images 59 / 41 / 31 / 31 us, 64 -> 96 at 35 x 35, 32 images 75 / 47 / 45 / 42,
-// 64 -> 64 at 56 x 56, 16 images 46 / 37 / 37 / 39).  The others run on the persistent kernel: the number of ranges is chosen so that the units (tiles x ranges x
+// share the depth, one tile per block, with as many ranges as give three blocks per compute unit, of at least 1024 each.
+// Where that is fewer than one and a half blocks per compute unit, the same chains of sums run on tiles of 32 rows and give the
+// same bits (whole call, the wider tiles and these: 36 blocks, 64 -> 128 at 32 x 32, 16 images 59 and 31 us; 72, 64 -> 96 at 35 x 35,
+// 32 images 75 and 39; 108, 64 -> 64 at 56 x 56, 16 images 45 and 34; 324, 54 x 54, 48 images 94 and 89; 360, 96 -> 64 at 71 x 71, 32
+// images 167 and 159; 432, 64 -> 64 at 54 x 54, 64 images 133 and 141; 720, 64 -> 512 at 50 x 50, 64 images 511 and 545).
+// The others run on the persistent kernel: the number of ranges is chosen so that the units (tiles x ranges x
 // 36) fill one, two or three rounds of the grid as fully as possible, fewer rounds winning unless more
 // rounds fill at least 7 % better; a range keeps at least 12 k-steps.
 struct GradPlan {
@@ -493,6 +495,7 @@ struct GradPlan {
   int tm, tn;           // tiles
   int kchunk;           // depth per range
   int grid;             // persistent grid (128 x 128 tiles), else 0
+  bool fine;            // narrow layers: tiles of 32 rows
 };
 constexpr int kGradBlocksPerCu = 3;
 
@@ -506,9 +509,10 @@ inline GradPlan plan_grad_gemm(int O, int C, int ld, int cus) {
     g.tn = (C + g.tile_n - 1) / g.tile_n;
     const int per = kXi * g.tm * g.tn;
     int ranges = std::max(1, (slots + per / 2) / per);
-    ranges = std::min(ranges, std::max(1, ld / (12 * BK)));
+    ranges = std::min(ranges, std::max(1, ld / 1024));
     g.kchunk = ((ld + ranges - 1) / ranges + 63) / 64 * 64;
     g.grid = 0;
+    g.fine = 2 * per * ranges < 3 * cus;
     return g;
   }
   g.tile_m = g.tile_n = 128;
@@ -543,6 +547,13 @@ inline void launch_grad_gemm(const GradPlan &g, wg::GradProblem p, int here, hip
       hipLaunchKernelGGL((wg::wino_grad_gemm_split_kernel<kGradBlocksPerCu>), dim3(grid), dim3(kThreads), 0, st, p, units);
     else
       hipLaunchKernelGGL((wg::wino_grad_gemm_kernel<kGradBlocksPerCu>), dim3(grid), dim3(kThreads), 0, st, p, units);
+    return;
+  }
+  if (g.fine) {
+    const bool both = g.tile_m == 64 && g.tile_n == 64;   // four k-groups
+    const int tm = (p.rows + 31) / 32, tn = both ? (p.cols + 31) / 32 : (p.cols + 63) / 64;
+    hipLaunchKernelGGL((both ? wg::wino_grad_gemm_fine_kernel<4> : wg::wino_grad_gemm_fine_kernel<2>), dim3(grid_blocks(tm, tn, kXi * here)),
+                       dim3(kThreads), 0, st, p, TileGrid{tm, tn, tm * tn * kXi * here});
     return;
   }
   const TileGrid tg{g.tm, g.tn, units};
