@@ -428,10 +428,17 @@ class Tape(object):
         self._nodes.append(node)
         self._readers.append(0)
         for i in inputs:
-            if i.node >= 0:
-                self._readers[i.node] += 1
+            n = self._call_of(i)
+            if n >= 0:
+                self._readers[n] += 1
         self._after_forward(node)
         return v
+
+    def _call_of(self, var):
+        """The index of the operator call on this tape that produced var; -1 for a leaf, and for a value that was carried here from
+        another tape or from before a reverse sweep, whose `node` counts other calls."""
+        n = var.node
+        return n if 0 <= n < len(self._nodes) and self._nodes[n].out is var else -1
 
     # hooks of executors that manage memory (tsplit_amd.tape_budget)
     def _after_forward(self, node):
@@ -458,7 +465,7 @@ class Tape(object):
 
     def _owns(self, var, fresh):
         var.own = fresh and self._can("add_to")
-        if var.own and var.node < 0:
+        if var.own and self._call_of(var) < 0:
             self._leaves.append(var)      # a leaf's gradient is the caller's once the sweep ends
 
     # ---- products with something behind them: one call where the backend has it, else the operators one by one
@@ -489,11 +496,12 @@ class Tape(object):
         """Adds op(a) op(b) to var's gradient."""
         if not var.needs_grad:
             return
-        if var.node in self._gates and self._readers[var.node] == 1 and var.grad is None:
+        n = self._call_of(var)
+        if n in self._gates and self._readers[n] == 1 and var.grad is None:
             # a Relu's output that goes nowhere else: its gradient behind the product that makes it
-            var.grad = self.b.matmul_add(a, ta, b, tb, var.shape, gate=self._gates[var.node].value)[0]
+            var.grad = self.b.matmul_add(a, ta, b, tb, var.shape, gate=self._gates[n].value)[0]
             self._owns(var, True)
-            self._gated.add(var.node)
+            self._gated.add(n)
         elif var.own:
             self.b.matmul_add(a, ta, b, tb, var.shape, addend=var.grad, out=var.grad)
         else:
@@ -596,7 +604,7 @@ class Tape(object):
         """gpu_ops/Relu.py:51,117."""
         def fwd():
             return self.b.relu(x.value, x.shape)
-        y = self._ready.pop(x.node, None)
+        y = self._ready.pop(self._call_of(x), None)
         out = None
 
         def back(g):
@@ -711,10 +719,12 @@ class Tape(object):
             known = _prod([s for s in shape if s != -1])
             shape[shape.index(-1)] = _prod(a.shape) // known
         shape = tuple(shape)
-        # operators' outputs and gradients are written once, so another shape of one is a view of it; parameters and inputs are
-        # the caller's to write again, so they are copied
+        # this tape's outputs and gradients are written once, so another shape of one is a view of it; parameters, inputs and what
+        # other tapes left are the caller's to write again, so they are copied
+        made_here = self._call_of(a) >= 0
+
         def fwd():
-            return self._seen_as(a.value, shape) if a.node >= 0 else self.b.reshape(a.value, shape)
+            return self._seen_as(a.value, shape) if made_here else self.b.reshape(a.value, shape)
         return self._out(fwd(), shape, [a], lambda g: self._acc(a, self._seen_as(g, a.shape)), saved=[], redo=fwd)
 
     @_op
@@ -855,13 +865,14 @@ class Tape(object):
                 self._owns(v, True)
             if scores.needs_grad:
                 # scores that go nowhere else take their scale and their selection behind this product
-                alone = scores.node in self._scores and self._readers[scores.node] == 1 and scores.grad is None
-                scale, causal = self._scores[scores.node] if alone else (1.0, False)
+                n = self._call_of(scores)
+                alone = n in self._scores and self._readers[n] == 1 and scores.grad is None
+                scale, causal = self._scores[n] if alone else (1.0, False)
                 scores.grad = self._heads_product(g, ys, False, v.value, v.shape, True, scores.shape, heads, scale, causal=causal,
                                                   addend=scores.grad)
                 self._owns(scores, True)
                 if alone:
-                    self._scaled.add(scores.node)
+                    self._scaled.add(n)
         return self._out(y, ys, [u for u in (scores, v, residual) if u is not None], back, saved=[scores, v])
 
     def takes_cells(self, x, initial, steps, units):
