@@ -4,42 +4,8 @@ primitives that a device backend has for products with something behind them."""
 import numpy as np
 import pytest
 
-from oracle_backend import OracleBackend, _s
+from oracle_backend import OracleBackend, WithMore
 from tsplit_amd import graph
-
-
-class WithMore(OracleBackend):
-    """The oracle's operators behind the device backend's calls that do several at once."""
-
-    def view(self, x, shape):
-        return np.asarray(x).reshape(shape)
-
-    def add_to(self, a, b):
-        a[...] = self.add(a, b, a.shape)
-
-    def matmul_add(self, a, ta, b, tb, out_shape, bias=None, addend=None, relu=False, out=None, gate=None):
-        c = self.matmul(a.reshape(-1, a.shape[-1]), ta, b.reshape(-1, b.shape[-1]), tb, None)
-        if bias is not None:
-            c = self.add(c, self.broadcast_to(bias, c.shape), None)
-        c = c.reshape(out_shape)
-        if addend is not None:
-            c = self.add(c, addend, None)
-        if gate is not None:
-            c = self.relu_grad(gate, c, None)
-        if out is not None:
-            out[...] = c
-            c = out
-        return c, self.relu(c, None) if relu else None
-
-    def heads_matmul(self, a, ta, b, tb, out_shape, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0, addend=None):
-        def split(v):
-            return v if v.ndim == 4 else v.reshape(v.shape[0], v.shape[1], heads, -1).transpose(0, 2, 1, 3)
-        y = _s(alpha) * self.batch_matmul(split(a), ta, split(b), tb, None)
-        if causal:
-            y = _s(np.where(np.tril(np.ones(y.shape[2:], bool)), y, fill))
-        if len(out_shape) == 3:
-            y = y.transpose(0, 2, 1, 3).reshape(out_shape)
-        return _s(y if addend is None else y + addend)
 
 
 BACKENDS = [OracleBackend, WithMore]

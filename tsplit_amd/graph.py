@@ -996,14 +996,20 @@ class Tape(object):
         """scale * table[id] + positions, those left out where the id is 0 (examples/transformer.py:189-232 node by node)."""
         ys = tuple(ids.shape) + (table.shape[1],)
         fused = self._can("embedding_add")
+
+        def where_an_id(v):
+            cond = self.b.broadcast_shape(self.b.reshape(ids.value, tuple(ids.shape) + (1,)), ys)
+            return self.b.where(cond, v, self.b.zeros(ys), ys)
         if fused:
             y = self.b.embedding_add(table.value, ids.value, scale, positions.value, ys)
         else:
-            cond = self.b.broadcast_shape(self.b.reshape(ids.value, tuple(ids.shape) + (1,)), ys)
-            y = self.b.add(self.b.mul_const(self.b.embedding(table.value, ids.value, ys), scale, ys),
-                           self.b.where(cond, positions.value, self.b.zeros(ys), ys), ys)
+            y = self.b.add(self.b.mul_const(self.b.embedding(table.value, ids.value, ys), scale, ys), where_an_id(positions.value), ys)
 
         def back(g):
+            if positions.needs_grad:
+                self._acc(positions, where_an_id(g), fresh=True)
+            if not table.needs_grad:
+                return
             if fused and table.own:
                 self.b.embedding_add_grad(g, ids.value, scale, table.shape, table.grad)
             elif fused:
