@@ -29,3 +29,17 @@ def test_embedding_and_positions_both_get_their_gradients(backend, learned):
         assert (got is not None) == (want is not None) == yes
         if yes:
             np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("learned", ["x", "initial"])
+def test_lstm_cells_refuse_what_they_give_no_gradient(learned):
+    class WithCells(WithMore):
+        def lstm(self, x, params, initial, steps):
+            return np.zeros((x.shape[0], 3), np.float32), None
+
+    t = graph.Tape(WithCells())
+    x, initial = [(t.param if name == learned else t.const)(np.zeros(s, np.float32), s) for name, s in (("x", (2, 8)), ("initial", (1,)))]
+    params = [t.param(np.zeros(s, np.float32), s) for _ in range(4) for s in ((2, 3), (3, 3), (3,))]
+    assert not t.takes_cells(x, initial, 4, 3)
+    with pytest.raises(ValueError, match="gradient"):
+        t.lstm_cells(x, params, initial, 4)

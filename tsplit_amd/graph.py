@@ -886,6 +886,8 @@ class Tape(object):
     def lstm_cells(self, x, params, initial, steps):
         """The last hidden state of `steps` LSTM cells on the frames of x, from a state of one value everywhere; params: W, U and b of
         the forget, input, output and candidate gates.  The reference's graph spells out every cell (examples/LSTM.py:52-84)."""
+        if x.needs_grad or initial.needs_grad:
+            raise ValueError("lstm_cells gives the frames and the initial state no gradient: spell the cells out (takes_cells)")
         values = [p.value for p in params]
         y, saved = self.b.lstm(x.value, values, initial.value, steps)
 
