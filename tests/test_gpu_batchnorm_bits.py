@@ -53,3 +53,37 @@ def digests(shape):
 @pytest.mark.parametrize("shape", SHAPES)
 def test_results_keep_their_bits(shape):
     assert digests(shape) == GOLDEN[shape]
+
+
+# the same kernels, planes of whole words in memory order (56 x 56 and 112 x 112) and short planes in words (4 x 4)
+@pytest.mark.parametrize("shape", SHAPES + [(1030, 3, 4, 4), (16, 3, 56, 56)])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+def test_pair_passes_on_nan_as_the_two_calls_do(shape, bad):
+    """A NaN or an infinity makes its channel's statistics NaN: the gradients of BatchNorm + Relu in one call, with saved doubles or with
+    both layers' arrays, are NaN where those of the two calls are, beta's among them."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    ctx = nd.gpu(0)
+    rng = np.random.RandomState(sum(shape))
+    c = shape[1]
+    x = rng.normal(size=shape).astype(np.float32)
+    x[1, 1, 1, 1] = bad
+    gx, dy = nd.array(x, ctx), nd.array(rng.normal(size=shape).astype(np.float32), ctx)
+    gamma, beta = [nd.array(rng.normal(size=(1, c, 1, 1)).astype(np.float32), ctx) for _ in range(2)]
+    bn, y, dbn = [nd.empty(shape, ctx) for _ in range(3)]
+
+    def gradients():
+        return nd.empty(shape, ctx), nd.empty((1, c, 1, 1), ctx), nd.empty((1, c, 1, 1), ctx)
+    two, one, both = gradients(), gradients(), gradients()
+    L.CuDNN_Batch_Normalization(gx, gamma, beta, bn, None, None, 0.99, 0.01)
+    L.relu(bn, y)
+    L.relu_gradient(bn, dy, dbn)
+    L.CuDNN_Batch_Normalization_gradient(dbn, gx, gamma, *two, None, None, 0.01)
+    assert np.isnan(two[2].asnumpy()[0, 1]) and np.isfinite(two[2].asnumpy()[0, [0, 2]]).all()
+    y1, mean, istd = nd.empty(shape, ctx), nd.empty((c, 2), ctx), nd.empty((c, 2), ctx)
+    L.batch_norm_relu(gx, gamma, beta, y1, mean, istd, 0.01)
+    L.batch_norm_relu_gradient(dy, gx, gamma, beta, *one, mean, istd, 0.01)
+    pair, bn1, r1, dbn1 = nd.empty((c, 2), ctx), nd.empty(shape, ctx), nd.empty(shape, ctx), nd.empty(shape, ctx)
+    L.batch_norm_then_relu(gx, gamma, beta, bn1, r1, pair, None, None, 0.01)
+    L.batch_norm_then_relu_gradient(dy, gx, gamma, pair, dbn1, *both, None, None, 0.01)
+    for got, want in [(y1, y), (bn1, bn), (r1, y), (dbn1, dbn)] + list(zip(one, two)) + list(zip(both, two)):
+        np.testing.assert_array_equal(got.asnumpy(), want.asnumpy())

@@ -94,18 +94,23 @@ __device__ __forceinline__ f32x4 relu_w(const f32x4 &z) {
 }
 __device__ __forceinline__ float relu_w(const float &z) { return relu1(z); }
 __device__ __forceinline__ float gate1(float z) { return z > 0.f ? 1.f : (z < 0.f ? 0.f : 0.5f); }
-// dy * relu'(a*x + b)
-__device__ __forceinline__ float gated(const float &dy, const float &x, float a, float b) { return dy * gate1(axpb(x, a, b)); }
+// dy * relu'(a*x + b).  kHalf takes the factor of a NaN for 0.5 (the fused pair with saved floats); kOperator is Relu's gradient
+// operator, NaN included (the forms that have the bits of the two calls).
+enum Gate { kNone, kHalf, kOperator };
+template <int GATE>
+__device__ __forceinline__ float gated(const float &dy, const float &x, float a, float b) {
+  return GATE == kOperator ? relu_grad_of(axpb(x, a, b), dy) : GATE == kHalf ? dy * gate1(axpb(x, a, b)) : dy;
+}
+template <int GATE>
 __device__ __forceinline__ f32x4 gated(const f32x4 &dy, const f32x4 &x, float a, float b) {
-  const f32x4 r = {gated(dy.x, x.x, a, b), gated(dy.y, x.y, a, b), gated(dy.z, x.z, a, b), gated(dy.w, x.w, a, b)};
+  const f32x4 r = {gated<GATE>(dy.x, x.x, a, b), gated<GATE>(dy.y, x.y, a, b), gated<GATE>(dy.z, x.z, a, b), gated<GATE>(dy.w, x.w, a, b)};
   return r;
 }
-// the same as Relu's gradient operator has it, NaN included
-__device__ __forceinline__ float gated_op(const float &dy, const float &x, float a, float b) { return relu_grad_of(axpb(x, a, b), dy); }
-__device__ __forceinline__ f32x4 gated_op(const f32x4 &dy, const f32x4 &x, float a, float b) {
-  const f32x4 r = {gated_op(dy.x, x.x, a, b), gated_op(dy.y, x.y, a, b), gated_op(dy.z, x.z, a, b), gated_op(dy.w, x.w, a, b)};
-  return r;
-}
+// What a gradient kernel's form does with the gradient behind a Relu.  kAlone: there is none.  kFused: y is Relu's result, the BatchNorm's
+// own never leaves; with saved doubles (which also means that the kernel sums the statistics again) it has the bits of the two calls.
+// kBoth: y is the BatchNorm's, r Relu's of it; bits of the two calls.
+enum Pair { kAlone, kFused, kBoth };
+constexpr int gate_of(int pair, bool stats) { return pair == kBoth || (pair == kFused && stats) ? kOperator : pair == kFused ? kHalf : kNone; }
 // k1 dy + k2 x + k3; in the one-pass kernels the other product is the fused one
 __device__ __forceinline__ float lin2(const float &dy, const float &x, float k1, float k2, float k3) { return fmaf(k2, x, k1 * dy) + k3; }
 __device__ __forceinline__ f32x4 lin2(const f32x4 &dy, const f32x4 &x, float k1, float k2, float k3) {
@@ -215,8 +220,6 @@ __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restr
 
 // y = a*x + b (then Relu) over a (split, channel) grid: for planes too short for the plane-major kernel
 // and for arrays without 16-byte words
-// kFused: y is Relu's result, the BatchNorm's own never leaves.  kBoth: y is the BatchNorm's, r Relu's of it.
-enum Pair { kAlone, kFused, kBoth };
 template <int VEC, int RELU>
 __global__ __launch_bounds__(kThreads) void bn_apply_kernel(const float *__restrict__ x, float *__restrict__ y, float *__restrict__ r,
                                                             const float *__restrict__ coef, Geo g) {
@@ -288,6 +291,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
                                                                  const float *__restrict__ pair, float *__restrict__ dg) {
   using W = typename Word<VEC>::T;
   constexpr bool kLast = RELU == kFused && !STATS;
+  constexpr int kGate = gate_of(RELU, STATS);
   __shared__ double sm[4 * kWaves];
   const int c = blockIdx.y, s = blockIdx.x;
   float ga = 0.f, gb = 0.f;
@@ -314,11 +318,8 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
     }
 #pragma unroll
     for (int u = 0; u < kReadAhead; ++u) {
-      if (RELU == kFused) dv[u] = gated(dv[u], xv[u], ga, gb);
-      if (RELU == kBoth) {
-        dv[u] = gated_op(dv[u], xv[u], ga, gb);
-        reinterpret_cast<W *>(dg)[word_addr<VEC>(g, i + u * kThreads, c)] = dv[u];
-      }
+      dv[u] = gated<kGate>(dv[u], xv[u], ga, gb);
+      if (RELU == kBoth) reinterpret_cast<W *>(dg)[word_addr<VEC>(g, i + u * kThreads, c)] = dv[u];
       acc_dot<kLast>(dv[u], xv[u], sdy, sdx);
       if (STATS) acc2(xv[u], sx, sq);
     }
@@ -326,8 +327,8 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_reduce_kernel(const float *__
   for (; i < end; i += kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c);
     W x0 = xw[a0], d0 = dw[a0];
-    if (RELU == kFused) d0 = gated(d0, x0, ga, gb);
-    if (RELU == kBoth) reinterpret_cast<W *>(dg)[a0] = d0 = gated_op(d0, x0, ga, gb);
+    d0 = gated<kGate>(d0, x0, ga, gb);
+    if (RELU == kBoth) reinterpret_cast<W *>(dg)[a0] = d0;
     acc_dot(d0, x0, sdy, sdx);
     if (STATS) acc2(x0, sx, sq);
   }
@@ -410,14 +411,14 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_coef_kernel(const double *__r
   }
 }
 
-template <int VEC, bool RELU>
+template <int VEC, int GATE>
 __global__ __launch_bounds__(kThreads) void bn_bwd_dx_kernel(const float *__restrict__ dy, const float *__restrict__ x,
                                                              float *__restrict__ dx, const float *__restrict__ coef,
                                                              Geo g) {
   using W = typename Word<VEC>::T;
   const int c = blockIdx.y;
   const float k1 = coef[5 * c], k2 = coef[5 * c + 1], k3 = coef[5 * c + 2];
-  const float ga = RELU ? coef[5 * c + 3] : 0.f, gb = RELU ? coef[5 * c + 4] : 0.f;
+  const float ga = GATE ? coef[5 * c + 3] : 0.f, gb = GATE ? coef[5 * c + 4] : 0.f;
   const uint32_t begin = blockIdx.x * g.chunk;
   const uint32_t end = min(begin + g.chunk, g.words);
   const W *xw = reinterpret_cast<const W *>(x);
@@ -428,18 +429,18 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_dx_kernel(const float *__rest
     const int64_t a0 = word_addr<VEC>(g, i, c), a1 = word_addr<VEC>(g, i + kThreads, c);
     const W x0 = __builtin_nontemporal_load(xw + a0), d0 = __builtin_nontemporal_load(dw + a0);
     const W x1 = __builtin_nontemporal_load(xw + a1), d1 = __builtin_nontemporal_load(dw + a1);
-    __builtin_nontemporal_store(lin2(RELU ? gated(d0, x0, ga, gb) : d0, x0, k1, k2, k3), ow + a0);
-    __builtin_nontemporal_store(lin2(RELU ? gated(d1, x1, ga, gb) : d1, x1, k1, k2, k3), ow + a1);
+    __builtin_nontemporal_store(lin2(gated<GATE>(d0, x0, ga, gb), x0, k1, k2, k3), ow + a0);
+    __builtin_nontemporal_store(lin2(gated<GATE>(d1, x1, ga, gb), x1, k1, k2, k3), ow + a1);
   }
   for (; i < end; i += kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c);
     const W x0 = __builtin_nontemporal_load(xw + a0), d0 = __builtin_nontemporal_load(dw + a0);
-    __builtin_nontemporal_store(lin2(RELU ? gated(d0, x0, ga, gb) : d0, x0, k1, k2, k3), ow + a0);
+    __builtin_nontemporal_store(lin2(gated<GATE>(d0, x0, ga, gb), x0, k1, k2, k3), ow + a0);
   }
 }
 
 // in the order of memory, as bn_apply_plane_kernel
-template <bool RELU>
+template <int GATE>
 __global__ __launch_bounds__(kThreads) void bn_bwd_dx_plane_kernel(const f32x4 *__restrict__ dy, const f32x4 *__restrict__ x,
                                                                    f32x4 *__restrict__ dx, const float *__restrict__ coef,
                                                                    PlaneGeo g) {
@@ -447,9 +448,9 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_dx_plane_kernel(const f32x4 *
   if (i >= g.words) return;
   const uint32_t c = word_channel(g, i);
   const float k1 = coef[5 * c], k2 = coef[5 * c + 1], k3 = coef[5 * c + 2];
-  const float ga = RELU ? coef[5 * c + 3] : 0.f, gb = RELU ? coef[5 * c + 4] : 0.f;
+  const float ga = GATE ? coef[5 * c + 3] : 0.f, gb = GATE ? coef[5 * c + 4] : 0.f;
   const f32x4 xv = __builtin_nontemporal_load(x + i), dv = __builtin_nontemporal_load(dy + i);
-  __builtin_nontemporal_store(lin2(RELU ? gated(dv, xv, ga, gb) : dv, xv, k1, k2, k3), dx + i);
+  __builtin_nontemporal_store(lin2(gated<GATE>(dv, xv, ga, gb), xv, k1, k2, k3), dx + i);
 }
 
 // ---- one block per channel, the channel in registers ------------------------------------
@@ -539,6 +540,7 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
                                                                   const float *__restrict__ save_istd, bool wide,
                                                                   float *__restrict__ dgamma, float *__restrict__ dbeta,
                                                                   const float *__restrict__ pair, float *__restrict__ dg) {
+  constexpr int kGate = gate_of(RELU, STATS);
   __shared__ double sm[kWaves];
   __shared__ float coef[3];
   const int c = blockIdx.x;
@@ -558,18 +560,18 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     const int64_t at = ok ? chan_addr(hw, e, c, C) : 0;
     xv[r] = ok ? __builtin_nontemporal_load(x + at) : 0.f;
     dv[r] = ok ? __builtin_nontemporal_load(dy + at) : 0.f;
-    if constexpr (RELU != kBoth) {
-      if (RELU == kFused) dv[r] = gated(dv[r], xv[r], ga, gb);
+    if constexpr (kGate != kOperator) {
+      dv[r] = gated<kGate>(dv[r], xv[r], ga, gb);
       acc_dot(dv[r], xv[r], sdy, sdx);
       if (STATS) squares_onepass(xv, r, sx, sq);
     }
   }
-  if constexpr (RELU == kBoth) {
+  if constexpr (kGate == kOperator) {
     // (with its selects the compiler waits for every load by itself unless all are asked for first: 43 us for 17)
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      dv[r] = r * kThreads + threadIdx.x < m ? gated_op(dv[r], xv[r], ga, gb) : 0.f;
+      dv[r] = r * kThreads + threadIdx.x < m ? gated<kOperator>(dv[r], xv[r], ga, gb) : 0.f;
       acc_dot(dv[r], xv[r], sdy, sdx);
       if (STATS) squares_onepass(xv, r, sx, sq);
     }
@@ -690,7 +692,7 @@ __global__ __launch_bounds__(kThreads) void bn_gate_kernel(const float *__restri
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
   if (i >= g.words) return;
   const uint32_t c = word_channel(g, i);
-  reinterpret_cast<W *>(dg)[i] = gated_op(reinterpret_cast<const W *>(dy)[i], reinterpret_cast<const W *>(x)[i], pair[2 * c], pair[2 * c + 1]);
+  reinterpret_cast<W *>(dg)[i] = gated<kOperator>(reinterpret_cast<const W *>(dy)[i], reinterpret_cast<const W *>(x)[i], pair[2 * c], pair[2 * c + 1]);
 }
 
 // ---------------------------------------------------------------- BatchNorm + Relu + 2x2 / stride 2 max pooling
@@ -1209,10 +1211,10 @@ static int bn_backward(const char *who, int relu, const DLArrayHandle gradient_Y
     hipLaunchKernelGGL((bn_bwd_coef_kernel<R == kFused>), dim3(Cu), dim3(kThreads), 0, s, static_cast<const double *>(part),  \
                        rd.S, cf(bn_scale), bias, eps, inv_m, sm, sv, wide, coef, dg, db);                                 \
     if (V == 4 && plane_major)                                                                                      \
-      hipLaunchKernelGGL((bn_bwd_dx_plane_kernel<R == kFused>), dim3(blocks), dim3(kThreads), 0, s, dyw, xw, dxw,             \
+      hipLaunchKernelGGL((bn_bwd_dx_plane_kernel<R == kFused ? gate_of(R, ST) : kNone>), dim3(blocks), dim3(kThreads), 0, s, dyw, xw, dxw,             \
                          static_cast<const float *>(coef), pg);                                                     \
     else                                                                                                            \
-      hipLaunchKernelGGL((bn_bwd_dx_kernel<V, R == kFused>), gd, dim3(kThreads), 0, s, dr ? dr : cf(gradient_Y), cf(input_X),           \
+      hipLaunchKernelGGL((bn_bwd_dx_kernel<V, R == kFused ? gate_of(R, ST) : kNone>), gd, dim3(kThreads), 0, s, dr ? dr : cf(gradient_Y), cf(input_X),           \
                          mf(gradient_X), static_cast<const float *>(coef), dxp.g);                                  \
   } while (0)
   if (rd.vec == 4) {
