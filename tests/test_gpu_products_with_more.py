@@ -86,6 +86,20 @@ def test_product_with_column_sums(shape, rng):
         L.matrix_multiply_sums(ga, gb, plain, _full((N + 1,)))
 
 
+def test_column_sums_of_ranges_deeper_than_16384_rows_are_the_reductions_own(rng):
+    """(1344 x 1472 fill the chip, so 16640 rows stay one range)"""
+    from tsplit_amd import gpu_links as L
+    M, N, K = 1344, 1472, 16640
+    draw = np.random.default_rng(rng.randint(1 << 30))
+    ga, gb = _dev(draw.standard_normal((K, M), np.float32), draw.standard_normal((K, N), np.float32))
+    plain, c, want, sums = _full((M, N)), _full((M, N)), _full((N,)), _full((N,))
+    L.matrix_multiply(ga, True, gb, False, plain)
+    L.reduce_sum_axis_zero(gb, want)
+    L.matrix_multiply_sums(ga, gb, c, sums)
+    np.testing.assert_array_equal(c.asnumpy(), plain.asnumpy())
+    np.testing.assert_array_equal(sums.asnumpy(), want.asnumpy())
+
+
 def test_product_with_more_split_bf16_and_arrays_of_more_axes(rng):
     from tsplit_amd import gpu_links as L
     x, w, add = rng.normal(size=(3, 7, 40)).astype(np.float32), rng.normal(size=(40, 36)).astype(np.float32), rng.normal(size=(3, 7, 36)).astype(np.float32)

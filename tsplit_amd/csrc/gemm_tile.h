@@ -235,8 +235,8 @@ struct Core {
     run<false>(la, lb, kbegin, kend, lds, acc, false, none);
   }
   // SUMS, where `on`: col[t] is also the sum over the range of what this lane supplies of B's column of tile t (of lane group g the
-  // k = 4 g + i of every half).  Eight of a step are added pairwise, eight steps one by one, then those: no longer a chain of
-  // roundings than a reduction in slices has.
+  // k = 4 g + i of every half).  Eight of a step are added pairwise, eight steps one by one, then those: in ranges of up to
+  // 16 K rows no longer a chain of roundings than a reduction in slices has.
   template <bool SUMS>
   static __device__ __forceinline__ void run(AL &la, BL &lb, int kbegin, int kend, float *lds, f32x4 (&acc)[TM][TN], bool on, float (&col)[TN]) {
     const int lane = threadIdx.x & 63, wm0 = wave_m0(), wn0 = wave_n0();
