@@ -155,17 +155,10 @@ struct Parts {
   int count;
 };
 template <typename W, bool SPLIT>
-__global__ __launch_bounds__(kThreads) void parts_kernel(Parts parts, W *__restrict__ whole, FastDiv row, int64_t total) {
-  const int64_t idx = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+__global__ __launch_bounds__(kThreads) void parts_kernel(Parts parts, W *__restrict__ whole, FastDiv row, uint32_t total) {
+  const uint32_t idx = blockIdx.x * kThreads + threadIdx.x;
   if (idx >= total) return;
-  uint32_t r, j;
-  if (total < (1ll << 32)) {
-    r = row.div(static_cast<uint32_t>(idx));
-    j = static_cast<uint32_t>(idx) - r * row.d;
-  } else {
-    r = static_cast<uint32_t>(idx / row.d);
-    j = static_cast<uint32_t>(idx - static_cast<int64_t>(r) * row.d);
-  }
+  const uint32_t r = row.div(idx), j = idx - r * row.d;
   float *p = parts.p[0];
   uint32_t from = 0, to = parts.at[1];
 #pragma unroll
@@ -194,11 +187,12 @@ int join_or_split(const char *who, const DLArrayHandle *arrays, int count, const
     vec = vec && aligned16(arrays[k]->data) && arrays[k]->shape[axis] * inner % 4 == 0;
   }
   TS_REQUIRE(extent == whole->shape[axis], "%s: the parts' extents on the axis add up to %lld", who, (long long)extent);
+  const int64_t words = extent * inner / (vec ? 4 : 1), total = outer * words;
+  // (a launch has fewer than 2^32 threads)
+  TS_REQUIRE(total <= (1ll << 32) - kThreads - 1, "%s: %lld words, a launch moves fewer than 2^32", who, (long long)total);
   hipStream_t s = stream_of(stream_handle);
   ProfileScope ps(nullptr, s, 0, 0, 0);
-  const int64_t words = extent * inner / (vec ? 4 : 1), total = outer * words;
   if (total == 0) return ps.finish();
-  TS_REQUIRE(words < (1ll << 32) && (total + kThreads - 1) / kThreads < (1ll << 31), "%s: array too large", who);
   Parts parts{};
   parts.count = count;
   for (int k = 0; k < count; ++k) {
@@ -208,9 +202,9 @@ int join_or_split(const char *who, const DLArrayHandle *arrays, int count, const
   const dim3 grid(static_cast<unsigned>((total + kThreads - 1) / kThreads));
   const FastDiv row(static_cast<uint32_t>(words));
   if (vec)
-    hipLaunchKernelGGL((parts_kernel<float4, SPLIT>), grid, dim3(kThreads), 0, s, parts, static_cast<float4 *>(whole->data), row, total);
+    hipLaunchKernelGGL((parts_kernel<float4, SPLIT>), grid, dim3(kThreads), 0, s, parts, static_cast<float4 *>(whole->data), row, static_cast<uint32_t>(total));
   else
-    hipLaunchKernelGGL((parts_kernel<float, SPLIT>), grid, dim3(kThreads), 0, s, parts, static_cast<float *>(whole->data), row, total);
+    hipLaunchKernelGGL((parts_kernel<float, SPLIT>), grid, dim3(kThreads), 0, s, parts, static_cast<float *>(whole->data), row, static_cast<uint32_t>(total));
   return ps.finish();
 }
 

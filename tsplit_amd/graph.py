@@ -745,9 +745,10 @@ class Tape(object):
         return self._out(y, shape, [a, b], back, saved=[], redo=fwd)
 
     def concat_all(self, parts, axis):
-        """The parts one behind the other: one node where the backend joins any number, else chained concats of two
-        (examples/imagenet_inceptionv4.py concatenates in pairs)."""
-        if 2 < len(parts) <= 8 and self._ahead and self._can("join"):
+        """The parts one behind the other: one node where the backend joins any number and the whole is within one launch's reach, else
+        chained concats of two (examples/imagenet_inceptionv4.py concatenates in pairs)."""
+        values = sum(_prod(p.shape) for p in parts)
+        if 2 < len(parts) <= 8 and self._ahead and self._can("join") and values < (1 << 32) - (1 << 10):
             return self.join(parts, axis)
         x = parts[0]
         for p in parts[1:]:
