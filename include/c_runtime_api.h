@@ -515,6 +515,8 @@ int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transposeA, const D
                                DLArrayHandle matC, int heads, float alpha, const DLArrayHandle mask,
                                float mask_value, int causal, float fill, const DLArrayHandle addend,
                                DLStreamHandle stream);
+/* output = scale * input, with causal 0 in place of what lies right of the diagonal of the last two axes; output may be input. */
+int TSplit_HeadsScale(const DLArrayHandle input, float scale, int causal, DLArrayHandle output, DLStreamHandle stream);
 /* ---- Softmax cross-entropy with labels that are one class index a row (a float, as the reference's OneHot takes it),
  *      smoothed: label[j] = on * (j == id) + off (outside the reference's ABI; examples/transformer.py:184-186 builds
  *      the label array).  Otherwise DLGpuSoftmaxCrossEntropy and its gradient. ---- */

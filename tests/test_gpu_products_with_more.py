@@ -120,6 +120,23 @@ def test_product_with_more_split_bf16_and_arrays_of_more_axes(rng):
         L.matrix_multiply_add(gx, False, gw, True, c)
 
 
+# one row, one column, more rows than columns and fewer, columns beyond one pass of a block
+@pytest.mark.parametrize("shape", [(3, 1), (1, 4), (2, 3, 7, 5), (2, 2, 5, 9), (2, 70, 600), (0, 4)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_scale_and_causal_selection(shape, causal, in_place, rng):
+    from tsplit_amd import gpu_links as L
+    x = rng.normal(size=shape).astype(np.float32)
+    x.ravel()[::5] = np.inf
+    gx = _dev(x)[0]
+    out = gx if in_place else _full(shape)
+    L.heads_scale(gx, -0.3, causal, out)
+    want = (np.where(np.tril(np.ones(shape[-2:], bool)), x, np.float32(0)) if causal else x) * np.float32(-0.3)
+    np.testing.assert_array_equal(out.asnumpy().view(np.uint32), want.view(np.uint32))
+    with pytest.raises(RuntimeError):
+        L.heads_scale(gx, 1.0, causal, _full((3, 2, 2)))
+
+
 # heads' widths that are a word, none, larger than a tile; lengths off the tiles, few and many columns, wide results in words or not
 @pytest.mark.parametrize("n,heads,tq,tk,dh", [(2, 3, 5, 7, 4), (3, 2, 65, 33, 33), (1, 4, 128, 64, 64), (2, 1, 70, 130, 66), (5, 4, 50, 77, 64)])
 @pytest.mark.parametrize("causal", [False, True])

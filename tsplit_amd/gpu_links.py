@@ -27,7 +27,7 @@ __all__ = [
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
     "batch_norm_relu", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
-    "optimizer_update_multi", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply",
+    "optimizer_update_multi", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply", "heads_scale",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "join", "part", "lstm_sizes", "lstm", "lstm_gradient",
     "CuDNN_Dropout", "CuDNN_Dropout_gradient", "CuSparse_Csrmv", "CuSparse_Csrmm",
@@ -111,6 +111,11 @@ def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, ma
     check_call(_LIB.TSplit_HeadsMatrixMultiply(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(matC), int(heads),
                                                ctypes.c_float(alpha), _h(mask) if mask else None, ctypes.c_float(mask_value),
                                                int(bool(causal)), ctypes.c_float(fill), _h(addend) if addend else None, _s(stream)))
+
+
+def heads_scale(in_arr, scale, causal, out_arr, stream=None):
+    """out_arr = scale * in_arr, with `causal` 0 right of the diagonal of the last two axes; out_arr may be in_arr."""
+    check_call(_LIB.TSplit_HeadsScale(_h(in_arr), ctypes.c_float(scale), int(bool(causal)), _h(out_arr), _s(stream)))
 
 
 def join(parts, whole, axis, stream=None):

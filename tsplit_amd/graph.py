@@ -151,6 +151,12 @@ class GpuBackend(object):
         self.L.heads_matrix_multiply(a, ta, b, tb, c, heads, alpha, mask, mask_value, causal, fill, addend, self.stream)
         return c
 
+    def heads_scale(self, x, scale, causal, shape, out=None):
+        """scale * x, 0 right of the diagonals with `causal`.  out: the array to write (it may be x), or None for a new one."""
+        out = self.empty(shape) if out is None else out
+        self.L.heads_scale(x, scale, causal, out, self.stream)
+        return out
+
     # ---- normalisation, activations, pooling
     def bn(self, x, gamma, beta, xs, eps):
         y = self.empty(xs)
@@ -836,6 +842,8 @@ class Tape(object):
         def back(g):
             if out.node in self._scaled:
                 self._scaled.discard(out.node)
+            elif self._can("heads_scale"):      # (a gradient that nothing else holds in place: a planner counts no other array there)
+                g = self.b.heads_scale(g, scale, causal, ys, g if out.own else None)
             else:
                 if causal:
                     tril = self.b.broadcast_shape(self.b.from_numpy(np.tril(np.ones((tq, tk), np.float32))), ys)
@@ -1291,7 +1299,7 @@ class MicroTape(Tape):
         for v in outside_vars:
             whole = outside[id(v)][2]
             if whole is not None:
-                self._acc(v, whole)
+                self._acc(v, whole, fresh=True)
         self._put_off = []
         # on this tape the stretch is one operator: it read the outside values, its output is the loss
         # and its backward operators have run

@@ -76,13 +76,14 @@ def _bytes(shape):
 class OpRecord(object):
     """One operator call of a recorded graph.  Indices refer to operator calls (-1: a leaf)."""
     __slots__ = ["bytes", "inputs", "saved", "has_backward", "grad_inputs", "leaf_grad_bytes", "cheap", "name",
-                 "transient", "early_grads", "early_leaf_grad_bytes"]
+                 "transient", "early_grads", "early_leaf_grad_bytes", "back_bytes"]
 
     def __init__(self, nbytes, inputs, saved, has_backward, grad_inputs, leaf_grad_bytes, cheap=False, name=None):
         self.name = name                   # the Tape method of the call
         # a stretch of operators run per micro-tensor (split_tail): bytes it holds on top of its inputs while it
         # runs, the outside values whose gradients it leaves behind, and the parameter gradients it creates
         self.transient, self.early_grads, self.early_leaf_grad_bytes = 0, (), 0
+        self.back_bytes = 0                # held by the backward operators on top of what they read and leave behind
         self.cheap = cheap                 # the operator can compute its output again from its inputs
         self.bytes = nbytes                # of the output
         self.inputs = inputs               # producers of the values the forward operator reads
@@ -126,6 +127,12 @@ def record(build, inputs, fuse_bn_relu=False):
                             node.back is not None,
                             [v.node for v in node.inputs if v.node >= 0 and v.needs_grad] if node.back is not None else [],
                             leaf_grad, node.redo is not None, call[0]))
+    # the gradient of scores that no head_context scales in its product alone may be another operator's array too, so it is scaled into a new one
+    for node, call in zip(t._nodes, t._log):
+        if call[0] != "head_context":
+            for v in node.inputs:
+                if v.node >= 0 and ops[v.node].name == "head_scores":
+                    ops[v.node].back_bytes = ops[v.node].bytes
     leaves = sum(_bytes(s) for s in inputs.values()) + sum(_bytes(v.shape) for v in b.vars.values())
     leaves += sum(_bytes(shape) for _, shape in b._consts.values())
     assert loss.node == len(ops) - 1
@@ -273,6 +280,8 @@ def replay(ops, leaves_bytes, away=(), lead=3, redo=(), hold=1):
         if op.has_backward and (j == n - 1 or j in grads):
             # every input that takes a gradient gets a new array; adding to an earlier one holds the
             # sum and both terms for a moment
+            live += op.back_bytes
+            note(moment)
             for i in op.grad_inputs:
                 extra = ops[i].bytes
                 live += extra
@@ -285,6 +294,7 @@ def replay(ops, leaves_bytes, away=(), lead=3, redo=(), hold=1):
                 note(moment)
             live += op.leaf_grad_bytes
             note(moment)
+            live -= op.back_bytes
         if j in grads:
             live -= grads.pop(j)
         for i in by_last[j]:
