@@ -8,10 +8,13 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n,c,h,w,o,kh,kw,ph,pw,s", [(2, 500, 4, 3, 261, 3, 3, 1, 1, 1), (1, 520, 5, 4, 700, 1, 3, 0, 1, 1), (3, 263, 6, 7, 170, 5, 5, 2, 2, 2),
-                                                     (2, 513, 3, 3, 259, 3, 3, 0, 0, 1)])
-def test_large_filters(n, c, h, w, o, kh, kw, ph, pw, s, rng):
-    from tsplit_amd import gpu_links as L, ndarray as nd
+# (ranges: into how many the depth of the filter gradient is cut, which the fold adds up in fours)
+@pytest.mark.parametrize("n,c,h,w,o,kh,kw,ph,pw,s,ranges", [(2, 500, 4, 3, 261, 3, 3, 1, 1, 1, 1), (1, 520, 5, 4, 700, 1, 3, 0, 1, 1, 1),
+                                                            (3, 263, 6, 7, 170, 5, 5, 2, 2, 2, 1), (2, 513, 3, 3, 259, 3, 3, 0, 0, 1, 1),
+                                                            (64, 500, 4, 4, 261, 3, 3, 1, 1, 1, 2), (33, 263, 9, 7, 170, 5, 5, 2, 2, 2, 3),
+                                                            (64, 512, 4, 4, 512, 3, 3, 1, 1, 1, 4), (16, 500, 8, 8, 700, 1, 3, 0, 1, 1, 5)])
+def test_large_filters(n, c, h, w, o, kh, kw, ph, pw, s, ranges, rng):
+    from tsplit_amd import gpu_links as L, ndarray as nd, profiler
     ctx = nd.gpu(0)
     oh, ow = (h + 2 * ph - kh) // s + 1, (w + 2 * pw - kw) // s + 1
     assert c * o * kh * kw >= 1 << 20
@@ -20,7 +23,9 @@ def test_large_filters(n, c, h, w, o, kh, kw, ph, pw, s, rng):
     y, dx, dw = nd.empty(g.shape, ctx), nd.empty(x.shape, ctx), nd.empty(f.shape, ctx)
     L.CuDNN_conv2d(gx, gf, y, ph, pw, s)
     L.CuDNN_conv2d_gradient_of_data(gf, gg, dx, ph, pw, s)
-    L.CuDNN_conv2d_gradient_of_filter(gx, gg, dw, ph, pw, s)
+    p = profiler.CreateProfiler()
+    L.CuDNN_conv2d_gradient_of_filter(gx, gg, dw, ph, pw, s, None, p)
+    assert abs(p.workspace_memory * 2 ** 18 / f.size - ranges) < 1e-3
     # the sums in float64: patches of the padded input, [n, oh * ow, c * kh * kw]
     xp = np.pad(x.astype(np.float64), ((0, 0), (0, 0), (ph, ph), (pw, pw)))
     patches = np.stack([xp[:, :, u:u + s * (oh - 1) + 1:s, v:v + s * (ow - 1) + 1:s] for u in range(kh) for v in range(kw)], axis=2)
