@@ -501,14 +501,14 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
  *      DLGpuBroadcastTo + DLGpuMatrixElementwiseAdd, DLGpuRelu and DLGpuReluGradient round it: the same bits.
  *      TSplit_HeadsMatrixMultiply: for every n and head, C = alpha * op(A) op(B), + mask_value in the columns where
  *      mask (of n x columns values) is 0, then `fill` in the columns right of the row where causal != 0, then
- *      + addend (laid out as C, not C).  A, B and C are each [n, heads, rows, columns], or [n, rows, heads *
+ *      + addend (laid out as C, not C); alpha * product + mask_value is rounded once.  A, B and C are each [n, heads, rows, columns], or [n, rows, heads *
  *      columns] with a head's columns side by side: heads are neither split off nor merged by a transpose.
  *      The reference's graph spells these out node by node (examples/transformer.py:56-171). ---- */
 int TSplit_MatrixMultiplyAdd(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
                              const DLArrayHandle bias, const DLArrayHandle addend, const DLArrayHandle gate,
                              DLArrayHandle matC, DLArrayHandle relu, DLStreamHandle stream);
 /* C [M, N] = A' B and sums [N] = the sums of B's columns, A and B of K rows (the last axis' columns): a linear layer's parameter
- * gradients.  C has the bits of DLGpuMatrixMultiply. */
+ * gradients.  C has the bits of DLGpuMatrixMultiply, sums those of DLGpuReduceSumAxisZero to rounding. */
 int TSplit_MatrixMultiplySums(const DLArrayHandle matA, const DLArrayHandle matB, DLArrayHandle matC, DLArrayHandle sums,
                               DLStreamHandle stream);
 int TSplit_HeadsMatrixMultiply(const DLArrayHandle matA, int transposeA, const DLArrayHandle matB, int transposeB,
@@ -538,7 +538,7 @@ int TSplit_LstmGradient(const DLArrayHandle dlast, const DLArrayHandle x, const 
                         const DLArrayHandle initial, int steps, const DLArrayHandle rows, const DLArrayHandle packed,
                         const DLArrayHandle gates, const DLArrayHandle cells, DLArrayHandle dgates,
                         DLArrayHandle *dparams, DLStreamHandle stream);
-/* ---- output = scale * table[id] + (id != 0 ? positions : 0), positions of the output's size, and the table's gradient,
+/* ---- output = scale * table[id] + (id != 0 ? positions : 0), positions of the output's size (rounded once), and the table's gradient,
  *      added to what table_grad holds where add_to != 0 (outside the reference's ABI; examples/transformer.py:189-232 node by node). ---- */
 int TSplit_EmbeddingAdd(const DLArrayHandle table, const DLArrayHandle ids, float scale, const DLArrayHandle positions,
                         DLArrayHandle output, DLStreamHandle stream);

@@ -163,10 +163,6 @@ __global__ __launch_bounds__(kThreads) void bn_stats_kernel(const float *__restr
   }
 }
 
-// Folds the partials of channel c (the pair k at part[(c * part_c + k * part_k) * 2]; fixed order per
-// thread, fixed tree: deterministic) into the coefficients of y = a*x + b, coef[2c] and coef[2c + 1],
-// and the saved statistics.  One block per channel, so that the streaming pass behind it starts with
-// two loads instead of a reduction in every block.
 // Saved statistics: one float a channel, or (wide, the fused forms only) one double in the place of two floats.  From floats the
 // fused backward pass cannot rebuild the a and b of an unfused forward pass, so the fused forward pass then takes rounded statistics too;
 // from doubles it can, and the fused pair has the bits of BatchNorm and Relu one by one; its gradient then forms the statistics of
@@ -181,6 +177,10 @@ __device__ __forceinline__ void save_stat(float *p, int c, bool wide, double v) 
     p[c] = static_cast<float>(v);
 }
 
+// Folds the partials of channel c (the pair k at part[(c * part_c + k * part_k) * 2]; fixed order per
+// thread, fixed tree: deterministic) into the coefficients of y = a*x + b, coef[2c] and coef[2c + 1],
+// and the saved statistics.  One block per channel, so that the streaming pass behind it starts with
+// two loads instead of a reduction in every block.
 template <bool RELU>
 __global__ __launch_bounds__(kThreads) void bn_coef_kernel(const double *__restrict__ part, int S, int64_t part_c,
                                                            int64_t part_k, const float *__restrict__ gamma,
@@ -1152,6 +1152,11 @@ static int bn_backward(const char *who, int relu, const DLArrayHandle gradient_Y
       dy1 = dr;
       relu = kAlone;
     }
+// The kernels' forms <statistics summed again, Pair> by what the call brings, here and in the two-pass kernels below:
+//   kAlone, saved arrays  <no, kAlone>      kFused, saved floats   <no, kFused>     kBoth, saved arrays  <no, kBoth>
+//   kAlone, none          <yes, kAlone>     kFused, saved doubles  <yes, kFused>    kBoth, none          <yes, kBoth>
+// kFused always has saved arrays, and `wide` says that they are doubles; `pair` and `dr` are kBoth's alone; `sm` and `sv` are null
+// unless both saved arrays are given.
 #define BN_BWD1(R, ST, RL)                                                                                          \
   hipLaunchKernelGGL((bn_bwd_onepass_kernel<R, ST, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,     \
                      dy1, cf(input_X), mf(gradient_X), cf(bn_scale), bias1, FastDiv(hw),                 \

@@ -467,10 +467,10 @@ static __global__ __launch_bounds__(256) void conv_relay_kernel(Relay R) {
   R.out[idx] = ch < R.chans ? R.w[row * R.w_row + ch * R.w_chan + (F.a + R.s * u) * R.f_w + F.b + R.s * v] : 0.f;
 }
 
-// The same for a filter of one phase with all its taps, kTurnRows rows x kTurnChans channels a block, through LDS: `along` the rows of the
-// output, memory holds a row's channels (forward) or a channel's rows (data gradient) side by side, and runs of either are read, and
-// written, whole.  One thread a value fetched every value by itself: 512 x 512 x 9 behind other
-// layers 14.5 us, 1.3 TB/s (five such layers both ways: 2.117 -> 2.092 ms a step).
+// The same for a filter of one phase with all its taps, kRelayRows rows x kRelayChans channels a block, through LDS: memory
+// holds a row's channels (forward) or a channel's rows (data gradient, `across`) side by side, and runs of either are read, and of the
+// output's rows written, whole.  One thread a value fetched every value by itself: 512 x 512 x 9 behind other layers 14.5 us, 1.3 TB/s
+// (five such layers both ways: 2.117 -> 2.092 ms a step).
 constexpr int kRelayRows = 8, kRelayChans = 32;
 static __global__ __launch_bounds__(256) void conv_relay_tiles_kernel(const float *__restrict__ w, float *__restrict__ out, int rows, int chans, int padded,
                                                                       FastDiv taps, int64_t w_row, int64_t w_chan, FastDiv tiles) {

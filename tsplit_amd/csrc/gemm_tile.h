@@ -422,7 +422,8 @@ static __global__ __launch_bounds__(256) void fold_two_kernel(const float *__res
 }
 
 // ---- products whose result is worked on before it is stored
-// What follows the sum of products, in this order and with a rounding each, as the operators behind a product would do it:
+// What follows the sum of products, in this order and with a rounding each, as the operators behind a product would do it (but for alpha *
+// sum + mask_value, rounded once; alpha is 1 where there is a bias):
 // v = alpha * sum; + bias[column]; + mask_value where mask[column] is 0; fill where the column lies right of the row; + add; stored, and
 // max(v, 0) stored as well; or the result, as the gradient behind a Relu, taken through it: as a second array or in place of the result.
 // Each of these as an operator of its own reads and writes the whole result again: scores of 32 x 8 x 256 x

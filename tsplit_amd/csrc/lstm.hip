@@ -7,8 +7,8 @@
 // has dh = dz_{t+1} U' with the cell's gradient behind it, and the parameters' gradients are one product over all steps of the
 // rows with dz.
 //
-// What bounds a step is latency: the launch, one trip to memory for h (written on other XCDs a launch ago) and the products' own
-// chain.  So a block is a tile of 16 samples x 16 units (64 blocks at 128 x 128), a wave is one gate of it, everything a wave
+// What bounds a launch a step is latency: the launch, one trip to memory for h (written on other XCDs a launch ago) and the products' own
+// chain.  So a block is a tile of 16 samples x 16 units (128 blocks at 128 samples and 256 units), a wave is one gate of it, everything a wave
 // multiplies is asked for before the first product, and the weights lie in the order of the matrix instruction's lanes, 16 bytes a
 // lane.  v_mfma_f32_16x16x4_f32 sums k = 4 (lane / 16) + i with i its number of four: any order of k will do as long as both
 // operands have it, and this one loads float4 on both sides.

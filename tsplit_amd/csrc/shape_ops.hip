@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kThreads) void embedding_kernel(const W *__restrict
 }
 
 // out[row, :] = scale * table[int(ids[row]), :] + (ids[row] != 0 ? pos[row, :] : 0): the look-up of a token and the position behind it
-// in one pass of 12 bytes a value (as operators of their own: 52, and six launches)
+// in one pass of 12 bytes a value (as operators of their own: 52, and six launches); product and sum are rounded once
 template <typename W>
 __global__ __launch_bounds__(kThreads) void embedding_add_kernel(const W *__restrict__ table, const float *__restrict__ ids, float scale,
                                                                  const W *__restrict__ pos, W *__restrict__ out, FastDiv per_row, int64_t vocab,
