@@ -20,11 +20,12 @@ from . import ndarray
 class Var(object):
     """A value on the tape: backend array, shape, accumulated gradient; `node` is the index of the
     operator call that produced it on its tape (-1 for parameters, inputs and constants)."""
-    __slots__ = ["value", "shape", "grad", "needs_grad", "name", "node", "own"]
+    __slots__ = ["value", "shape", "grad", "needs_grad", "name", "node", "home", "own"]
 
     def __init__(self, value, shape, needs_grad, name=None):
         self.value, self.shape, self.grad, self.needs_grad, self.name = value, tuple(shape), None, needs_grad, name
         self.node = -1
+        self.home = None     # the sweep of the tape that `node` counts in
         self.own = False     # during a reverse sweep: `grad` is an array of this value alone, so more may be added in place
 
 
@@ -402,6 +403,7 @@ class Tape(object):
     def __init__(self, backend):
         self.b = backend
         self._nodes = []     # every operator call, in order (Node)
+        self._sweep = object()   # stands for these calls; the next sweep's are another's
         self._readers = []   # per operator call: how many inputs of later calls its output is
         self._ready = {}     # operator call -> the Relu of its output, where its launch has left that too
         self._leaves = []    # leaves whose gradient arrays are this sweep's
@@ -430,21 +432,19 @@ class Tape(object):
         v = Var(value, shape, any(i.needs_grad for i in inputs))
         saved = inputs if saved is None else [v if s is SELF else s for s in saved]
         node = Node(v, backward if v.needs_grad else None, inputs, saved if v.needs_grad else (), len(self._nodes), redo)
-        v.node = node.index
+        v.node, v.home = node.index, self._sweep
         self._nodes.append(node)
         self._readers.append(0)
         for i in inputs:
-            n = self._call_of(i)
-            if n >= 0:
-                self._readers[n] += 1
+            if i.home is v.home:
+                self._readers[i.node] += 1
         self._after_forward(node)
         return v
 
     def _call_of(self, var):
         """The index of the operator call on this tape that produced var; -1 for a leaf, and for a value that was carried here from
         another tape or from before a reverse sweep, whose `node` counts other calls."""
-        n = var.node
-        return n if 0 <= n < len(self._nodes) and self._nodes[n].out is var else -1
+        return var.node if var.home is self._sweep else -1
 
     # hooks of executors that manage memory (tsplit_amd.tape_budget)
     def _after_forward(self, node):
@@ -471,7 +471,7 @@ class Tape(object):
 
     def _owns(self, var, fresh):
         var.own = fresh and self._can("add_to")
-        if var.own and self._call_of(var) < 0:
+        if var.own and var.home is not self._sweep:
             self._leaves.append(var)      # a leaf's gradient is the caller's once the sweep ends
 
     # ---- products with something behind them: one call where the backend has it, else the operators one by one
@@ -1076,7 +1076,7 @@ class Tape(object):
                     v.grad, v.own = None, False      # interior gradients are dropped as soon as they are consumed
             self._after_backward(node)
         self._release_leaves()
-        self._nodes, self._readers = [], []
+        self._nodes, self._readers, self._sweep = [], [], object()
         self._ready, self._scores, self._scaled, self._gates, self._gated = {}, {}, set(), {}, set()
 
 
