@@ -204,6 +204,28 @@ def test_cross_entropy_with_class_indices_and_with_label_arrays(rows, cols, rng)
         assert (np.abs(g.asnumpy() - grad) <= 100 * EPS * (e / s + lab) * 0.5 / rows).all()
 
 
+# a wave's row, a block's in words and not, rows that registers do not hold; a loss without smoothing and with
+@pytest.mark.parametrize("cols", [200, 1000, 5000, 5003, 40000, 40001])
+@pytest.mark.parametrize("smoothing", [0.0, 0.1])
+def test_cross_entropy_of_logits_masked_with_the_lowest_value(cols, smoothing, rng):
+    from tsplit_amd import gpu_links as L
+    y = rng.normal(size=(3, cols)).astype(np.float32)
+    masked = rng.rand(3, cols) < 0.5
+    masked[:, :2] = False
+    y[masked] = np.finfo(np.float32).min
+    ids = np.float32([0, 1, 1])
+    on, off = 1.0 - smoothing, smoothing / cols
+    lab = on * (np.arange(cols) == ids[:, None]) + off
+    gy, gids, glab, loss, other = _dev(y, ids, lab.astype(np.float32)) + [_full((1,)), _full((1,))]
+    L.softmax_cross_entropy_ids(gy, gids, on, off, loss)
+    L.softmax_cross_entropy(gy, glab, other)
+    y64 = y.astype(np.float64)
+    m = y64.max(1, keepdims=True)
+    per = lab * (np.log(np.exp(y64 - m).sum(1, keepdims=True)) - (y64 - m))
+    for got in (loss, other):
+        assert abs(got.asnumpy()[0] - per.sum(1).mean()) <= 100 * EPS * (np.abs(per).sum(1).mean() + 1)
+
+
 @pytest.mark.parametrize("width", [64, 37])
 def test_look_up_with_positions(width, rng):
     from tsplit_amd import gpu_links as L

@@ -136,8 +136,8 @@ __global__ __launch_bounds__(THREADS == kWave ? 4 * kWave : THREADS) __attribute
 #pragma unroll
       for (int i = 1; i < kWaves; ++i) m = fmaxf(m, sm[i]);
     }
-    // the loss, sum of label * (lse - (x - m)), is lse * sum(label) - sum(label * (x - m)): two terms of one sign.  Of class indices it needs
-    // the sum of x - m and one value more.
+    // the loss, sum of label * (lse - (x - m)), is lse * sum(label) - sum(label * (x - m)): two terms of one sign.  Of class indices
+    // label is `off` (and one value more): weighted as they are added, so that logits masked with the type's lowest value add up.
     float s = 0.f, labels = 0.f, below = 0.f;
     each([&](int w, float(&x)[VEC]) {
       const int j = (w * THREADS + thread) * VEC;
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(THREADS == kWave ? 4 * kWave : THREADS) __attribute
       for (int i = 0; i < VEC; ++i) {
         const float e = j < ncol ? expf(x[i] - m) : 0.f;
         if constexpr (GRAD && WORDS != 0) x[i] = e;
-        if constexpr (!GRAD && Label::kIds) below += j < ncol ? x[i] - m : 0.f;
+        if constexpr (!GRAD && Label::kIds) below = j < ncol ? fmaf(lab.off, x[i] - m, below) : below;
         if constexpr (!GRAD && !Label::kIds) {
           labels += l[i];
           below += j < ncol ? l[i] * (x[i] - m) : 0.f;
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(THREADS == kWave ? 4 * kWave : THREADS) __attribute
         if constexpr (Label::kIds) {
           const float id = lab.ids[r];
           const int hit = id >= 0.f && id < static_cast<float>(ncol) ? static_cast<int>(id) : -1;
-          float loss = lab.off * (static_cast<float>(ncol) * lse - below);
+          float loss = lab.off * static_cast<float>(ncol) * lse - below;
           if (hit >= 0 && static_cast<float>(hit) == id) loss += lab.on * (lse - (row[hit] - m));
           out[r] = loss;
         } else {
