@@ -87,3 +87,34 @@ def test_pair_passes_on_nan_as_the_two_calls_do(shape, bad):
     L.batch_norm_then_relu_gradient(dy, gx, gamma, pair, dbn1, *both, None, None, 0.01)
     for got, want in [(y1, y), (bn1, bn), (r1, y), (dbn1, dbn)] + list(zip(one, two)) + list(zip(both, two)):
         np.testing.assert_array_equal(got.asnumpy(), want.asnumpy())
+
+
+# planes in words and not, a channel in registers and not
+@pytest.mark.parametrize("shape", [(16, 4, 14, 14), (8, 4, 112, 112), (16, 3, 71, 71)])
+def test_a_tape_that_is_asked_to_fuse_takes_saved_floats_and_one_that_is_not_gives_the_bits_of_two_calls(shape):
+    from tsplit_amd import gpu_links as L, graph, ndarray as nd
+    ctx = nd.gpu(0)
+    rng = np.random.RandomState(sum(shape))
+    c = shape[1]
+    x, dy = [nd.array(rng.normal(size=shape).astype(np.float32), ctx) for _ in range(2)]
+    gamma, beta = [nd.array(rng.normal(size=(1, c, 1, 1)).astype(np.float32), ctx) for _ in range(2)]
+    bn, y, dbn, dx = [nd.empty(shape, ctx) for _ in range(4)]
+    mean, istd, dg, db = [nd.empty((1, c, 1, 1), ctx) for _ in range(4)]
+    want = {}
+    L.batch_norm_relu(x, gamma, beta, y, mean, istd, 0.01)
+    L.batch_norm_relu_gradient(dy, x, gamma, beta, dx, dg, db, mean, istd, 0.01)
+    want[True] = [a.asnumpy() for a in (y, dx, dg, db)]
+    L.CuDNN_Batch_Normalization(x, gamma, beta, bn, None, None, 0.99, 0.01)
+    L.relu(bn, y)
+    L.relu_gradient(bn, dy, dbn)
+    L.CuDNN_Batch_Normalization_gradient(dbn, x, gamma, dx, dg, db, None, None, 0.01)
+    want[False] = [a.asnumpy() for a in (y, dx, dg, db)]
+    for fuse in (True, False):
+        t = graph.Tape(graph.GpuBackend(ctx))
+        t.fuse_bn_relu = fuse
+        leaves = [t.param(v, v.shape) for v in (x, gamma, beta)]
+        out = t.bn_then_relu(*leaves)
+        assert [n.out is out for n in t._nodes] == [True]
+        t._nodes[0].back(dy)
+        for a, b in zip([out.value] + [v.grad for v in leaves], want[fuse]):
+            np.testing.assert_array_equal(a.asnumpy(), b)

@@ -69,7 +69,7 @@ def conv_out(size, k, pad, stride):
 class GpuBackend(object):
     """Primitives on device arrays, one `gpu_links` call each (plus the output allocation)."""
 
-    fuses_pairs = True   # bn_relu is bn and relu, bit for bit
+    fuses_pairs = True   # bn_relu has an exact form
     L = L        # the links module; a subclass that only counts memory puts a stand-in here
 
     def __init__(self, ctx=None, stream=None):
@@ -169,10 +169,11 @@ class GpuBackend(object):
         self.L.CuDNN_Batch_Normalization_gradient(dy, x, gamma, dx, dg, db, None, None, eps, self.stream)
         return dx, dg, db
 
-    def bn_relu(self, x, gamma, beta, xs, eps):
-        """-> (relu(bn(x)), saved mean, saved inverse deviation): one call, the BatchNorm output is never written."""
-        # (statistics as doubles: the pair then has the bits of bn and relu)
-        y, mean, istd = self.empty(xs), self.empty((xs[1], 2)), self.empty((xs[1], 2))
+    def bn_relu(self, x, gamma, beta, xs, eps, exact=False):
+        """-> (relu(bn(x)), saved mean, saved inverse deviation): one call, the BatchNorm output is never written.  exact: the statistics
+        are saved as doubles, and the pair has the bits of bn and relu."""
+        saved = (xs[1], 2) if exact else (1, xs[1], 1, 1)
+        y, mean, istd = self.empty(xs), self.empty(saved), self.empty(saved)
         self.L.batch_norm_relu(x, gamma, beta, y, mean, istd, eps, stream=self.stream)
         return y, mean, istd
 
@@ -577,14 +578,15 @@ class Tape(object):
         return self._out(fwd(), x.shape, [x, gamma, beta], back, saved=[x, gamma], redo=fwd)
 
     @_op
-    def batch_norm_relu(self, x, gamma, beta, eps=0.01):
+    def batch_norm_relu(self, x, gamma, beta, eps=0.01, exact=False):
         """BatchNorm and the Relu behind it as one node (TSplit_BatchNormRelu / _gradient; the reference's graph
         has two nodes, gpu_ops/BatchNorm.py and gpu_ops/Relu.py): the BatchNorm output is never written, and
-        the gradient reads the BatchNorm's input, the parameters and the two saved statistics vectors."""
-        stats = [None, None]
+        the gradient reads the BatchNorm's input, the parameters and the two saved statistics vectors.
+        exact (device backends): with the bits of the two nodes."""
+        stats, form = [None, None], {"exact": True} if exact else {}
 
         def fwd():
-            r = self.b.bn_relu(x.value, gamma.value, beta.value, x.shape, eps)
+            r = self.b.bn_relu(x.value, gamma.value, beta.value, x.shape, eps, **form)
             if r is None:                      # a backend that only records shapes
                 return None
             y, stats[0], stats[1] = r
@@ -601,8 +603,10 @@ class Tape(object):
         """The pair as the reference's graph has it (two nodes), or as one node: when the tape was asked to fuse, and on the device
         on a tape that accounts for no value, where nothing can read the BatchNorm's output (the same values from two passes of
         five less going forward, three of eight less going back)."""
-        if self.fuse_bn_relu or (self._ahead and getattr(type(self.b), "fuses_pairs", False)):
+        if self.fuse_bn_relu:
             return self.batch_norm_relu(x, gamma, beta, eps)
+        if self._ahead and getattr(type(self.b), "fuses_pairs", False):
+            return self.batch_norm_relu(x, gamma, beta, eps, exact=True)
         return self.relu(self.batch_norm(x, gamma, beta, eps))
 
     @_op
