@@ -5,7 +5,7 @@
 // operand is simply one whose other index is contiguous); nothing is ever transposed in memory.
 // The tile (128x128, 64x128, 128x64 or 64x64) and the number of ranges K is cut into come from a
 // small model of the chip (tile_plan.h); the ranges' results are added in ascending order by a
-// second kernel.  The batched form runs every leading index as one more grid dimension of the same
+// second kernel.  Small products run on the kernel of gemm_waves.h, in one launch.  The batched form runs every leading index as one more grid dimension of the same
 // kernel.  Operands of 2 GiB and more, and results whose 64 rows reach that far, stay on the engine
 // of mfma_gemm.h, which takes 64-bit addresses, with its own tiles and ranges.
 #include <algorithm>
@@ -14,6 +14,7 @@
 #include "gemm_tile.h"
 #include "mfma_gemm.h"
 #include "gemm_split.h"
+#include "gemm_waves.h"
 #include "tile_plan.h"
 
 namespace tsplit {
@@ -26,13 +27,16 @@ inline int64_t stored_rows(bool k_rows, int mn, int K) { return k_rows ? K : mn;
 
 struct Plan {
   int tile, S, kchunk;
+  WavesPlan waves;   // with waves: one launch of gemm_waves.h instead, S is 1
 };
 
 Plan best_plan(int M, int N, int K, int batch, bool may_split) {
   const int64_t cols = N;
   const int steps = std::max(1, (K + gt::BK - 1) / gt::BK);
   const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, kProductCost);
-  Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK};
+  const WavesPlan waves = plan_waves(M, N, K, batch, t.us);
+  if (waves.waves) return {0, 1, K, waves};
+  Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK, waves};
   p.S = std::max(1, (K + p.kchunk - 1) / p.kchunk);
   if (p.S == 1) p.kchunk = K;
   return p;
@@ -97,6 +101,30 @@ void launch_epilogue(int tile, const float *A, int64_t lda, const float *B, int6
   }
 }
 
+constexpr gt::Epilogue kNothingMore{1.f, nullptr, nullptr, 0.f, 0, 0.f, nullptr, nullptr, nullptr};
+constexpr gt::BatchOf kOneProduct{1, 0, 0, 0, 0, 0, 0};
+
+// small products: the depth shared by the waves of a block (gemm_waves.h)
+template <int TM, int TN, bool TA, bool TB, bool SUMS>
+void launch_waves_tile(const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch, int M, int N,
+                       int K, const gt::Epilogue &ep, float *sums, int waves, hipStream_t s) {
+  const int tm = (M + 16 * TM - 1) / (16 * TM), tn = (N + 16 * TN - 1) / (16 * TN);
+  const bool wide = TN > 1 && N % 2 == 0 && ldc % 2 == 0 && zs.co % 2 == 0 && zs.ci % 2 == 0 && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu) && aligned16(ep.gate);
+  const size_t lds = static_cast<size_t>(waves) * (256 * TM * TN + (SUMS ? 16 * TN : 0)) * sizeof(float);
+  hipLaunchKernelGGL((gw::gemm_waves_kernel<TM, TN, TA, TB, SUMS>), dim3(grid_blocks(tm, tn, batch)), dim3(64 * waves), lds, s, DenseParams{A, lda, M, K},
+                     DenseParams{B, ldb, N, K}, out, ldc, zs, ep, sums, wide, M, N, K, TileGrid{tm, tn, tm * tn * batch});
+}
+template <bool TA, bool TB, bool SUMS = false>
+void launch_waves(const WavesPlan &p, const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch,
+                  int M, int N, int K, const gt::Epilogue &ep, float *sums, hipStream_t s) {
+  switch (p.tile) {
+    case 0: return launch_waves_tile<1, 1, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
+    case 1: return launch_waves_tile<1, 2, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
+    case 2: return launch_waves_tile<2, 1, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
+    default: return launch_waves_tile<2, 2, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
+  }
+}
+
 // the results of S ranges (or of one) summed, with what follows
 int launch_epilogue_fold(const float *part, float *out, int64_t mn, int N, int S, const gt::Epilogue &ep, hipStream_t s) {
   if (N % 4 == 0 && aligned16(part) && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu) && aligned16(ep.gate))
@@ -109,6 +137,10 @@ int launch_epilogue_fold(const float *part, float *out, int64_t mn, int N, int S
 template <bool TA, bool TB>
 int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws_elems) {
   const Plan plan = plan_product(M, N, K, 1, true);
+  if (plan.waves.waves) {
+    launch_waves<TA, TB>(plan.waves, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, kNothingMore, nullptr, s);
+    return 0;
+  }
   const int64_t mn = static_cast<int64_t>(M) * N;
   float *out = C;
   if (plan.S > 1) {
@@ -137,6 +169,10 @@ void launch_sums_tile(const float *A, int64_t lda, const float *B, int64_t ldb, 
 }
 int launch_sums(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, float *sums, int M, int N, int K, hipStream_t s) {
   const Plan plan = plan_product(M, N, K, 1, true);
+  if (plan.waves.waves) {
+    launch_waves<true, false, true>(plan.waves, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, kNothingMore, sums, s);
+    return 0;
+  }
   const int64_t mn = static_cast<int64_t>(M) * N, n = mn + N;
   float *out = C, *to = sums;
   if (plan.S > 1) {
@@ -261,8 +297,12 @@ int dispatch_epilogue(const float *A, int64_t lda, const float *B, int64_t ldb, 
   const int64_t mn = static_cast<int64_t>(M) * N;
   if (near<TA, TB>(lda, ldb, M, N, K) && rows_reach(N) && !(split_bf16_enabled() && K % 4 == 0 && K >= BK)) {
     const Plan plan = plan_product(M, N, K, 1, true);
+    if (plan.waves.waves) {
+      launch_waves<TA, TB>(plan.waves, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, ep, nullptr, s);
+      return 0;
+    }
     if (plan.S == 1) {
-      launch_epilogue<TA, TB>(plan.tile, A, lda, B, ldb, C, N, gt::BatchOf{1, 0, 0, 0, 0, 0, 0}, 1, M, N, K, ep, s);
+      launch_epilogue<TA, TB>(plan.tile, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, ep, s);
       return 0;
     }
     float *part = static_cast<float *>(scratch_get(s, 2, static_cast<size_t>(plan.S) * mn * 4));
@@ -290,7 +330,11 @@ int dispatch_batched(const float *A, int64_t lda, int64_t sa, const float *B, in
     if (N <= 64) return launch_far_batched<256, 64, 4, 1, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
     return launch_far_batched<128, 128, 2, 2, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
   }
-  Plan plan = plan_product(M, N, K, batch, false);
+  const Plan plan = plan_product(M, N, K, batch, false);
+  if (plan.waves.waves) {
+    launch_waves<TA, TB>(plan.waves, A, lda, B, ldb, C, N, gt::BatchOf{1, sa, 0, sb, 0, static_cast<int64_t>(M) * N, 0}, batch, M, N, K, kNothingMore, nullptr, s);
+    return 0;
+  }
   launch_planned<TA, TB>(A, lda, sa, B, ldb, sb, C, static_cast<int64_t>(M) * N, batch, M, N, K, plan, s);
   return 0;
 }
@@ -324,8 +368,11 @@ int dispatch_heads(const HeadArray &a, const HeadArray &b, const HeadArray &c, i
              "TSplit_HeadsMatrixMultiply: a matrix reaches beyond 32-bit byte offsets");
   const int batch = static_cast<int>(c.n) * heads;
   const Plan plan = plan_product(M, N, K, batch, false);
-  launch_epilogue<TA, TB>(plan.tile, a.p, a.ld, b.p, b.ld, c.p, c.ld, gt::BatchOf{heads, a.outer, a.inner, b.outer, b.inner, c.outer, c.inner}, batch,
-                          M, N, K, ep, s);
+  const gt::BatchOf zs{heads, a.outer, a.inner, b.outer, b.inner, c.outer, c.inner};
+  if (plan.waves.waves)
+    launch_waves<TA, TB>(plan.waves, a.p, a.ld, b.p, b.ld, c.p, c.ld, zs, batch, M, N, K, ep, nullptr, s);
+  else
+    launch_epilogue<TA, TB>(plan.tile, a.p, a.ld, b.p, b.ld, c.p, c.ld, zs, batch, M, N, K, ep, s);
   return 0;
 }
 

@@ -55,14 +55,14 @@ constexpr TileCost kFilterTapsCost = {{2, 3, 3, 4},
                                       {0.6, 0.5, 0, 0}, 2.0, 6.2};
 struct TilePlan {
   int tile, S;
+  double us = 0;   // what the model takes it to cost
 };
 
 // A launch of `parts` products of M rows each (the phases of a strided data gradient; 1 otherwise), every one `batch` times:
 // part i has cols[i] columns and a depth of steps[i] x 32.  max_split 1: the depth stays whole.
 inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int parts, int64_t batch, int max_split, double out_values,
                            const TileCost &cost) {
-  TilePlan best{0, 1};
-  double least = 1e300;
+  TilePlan best{0, 1, 1e300};
   int deepest = 1;
   for (int i = 0; i < parts; ++i) deepest = std::max(deepest, steps[i]);
   for (int t = 0; t < 4; ++t) {
@@ -83,10 +83,7 @@ inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int
       double us = whole * (mean * cost.step[t][resident - 1] + cost.round[t]);
       if (rest) us += mean * cost.step[t][rest - 1] + cost.round[t];
       if (S > 1) us += cost.fold + (2 * S + 1) * out_values * 4 / (cost.fold_tb * 1e6);
-      if (us < least) {
-        least = us;
-        best = {t, S};
-      }
+      if (us < best.us) best = {t, S, us};
     };
     const int most = tiles > 1024 ? 1 : std::min(max_split, deepest);
     for (int S = 1, by = 1; S <= most; S += by) {   // 1 to 8, then four to every doubling
@@ -96,6 +93,35 @@ inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int
     // as many ranges as give every CU the same number of blocks
     for (int n = 1; n <= 10; ++n)
       if (const int64_t S = tiles > 0 ? 256 * n / tiles : 0; S > 1 && S <= most) consider(static_cast<int>(S));
+  }
+  return best;
+}
+
+// Small products go to the kernel whose blocks share the depth of one small tile among their waves (gemm_waves.h), where that takes less.
+// A launch there costs what any launch does, and for every block of the busiest CU a part of its own and one for each value of the depth.
+// From 60 shapes, rows 1 to 2048, columns 10 to 5003, depth 16 to 5003, in the four forms on four tiles with 2 to 16 waves: 9 % rms off, the
+// tile kernel's model (launches included) 12 %.  Over those shapes 1.25 times faster than the tile kernel alone, with the best of both by
+// hindsight 1.30: 128 x 256 over 784 7.3 -> 5.1-5.8 us, over 256 6.6 -> 4.3, 784 x 256 over 128 6.0 -> 4.6, 385 x 256 over 1024 9.9 -> 7.2, 32 x
+// 4096 over 1024 11.6 -> 7.3, 1 x 1908 over 308 6.9 -> 4.6; where the tile kernel stays: 250 x 5003 over 256 12.0 (14.5 here), 100 x 4096 over
+// 4096 39 (41-60).
+constexpr TileKind kWaveTiles[] = {{16, 16}, {16, 32}, {32, 16}, {32, 32}};
+struct WavesPlan {
+  int tile, waves;   // waves 0: the tile kernel
+};
+inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, double tile_kernel_us) {
+  constexpr double kLaunch = 3.6, kBlock[] = {0.18, 0.40, 0.47, 0.76}, kDepth[] = {0.0022, 0.0031, 0.0031, 0.0045};
+  WavesPlan best{0, 0};
+  double least = 2.3 + 1.15 * tile_kernel_us;
+  for (int t = 0; t < 4; ++t) {
+    const int64_t blocks = ((M + kWaveTiles[t].bm - 1) / kWaveTiles[t].bm) * ((N + kWaveTiles[t].bn - 1) / kWaveTiles[t].bn) * batch;
+    if (blocks > 1024) continue;
+    const int64_t n = (blocks + 255) / 256;
+    const double us = kLaunch + n * (kBlock[t] + kDepth[t] * K);
+    if (us < least && (n == 1 || us < 12)) {   // (beyond that the tile kernel fills the chip as well: 100 x 4096 over 4096)
+      least = us;
+      // sixteen waves gain nothing on a CU of their own, and eight lose where blocks share one; 32 values of the depth a wave
+      best = {t, static_cast<int>(std::max<int64_t>(2, std::min<int64_t>(n == 1 ? 8 : 4, (K + 31) / 32)))};
+    }
   }
   return best;
 }
