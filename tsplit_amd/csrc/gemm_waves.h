@@ -2,7 +2,7 @@
 //
 // A product of a few hundred rows and columns has few 64 x 64 tiles, so on the kernel of gemm_tile.h its depth was cut into ranges and a
 // second launch added them; either launch takes what any launch takes, and a range of one or two steps is a chain of memory latencies
-// behind one barrier each.  Here a block owns 16 TM x 16 TN of the result, up to sixteen waves deal the depth among them 32 values at a time,
+// behind one barrier each.  Here a block owns 16 TM x 16 TN of the result, its two to four waves deal the depth among them 32 values at a time,
 // operands go from memory to the registers the matrix instruction reads (no LDS, no barrier on the way), and the waves' sums are added
 // through LDS in ascending order.  What bounds it is latency: one for the operands, one for LDS, and the launch.
 #pragma once
@@ -85,7 +85,7 @@ struct Loader {
 
 // SUMS: the blocks of the first row of tiles also leave the sums of B's columns.
 template <int TM, int TN, bool TA, bool TB, bool SUMS>
-__global__ __launch_bounds__(1024) void gemm_waves_kernel(mg::DenseParams ap, mg::DenseParams bp, float *out, int64_t ldc, gt::BatchOf zs,
+__global__ __launch_bounds__(256) void gemm_waves_kernel(mg::DenseParams ap, mg::DenseParams bp, float *out, int64_t ldc, gt::BatchOf zs,
                                                           gt::Epilogue ep, float *sums, bool wide, int M, int N, int K, mg::TileGrid tg) {
   extern __shared__ __attribute__((aligned(16))) float lds[];   // [wave][tm][e][lane][tn]; with SUMS [wave][16 TN] behind it
   int z, tile_m, tile_n;

@@ -117,10 +117,11 @@ inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, doub
     if (blocks > 1024) continue;
     const int64_t n = (blocks + 255) / 256;
     const double us = kLaunch + n * (kBlock[t] + kDepth[t] * K);
-    if (us < least && (n == 1 || us < 12)) {   // (beyond that the tile kernel fills the chip as well: 100 x 4096 over 4096)
+    if (us < least && (n == 1 || us < 8)) {   // (of several blocks a CU the tile kernel fills the chip as well: 100 x 4096 over 4096)
       least = us;
-      // sixteen waves gain nothing on a CU of their own, and eight lose where blocks share one; 32 values of the depth a wave
-      best = {t, static_cast<int>(std::max<int64_t>(2, std::min<int64_t>(n == 1 ? 8 : 4, (K + 31) / 32)))};
+      // 32 values of the depth a wave; eight or sixteen waves gain nothing on a CU of their own (over the shapes 0.2 %) and lose where
+      // blocks share one
+      best = {t, static_cast<int>(std::max<int64_t>(2, std::min<int64_t>(4, (K + 31) / 32)))};
     }
   }
   return best;
