@@ -1,0 +1,51 @@
+"""The extension module that Python's calls go through (csrc/python/calls.cpp): what arrays own, and what operator calls refuse."""
+import ctypes
+import gc
+
+import numpy as np
+import pytest
+
+from tsplit_amd import _calls, gpu_links as L, ndarray as nd
+from tsplit_amd._base import _LIB
+
+
+def test_arrays_own_their_memory_and_views_keep_their_parent():
+    a = nd.array(np.arange(12, dtype=np.float32).reshape(3, 4), nd.cpu(0))
+    assert a.shape == (3, 4) and a.handle is a.handle and a.data_ptr == a.handle.contents.data and a.ctx.device_type == 1
+    v = nd.view(a, (12,))
+    assert v._owner is a
+    a.split_tensor(3)                            # the array lists views that refer to it: a cycle
+    assert [p.asnumpy()[0, 0] for p in a.sTensor] == [0, 4, 8] and a.split_number == 3 and a.splitted
+    del a
+    gc.collect()
+    np.testing.assert_array_equal(v.asnumpy(), np.arange(12))
+    for shape in ((), (0, 3), [2, np.int64(5)], (1,) * 20):
+        assert nd.empty(shape).shape == tuple(int(s) for s in shape)
+
+
+def test_an_array_lives_through_assigned_attributes_and_a_raw_handle():
+    h = nd.DLArrayHandle()
+    shape = (ctypes.c_int64 * 2)(2, 3)
+    assert _LIB.DLArrayAlloc(shape, ctypes.c_int64(2), nd.cpu(0), ctypes.byref(h), ctypes.c_int(1)) == 0
+    a = nd.NDArray(h)
+    assert a.handle is h and a.shape == (2, 3) and (a.swap, a.in_gpu, a._keeper) == (False, True, None)
+    a.to_swap()
+    a.in_gpu = False
+    assert a.swap is True and a.in_gpu is False and a._events == {}
+
+
+def test_calls_refuse_what_they_cannot_take():
+    a = nd.empty((2, 3))
+    for bad in (None, 3, "x", np.zeros((2, 3), np.float32)):
+        with pytest.raises(AssertionError):
+            L.relu(a, bad)
+    with pytest.raises(RuntimeError):
+        L.matrix_multiply(a, False, a, False, a)            # shapes do not conform: refused before any launch
+    with pytest.raises(TypeError):
+        L.CuDNN_max_pooling2d(a, 2.5, 2, a)
+    with pytest.raises(TypeError):
+        _calls.DLGpuRelu(a, a)
+    with pytest.raises(ValueError):
+        nd.empty("ab")
+    with pytest.raises(TypeError):
+        nd.empty((2, 3), 5)

@@ -3,7 +3,8 @@
     python -m tsplit_amd.build            # incremental
     python -m tsplit_amd.build --force    # recompile everything
 
-Also builds the host-only pool test library used by the CPU tests.
+Also builds the extension module that Python's calls go through (_calls.so, plain g++) and the host-only pool test library
+used by the CPU tests.
 """
 import argparse
 import concurrent.futures
@@ -11,12 +12,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "_obj")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libc_runtime_api.so")
+CALLS = os.path.join(HERE, "_calls.so")
 POOL_TEST_LIB = os.path.join(LIBDIR, "libtsplit_pool_host.so")
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
@@ -65,6 +68,12 @@ def build(force=False, jobs=8, verbose=True):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    calls_src = os.path.join(CSRC, "python", "calls.cpp")
+    if force or not os.path.exists(CALLS) or os.path.getmtime(CALLS) < max(os.path.getmtime(calls_src), hmtime):
+        r = subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall",
+                            "-I" + sysconfig.get_paths()["include"], calls_src, "-o", CALLS], capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"g++ failed on python/calls.cpp:\n{r.stderr}")
     # host-only pool library for the CPU tests (plain g++, no HIP)
     pool_src = os.path.join(CSRC, "pool_capi.cpp")
     if os.path.exists(pool_src):

@@ -3,10 +3,12 @@
 Mirror of the reference's python/athena/gpu_links/*.py: same function names, argument
 order and defaults (cited per function), so a graph op written against the reference's
 `gpu_links` runs unchanged on this library.  Return values of the C calls are checked
-here (the reference's wrappers ignore them).
+(the reference's wrappers ignore them); calls of arrays, numbers, a stream and a profiler
+go through the extension module _calls, which does that itself.
 """
 import ctypes
 
+from . import _calls
 from . import ndarray as _nd
 from ._base import _LIB, c_array, check_call
 
@@ -50,72 +52,65 @@ def _p(profiler):
 # ---- graph-closure ops (gpu_links/ArraySetLink.py:8, AddElewiseLink.py, AddConstLink.py,
 #      MultiplyElewiseLink.py, MultiplyConstLink.py, ReshapeLink.py:8) ----
 def array_set(arr, value, stream=None, profiler=None):
-    check_call(_LIB.DLGpuArraySet(_h(arr), ctypes.c_float(value), _s(stream), _p(profiler)))
+    _calls.DLGpuArraySet(arr, value, stream, profiler)
 
 
 def matrix_elementwise_add(matA, matB, matC, stream=None, profiler=None):
-    check_call(_LIB.DLGpuMatrixElementwiseAdd(_h(matA), _h(matB), _h(matC), _s(stream), _p(profiler)))
+    _calls.DLGpuMatrixElementwiseAdd(matA, matB, matC, stream, profiler)
 
 
 def matrix_elementwise_add_by_const(in_mat, val, out_mat, stream=None, profiler=None):
-    check_call(_LIB.DLGpuMatrixElementwiseAddByConst(_h(in_mat), ctypes.c_float(val), _h(out_mat),
-                                                     _s(stream), _p(profiler)))
+    _calls.DLGpuMatrixElementwiseAddByConst(in_mat, val, out_mat, stream, profiler)
 
 
 def matrix_elementwise_multiply(matA, matB, matC, stream=None, profiler=None):
-    check_call(_LIB.DLGpuMatrixElementwiseMultiply(_h(matA), _h(matB), _h(matC), _s(stream), _p(profiler)))
+    _calls.DLGpuMatrixElementwiseMultiply(matA, matB, matC, stream, profiler)
 
 
 def matrix_elementwise_multiply_by_const(in_mat, val, out_mat, stream=None, profiler=None):
-    check_call(_LIB.DLGpuMatrixMultiplyByConst(_h(in_mat), ctypes.c_float(val), _h(out_mat),
-                                               _s(stream), _p(profiler)))
+    _calls.DLGpuMatrixMultiplyByConst(in_mat, val, out_mat, stream, profiler)
 
 
 def array_reshape(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuReshape(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuReshape(in_arr, out_arr, stream, profiler)
 
 
 # ---- Relu (gpu_links/ReluLink.py:8,14) ----
 def relu(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuRelu(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuRelu(in_arr, out_arr, stream, profiler)
 
 
 def relu_gradient(in_arr, in_grad_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuReluGradient(_h(in_arr), _h(in_grad_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuReluGradient(in_arr, in_grad_arr, out_arr, stream, profiler)
 
 
 # ---- MatMul (gpu_links/MatrixMultLink.py:8) ----
 def matrix_multiply(matA, transA, matB, transB, matC, stream=None, profiler=None):
-    check_call(_LIB.DLGpuMatrixMultiply(_h(matA), ctypes.c_bool(bool(transA)), _h(matB),
-                                        ctypes.c_bool(bool(transB)), _h(matC), _s(stream), _p(profiler)))
+    _calls.DLGpuMatrixMultiply(matA, transA, matB, transB, matC, stream, profiler)
 
 
 def matrix_multiply_add(matA, transA, matB, transB, matC, bias=None, addend=None, relu=None, stream=None, gate=None):
     """matC = op(matA) op(matB) + bias + addend, relu = max(matC, 0), each where given: the bits of matrix_multiply,
     broadcast_to and matrix_elementwise_add, and relu (no counterpart in the reference's gpu_links).  With `gate`, a Relu's input,
     that Relu's gradient of the result: in relu where it is given, else in matC."""
-    check_call(_LIB.TSplit_MatrixMultiplyAdd(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(bias) if bias else None,
-                                             _h(addend) if addend else None, _h(gate) if gate else None, _h(matC),
-                                             _h(relu) if relu else None, _s(stream)))
+    _calls.TSplit_MatrixMultiplyAdd(matA, bool(transA), matB, bool(transB), bias, addend, gate, matC, relu, stream)
 
 
 def matrix_multiply_sums(matA, matB, matC, sums, stream=None):
     """matC = matA' matB (the bits of matrix_multiply), sums = the sums of matB's columns (no counterpart in the reference's gpu_links)."""
-    check_call(_LIB.TSplit_MatrixMultiplySums(_h(matA), _h(matB), _h(matC), _h(sums), _s(stream)))
+    _calls.TSplit_MatrixMultiplySums(matA, matB, matC, sums, stream)
 
 
 def heads_matrix_multiply(matA, transA, matB, transB, matC, heads, alpha=1.0, mask=None, mask_value=0.0, causal=False, fill=0.0,
                           addend=None, stream=None):
     """For every sample and head matC = alpha * op(matA) op(matB), + mask_value in columns where mask is 0, `fill` right of the
     diagonal with `causal`, + addend.  Arrays are [n, heads, rows, columns] or [n, rows, heads * columns]."""
-    check_call(_LIB.TSplit_HeadsMatrixMultiply(_h(matA), int(bool(transA)), _h(matB), int(bool(transB)), _h(matC), int(heads),
-                                               ctypes.c_float(alpha), _h(mask) if mask else None, ctypes.c_float(mask_value),
-                                               int(bool(causal)), ctypes.c_float(fill), _h(addend) if addend else None, _s(stream)))
+    _calls.TSplit_HeadsMatrixMultiply(matA, bool(transA), matB, bool(transB), matC, heads, alpha, mask, mask_value, bool(causal), fill, addend, stream)
 
 
 def heads_scale(in_arr, scale, causal, out_arr, stream=None):
     """out_arr = scale * in_arr, with `causal` 0 right of the diagonal of the last two axes; out_arr may be in_arr."""
-    check_call(_LIB.TSplit_HeadsScale(_h(in_arr), ctypes.c_float(scale), int(bool(causal)), _h(out_arr), _s(stream)))
+    _calls.TSplit_HeadsScale(in_arr, scale, bool(causal), out_arr, stream)
 
 
 def join(parts, whole, axis, stream=None):
@@ -153,11 +148,11 @@ def lstm_gradient(dlast, x, params, initial, steps, rows, packed, gates, cells, 
 
 # ---- Softmax / CE (gpu_links/SoftmaxLink.py, SoftmaxCrossEntropyLink.py:8,17) ----
 def softmax(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuSoftmax(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuSoftmax(in_arr, out_arr, stream, profiler)
 
 
 def softmax_cross_entropy(in_arr_a, in_arr_b, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuSoftmaxCrossEntropy(_h(in_arr_a), _h(in_arr_b), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuSoftmaxCrossEntropy(in_arr_a, in_arr_b, out_arr, stream, profiler)
 
 
 def softmax_cross_entropy_no_alloc(in_arr_a, in_arr_b, out_arr, stream=None):
@@ -167,50 +162,43 @@ def softmax_cross_entropy_no_alloc(in_arr_a, in_arr_b, out_arr, stream=None):
 
 
 def softmax_cross_entropy_gradient(in_arr_a, in_arr_b, in_arr_c, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuSoftmaxCrossEntropy_Gradient(_h(in_arr_a), _h(in_arr_b), _h(in_arr_c), _h(out_arr),
-                                                      _s(stream), _p(profiler)))
+    _calls.DLGpuSoftmaxCrossEntropy_Gradient(in_arr_a, in_arr_b, in_arr_c, out_arr, stream, profiler)
 
 
 def softmax_cross_entropy_ids(logits, ids, on, off, out_arr, stream=None):
     """softmax_cross_entropy with labels on * one_hot(ids) + off that are never written."""
-    check_call(_LIB.TSplit_SoftmaxCrossEntropyIds(_h(logits), _h(ids), ctypes.c_float(on), ctypes.c_float(off), _h(out_arr), _s(stream)))
+    _calls.TSplit_SoftmaxCrossEntropyIds(logits, ids, on, off, out_arr, stream)
 
 
 def softmax_cross_entropy_ids_gradient(logits, ids, on, off, adjoint, out_arr, stream=None):
-    check_call(_LIB.TSplit_SoftmaxCrossEntropyIds_Gradient(_h(logits), _h(ids), ctypes.c_float(on), ctypes.c_float(off), _h(adjoint),
-                                                           _h(out_arr), _s(stream)))
+    _calls.TSplit_SoftmaxCrossEntropyIds_Gradient(logits, ids, on, off, adjoint, out_arr, stream)
 
 
 def embedding_add(table, ids, scale, positions, out_arr, stream=None):
     """scale * table[id] + (id != 0 ? positions : 0)."""
-    check_call(_LIB.TSplit_EmbeddingAdd(_h(table), _h(ids), ctypes.c_float(scale), _h(positions), _h(out_arr), _s(stream)))
+    _calls.TSplit_EmbeddingAdd(table, ids, scale, positions, out_arr, stream)
 
 
 def embedding_add_gradient(out_grad, ids, scale, table_grad, add_to=False, stream=None):
-    check_call(_LIB.TSplit_EmbeddingAdd_Gradient(_h(out_grad), _h(ids), ctypes.c_float(scale), int(bool(add_to)), _h(table_grad), _s(stream)))
+    _calls.TSplit_EmbeddingAdd_Gradient(out_grad, ids, scale, bool(add_to), table_grad, stream)
 
 
 # ---- Conv2d (gpu_links/CudnnConv2d.py:8,21,33; gpu_links/Conv2dLink.py:8,24,35) ----
 def CuDNN_conv2d(in_arr_x, in_arr_f, out_arr, padding=0, padding2=None, stride=1, stream=None, profiler=None):
     pad2 = padding if padding2 is None else padding2
-    check_call(_LIB.CuDNN_DLGpuConv2d(_h(in_arr_x), _h(in_arr_f), _h(out_arr), int(padding), int(pad2),
-                                      int(stride), _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuConv2d(in_arr_x, in_arr_f, out_arr, padding, pad2, stride, stream, profiler)
 
 
 def CuDNN_conv2d_gradient_of_filter(in_arr_x, in_gradient_y, out_gradient_f, padding=0, padding2=None,
                                     stride=1, stream=None, profiler=None):
     pad2 = padding if padding2 is None else padding2
-    check_call(_LIB.CuDNN_DLGpuConv2d_Gradient_of_Filter(_h(in_arr_x), _h(in_gradient_y), _h(out_gradient_f),
-                                                         int(padding), int(pad2), int(stride),
-                                                         _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuConv2d_Gradient_of_Filter(in_arr_x, in_gradient_y, out_gradient_f, padding, pad2, stride, stream, profiler)
 
 
 def CuDNN_conv2d_gradient_of_data(in_arr_f, in_gradient_y, out_gradient_x, padding=0, padding2=None,
                                   stride=1, stream=None, profiler=None):
     pad2 = padding if padding2 is None else padding2
-    check_call(_LIB.CuDNN_DLGpuConv2d_Gradient_of_Data(_h(in_arr_f), _h(in_gradient_y), _h(out_gradient_x),
-                                                       int(padding), int(pad2), int(stride),
-                                                       _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuConv2d_Gradient_of_Data(in_arr_f, in_gradient_y, out_gradient_x, padding, pad2, stride, stream, profiler)
 
 
 def conv2d(in_arr_x, in_arr_f, out_arr, workspace_arr, padding=0, stride=1, stream=None, profiler=None):
@@ -235,56 +223,42 @@ def conv2d_gradient_of_data(in_arr_f, in_gradient_y, out_gradient_x, workspace_i
 # ---- BatchNorm (gpu_links/CudnnBnLink.py:8,17) ----
 def CuDNN_Batch_Normalization(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var,
                               momentum=0.99, eps=0.001, stream=None, profiler=None):
-    check_call(_LIB.CuDNN_DLGpuBatch_Normalization(
-        _h(in_arr), _h(bn_scale_arr), _h(bn_bias_arr), _h(out_arr), ctypes.c_float(momentum),
-        ctypes.c_float(eps), save_mean.handle if save_mean else None,
-        save_var.handle if save_var else None, _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuBatch_Normalization(in_arr, bn_scale_arr, bn_bias_arr, out_arr, momentum, eps, save_mean, save_var, stream, profiler)
 
 
 def CuDNN_Batch_Normalization_gradient(in_gradient_y, in_arr_x, in_bn_scale, out_gradient_x,
                                        out_gradient_bn_scale, out_gradient_bn_bias, saved_mean, saved_var,
                                        eps=0.001, stream=None, profiler=None):
-    check_call(_LIB.CuDNN_DLGpuBatch_Normalization_gradient(
-        _h(in_gradient_y), _h(in_arr_x), _h(in_bn_scale), _h(out_gradient_x), _h(out_gradient_bn_scale),
-        _h(out_gradient_bn_bias), ctypes.c_float(eps), saved_mean.handle if saved_mean else None,
-        saved_var.handle if saved_var else None, _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuBatch_Normalization_gradient(in_gradient_y, in_arr_x, in_bn_scale, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
 
 
 # ---- MaxPool (gpu_links/MaxPoolLink.py:8,15; gpu_links/CudnnMaxPoolLink.py:8,15) ----
 def max_pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding=0, stride=1, stream=None, profiler=None):
-    check_call(_LIB.DLGpuMax_Pooling2d(_h(in_arr), int(kernel_H), int(kernel_W), _h(pooled_layer),
-                                       int(padding), int(stride), _s(stream), _p(profiler)))
+    _calls.DLGpuMax_Pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding, stride, stream, profiler)
 
 
 def max_pooling2d_gradient(in_arr, in_grad_arr, kernel_H, kernel_W, out_grad_arr, padding=0, stride=1,
                            stream=None, profiler=None):
-    check_call(_LIB.DLGpuMax_Pooling2d_gradient(_h(in_arr), _h(in_grad_arr), int(kernel_H), int(kernel_W),
-                                                _h(out_grad_arr), int(padding), int(stride),
-                                                _s(stream), _p(profiler)))
+    _calls.DLGpuMax_Pooling2d_gradient(in_arr, in_grad_arr, kernel_H, kernel_W, out_grad_arr, padding, stride, stream, profiler)
 
 
 def CuDNN_max_pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding=0, stride=1, stream=None,
                         profiler=None):
-    check_call(_LIB.CuDNN_DLGpuMax_Pooling2d(_h(in_arr), ctypes.c_size_t(kernel_H), ctypes.c_size_t(kernel_W),
-                                             _h(pooled_layer), ctypes.c_size_t(padding),
-                                             ctypes.c_size_t(stride), _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuMax_Pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding, stride, stream, profiler)
 
 
 def CuDNN_max_pooling2d_gradient(in_arr_y, in_gradient_y, in_arr_x, kernel_H, kernel_W, out_gradient_x,
                                  padding=0, stride=1, stream=None, profiler=None):
-    check_call(_LIB.CuDNN_DLGpuMax_Pooling2d_gradient(
-        _h(in_arr_y), _h(in_gradient_y), _h(in_arr_x), ctypes.c_size_t(kernel_H), ctypes.c_size_t(kernel_W),
-        _h(out_gradient_x), ctypes.c_size_t(padding), ctypes.c_size_t(stride), _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuMax_Pooling2d_gradient(in_arr_y, in_gradient_y, in_arr_x, kernel_H, kernel_W, out_gradient_x, padding, stride, stream, profiler)
 
 
 # ---- Concat / Slice (gpu_links/ConcatLink.py:8,14; gpu_links/SliceLink.py:8,16) ----
 def concat(in_arr1, in_arr2, out_arr, axis=0, stream=None, profiler=None):
-    check_call(_LIB.DLGpuConcat(_h(in_arr1), _h(in_arr2), _h(out_arr), int(axis), _s(stream), _p(profiler)))
+    _calls.DLGpuConcat(in_arr1, in_arr2, out_arr, axis, stream, profiler)
 
 
 def concat_gradient(out_grad_arr, in_arr, axis=0, idx=0, stream=None, profiler=None):
-    check_call(_LIB.DLGpuConcat_gradient(_h(out_grad_arr), _h(in_arr), int(axis), int(idx),
-                                         _s(stream), _p(profiler)))
+    _calls.DLGpuConcat_gradient(out_grad_arr, in_arr, axis, idx, stream, profiler)
 
 
 def matrix_slice(in_arr, out_arr, begin_pos, stream=None, profiler=None):
@@ -299,12 +273,11 @@ def matrix_slice_gradient(in_arr, out_arr, begin_pos, stream=None, profiler=None
 
 # ---- Optimizers (gpu_links/OptimizerLink.py:7-30) ----
 def sgd_update(param, grad, lr, stream=None):
-    check_call(_LIB.SGDOptimizerUpdate(_h(param), _h(grad), ctypes.c_float(lr), _s(stream)))
+    _calls.SGDOptimizerUpdate(param, grad, lr, stream)
 
 
 def momentum_update(param, grad, velocity, lr, momentum, nesterov, stream=None):
-    check_call(_LIB.MomentumOptimizerUpdate(_h(param), _h(grad), _h(velocity), ctypes.c_float(lr),
-                                            ctypes.c_float(momentum), ctypes.c_bool(bool(nesterov)), _s(stream)))
+    _calls.MomentumOptimizerUpdate(param, grad, velocity, lr, momentum, nesterov, stream)
 
 
 def optimizer_update_multi(params, grads, velocities, lr, momentum=0.0, nesterov=False, stream=None):
@@ -328,40 +301,32 @@ def adam_update(param, grad, expavg, expavgsq, lr, beta1, beta2, beta1t, beta2t,
 
 # ---- AvgPool (gpu_links/AvgPoolLink.py:8,15; gpu_links/CudnnAvgPoolLink.py:8,15) ----
 def average_pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding=0, stride=1, stream=None, profiler=None):
-    check_call(_LIB.DLGpuAvgerage_Pooling2d(_h(in_arr), ctypes.c_size_t(kernel_H), ctypes.c_size_t(kernel_W),
-                                            _h(pooled_layer), ctypes.c_size_t(padding), ctypes.c_size_t(stride),
-                                            _s(stream), _p(profiler)))
+    _calls.DLGpuAvgerage_Pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding, stride, stream, profiler)
 
 
 def average_pooling2d_gradient(in_gradient_y, kernel_H, kernel_W, out_gradient_x, padding=0, stride=1,
                                stream=None, profiler=None):
-    check_call(_LIB.DLGpuAvgerage_Pooling2d_gradient(
-        _h(in_gradient_y), ctypes.c_size_t(kernel_H), ctypes.c_size_t(kernel_W), _h(out_gradient_x),
-        ctypes.c_size_t(padding), ctypes.c_size_t(stride), _s(stream), _p(profiler)))
+    _calls.DLGpuAvgerage_Pooling2d_gradient(in_gradient_y, kernel_H, kernel_W, out_gradient_x, padding, stride, stream, profiler)
 
 
 def CuDNN_average_pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding=0, stride=1, stream=None,
                             profiler=None):
-    check_call(_LIB.CuDNN_DLGpuAvgerage_Pooling2d(
-        _h(in_arr), ctypes.c_size_t(kernel_H), ctypes.c_size_t(kernel_W), _h(pooled_layer),
-        ctypes.c_size_t(padding), ctypes.c_size_t(stride), _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuAvgerage_Pooling2d(in_arr, kernel_H, kernel_W, pooled_layer, padding, stride, stream, profiler)
 
 
 def CuDNN_average_pooling2d_gradient(in_arr_y, in_gradient_y, in_arr_x, kernel_H, kernel_W, out_gradient_x,
                                      padding=0, stride=1, stream=None, profiler=None):
-    check_call(_LIB.CuDNN_DLGpuAvgerage_Pooling2d_gradient(
-        _h(in_arr_y), _h(in_gradient_y), _h(in_arr_x), ctypes.c_size_t(kernel_H), ctypes.c_size_t(kernel_W),
-        _h(out_gradient_x), ctypes.c_size_t(padding), ctypes.c_size_t(stride), _s(stream), _p(profiler)))
+    _calls.CuDNN_DLGpuAvgerage_Pooling2d_gradient(in_arr_y, in_gradient_y, in_arr_x, kernel_H, kernel_W, out_gradient_x, padding, stride, stream, profiler)
 
 
 # ---- Broadcast / reduce (gpu_links/BroadcastLink.py:8, ReduceSumAxisZeroLink.py:7,15,
 #      Conv2dBroadcastLink.py:8, Conv2dReduceSumLink.py:8, BroadcastShapeLink.py:8, ReduceSumLink.py:7) ----
 def broadcast_to(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuBroadcastTo(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuBroadcastTo(in_arr, out_arr, stream, profiler)
 
 
 def reduce_sum_axis_zero(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuReduceSumAxisZero(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuReduceSumAxisZero(in_arr, out_arr, stream, profiler)
 
 
 def _reduce_sum_axis_zero(in_arr, out_arr, workspace_arr, stream=None, profiler=None):
@@ -369,11 +334,11 @@ def _reduce_sum_axis_zero(in_arr, out_arr, workspace_arr, stream=None, profiler=
 
 
 def conv2d_broadcast_to(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuConv2d_broadcast_to(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuConv2d_broadcast_to(in_arr, out_arr, stream, profiler)
 
 
 def conv2d_reduce_sum(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuConv2d_reduce_sum(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuConv2d_reduce_sum(in_arr, out_arr, stream, profiler)
 
 
 def broadcast_shape(in_arr, out_arr, add_axes=None, stream=None):
@@ -414,25 +379,24 @@ def matrix_transpose(in_mat, out_mat, perm, stream=None, profiler=None):
 
 
 def batch_matrix_multiply(matA, transA, matB, transB, matC, stream=None):
-    check_call(_LIB.DLGpuBatchMatrixMultiply(_h(matA), ctypes.c_bool(bool(transA)), _h(matB),
-                                             ctypes.c_bool(bool(transB)), _h(matC), _s(stream)))
+    _calls.DLGpuBatchMatrixMultiply(matA, transA, matB, transB, matC, stream)
 
 
 # ---- OneHot / Where / Embedding (gpu_links/OneHotLink.py:8, WhereLink.py:8, EmbeddingLookUpLink.py:8,15) ----
 def one_hot(in_arr, out_arr, stream=None):
-    check_call(_LIB.DLGpuOneHot(_h(in_arr), _h(out_arr), _s(stream)))
+    _calls.DLGpuOneHot(in_arr, out_arr, stream)
 
 
 def where(cond, arr1, arr2, out_arr, stream=None):
-    check_call(_LIB.DLGpuWhere(_h(cond), _h(arr1), _h(arr2), _h(out_arr), _s(stream)))
+    _calls.DLGpuWhere(cond, arr1, arr2, out_arr, stream)
 
 
 def embedding_lookup(in_mat, ids, out_mat, stream=None, profiler=None):
-    check_call(_LIB.DLGpuEmbeddingLookUp(_h(in_mat), _h(ids), _h(out_mat), _s(stream), _p(profiler)))
+    _calls.DLGpuEmbeddingLookUp(in_mat, ids, out_mat, stream, profiler)
 
 
 def embedding_lookup_gradient(grad_out, ids, grad_in, stream=None, profiler=None):
-    check_call(_LIB.DLGpuEmbeddingLookUp_Gradient(_h(grad_out), _h(ids), _h(grad_in), _s(stream), _p(profiler)))
+    _calls.DLGpuEmbeddingLookUp_Gradient(grad_out, ids, grad_in, stream, profiler)
 
 
 # ---- Dropout (gpu_links/CudnnDropoutLink.py:8,15).  reserve_size is a ctypes.c_int and
@@ -489,11 +453,11 @@ def matrix_rsqrt(in_arr, out_arr, stream=None, profiler=None):
 
 
 def tanh(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuTanh(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuTanh(in_arr, out_arr, stream, profiler)
 
 
 def sigmoid(in_arr, out_arr, stream=None, profiler=None):
-    check_call(_LIB.DLGpuSigmoid(_h(in_arr), _h(out_arr), _s(stream), _p(profiler)))
+    _calls.DLGpuSigmoid(in_arr, out_arr, stream, profiler)
 
 
 # ---- Which routine a convolution takes (no counterpart in the reference's gpu_links) ----
@@ -545,26 +509,20 @@ def winograd_gemm_times(filter_gradient=False, kind=None):
 # ---- Fused BatchNorm + Relu (no counterpart in the reference's gpu_links) ----
 def batch_norm_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var, eps=0.01, stream=None,
                     profiler=None):
-    check_call(_LIB.TSplit_BatchNormRelu(_h(in_arr), _h(bn_scale_arr), _h(bn_bias_arr), _h(out_arr),
-                                         ctypes.c_float(eps), _h(save_mean), _h(save_var), _s(stream), _p(profiler)))
+    _calls.TSplit_BatchNormRelu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, eps, save_mean, save_var, stream, profiler)
 
 
 def batch_norm_then_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, relu_arr, pair, save_mean=None, save_var=None, eps=0.01, stream=None,
                          profiler=None):
     """out_arr = BatchNorm, relu_arr = Relu of it: CuDNN_Batch_Normalization and relu in one call, with their bits; `pair` (2 C
     values) is what the gradient reads again."""
-    check_call(_LIB.TSplit_BatchNormThenRelu(_h(in_arr), _h(bn_scale_arr), _h(bn_bias_arr), _h(out_arr), _h(relu_arr), _h(pair),
-                                             ctypes.c_float(eps), _h(save_mean) if save_mean else None, _h(save_var) if save_var else None,
-                                             _s(stream), _p(profiler)))
+    _calls.TSplit_BatchNormThenRelu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, relu_arr, pair, eps, save_mean, save_var, stream, profiler)
 
 
 def batch_norm_then_relu_gradient(in_gradient, in_arr, in_bn_scale, pair, out_gradient_y, out_gradient_x, out_gradient_bn_scale,
                                   out_gradient_bn_bias, saved_mean=None, saved_var=None, eps=0.01, stream=None, profiler=None):
     """relu_gradient and CuDNN_Batch_Normalization_gradient in one call, with their bits; out_gradient_y: between the two."""
-    check_call(_LIB.TSplit_BatchNormThenRelu_gradient(
-        _h(in_gradient), _h(in_arr), _h(in_bn_scale), _h(pair), _h(out_gradient_y), _h(out_gradient_x), _h(out_gradient_bn_scale),
-        _h(out_gradient_bn_bias), ctypes.c_float(eps), _h(saved_mean) if saved_mean else None, _h(saved_var) if saved_var else None,
-        _s(stream), _p(profiler)))
+    _calls.TSplit_BatchNormThenRelu_gradient(in_gradient, in_arr, in_bn_scale, pair, out_gradient_y, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
 
 
 def batch_norm_relu_max_pool(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var, eps=0.01, stats=None, slots=0,
@@ -593,22 +551,15 @@ def conv2d_batch_norm_stats(in_arr_x, in_arr_f, out_arr, stats, slot, padding=0,
     """CuDNN_conv2d that also writes the per-channel (sum, sum of squares) of out_arr into row `slot` of
     `stats` (float32 array of at least (slot + 1) * out_channels * 4 elements, read as doubles)."""
     pad2 = padding if padding2 is None else padding2
-    check_call(_LIB.TSplit_Conv2dBatchNormStats(_h(in_arr_x), _h(in_arr_f), _h(out_arr), int(padding), int(pad2),
-                                                int(stride), _h(stats), int(slot), _s(stream), _p(profiler)))
+    _calls.TSplit_Conv2dBatchNormStats(in_arr_x, in_arr_f, out_arr, padding, pad2, stride, stats, slot, stream, profiler)
 
 
 def batch_norm_from_stats(in_arr, stats, slots, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var, eps=0.01,
                           relu=False, stream=None, profiler=None):
     """BatchNorm (+ Relu) forward with the batch statistics taken from rows 0 .. slots-1 of `stats`."""
-    check_call(_LIB.TSplit_BatchNormFromStats(_h(in_arr), _h(stats), int(slots), _h(bn_scale_arr), _h(bn_bias_arr),
-                                              _h(out_arr), ctypes.c_float(eps), _h(save_mean) if save_mean else None,
-                                              _h(save_var) if save_var else None, int(bool(relu)), _s(stream),
-                                              _p(profiler)))
+    _calls.TSplit_BatchNormFromStats(in_arr, stats, slots, bn_scale_arr, bn_bias_arr, out_arr, eps, save_mean, save_var, bool(relu), stream, profiler)
 
 
 def batch_norm_relu_gradient(in_gradient_y, in_arr_x, in_bn_scale, in_bn_bias, out_gradient_x, out_gradient_bn_scale,
                              out_gradient_bn_bias, saved_mean, saved_var, eps=0.01, stream=None, profiler=None):
-    check_call(_LIB.TSplit_BatchNormRelu_gradient(
-        _h(in_gradient_y), _h(in_arr_x), _h(in_bn_scale), _h(in_bn_bias), _h(out_gradient_x),
-        _h(out_gradient_bn_scale), _h(out_gradient_bn_bias), ctypes.c_float(eps), _h(saved_mean), _h(saved_var),
-        _s(stream), _p(profiler)))
+    _calls.TSplit_BatchNormRelu_gradient(in_gradient_y, in_arr_x, in_bn_scale, in_bn_bias, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)

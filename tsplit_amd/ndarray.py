@@ -12,8 +12,10 @@ import ctypes
 
 import numpy as np
 
+from . import _calls
+from . import stream as _stream
 from ._base import _LIB, c_array, check_call
-from .stream import create_event_handle, current_keeper
+from .stream import create_event_handle
 
 # 0: raw device malloc/free per tensor; != 0: pooled allocator (ndarray.py:8)
 MEMORY_MANAGE_RULE = 1
@@ -51,8 +53,6 @@ def _prototype(name, *argtypes):
 
 
 _int64_p, _handle_p = ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(DLArrayHandle)
-_alloc = _prototype("DLArrayAlloc", _int64_p, ctypes.c_int64, DLContext, _handle_p, ctypes.c_int)
-_free = _prototype("DLArrayFree", DLArrayHandle, ctypes.c_int)
 _array_view = _prototype("TSplit_ArrayView", DLArrayHandle, _int64_p, ctypes.c_int, _handle_p)
 _shapes = {}     # shape -> the same as a C array, which the library copies
 
@@ -68,6 +68,10 @@ def _c_shape(shape):
         return c
 
 
+_calls.bind({name: ctypes.cast(_LIB[name], ctypes.c_void_p).value for name in _calls.SYMBOLS + ["DLArrayAlloc", "DLArrayFree"]}, globals(),
+            vars(_stream), lambda address: ctypes.cast(address, DLArrayHandle))
+
+
 def cpu(dev_id=0):
     return DLContext(dev_id, 1)
 
@@ -80,39 +84,13 @@ def is_gpu_ctx(ctx):
     return bool(ctx) and ctx.device_type == 2
 
 
-class NDArray(object):
-    """A buffer object: no arithmetic, only allocation, copies and micro-tensor views."""
-    __slots__ = ["handle", "auto_deleted", "swap", "in_gpu", "_events", "splitted", "sTensor",
-                 "split_number", "split_dimension", "_owner", "_is_view", "_keeper"]
+class NDArray(_calls.Array):
+    """A buffer object: no arithmetic, only allocation, copies and micro-tensor views.
 
-    def __init__(self, handle, auto_deleted=True, owner=None, is_view=False):
-        self.handle = handle
-        self.auto_deleted = auto_deleted
-        self.splitted = False
-        self.sTensor = []
-        self.split_number = 1
-        self.split_dimension = None
-        self.swap = False
-        self.in_gpu = True
-        self._events = {}
-        self._owner = owner          # keeps the parent allocation alive for views
-        self._is_view = is_view
-        self._keeper = current_keeper()     # set while a step is being recorded into a graph
-
-    def __del__(self, _free=_free):
-        h = getattr(self, "handle", None)
-        if not h or MEMORY_MANAGE_RULE is None:      # (None: the interpreter is going down)
-            return
-        if self._is_view:
-            # a view owns its struct and shape but not its data
-            h.contents.data = None
-            _free(h, MEMORY_MANAGE_RULE)
-        elif self.auto_deleted:
-            # an array born inside a recorded step outlives this object: the graph replays into it
-            keeper = self._keeper
-            if keeper is None or h.contents.ctx.device_type != 2 or not keeper.take(h, MEMORY_MANAGE_RULE):
-                _free(h, MEMORY_MANAGE_RULE)
-        self.handle = None
+    NDArray(handle, auto_deleted=True, owner=None, is_view=False) takes the DLArray of `handle` over and frees it when collected: a view its
+    struct only (`owner` keeps the parent allocation alive), an array born inside a recorded step by way of the recording.  `handle`, `shape`
+    and `data_ptr` read that DLArray; swap, in_gpu, splitted, sTensor, split_number and split_dimension are the host's notes."""
+    __slots__ = []
 
     # ---- events used by swapping executors (created lazily) ----
     def _event(self, name):
@@ -162,17 +140,8 @@ class NDArray(object):
         self.in_gpu = True
 
     @property
-    def shape(self):
-        c = self.handle.contents
-        return tuple(c.shape[:c.ndim])
-
-    @property
     def ctx(self):
         return self.handle.contents.ctx
-
-    @property
-    def data_ptr(self):
-        return self.handle.contents.data
 
     def __setitem__(self, in_slice, value):
         if not isinstance(in_slice, slice) or in_slice.start is not None or in_slice.stop is not None:
@@ -252,10 +221,7 @@ def array(arr, ctx, stream_handle=None, event_handle=None):
 
 
 def empty(shape, ctx=cpu(0)):
-    cshape = _c_shape(shape)
-    handle = DLArrayHandle()
-    check_call(_alloc(cshape, len(cshape), ctx, ctypes.byref(handle), MEMORY_MANAGE_RULE))
-    return NDArray(handle)
+    return _calls.new_array(NDArray, shape, ctx)
 
 
 class ND_Sparse_Array(object):
