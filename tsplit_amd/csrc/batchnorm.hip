@@ -18,9 +18,17 @@
 // Small channels (N*H*W <= 16384: 14x14 and smaller planes at batch 64, 17x17 at batch 32) take
 // one-pass kernels instead: one block per channel keeps the channel's values in registers, so
 // x (and dy) are read once - the algorithmic 8 and 12 B/elem - in one launch per direction.
+// What bounds those is latency: a block's loads, the walk through LDS in the order of the sums (about
+// 1 us a direction), the stores.  Forward and gradient behind a Relu, against four waves a block
+// that loaded value by value: 16 x 128 x 32 x 32 12.9 and 16.1 -> 7.8 and 9.7 us, 32 x 192 x 17 x 17
+// 11.0 and 13.9 -> 7.6 and 9.2, 64 x 256 x 14 x 14 12.0 and 14.8 -> 8.6 and 11.1, 64 x 1024 x 14 x 14 28.9
+// and 56.6 -> 25.0 and 35.5 (5.8 TB/s of 12 B/elem would be 26.5), 64 x 512 x 7 x 7 6.9 and 9.0 -> 7.5 and 9.2.
+#include <algorithm>
+
 #include "activations.h"
 #include "common.h"
 #include "fastdiv.h"
+#include "mfma_gemm.h"
 #include "reduce.h"
 
 namespace tsplit {
@@ -454,52 +462,175 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_dx_plane_kernel(const f32x4 *
 }
 
 // ---- one block per channel, the channel in registers ------------------------------------
-constexpr int kOnePassMax = 64 * kThreads;      // elements per channel
+constexpr int kRow = 256;                // values that the sums take side by side
+constexpr int kOnePassMax = 64 * kRow;   // elements per channel
 
-// element e of channel c: plane e / HW, offset e % HW
-__device__ __forceinline__ int64_t chan_addr(const FastDiv &hw, uint32_t e, int c, int C) {
-  const uint32_t n = hw.div(e);
-  return (static_cast<int64_t>(n) * C + c) * hw.d + (e - n * hw.d);
+// A channel's values e = 0, 1, ... lie in planes of hw.  They are taken in rows of 256, value l of a row by sum l, which adds its values in the
+// order of the rows; the 256 sums are added as doubles: the bits of 256 threads of which thread l takes the values e = 256 r + l one by one.
+// Loaded that way, with a division and a 64-bit address a value in four waves, the loads were what took the time.  So wave w of W holds the
+// rows w, w + W, ..., four values a lane, and hands them, two rows of every wave at a time, through LDS to the 256 threads that add.
+// A lane's four values are one word where planes are of whole words, else they lie 64 apart (words that run over the edge of a plane into
+// the next, with a second load and a join, took 8.5 us for 7.5 at 32 x 192 x 17 x 17).  kFar: 64 apart, by 64-bit addresses, where a row's
+// planes lie 2 GiB and more apart.
+enum Layout { kWords, kValues, kFar };
+template <int W, int LAYOUT>
+struct Rows {
+  FastDiv hw;
+  int C, c;
+  uint32_t m, per;      // values of the channel; rows a wave
+  uint32_t wave, lane;
+  int64_t left;         // values of the tensor from the channel on
+  __device__ __forceinline__ Rows(const FastDiv &plane, int chans, uint32_t values) : hw(plane), C(chans), c(blockIdx.x), m(values) {
+    per = ((m + kRow - 1) / kRow + W - 1) / W;
+    wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    lane = threadIdx.x & 63;
+    left = static_cast<int64_t>(m) * C - static_cast<int64_t>(c) * hw.d;
+  }
+  // the lane's value i of row r of this wave, m and more where there is none
+  __device__ __forceinline__ uint32_t value(uint32_t r, uint32_t i) const { return (r * W + wave) * kRow + (LAYOUT == kWords ? 4 * lane + i : 64 * i + lane); }
+  // a buffer from the first plane of row r on, and the byte offset of value e in it (out of range where there is none)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const float *p, uint32_t r, uint32_t &n0) const {
+    const uint32_t first = (r * W + wave) * kRow;
+    n0 = hw.div(first < m ? first : 0);
+    const int64_t before = static_cast<int64_t>(n0) * C * hw.d, bytes = (left - before) * 4;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p) + static_cast<int64_t>(c) * hw.d + before, 0,
+                                             static_cast<int>(bytes < 0x7fffffffll ? bytes : 0x7fffffffll), mg::kBufFlags);
+  }
+  __device__ __forceinline__ unsigned offset(uint32_t n0, uint32_t e) const {
+    const uint32_t n = hw.div(e);
+    return e < m ? ((n - n0) * static_cast<uint32_t>(C) * hw.d + e - n * hw.d) * 4u : mg::kOobOffset;
+  }
+  __device__ __forceinline__ int64_t at(uint32_t e) const {
+    const uint32_t n = hw.div(e);
+    return (static_cast<int64_t>(n) * C + c) * hw.d + e - n * hw.d;
+  }
+  __device__ __forceinline__ f32x4 load(const float *p, uint32_t r) const {
+    if constexpr (LAYOUT == kFar) {
+      f32x4 v;
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) v[i] = value(r, i) < m ? p[at(value(r, i))] : 0.f;
+      return v;
+    }
+    uint32_t n0;
+    const __amdgpu_buffer_rsrc_t from = buffer(p, r, n0);
+    f32x4 v;
+    if constexpr (LAYOUT == kWords) {
+      v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, offset(n0, value(r, 0)), 0, kStream));
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, offset(n0, value(r, i)), 0, kStream));
+    }
+    return v;
+  }
+  __device__ __forceinline__ void store(float *p, uint32_t r, const f32x4 &v) const {
+    if constexpr (LAYOUT == kFar) {
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i)
+        if (value(r, i) < m) p[at(value(r, i))] = v[i];
+      return;
+    }
+    uint32_t n0;
+    const __amdgpu_buffer_rsrc_t to = buffer(p, r, n0);
+    if constexpr (LAYOUT == kWords) {
+      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(mg::u32x4, v), to, offset(n0, value(r, 0)), 0, kStream);
+    } else {
+#pragma unroll
+      for (uint32_t i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[i]), to, offset(n0, value(r, i)), 0, kStream);
+    }
+  }
+  static constexpr int kStream = 2;   // non-temporal
+};
+// Goes through the rows in order: value(k, r) are this lane's values of the wave's row r of array k, add(row, v) runs on the first 256
+// threads with each thread's value of every array.
+template <int R, int ARRAYS, int W, int LAYOUT, class Value, class Add>
+__device__ __forceinline__ void in_rows(const Rows<W, LAYOUT> &rows, float (*stage)[ARRAYS][2 * W][kRow], Value value, Add add) {
+#pragma unroll
+  for (int b = 0; b < R; b += 2) {
+    if (b >= static_cast<int>(rows.per)) break;
+    float(*const to)[2 * W][kRow] = stage[b >> 1 & 1];
+#pragma unroll
+    for (int r = 0; r < 2 && b + r < R; ++r)
+#pragma unroll
+      for (int k = 0; k < ARRAYS; ++k) {
+        float *const row = to[k][r * W + rows.wave];
+        const f32x4 v = value(k, b + r);
+        if constexpr (LAYOUT == kWords) {
+          *reinterpret_cast<f32x4 *>(row + 4 * rows.lane) = v;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) row[64 * i + rows.lane] = v[i];
+        }
+      }
+    __syncthreads();
+    if (W * kWave == kRow || threadIdx.x < kRow) {
+#pragma unroll
+      for (int q = 0; q < (b + 1 < R ? 2 * W : W); ++q) {
+        float v[ARRAYS];
+#pragma unroll
+        for (int k = 0; k < ARRAYS; ++k) v[k] = to[k][q][threadIdx.x];
+        add(b * W + q, v);
+      }
+    }
+  }
+}
+// the totals of the 256 threads' sums, as doubles, to all threads
+template <int NS>
+__device__ __forceinline__ void totals(const float (&s)[NS], double (*sm)[kRow / kWave], double (&total)[NS]) {
+  if (threadIdx.x < kRow) {
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+      const double v = wave_sum(static_cast<double>(s[k]));
+      if ((threadIdx.x & 63) == 0) sm[k][threadIdx.x >> 6] = v;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    total[k] = sm[k][0];
+#pragma unroll
+    for (int i = 1; i < kRow / kWave; ++i) total[k] += sm[k][i];
+  }
 }
 
-// v[r] into a channel's sums: of the first two squares the first is the fused one
-template <int R>
-__device__ __forceinline__ void squares_onepass(const float (&v)[R], int r, float &s, float &q) {
-  s += v[r];
-  if (r > 0) q = fmaf(v[r == 1 ? 0 : r], v[r == 1 ? 0 : r], r == 1 ? v[1] * v[1] : q);
-}
-
-// R: values per thread (compile-time bound of the register arrays)
-template <int R, int RELU>
-__global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *__restrict__ x, float *__restrict__ y,
+// W waves of up to R rows each
+template <int W, int R, int LAYOUT, int RELU>
+__global__ __launch_bounds__(W *kWave) void bn_fwd_onepass_kernel(const float *__restrict__ x, float *__restrict__ y,
                                                                   const float *__restrict__ gamma,
                                                                   const float *__restrict__ beta, FastDiv hw, int C,
                                                                   uint32_t m, float eps, double inv_m,
                                                                   float *__restrict__ save_mean,
                                                                   float *__restrict__ save_istd, bool wide,
                                                                   float *__restrict__ rl, float *__restrict__ pair) {
-  __shared__ double sm[kWaves];
+  __shared__ __attribute__((aligned(16))) float stage[2][1][2 * W][kRow];
+  __shared__ double sm[2][kRow / kWave];
   __shared__ float coef[2];
-  const int c = blockIdx.x;
-  float v[R];
-  float s = 0.f;
+  const Rows<W, LAYOUT> rows(hw, C, m);
+  const int c = rows.c;
+  f32x4 v[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const uint32_t e = r * kThreads + threadIdx.x;
-    v[r] = e < m ? __builtin_nontemporal_load(x + chan_addr(hw, e, c, C)) : 0.f;
-    s += v[r];
-  }
-  const double mean = block_sum<double, kWaves>(static_cast<double>(s), sm) * inv_m;
+  for (int r = 0; r < R; ++r) v[r] = rows.load(x, r);
+  __builtin_amdgcn_sched_barrier(0);   // (all loads are asked for before the first is waited for)
+  float s[1] = {0.f}, q[1] = {0.f};
+  double total[1];
+  in_rows<R, 1>(rows, stage, [&](int, int r) { return v[r]; }, [&](int, const float (&u)[1]) { s[0] += u[0]; });
+  totals(s, sm, total);
+  const double mean = total[0] * inv_m;
   // the values are at hand: the variance is the mean squared distance from the mean
   const float mf32 = static_cast<float>(mean);
-  float q = 0.f;
+  in_rows<R, 1>(
+      rows, stage,
+      [&](int, int r) {
+        f32x4 d;
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const uint32_t e = r * kThreads + threadIdx.x;
-    const float d = v[r] - mf32;
-    q += e < m ? d * d : 0.f;
-  }
-  double var = block_sum<double, kWaves>(static_cast<double>(q), sm) * inv_m;
+        for (uint32_t i = 0; i < 4; ++i) {
+          const float u = v[r][i] - mf32;
+          d[i] = rows.value(r, i) < m ? __fmul_rn(u, u) : 0.f;
+        }
+        return d;
+      },
+      [&](int, const float (&u)[1]) { q[0] += u[0]; });
+  totals(q, sm + 1, total);
+  double var = total[0] * inv_m;
   // (x - float(mean)) leaves out mean - float(mean): var = E[(x - mf)^2] - (mean - mf)^2
   const double dm = mean - static_cast<double>(mf32);
   var -= dm * dm;
@@ -522,17 +653,14 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_onepass_kernel(const float *_
   if (RELU == kBoth && threadIdx.x < 2) pair[2 * c + threadIdx.x] = coef[threadIdx.x];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const uint32_t e = r * kThreads + threadIdx.x;
-    if (e < m) {
-      const float z = axpb(v[r], a, b);
-      __builtin_nontemporal_store(RELU == kFused ? relu1(z) : z, y + chan_addr(hw, e, c, C));
-      if (RELU == kBoth) __builtin_nontemporal_store(relu1(z), rl + chan_addr(hw, e, c, C));
-    }
+    const f32x4 z = axpb(v[r], a, b);
+    rows.store(y, r, RELU == kFused ? relu_w(z) : z);
+    if (RELU == kBoth) rows.store(rl, r, relu_w(z));
   }
 }
 
-template <int R, bool STATS, int RELU>
-__global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *__restrict__ dy, const float *__restrict__ x,
+template <int W, int R, int LAYOUT, bool STATS, int RELU>
+__global__ __launch_bounds__(W *kWave) void bn_bwd_onepass_kernel(const float *__restrict__ dy, const float *__restrict__ x,
                                                                   float *__restrict__ dx, const float *__restrict__ gamma,
                                                                   const float *__restrict__ beta, FastDiv hw, int C,
                                                                   uint32_t m, float eps, double inv_m,
@@ -540,10 +668,12 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
                                                                   const float *__restrict__ save_istd, bool wide,
                                                                   float *__restrict__ dgamma, float *__restrict__ dbeta,
                                                                   const float *__restrict__ pair, float *__restrict__ dg) {
-  constexpr int kGate = gate_of(RELU, STATS);
-  __shared__ double sm[kWaves];
+  constexpr int kGate = gate_of(RELU, STATS), kSums = STATS ? 4 : 2;
+  __shared__ __attribute__((aligned(16))) float stage[2][2][2 * W][kRow];
+  __shared__ double sm[kSums][kRow / kWave];
   __shared__ float coef[3];
-  const int c = blockIdx.x;
+  const Rows<W, LAYOUT> rows(hw, C, m);
+  const int c = rows.c;
   float ga = 0.f, gb = 0.f;
   if (RELU == kBoth) ga = pair[2 * c], gb = pair[2 * c + 1];
   if (RELU == kFused) {
@@ -551,51 +681,47 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
     ga = static_cast<float>(a);
     gb = static_cast<float>(static_cast<double>(beta[c]) - saved_stat(save_mean, c, wide) * a);
   }
-  float xv[R], dv[R];
-  float sdy = 0.f, sdx = 0.f, sx = 0.f, sq = 0.f;
+  f32x4 xv[R], dv[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const uint32_t e = r * kThreads + threadIdx.x;
-    const bool ok = e < m;
-    const int64_t at = ok ? chan_addr(hw, e, c, C) : 0;
-    xv[r] = ok ? __builtin_nontemporal_load(x + at) : 0.f;
-    dv[r] = ok ? __builtin_nontemporal_load(dy + at) : 0.f;
-    if constexpr (kGate != kOperator) {
-      dv[r] = gated<kGate>(dv[r], xv[r], ga, gb);
-      acc_dot(dv[r], xv[r], sdy, sdx);
-      if (STATS) squares_onepass(xv, r, sx, sq);
-    }
+    xv[r] = rows.load(x, r);
+    dv[r] = rows.load(dy, r);
   }
-  if constexpr (kGate == kOperator) {
-    // (with its selects the compiler waits for every load by itself unless all are asked for first: 43 us for 17)
-    __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_sched_barrier(0);   // (all loads are asked for before the first is waited for)
+  float s[kSums] = {};
+  double total[kSums];
+  in_rows<R, 2>(
+      rows, stage,
+      [&](int k, int r) {
+        if (k == 0) return xv[r];
+        if constexpr (kGate != kNone) {
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      dv[r] = r * kThreads + threadIdx.x < m ? gated<kOperator>(dv[r], xv[r], ga, gb) : 0.f;
-      acc_dot(dv[r], xv[r], sdy, sdx);
-      if (STATS) squares_onepass(xv, r, sx, sq);
-    }
-  }
-  const double r0 = block_sum<double, kWaves>(static_cast<double>(sdy), sm);
-  const double r1 = block_sum<double, kWaves>(static_cast<double>(sdx), sm);
-  double r2 = 0.0, r3 = 0.0;
-  if (STATS) {
-    r2 = block_sum<double, kWaves>(static_cast<double>(sx), sm);
-    r3 = block_sum<double, kWaves>(static_cast<double>(sq), sm);
-  }
+          for (uint32_t i = 0; i < 4; ++i) dv[r][i] = rows.value(r, i) < m ? gated<kGate>(dv[r][i], xv[r][i], ga, gb) : 0.f;
+        }
+        return dv[r];
+      },
+      [&](int row, const float (&u)[2]) {
+        acc_dot(u[1], u[0], s[0], s[1]);
+        if constexpr (STATS) {   // of the first two squares the first is the fused one (it waits in the sum until then)
+          s[kSums - 2] += u[0];
+          float &q = s[kSums - 1];
+          q = row == 0 ? u[0] : row == 1 ? fmaf(q, q, u[0] * u[0]) : fmaf(u[0], u[0], q);
+        }
+      });
+  totals(s, sm, total);
   if (threadIdx.x == 0) {
     double mean, istd;
     if (!STATS) {
       mean = save_mean[c];
       istd = save_istd[c];
     } else {
-      mean = r2 * inv_m;
-      double var = r3 * inv_m - mean * mean;
+      mean = total[kSums - 2] * inv_m;
+      double var = total[kSums - 1] * inv_m - mean * mean;
       if (var < 0.0) var = 0.0;
       istd = 1.0 / sqrt(var + static_cast<double>(eps));
     }
-    const double dbias = r0;
-    const double dscale = (r1 - mean * r0) * istd;
+    const double dbias = total[0];
+    const double dscale = (total[1] - mean * total[0]) * istd;
     const double k1 = static_cast<double>(gamma[c]) * istd;
     const double k2 = -k1 * istd * dscale * inv_m;
     const double k3 = -k1 * dbias * inv_m - k2 * mean;
@@ -609,12 +735,42 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_onepass_kernel(const float *_
   const float k1 = coef[0], k2 = coef[1], k3 = coef[2];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
-    const uint32_t e = r * kThreads + threadIdx.x;
-    if (e < m) {
-      if (RELU == kBoth) __builtin_nontemporal_store(dv[r], dg + chan_addr(hw, e, c, C));
-      __builtin_nontemporal_store(lin2_onepass(dv[r], xv[r], k1, k2, k3), dx + chan_addr(hw, e, c, C));
-    }
+    if (RELU == kBoth) rows.store(dg, r, dv[r]);
+    f32x4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = lin2_onepass(dv[r][i], xv[r][i], k1, k2, k3);
+    rows.store(dx, r, o);
   }
+}
+
+// a one-pass kernel by the size of a channel: four waves of 4 rows, or eight of 4, 5, 7 or 8 (a wave's rows that do not exist cost what others do:
+// 32 x 192 x 17 x 17 as 8 x 8 rows 8.7 us, as 8 x 5 7.6)
+#define BN_ONEPASS_SIZE(LAUNCH, LAYOUT, ...) \
+  do {                                       \
+    if (m <= 16 * kRow)                      \
+      LAUNCH(4, 4, LAYOUT, __VA_ARGS__);     \
+    else if (m <= 32 * kRow)                 \
+      LAUNCH(8, 4, LAYOUT, __VA_ARGS__);     \
+    else if (m <= 40 * kRow)                 \
+      LAUNCH(8, 5, LAYOUT, __VA_ARGS__);     \
+    else if (m <= 56 * kRow)                 \
+      LAUNCH(8, 7, LAYOUT, __VA_ARGS__);     \
+    else                                     \
+      LAUNCH(8, 8, LAYOUT, __VA_ARGS__);     \
+  } while (0)
+#define BN_ONEPASS(LAUNCH, ...)                       \
+  do {                                                \
+    if (rows_far(m, hw, C))                           \
+      LAUNCH(8, 8, kFar, __VA_ARGS__);                \
+    else if (hw % 4 == 0)                             \
+      BN_ONEPASS_SIZE(LAUNCH, kWords, __VA_ARGS__);   \
+    else                                              \
+      BN_ONEPASS_SIZE(LAUNCH, kValues, __VA_ARGS__);  \
+  } while (0)
+// the last plane of a row beyond 32-bit byte offsets from its first one
+inline bool rows_far(int64_t m, int64_t hw, int64_t C) {
+  const int64_t planes = std::min(m / hw, kRow / hw + 2);
+  return ((planes - 1) * C + 1) * hw * 4 >= (1ll << 31);
 }
 
 inline bool one_pass_ok(const DLArray *x) {
@@ -1012,27 +1168,16 @@ static int bn_forward(const char *who, int relu, const DLArrayHandle input_X, co
     ProfileScope ps1(p, s, numel(input_X) + 2 * C, numel(output_Y), 0);
     float *sm1 = save_mean_arr ? mf(save_mean_arr) : nullptr;
     float *sv1 = save_var_arr ? mf(save_var_arr) : nullptr;
-    const int per = static_cast<int>((m + kThreads - 1) / kThreads);
-#define BN_FWD1(R, RL)                                                                                              \
-  hipLaunchKernelGGL((bn_fwd_onepass_kernel<R, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,         \
-                     cf(input_X), mf(output_Y), cf(bn_scale), cf(bn_bias), FastDiv(hw), static_cast<int>(C), m, eps, \
-                     1.0 / static_cast<double>(m), sm1, sv1, relu == kFused && wide_stats(save_mean_arr, C), r, pair)
-#define BN_FWD1_R(RL)   \
-  do {                  \
-    if (per <= 16)      \
-      BN_FWD1(16, RL);  \
-    else if (per <= 32) \
-      BN_FWD1(32, RL);  \
-    else                \
-      BN_FWD1(64, RL);  \
-  } while (0)
+#define BN_FWD1(W, R, LAYOUT, RL)                                                                                                          \
+  hipLaunchKernelGGL((bn_fwd_onepass_kernel<W, R, LAYOUT, RL>), dim3(static_cast<unsigned>(C)), dim3(W * kWave), 0, s, cf(input_X),          \
+                     mf(output_Y), cf(bn_scale), cf(bn_bias), FastDiv(hw), static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, \
+                     sv1, relu == kFused && wide_stats(save_mean_arr, C), r, pair)
     if (relu == kBoth)
-      BN_FWD1_R(kBoth);
+      BN_ONEPASS(BN_FWD1, kBoth);
     else if (relu == kFused)
-      BN_FWD1_R(kFused);
+      BN_ONEPASS(BN_FWD1, kFused);
     else
-      BN_FWD1_R(kAlone);
-#undef BN_FWD1_R
+      BN_ONEPASS(BN_FWD1, kAlone);
 #undef BN_FWD1
     return ps1.finish();
   }
@@ -1137,9 +1282,8 @@ static int bn_backward(const char *who, int relu, const DLArrayHandle gradient_Y
     const float *bias1 = bn_bias ? cf(bn_bias) : nullptr;
     float *dg1 = gradient_bn_scale ? mf(gradient_bn_scale) : nullptr;
     float *db1 = gradient_bn_bias ? mf(gradient_bn_bias) : nullptr;
-    const int per = static_cast<int>((m + kThreads - 1) / kThreads);
     const float *dy1 = cf(gradient_Y);
-    if (relu == kBoth && per > 16) {
+    if (relu == kBoth && m > 16 * kRow) {
       // a block a channel writes two arrays of this size no faster than one after the other, a launch over all of them does (128
       // channels of 16 K values: one launch 34 us, 17 + 5 as two; 512 of 4 K or less 7 and 6 + 4)
       PlaneGeo pg;
@@ -1157,32 +1301,22 @@ static int bn_backward(const char *who, int relu, const DLArrayHandle gradient_Y
 //   kAlone, none          <yes, kAlone>     kFused, saved doubles  <yes, kFused>    kBoth, none          <yes, kBoth>
 // kFused always has saved arrays, and `wide` says that they are doubles; `pair` and `dr` are kBoth's alone; `sm` and `sv` are null
 // unless both saved arrays are given.
-#define BN_BWD1(R, ST, RL)                                                                                          \
-  hipLaunchKernelGGL((bn_bwd_onepass_kernel<R, ST, RL>), dim3(static_cast<unsigned>(C)), dim3(kThreads), 0, s,     \
-                     dy1, cf(input_X), mf(gradient_X), cf(bn_scale), bias1, FastDiv(hw),                 \
-                     static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, sv1, wide, dg1, db1, pair, dr)
-#define BN_BWD1_R(ST, RL)   \
-  do {                      \
-    if (per <= 16)          \
-      BN_BWD1(16, ST, RL);  \
-    else if (per <= 32)     \
-      BN_BWD1(32, ST, RL);  \
-    else                    \
-      BN_BWD1(64, ST, RL);  \
-  } while (0)
+#define BN_BWD1(W, R, LAYOUT, ST, RL)                                                                                                      \
+  hipLaunchKernelGGL((bn_bwd_onepass_kernel<W, R, LAYOUT, ST, RL>), dim3(static_cast<unsigned>(C)), dim3(W * kWave), 0, s, dy1, cf(input_X), \
+                     mf(gradient_X), cf(bn_scale), bias1, FastDiv(hw), static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, sv1, \
+                     wide, dg1, db1, pair, dr)
     if (relu == kBoth && saved)
-      BN_BWD1(16, false, kBoth);
+      BN_ONEPASS(BN_BWD1, false, kBoth);
     else if (relu == kBoth)
-      BN_BWD1(16, true, kBoth);
+      BN_ONEPASS(BN_BWD1, true, kBoth);
     else if (wide)
-      BN_BWD1_R(true, kFused);
+      BN_ONEPASS(BN_BWD1, true, kFused);
     else if (relu)
-      BN_BWD1_R(false, kFused);
+      BN_ONEPASS(BN_BWD1, false, kFused);
     else if (saved)
-      BN_BWD1_R(false, kAlone);
+      BN_ONEPASS(BN_BWD1, false, kAlone);
     else
-      BN_BWD1_R(true, kAlone);
-#undef BN_BWD1_R
+      BN_ONEPASS(BN_BWD1, true, kAlone);
 #undef BN_BWD1
     return ps1.finish();
   }
