@@ -108,15 +108,20 @@ constexpr TileKind kWaveTiles[] = {{16, 16}, {16, 32}, {32, 16}, {32, 32}};
 struct WavesPlan {
   int tile, waves;   // waves 0: the tile kernel
 };
-inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, double tile_kernel_us) {
+//
+// Deep products (from 1024 on) and those with the depth contiguous in both operands (`deep_words`: a lane's words lie a row apart) take
+// more a value on the wider tiles, whose loads then bound them; without that line 512 x 512 over 4096 took 29.9-34.5 us here and 27.7-28.4
+// on the tile kernel, over 8192 54-63 and 43-45, with `deep_words` 384 x 512 over 2048 19.4 and 16.7, 256 x 512 over 2048 15.0 and 14.2.
+inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, bool deep_words, double tile_kernel_us) {
   constexpr double kLaunch = 3.6, kBlock[] = {0.18, 0.40, 0.47, 0.76}, kDepth[] = {0.0022, 0.0031, 0.0031, 0.0045};
+  constexpr double kBeyond[] = {0, 0.0009, 0.0009, 0.0020}, kWords[] = {0, 0.0014, 0.0014, 0.0014};
   WavesPlan best{0, 0};
   double least = 2.3 + 1.15 * tile_kernel_us;
   for (int t = 0; t < 4; ++t) {
     const int64_t blocks = ((M + kWaveTiles[t].bm - 1) / kWaveTiles[t].bm) * ((N + kWaveTiles[t].bn - 1) / kWaveTiles[t].bn) * batch;
     if (blocks > 1024) continue;
     const int64_t n = (blocks + 255) / 256;
-    const double us = kLaunch + n * (kBlock[t] + kDepth[t] * K);
+    const double us = kLaunch + n * (kBlock[t] + kDepth[t] * K + (K > 1024 ? kBeyond[t] * (K - 1024) + (deep_words ? kWords[t] * K : 0) : 0));
     if (us < least && (n == 1 || us < 8)) {   // (of several blocks a CU the tile kernel fills the chip as well: 100 x 4096 over 4096)
       least = us;
       // 32 values of the depth a wave; eight or sixteen waves gain nothing on a CU of their own (over the shapes 0.2 %) and lose where
