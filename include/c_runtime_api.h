@@ -493,6 +493,12 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
                                          DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                                          DLStreamHandle stream_handle, ProfilerHandle p);
 
+/* ---- gradient_x = the convolution's data gradient + addend (of gradient_x's size; it may be gradient_x): a gradient of several
+ *      terms without a pass of its own (outside the reference's ABI, whose graph sums them with DLGpuMatrixElementwiseAdd: the
+ *      same bits).  In one launch for 1 x 1 filters of stride 1 and 2 without padding, else in the two it stands for. ---- */
+int TSplit_Conv2dGradientOfDataAdd(const DLArrayHandle input_f, const DLArrayHandle gradient_y, const DLArrayHandle addend,
+                                   DLArrayHandle gradient_x, const int padding, const int padding2, const int stride,
+                                   DLStreamHandle stream_handle);
 /* ---- Matrix products with the operators behind them in the same launch (outside the reference's ABI).
  *      TSplit_MatrixMultiplyAdd: C = op(A) op(B), + bias[column] where given, + addend where given (an array of
  *      C's size; it may be C), and, where given, relu = max(C, 0).  With `gate`, the input of a Relu of C's size, C is

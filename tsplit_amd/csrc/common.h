@@ -114,7 +114,9 @@ struct StatsSink {
 struct ConvTileGeo;   // conv_reach.h
 bool conv_tile_takes(const ConvTileGeo &g, bool bwd);
 int conv_tile_forward(const float *x, const float *w, float *y, const ConvTileGeo &g, hipStream_t st, StatsSink *sink);
-int conv_tile_bwd_data(const float *dy, const float *w, float *dx, const ConvTileGeo &g, hipStream_t st);
+// add: what the gradient is added to (it may be dx), null for nothing; only where conv_tile_bwd_data_adds.
+bool conv_tile_bwd_data_adds(const ConvTileGeo &g);
+int conv_tile_bwd_data(const float *dy, const float *w, const float *add, float *dx, const ConvTileGeo &g, hipStream_t st);
 
 // The filter gradient on the tile kernel (conv_wgrad_tile.hip); a block addresses `reach` bytes from the first image of its range.
 bool conv_tile_bwd_filter_takes(const ConvTileGeo &g, int64_t reach);

@@ -1487,10 +1487,15 @@ int conv_forward(const char *who, const DLArray *x, const DLArray *w, DLArray *y
   return ps.finish();
 }
 
+// added: what the gradient is added to (it may be dx), or null.  Only one launch of the tile kernel adds: elsewhere 1 is
+// returned, nothing launched.
 int conv_bwd_data(const char *who, const DLArray *w, const DLArray *dy, DLArray *dx, int ph, int pw, int s,
-                  DLStreamHandle sh, ProfilerHandle p) {
+                  DLStreamHandle sh, ProfilerHandle p, const DLArray *added = nullptr) {
   ConvGeo g;
   if (geo_from(who, dx, w, dy, ph, pw, s, g)) return -1;
+  if (added && (numel(dx) == 0 || numel(dy) == 0 || numel(w) == 0 || winograd_pays(g, g.O) || !conv_tile_bwd_data_adds(g) || !conv_tile_takes(g, true) ||
+                tile_kernel_images(g, static_cast<int64_t>(g.O) * g.oH * g.oW) <= 0))
+    return 1;
   hipStream_t st = stream_of(sh);
   ProfileScope ps(p, st, numel(dy) + numel(w), numel(dx), numel(w));
   if (numel(dx) > 0 && (numel(dy) == 0 || numel(w) == 0)) {
@@ -1503,7 +1508,7 @@ int conv_bwd_data(const char *who, const DLArray *w, const DLArray *dy, DLArray 
     const int per = conv_tile_takes(g, true) ? tile_kernel_images(g, dy_img) : 0;
     if (per > 0) {
       const int rc = for_image_runs(g, per, [&](const ConvGeo &run, int64_t first) {
-        return conv_tile_bwd_data(cf(dy) + first * dy_img, cf(w), mf(dx) + first * dx_img, run, st);
+        return conv_tile_bwd_data(cf(dy) + first * dy_img, cf(w), added ? cf(added) + first * dx_img : nullptr, mf(dx) + first * dx_img, run, st);
       });
       if (rc) return rc;
       return ps.finish();
@@ -1625,6 +1630,24 @@ int CuDNN_DLGpuConv2d_Gradient_of_Data(const DLArrayHandle input_f, const DLArra
                                        const int stride, DLStreamHandle stream_handle, ProfilerHandle p) {
   return conv_bwd_data("CuDNN_DLGpuConv2d_Gradient_of_Data", input_f, gradient_y, gradient_x, padding, padding2,
                        stride, stream_handle, p);
+}
+
+int TSplit_Conv2dGradientOfDataAdd(const DLArrayHandle input_f, const DLArrayHandle gradient_y, const DLArrayHandle addend,
+                                   DLArrayHandle gradient_x, const int padding, const int padding2, const int stride,
+                                   DLStreamHandle stream_handle) {
+  const char *who = "TSplit_Conv2dGradientOfDataAdd";
+  TS_REQUIRE(input_f && gradient_y && addend && gradient_x, "%s: NULL array", who);
+  TS_REQUIRE(numel(addend) == numel(gradient_x), "%s: the addend's size differs", who);
+  const int rc = conv_bwd_data(who, input_f, gradient_y, gradient_x, padding, padding2, stride, stream_handle, nullptr, addend);
+  if (rc <= 0) return rc;
+  // the gradient and the sum by themselves
+  DLArray alone = *gradient_x;
+  if (addend->data == gradient_x->data && numel(addend) > 0) {
+    alone.data = scratch_get(stream_of(stream_handle), 10, static_cast<size_t>(numel(gradient_x)) * sizeof(float));
+    TS_REQUIRE(alone.data, "%s: no scratch memory", who);
+  }
+  if (const int bad = conv_bwd_data(who, input_f, gradient_y, &alone, padding, padding2, stride, stream_handle, nullptr)) return bad;
+  return DLGpuMatrixElementwiseAdd(addend, &alone, gradient_x, stream_handle, nullptr);
 }
 
 // The plain symbols take one padding int and caller-provided im2col workspaces

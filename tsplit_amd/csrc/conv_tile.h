@@ -57,6 +57,7 @@ struct Params {
   FastDiv tm, tiles;             // M tiles; tiles of all phases (of all pairs)
   int phases;
   float *stats;
+  const float *add;              // laid out as out, which it may be (a lane reads a value before it writes it)
   Phase phase[kMaxPhases];
 };
 
@@ -244,9 +245,10 @@ __device__ __forceinline__ void halve(float *sum, float *sq, int lane) {
 // Stores a tile of a one-tap data gradient of stride 2: position (r, c) of a column covers the 2 x 2 input positions from (2 r, 2 c)
 // on; the value belongs to the first of them, no tap reaches the others.  Both rows of positions leave from here, in words of two
 // columns, so that dx is written once and in whole rows (a phase at a time, 64 x 512 x 28 x 28 into 64 x 256 x 56 x 56: 300 us).
-template <int TM, int TN, class StepRow>
-__device__ __forceinline__ void spread(const Params &P, const Phase &F, const f32x4 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t to, int m, int n,
-                                       int img0, int lane_row, StepRow step_row) {
+// ADD: `from` holds what is added, at every position.
+template <int TM, int TN, bool ADD, class StepRow>
+__device__ __forceinline__ void spread(const Params &P, const Phase &F, const f32x4 (&acc)[TM][TN], __amdgpu_buffer_rsrc_t to,
+                                       __amdgpu_buffer_rsrc_t from, int m, int n, int img0, int lane_row, StepRow step_row) {
   const int plane_bytes = P.out_plane * 4, out_h = P.out_h;
   const unsigned at = static_cast<unsigned>(lane_row) * plane_bytes, down = static_cast<unsigned>(P.out_w) * 4u;
   unsigned off[TN];
@@ -270,18 +272,31 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
       if (words) {
 #pragma unroll
         for (int j = 0; j < TN; j += 2) {
-          const float v[4] = {acc[tm][j][e], 0.f, acc[tm][j + 1][e], 0.f}, zeros[4] = {0.f, 0.f, 0.f, 0.f};
-          gt::store_words<4>(to, past ? kOobOffset : off[j], soff, v);
-          gt::store_words<4>(to, past || !below[j] ? kOobOffset : off[j] + down, soff, zeros);
+          const unsigned o = past ? kOobOffset : off[j], under = past || !below[j] ? kOobOffset : off[j] + down;
+          float v[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (ADD) {
+            gt::load_words<4>(from, o, soff, v);
+            gt::load_words<4>(from, under, soff, w);
+          }
+          v[0] = ADD ? v[0] + acc[tm][j][e] : acc[tm][j][e];
+          v[2] = ADD ? v[2] + acc[tm][j + 1][e] : acc[tm][j + 1][e];
+          gt::store_words<4>(to, o, soff, v);
+          gt::store_words<4>(to, under, soff, w);
         }
       } else {
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
           const bool none = past || off[j] == kOobOffset;
-          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[tm][j][e]), to, (none ? kOobOffset : off[j]) + soff, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(0u, to, (none || !beside[j] ? kOobOffset : off[j] + 4u) + soff, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(0u, to, (none || !below[j] ? kOobOffset : off[j] + down) + soff, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b32(0u, to, (none || !below[j] || !beside[j] ? kOobOffset : off[j] + down + 4u) + soff, 0, 0);
+          const unsigned o[4] = {none ? kOobOffset : off[j], none || !beside[j] ? kOobOffset : off[j] + 4u, none || !below[j] ? kOobOffset : off[j] + down,
+                                 none || !below[j] || !beside[j] ? kOobOffset : off[j] + down + 4u};
+          float v[4] = {0.f, 0.f, 0.f, 0.f};
+          if constexpr (ADD) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, o[i] + soff, 0, 0));
+          }
+          v[0] = ADD ? v[0] + acc[tm][j][e] : acc[tm][j][e];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[i]), to, o[i] + soff, 0, 0);
         }
       }
     }
@@ -289,7 +304,9 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
 
 // STATS: each wave leaves the sums and sums of squares of its rows over its 16 TN columns, for column group
 // (first column) / (16 TN) at stats[(group * M + row) * 2].
-template <int TM, int TN, bool BWD, int GATHER, bool ACROSS, bool STATS>
+// ADD: the result and what P.add holds in one store.  A gradient with several terms was a pass of its own that read two arrays
+// and wrote a third (64 x 256 x 56 x 56: 95 us); here the other term is read once, between the products and the store.
+template <int TM, int TN, bool BWD, int GATHER, bool ACROSS, bool STATS, bool ADD>
 __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, int total) {
   using X = Pass<TM, TN, BWD, GATHER, ACROSS>;
   using C = typename X::C;
@@ -304,10 +321,12 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
   // the wave's first row; offsets count from the image its tile begins in (a tile's images lie within 2 GiB)
   const int lane = threadIdx.x & 63, m = m0 + C::wave_m0(), n = n0 + C::wave_n0() + TN * (lane & 15);
   const int img0 = F.plane.div(n0), plane_bytes = P.out_plane * 4;
-  const __amdgpu_buffer_rsrc_t to =
-      gt::output_buffer(P.out + z * P.z_stride + img0 * P.out_img_stride + static_cast<int64_t>(m) * P.out_plane, 0x7fffffffll);
+  const int64_t tile_at = img0 * P.out_img_stride + static_cast<int64_t>(m) * P.out_plane;
+  const __amdgpu_buffer_rsrc_t to = gt::output_buffer(P.out + z * P.z_stride + tile_at, 0x7fffffffll);
+  const __amdgpu_buffer_rsrc_t from = ADD ? gt::output_buffer(const_cast<float *>(P.add) + tile_at, 0x7fffffffll) : to;
   if constexpr (BWD && ACROSS)
-    if (P.out_s == 2) return spread<TM, TN>(P, F, acc, to, m, n, img0, C::lane_row(), [](int tm, int e) { return C::step_row(tm, e); });
+    if (P.out_s == 2)
+      return spread<TM, TN, ADD>(P, F, acc, to, from, m, n, img0, C::lane_row(), [](int tm, int e) { return C::step_row(tm, e); });
   // where the lane's TN columns go: together if they lie in one image of a plane without gaps
   const unsigned at = static_cast<unsigned>(C::lane_row()) * plane_bytes;
   unsigned off[TN];
@@ -334,13 +353,20 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
         const bool past = kRagged && m + row + C::lane_row() >= P.M;
         const int soff = past ? 0 : row * plane_bytes;   // (past M the product may leave 32 bits)
         if constexpr (decltype(in_words)::value) {
-          float v[TN];
+          float v[TN], more[TN] = {};
+          if constexpr (ADD) gt::load_words<TN>(from, past ? kOobOffset : off[0], soff, more);
 #pragma unroll
-          for (int j = 0; j < TN; ++j) v[j] = acc[tm][j][e];
+          for (int j = 0; j < TN; ++j) v[j] = ADD ? more[j] + acc[tm][j][e] : acc[tm][j][e];
           gt::store_words<TN>(to, past ? kOobOffset : off[0], soff, v);
         } else {
+          float v[TN];
 #pragma unroll
-          for (int j = 0; j < TN; ++j) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[tm][j][e]), to, (past ? kOobOffset : off[j]) + (kRagged ? soff : 0), kRagged ? 0 : soff, 0);
+          for (int j = 0; j < TN; ++j) {
+            v[j] = acc[tm][j][e];
+            if constexpr (ADD) v[j] += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, (past ? kOobOffset : off[j]) + soff, 0, 0));
+          }
+#pragma unroll
+          for (int j = 0; j < TN; ++j) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), to, (past ? kOobOffset : off[j]) + (kRagged ? soff : 0), kRagged ? 0 : soff, 0);
         }
       }
   };

@@ -16,10 +16,15 @@ template <int TM, int TN, bool BWD, int GATHER, bool ACROSS>
 void launch_one(const Params &P, unsigned grid, int total, hipStream_t st) {
   if constexpr (!BWD)
     if (P.stats) {
-      hipLaunchKernelGGL((conv_tile_kernel<TM, TN, BWD, GATHER, ACROSS, true>), dim3(grid), dim3(gt::kThreads), 0, st, P, total);
+      hipLaunchKernelGGL((conv_tile_kernel<TM, TN, BWD, GATHER, ACROSS, true, false>), dim3(grid), dim3(gt::kThreads), 0, st, P, total);
       return;
     }
-  hipLaunchKernelGGL((conv_tile_kernel<TM, TN, BWD, GATHER, ACROSS, false>), dim3(grid), dim3(gt::kThreads), 0, st, P, total);
+  if constexpr (ACROSS)
+    if (P.add) {
+      hipLaunchKernelGGL((conv_tile_kernel<TM, TN, BWD, GATHER, ACROSS, false, true>), dim3(grid), dim3(gt::kThreads), 0, st, P, total);
+      return;
+    }
+  hipLaunchKernelGGL((conv_tile_kernel<TM, TN, BWD, GATHER, ACROSS, false, false>), dim3(grid), dim3(gt::kThreads), 0, st, P, total);
 }
 
 template <bool BWD, int GATHER, bool ACROSS>
@@ -42,8 +47,9 @@ void launch_pair(const Params &P, int tile, unsigned grid, int total, hipStream_
 }
 
 // Runs the phases of P; tiles and ranges are filled in here.  out_values: elements of the output, negative if this launch does
-// not write all of them (the fold of ranges adds whole tensors).
-int run_phases(Params &P, bool bwd, int gather, bool across, bool pairs, float *out, int64_t out_values, hipStream_t st, StatsSink *sink) {
+// not write all of them (the fold of ranges adds whole tensors).  add: what the output is added to (`across` alone); null: nothing.
+int run_phases(Params &P, bool bwd, int gather, bool across, bool pairs, float *out, int64_t out_values, hipStream_t st, StatsSink *sink,
+               const float *add = nullptr) {
   int64_t cols[kMaxPhases];
   int steps[kMaxPhases];
   const int step = pairs ? 2 : 1;
@@ -79,6 +85,7 @@ int run_phases(Params &P, bool bwd, int gather, bool across, bool pairs, float *
     sink->used += groups;
   }
   P.out = out;
+  P.add = S > 1 ? nullptr : add;
   P.z_stride = 0;
   if (S > 1) {
     P.out = static_cast<float *>(scratch_get(st, 2, static_cast<size_t>(S) * out_values * sizeof(float)));
@@ -109,7 +116,7 @@ int run_phases(Params &P, bool bwd, int gather, bool across, bool pairs, float *
       default: launch_tile<true, kTaps64, false>(P, plan.tile, grid, total, st); break;
     }
   }
-  if (S > 1) gt::launch_fold(P.out, out, out_values, S, st);
+  if (S > 1) gt::launch_fold(P.out, out, out_values, S, st, add);
   return 0;
 }
 
@@ -196,7 +203,9 @@ int conv_tile_forward(const float *x, const float *w, float *y, const ConvTileGe
   return run_phases(P, false, gather, false, false, y, static_cast<int64_t>(g.imgs) * P.out_img_stride, st, sink);
 }
 
-int conv_tile_bwd_data(const float *dy, const float *w, float *dx, const ConvTileGeo &g, hipStream_t st) {
+bool conv_tile_bwd_data_adds(const ConvTileGeo &g) { return g.kH * g.kW == 1 && g.ph == 0 && g.pw == 0 && g.s <= 2; }
+
+int conv_tile_bwd_data(const float *dy, const float *w, const float *add, float *dx, const ConvTileGeo &g, hipStream_t st) {
   const int taps = g.kH * g.kW, s = g.s;
   Params P;
   P.src = dy;
@@ -220,7 +229,7 @@ int conv_tile_bwd_data(const float *dy, const float *w, float *dx, const ConvTil
     P.phases = 1;
     P.phase[0] = Phase{FastDiv(P.out_plane), FastDiv(g.W), FastDiv(taps), FastDiv(g.kW), g.imgs * P.out_plane,
                        (blocks ? padded(g.O) : g.O) * taps, g.ph, g.pw, (g.kH - 1) * g.oW + g.kW - 1, 0, 0, 0, 0, 0};
-    if (inside) return run_phases(P, true, P.out_plane % 4 == 0 ? kWords : kOneTap, true, false, dx, values, st, nullptr);
+    if (inside) return run_phases(P, true, P.out_plane % 4 == 0 ? kWords : kOneTap, true, false, dx, values, st, nullptr, add);
     const int none[1][2] = {{0, 0}};
     if (relay(P, w, g.C, g.O, taps, g.C * taps, g.kW, 1, none, !blocks, st)) return -1;
     return run_phases(P, true, !blocks ? kTaps64 : taps <= 32 ? kBlocks32 : kBlocks64, false, false, dx, values, st, nullptr);
@@ -228,7 +237,7 @@ int conv_tile_bwd_data(const float *dy, const float *w, float *dx, const ConvTil
   if (s == 2 && taps == 1 && g.ph == 0 && g.pw == 0) {   // the product over dy's positions, spread over dx
     P.phases = 1;
     P.phase[0] = Phase{FastDiv(P.chan_stride), FastDiv(g.oW), FastDiv(1), FastDiv(1), g.imgs * P.chan_stride, g.O, 0, 0, 0, 0, 0, 0, 0, 0};
-    return run_phases(P, true, P.chan_stride % 4 == 0 ? kWords : kOneTap, true, false, dx, values, st, nullptr);
+    return run_phases(P, true, P.chan_stride % 4 == 0 ? kWords : kOneTap, true, false, dx, values, st, nullptr, add);
   }
   // phases (a, b): input positions a0 + s i, b0 + s j, reached by the filter taps a + s u, b + s v; by rows of positions, in
   // ascending order of b0

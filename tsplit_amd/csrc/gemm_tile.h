@@ -584,8 +584,16 @@ static __global__ __launch_bounds__(256) void fold_splits_kernel(const f32x4 *__
   out[i] = s;
 }
 
-// out[i] = sum over the S ranges' results, n values apart in `part`
-inline void launch_fold(const float *part, float *out, int64_t n, int S, hipStream_t st) {
+// out[i] = sum over the S ranges' results, n values apart in `part`, + add[i] where given (it may be out)
+inline void launch_fold(const float *part, float *out, int64_t n, int S, hipStream_t st, const float *add = nullptr) {
+  if (add) {
+    const Epilogue ep{1.f, nullptr, nullptr, 0.f, 0, 0.f, add, nullptr, nullptr};
+    if (n % 4 == 0 && ((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(add)) & 15) == 0)
+      hipLaunchKernelGGL((fold_epilogue_kernel<4>), dim3(static_cast<unsigned>((n / 4 + 255) / 256)), dim3(256), 0, st, part, out, n, 4, S, ep);
+    else
+      hipLaunchKernelGGL((fold_epilogue_kernel<1>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, st, part, out, n, 1, S, ep);
+    return;
+  }
   if (n % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0)
     hipLaunchKernelGGL(fold_splits_kernel, dim3(static_cast<unsigned>((n / 4 + 255) / 256)), dim3(256), 0, st,
                        reinterpret_cast<const f32x4 *>(part), reinterpret_cast<f32x4 *>(out), n / 4, S);

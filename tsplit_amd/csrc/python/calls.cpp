@@ -381,7 +381,7 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   X(TSplit_HeadsMatrixMultiply, 1 << 7 | 1 << 11) X(TSplit_HeadsScale, 0) X(DLGpuSoftmax, 0) X(DLGpuSoftmaxCrossEntropy, 0)                    \
   X(DLGpuSoftmaxCrossEntropy_Gradient, 0) X(TSplit_SoftmaxCrossEntropyIds, 0) X(TSplit_SoftmaxCrossEntropyIds_Gradient, 0)                     \
   X(TSplit_EmbeddingAdd, 0) X(TSplit_EmbeddingAdd_Gradient, 0) X(CuDNN_DLGpuConv2d, 0) X(CuDNN_DLGpuConv2d_Gradient_of_Filter, 0)              \
-  X(CuDNN_DLGpuConv2d_Gradient_of_Data, 0) X(CuDNN_DLGpuBatch_Normalization, 1 << 6 | 1 << 7)                                                  \
+  X(CuDNN_DLGpuConv2d_Gradient_of_Data, 0) X(TSplit_Conv2dGradientOfDataAdd, 0) X(CuDNN_DLGpuBatch_Normalization, 1 << 6 | 1 << 7)              \
   X(CuDNN_DLGpuBatch_Normalization_gradient, 1 << 7 | 1 << 8) X(DLGpuMax_Pooling2d, 0) X(DLGpuMax_Pooling2d_gradient, 0)                       \
   X(CuDNN_DLGpuMax_Pooling2d, 0) X(CuDNN_DLGpuMax_Pooling2d_gradient, 0) X(SGDOptimizerUpdate, 0) X(MomentumOptimizerUpdate, 0)                \
   X(DLGpuAvgerage_Pooling2d, 0) X(DLGpuAvgerage_Pooling2d_gradient, 0) X(CuDNN_DLGpuAvgerage_Pooling2d, 0)                                     \

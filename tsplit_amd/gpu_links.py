@@ -29,7 +29,7 @@ __all__ = [
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
     "batch_norm_relu", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
-    "optimizer_update_multi", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply", "heads_scale",
+    "optimizer_update_multi", "conv2d_gradient_of_data_add", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply", "heads_scale",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "join", "part", "lstm_sizes", "lstm", "lstm_gradient",
     "CuDNN_Dropout", "CuDNN_Dropout_gradient", "CuSparse_Csrmv", "CuSparse_Csrmm",
@@ -199,6 +199,13 @@ def CuDNN_conv2d_gradient_of_data(in_arr_f, in_gradient_y, out_gradient_x, paddi
                                   stride=1, stream=None, profiler=None):
     pad2 = padding if padding2 is None else padding2
     _calls.CuDNN_DLGpuConv2d_Gradient_of_Data(in_arr_f, in_gradient_y, out_gradient_x, padding, pad2, stride, stream, profiler)
+
+
+def conv2d_gradient_of_data_add(in_arr_f, in_gradient_y, addend, out_gradient_x, padding=0, padding2=None, stride=1, stream=None):
+    """out_gradient_x = the data gradient + addend (it may be out_gradient_x): the bits of the call above and
+    matrix_elementwise_add (no counterpart in the reference's gpu_links)."""
+    pad2 = padding if padding2 is None else padding2
+    _calls.TSplit_Conv2dGradientOfDataAdd(in_arr_f, in_gradient_y, addend, out_gradient_x, padding, pad2, stride, stream)
 
 
 def conv2d(in_arr_x, in_arr_f, out_arr, workspace_arr, padding=0, stride=1, stream=None, profiler=None):

@@ -116,6 +116,12 @@ class GpuBackend(object):
         L.CuDNN_conv2d_gradient_of_data(w, dy, dx, ph, pw, s, self.stream)
         return dx
 
+    def conv2d_grad_data_add(self, w, dy, xs, ph, pw, s, addend, out=None):
+        """conv2d_grad_data + addend, into `out` (it may be the addend) or a new array."""
+        dx = self.empty(xs) if out is None else out
+        L.conv2d_gradient_of_data_add(w, dy, addend, dx, ph, pw, s, self.stream)
+        return dx
+
     def conv2d_grad_filter(self, x, dy, ws, ph, pw, s):
         dw = self.empty(ws)
         L.CuDNN_conv2d_gradient_of_filter(x, dy, dw, ph, pw, s, self.stream)
@@ -559,9 +565,17 @@ class Tape(object):
         def back(g):
             if w.needs_grad:
                 self._acc(w, self.b.conv2d_grad_filter(x.value, g, w.shape, ph, pw, stride), fresh=True)
-            if x.needs_grad:
+            if x.needs_grad and x.grad is not None and self._adds_data_gradient(w.shape, ph, pw, stride):
+                x.grad = self.b.conv2d_grad_data_add(w.value, g, x.shape, ph, pw, stride, x.grad, x.grad if x.own else None)
+                if not x.own:
+                    self._owns(x, True)
+            elif x.needs_grad:
                 self._acc(x, self.b.conv2d_grad_data(w.value, g, x.shape, ph, pw, stride), fresh=True)
         return self._out(y, ys, [x, w], back, saved=[x, w])
+
+    def _adds_data_gradient(self, ws, ph, pw, stride):
+        """Whether a data gradient's launch can add to what is there: filters of one tap (others would be two launches all the same)."""
+        return ws[2:] == (1, 1) and not ph and not pw and stride <= 2 and self._ahead and self._can("conv2d_grad_data_add")
 
     @_op
     def batch_norm(self, x, gamma, beta, eps=0.01):
