@@ -421,6 +421,11 @@ int TSplit_BatchNormRelu(const DLArrayHandle input_X, const DLArrayHandle bn_sca
                          const DLArrayHandle bn_bias, DLArrayHandle output_Y, float eps,
                          DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr,
                          DLStreamHandle stream_handle, ProfilerHandle p);
+/* output_Y = TSplit_BatchNormRelu's + addend (another array of that size), the sum's bits those of DLGpuMatrixElementwiseAdd behind it:
+ * a residual block's end in one pass that reads two arrays, where the calls by themselves read three and write two. */
+int TSplit_BatchNormReluAdd(const DLArrayHandle input_X, const DLArrayHandle bn_scale, const DLArrayHandle bn_bias,
+                            const DLArrayHandle addend, DLArrayHandle output_Y, float eps,
+                            DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr, DLStreamHandle stream_handle);
 int TSplit_BatchNormRelu_gradient(const DLArrayHandle gradient_Y, const DLArrayHandle input_X,
                                   const DLArrayHandle bn_scale, const DLArrayHandle bn_bias,
                                   DLArrayHandle gradient_X, DLArrayHandle gradient_bn_scale,

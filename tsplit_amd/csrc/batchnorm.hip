@@ -116,8 +116,14 @@ __device__ __forceinline__ f32x4 gated(const f32x4 &dy, const f32x4 &x, float a,
 }
 // What a gradient kernel's form does with the gradient behind a Relu.  kAlone: there is none.  kFused: y is Relu's result, the BatchNorm's
 // own never leaves; with saved doubles (which also means that the kernel sums the statistics again) it has the bits of the two calls.
-// kBoth: y is the BatchNorm's, r Relu's of it; bits of the two calls.
-enum Pair { kAlone, kFused, kBoth };
+// kBoth: y is the BatchNorm's, r Relu's of it; bits of the two calls.  kSum (forward alone): kFused, and y = Relu's result + r.
+enum Pair { kAlone, kFused, kBoth, kSum };
+constexpr bool fused_of(int pair) { return pair == kFused || pair == kSum; }
+// what is stored as y of z, the BatchNorm's result; more: what r holds there (kSum)
+template <int PAIR, class W>
+__device__ __forceinline__ W output_of(const W &z, const W &more) {
+  return PAIR == kSum ? relu_w(z) + more : PAIR == kFused ? relu_w(z) : z;
+}
 constexpr int gate_of(int pair, bool stats) { return pair == kBoth || (pair == kFused && stats) ? kOperator : pair == kFused ? kHalf : kNone; }
 // k1 dy + k2 x + k3; in the one-pass kernels the other product is the fused one
 __device__ __forceinline__ float lin2(const float &dy, const float &x, float k1, float k2, float k3) { return fmaf(k2, x, k1 * dy) + k3; }
@@ -243,9 +249,14 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(const float *__restr
   for (; i + kThreads < end; i += 2 * kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c), a1 = word_addr<VEC>(g, i + kThreads, c);
     const W v0 = __builtin_nontemporal_load(xw + a0), v1 = __builtin_nontemporal_load(xw + a1);
+    W m0 = {}, m1 = {};
+    if (RELU == kSum) {
+      m0 = __builtin_nontemporal_load(reinterpret_cast<const W *>(r) + a0);
+      m1 = __builtin_nontemporal_load(reinterpret_cast<const W *>(r) + a1);
+    }
     const W z0 = axpb(v0, a, b), z1 = axpb(v1, a, b);
-    __builtin_nontemporal_store(RELU == kFused ? relu_w(z0) : z0, yw + a0);
-    __builtin_nontemporal_store(RELU == kFused ? relu_w(z1) : z1, yw + a1);
+    __builtin_nontemporal_store(output_of<RELU>(z0, m0), yw + a0);
+    __builtin_nontemporal_store(output_of<RELU>(z1, m1), yw + a1);
     if (RELU == kBoth) {
       __builtin_nontemporal_store(relu_w(z0), reinterpret_cast<W *>(r) + a0);
       __builtin_nontemporal_store(relu_w(z1), reinterpret_cast<W *>(r) + a1);
@@ -253,8 +264,10 @@ __global__ __launch_bounds__(kThreads) void bn_apply_kernel(const float *__restr
   }
   for (; i < end; i += kThreads) {
     const int64_t a0 = word_addr<VEC>(g, i, c);
+    W more = {};
+    if (RELU == kSum) more = __builtin_nontemporal_load(reinterpret_cast<const W *>(r) + a0);
     const W z = axpb(__builtin_nontemporal_load(xw + a0), a, b);
-    __builtin_nontemporal_store(RELU == kFused ? relu_w(z) : z, yw + a0);
+    __builtin_nontemporal_store(output_of<RELU>(z, more), yw + a0);
     if (RELU == kBoth) __builtin_nontemporal_store(relu_w(z), reinterpret_cast<W *>(r) + a0);
   }
 }
@@ -279,8 +292,10 @@ __global__ __launch_bounds__(kThreads) void bn_apply_plane_kernel(const f32x4 *_
   if (i >= g.words) return;
   const uint32_t c = word_channel(g, i);
   const float a = coef[2 * c], b = coef[2 * c + 1];
+  f32x4 more = {};
+  if (RELU == kSum) more = __builtin_nontemporal_load(r + i);
   const f32x4 z = axpb(__builtin_nontemporal_load(x + i), a, b);
-  __builtin_nontemporal_store(RELU == kFused ? relu_w(z) : z, y + i);
+  __builtin_nontemporal_store(output_of<RELU>(z, more), y + i);
   if (RELU == kBoth) __builtin_nontemporal_store(relu_w(z), r + i);
 }
 
@@ -308,19 +323,20 @@ __global__ __launch_bounds__(kThreads) void bn_apply_edges_kernel(const float *_
   const float a = coef[2 * w.c], b = coef[2 * w.c + 1];
   if (e + 4 <= g.words) {
     const f32x4 v = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(x + e));
-    f32x4 z = axpb(v, a, b);
+    f32x4 z = axpb(v, a, b), more = {};
+    if (RELU == kSum) more = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(r + e));
     if (w.left < 4) {
       const float a1 = coef[2 * w.next], b1 = coef[2 * w.next + 1];
 #pragma unroll
       for (uint32_t i = 1; i < 4; ++i)
         if (i >= w.left) z[i] = axpb(v[i], a1, b1);
     }
-    __builtin_nontemporal_store(RELU == kFused ? relu_w(z) : z, reinterpret_cast<f32x4 *>(y + e));
+    __builtin_nontemporal_store(output_of<RELU>(z, more), reinterpret_cast<f32x4 *>(y + e));
     if (RELU == kBoth) __builtin_nontemporal_store(relu_w(z), reinterpret_cast<f32x4 *>(r + e));
   } else {   // the array's last values: of one plane
     for (uint32_t i = e; i < g.words; ++i) {
       const float z = axpb(x[i], a, b);
-      y[i] = RELU == kFused ? relu_w(z) : z;
+      y[i] = output_of<RELU>(z, RELU == kSum ? r[i] : 0.f);
       if (RELU == kBoth) r[i] = relu_w(z);
     }
   }
@@ -696,6 +712,10 @@ __global__ __launch_bounds__(W *kWave) void bn_fwd_onepass_kernel(const float *_
         return d;
       },
       [&](int, const float (&u)[1]) { q[0] += u[0]; });
+  f32x4 more[RELU == kSum ? R : 1];
+  if (RELU == kSum)
+#pragma unroll
+    for (int r = 0; r < R; ++r) more[r] = rows.load(rl, r);
   totals(q, sm + 1, total);
   double var = total[0] * inv_m;
   // (x - float(mean)) leaves out mean - float(mean): var = E[(x - mf)^2] - (mean - mf)^2
@@ -705,15 +725,15 @@ __global__ __launch_bounds__(W *kWave) void bn_fwd_onepass_kernel(const float *_
   if (threadIdx.x == 0) {
     double istd = 1.0 / sqrt(var + static_cast<double>(eps));
     double mean_used = mean;
-    if (RELU == kFused && !wide) {      // as in bn_coef_kernel: coefficients from the rounded statistics the backward pass will read
+    if (fused_of(RELU) && !wide) {      // as in bn_coef_kernel: coefficients from the rounded statistics the backward pass will read
       mean_used = static_cast<double>(static_cast<float>(mean));
       istd = static_cast<double>(static_cast<float>(istd));
     }
     const double a = static_cast<double>(gamma[c]) * istd;
     coef[0] = static_cast<float>(a);
     coef[1] = static_cast<float>(static_cast<double>(beta[c]) - mean_used * a);
-    if (save_mean) save_stat(save_mean, c, RELU == kFused && wide, mean);
-    if (save_istd) save_stat(save_istd, c, RELU == kFused && wide, istd);
+    if (save_mean) save_stat(save_mean, c, fused_of(RELU) && wide, mean);
+    if (save_istd) save_stat(save_istd, c, fused_of(RELU) && wide, istd);
   }
   __syncthreads();
   const float a = coef[0], b = coef[1];
@@ -721,7 +741,7 @@ __global__ __launch_bounds__(W *kWave) void bn_fwd_onepass_kernel(const float *_
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const f32x4 z = axpb(v[r], a, b);
-    rows.store(y, r, RELU == kFused ? relu_w(z) : z);
+    rows.store(y, r, output_of<RELU>(z, more[RELU == kSum ? r : 0]));
     if (RELU == kBoth) rows.store(rl, r, relu_w(z));
   }
 }
@@ -1177,8 +1197,8 @@ static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t par
   const double inv_m = 1.0 / static_cast<double>(ap.m);
   float *sm = save_mean_arr ? mf(save_mean_arr) : nullptr;
   float *sv = save_var_arr ? mf(save_var_arr) : nullptr;
-  const bool wide = relu == kFused && wide_stats(save_mean_arr, C);
-  if (relu == kFused)
+  const bool wide = fused_of(relu) && wide_stats(save_mean_arr, C);
+  if (fused_of(relu))
     hipLaunchKernelGGL(bn_coef_kernel<true>, dim3(C), dim3(kThreads), 0, s, part, S, part_c, part_k, cf(scale), cf(bias),
                        eps, inv_m, coef, sm, sv, wide);
   else
@@ -1189,19 +1209,19 @@ static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t par
   if (plane_major_ok(ap, x, pg, blocks)) {
     const f32x4 *xw = reinterpret_cast<const f32x4 *>(x->data);
     f32x4 *yw = reinterpret_cast<f32x4 *>(y->data), *rw = reinterpret_cast<f32x4 *>(r);
-    const auto kernel = relu == kBoth ? bn_apply_plane_kernel<kBoth> : relu == kFused ? bn_apply_plane_kernel<kFused> : bn_apply_plane_kernel<kAlone>;
+    const auto kernel = relu == kBoth ? bn_apply_plane_kernel<kBoth> : relu == kSum ? bn_apply_plane_kernel<kSum> : relu == kFused ? bn_apply_plane_kernel<kFused> : bn_apply_plane_kernel<kAlone>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, xw, yw, rw, coef, pg);
     return;
   }
   if (edges_ok(ap, x, aligned16(x->data) && aligned16(y->data) && aligned16(r), pg, blocks)) {
-    const auto kernel = relu == kBoth ? bn_apply_edges_kernel<kBoth> : relu == kFused ? bn_apply_edges_kernel<kFused> : bn_apply_edges_kernel<kAlone>;
+    const auto kernel = relu == kBoth ? bn_apply_edges_kernel<kBoth> : relu == kSum ? bn_apply_edges_kernel<kSum> : relu == kFused ? bn_apply_edges_kernel<kFused> : bn_apply_edges_kernel<kAlone>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), pg);
     return;
   }
   const dim3 ga(ap.S, C);
 #define BN_APPLY(V)                                                                                                                        \
-  hipLaunchKernelGGL((relu == kBoth ? bn_apply_kernel<V, kBoth> : relu == kFused ? bn_apply_kernel<V, kFused> : bn_apply_kernel<V, kAlone>), \
-                     ga, dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), ap.g)
+  hipLaunchKernelGGL((relu == kBoth ? bn_apply_kernel<V, kBoth> : relu == kSum ? bn_apply_kernel<V, kSum>                                  \
+                                    : relu == kFused ? bn_apply_kernel<V, kFused> : bn_apply_kernel<V, kAlone>), ga, dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), ap.g)
   if (ap.vec == 4)
     BN_APPLY(4);
   else
@@ -1221,9 +1241,10 @@ static int bn_forward(const char *who, int relu, const DLArrayHandle input_X, co
   TS_REQUIRE(relu != kBoth || (relu_R && pair_arr && numel(relu_R) == numel(input_X) && numel(pair_arr) == 2 * C &&
                                relu_R->data != output_Y->data && relu_R->data != input_X->data),
              "%s: Relu's result is another array of the input's size, the pair's coefficients take 2 C elements", who);
-  float *const r = relu == kBoth ? mf(relu_R) : nullptr, *const pair = relu == kBoth ? mf(pair_arr) : nullptr;
-  TS_REQUIRE(stats_fit(save_mean_arr, save_var_arr, C, relu == kFused), "%s: save_mean and save_var must hold C elements each", who);
-  TS_REQUIRE(relu != kFused || (save_mean_arr && save_var_arr), "%s: the fused form needs both save arrays", who);
+  TS_REQUIRE(relu != kSum || (relu_R && numel(relu_R) == numel(input_X) && relu_R->data != output_Y->data), "%s: the addend is another array of the input's size", who);
+  float *const r = relu == kBoth || relu == kSum ? mf(relu_R) : nullptr, *const pair = relu == kBoth ? mf(pair_arr) : nullptr;
+  TS_REQUIRE(stats_fit(save_mean_arr, save_var_arr, C, fused_of(relu)), "%s: save_mean and save_var must hold C elements each", who);
+  TS_REQUIRE(!fused_of(relu) || (save_mean_arr && save_var_arr), "%s: the fused form needs both save arrays", who);
   // sums a convolution left for exactly this tensor on this stream (common.h): looked up before
   // stream_of() ends all notes, since this call writes too
   const double *note_sums = nullptr;
@@ -1254,9 +1275,11 @@ static int bn_forward(const char *who, int relu, const DLArrayHandle input_X, co
 #define BN_FWD1(W, R, LAYOUT, RL)                                                                                                          \
   hipLaunchKernelGGL((bn_fwd_onepass_kernel<W, R, LAYOUT, RL>), dim3(static_cast<unsigned>(C)), dim3(W * kWave), 0, s, cf(input_X),          \
                      mf(output_Y), cf(bn_scale), cf(bn_bias), FastDiv(hw), static_cast<int>(C), m, eps, 1.0 / static_cast<double>(m), sm1, \
-                     sv1, relu == kFused && wide_stats(save_mean_arr, C), r, pair)
+                     sv1, fused_of(relu) && wide_stats(save_mean_arr, C), r, pair)
     if (relu == kBoth)
       BN_ONEPASS(BN_FWD1, kBoth);
+    else if (relu == kSum)
+      BN_ONEPASS(BN_FWD1, kSum);
     else if (relu == kFused)
       BN_ONEPASS(BN_FWD1, kFused);
     else
@@ -1298,6 +1321,12 @@ int TSplit_BatchNormRelu(const DLArrayHandle input_X, const DLArrayHandle bn_sca
                          DLStreamHandle stream_handle, ProfilerHandle p) {
   return bn_forward("TSplit_BatchNormRelu", kFused, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr,
                     save_var_arr, stream_handle, p);
+}
+
+int TSplit_BatchNormReluAdd(const DLArrayHandle input_X, const DLArrayHandle bn_scale, const DLArrayHandle bn_bias, const DLArrayHandle addend,
+                            DLArrayHandle output_Y, float eps, DLArrayHandle save_mean_arr, DLArrayHandle save_var_arr, DLStreamHandle stream_handle) {
+  return bn_forward("TSplit_BatchNormReluAdd", kSum, input_X, bn_scale, bn_bias, output_Y, eps, save_mean_arr, save_var_arr, stream_handle,
+                    nullptr, addend);
 }
 
 // BatchNorm (relu == 0) or BatchNorm + Relu (relu != 0) forward whose batch statistics come from sums a

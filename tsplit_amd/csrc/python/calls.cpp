@@ -387,7 +387,7 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   X(DLGpuAvgerage_Pooling2d, 0) X(DLGpuAvgerage_Pooling2d_gradient, 0) X(CuDNN_DLGpuAvgerage_Pooling2d, 0)                                     \
   X(CuDNN_DLGpuAvgerage_Pooling2d_gradient, 0) X(DLGpuBroadcastTo, 0) X(DLGpuReduceSumAxisZero, 0) X(DLGpuConv2d_broadcast_to, 0)              \
   X(DLGpuConv2d_reduce_sum, 0) X(DLGpuBatchMatrixMultiply, 0) X(DLGpuOneHot, 0) X(DLGpuWhere, 0) X(DLGpuEmbeddingLookUp, 0)                    \
-  X(DLGpuEmbeddingLookUp_Gradient, 0) X(DLGpuTanh, 0) X(DLGpuSigmoid, 0) X(TSplit_BatchNormRelu, 0)                                            \
+  X(DLGpuEmbeddingLookUp_Gradient, 0) X(DLGpuTanh, 0) X(DLGpuSigmoid, 0) X(TSplit_BatchNormRelu, 0) X(TSplit_BatchNormReluAdd, 0)                                            \
   X(TSplit_BatchNormThenRelu, 1 << 7 | 1 << 8) X(TSplit_BatchNormThenRelu_gradient, 1 << 9 | 1 << 10) X(TSplit_Conv2dBatchNormStats, 0)        \
   X(TSplit_BatchNormFromStats, 1 << 7 | 1 << 8) X(TSplit_BatchNormRelu_gradient, 0) X(DLGpuConcat, 0) X(DLGpuConcat_gradient, 0)
 

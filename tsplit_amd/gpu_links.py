@@ -28,7 +28,7 @@ __all__ = [
     "matrix_transpose", "batch_matrix_multiply", "one_hot", "where", "embedding_lookup",
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
-    "batch_norm_relu", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
+    "batch_norm_relu", "batch_norm_relu_add", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
     "optimizer_update_multi", "conv2d_gradient_of_data_add", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply", "heads_scale",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "join", "part", "lstm_sizes", "lstm", "lstm_gradient",
@@ -517,6 +517,11 @@ def winograd_gemm_times(filter_gradient=False, kind=None):
 def batch_norm_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var, eps=0.01, stream=None,
                     profiler=None):
     _calls.TSplit_BatchNormRelu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, eps, save_mean, save_var, stream, profiler)
+
+
+def batch_norm_relu_add(in_arr, bn_scale_arr, bn_bias_arr, addend, out_arr, save_mean, save_var, eps=0.01, stream=None):
+    """out_arr = batch_norm_relu's + addend (another array), with the bits of the two calls."""
+    _calls.TSplit_BatchNormReluAdd(in_arr, bn_scale_arr, bn_bias_arr, addend, out_arr, eps, save_mean, save_var, stream)
 
 
 def batch_norm_then_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, relu_arr, pair, save_mean=None, save_var=None, eps=0.01, stream=None,

@@ -183,6 +183,13 @@ class GpuBackend(object):
         self.L.batch_norm_relu(x, gamma, beta, y, mean, istd, eps, stream=self.stream)
         return y, mean, istd
 
+    def bn_relu_add(self, x, gamma, beta, addend, xs, eps, exact=False):
+        """bn_relu with relu(bn(x)) + addend in the place of relu(bn(x))."""
+        saved = (xs[1], 2) if exact else (1, xs[1], 1, 1)
+        y, mean, istd = self.empty(xs), self.empty(saved), self.empty(saved)
+        self.L.batch_norm_relu_add(x, gamma, beta, addend, y, mean, istd, eps, stream=self.stream)
+        return y, mean, istd
+
     def bn_relu_grad(self, dy, x, gamma, beta, mean, istd, xs, eps):
         dx, dg, db = self.empty(xs), self.empty((1, xs[1], 1, 1)), self.empty((1, xs[1], 1, 1))
         self.L.batch_norm_relu_gradient(dy, x, gamma, beta, dx, dg, db, mean, istd, eps, stream=self.stream)
@@ -592,26 +599,40 @@ class Tape(object):
         return self._out(fwd(), x.shape, [x, gamma, beta], back, saved=[x, gamma], redo=fwd)
 
     @_op
-    def batch_norm_relu(self, x, gamma, beta, eps=0.01, exact=False):
+    def batch_norm_relu(self, x, gamma, beta, eps=0.01, exact=False, residual=None):
         """BatchNorm and the Relu behind it as one node (TSplit_BatchNormRelu / _gradient; the reference's graph
         has two nodes, gpu_ops/BatchNorm.py and gpu_ops/Relu.py): the BatchNorm output is never written, and
         the gradient reads the BatchNorm's input, the parameters and the two saved statistics vectors.
-        exact (device backends): with the bits of the two nodes."""
+        exact (device backends): with the bits of the two nodes.  residual (likewise, and not on a tape that accounts for every
+        value): a Var that is added behind the Relu."""
         stats, form = [None, None], {"exact": True} if exact else {}
 
         def fwd():
-            r = self.b.bn_relu(x.value, gamma.value, beta.value, x.shape, eps, **form)
+            if residual is not None:
+                r = self.b.bn_relu_add(x.value, gamma.value, beta.value, residual.value, x.shape, eps, **form)
+            else:
+                r = self.b.bn_relu(x.value, gamma.value, beta.value, x.shape, eps, **form)
             if r is None:                      # a backend that only records shapes
                 return None
             y, stats[0], stats[1] = r
             return y
 
         def back(g):
+            if residual is not None:
+                self._acc(residual, g)
             dx, dg, db = self.b.bn_relu_grad(g, x.value, gamma.value, beta.value, stats[0], stats[1], x.shape, eps)
             self._acc(x, dx)
             self._acc(gamma, dg)
             self._acc(beta, db)
-        return self._out(fwd(), x.shape, [x, gamma, beta], back, saved=[x, gamma, beta], redo=fwd)
+        inputs = [x, gamma, beta] + ([] if residual is None else [residual])
+        return self._out(fwd(), x.shape, inputs, back, saved=[x, gamma, beta], redo=fwd)
+
+    def bn_relu_then_add(self, x, gamma, beta, residual, eps=0.01):
+        """bn_then_relu and the sum with `residual` behind it; where that is one node, the sum is part of it."""
+        if self._ahead and self._can("bn_relu_add") and (self.fuse_bn_relu or getattr(type(self.b), "fuses_pairs", False)):
+            assert residual.shape == x.shape, (residual.shape, x.shape)
+            return self.batch_norm_relu(x, gamma, beta, eps, not self.fuse_bn_relu, residual)
+        return self.add(self.bn_then_relu(x, gamma, beta, eps), residual)
 
     def bn_then_relu(self, x, gamma, beta, eps=0.01):
         """The pair as the reference's graph has it (two nodes), or as one node: when the tape was asked to fuse, and on the device

@@ -111,9 +111,10 @@ class ShapeBinder(Binder):
 
 
 # ------------------------------------------------------------------ ResNet (bottleneck)
-def _bn_relu(t, b, x, name, eps):
+def _bn_relu(t, b, x, name, eps, residual=None):
     c = x.shape[1]
-    return t.bn_then_relu(x, b.get(name + "_scale", (1, c, 1, 1), "one"), b.get(name + "_bias", (1, c, 1, 1), "zero"), eps)
+    scale, bias = b.get(name + "_scale", (1, c, 1, 1), "one"), b.get(name + "_bias", (1, c, 1, 1), "zero")
+    return t.bn_then_relu(x, scale, bias, eps) if residual is None else t.bn_relu_then_add(x, scale, bias, residual, eps)
 
 
 def _conv(t, b, x, cout, k, stride, pad, name):
@@ -128,14 +129,12 @@ def _bottleneck_stage(t, b, x, cout, num_blocks, first, name, eps):
     identity = _bn_relu(t, b, _conv(t, b, x, cout, 1, s, 0, name + "_conv0"), name + "_bn0", eps)
     x = _bn_relu(t, b, _conv(t, b, x, mid, 1, 1, 0, name + "_conv1"), name + "_bn1", eps)
     x = _bn_relu(t, b, _conv(t, b, x, mid, 3, s, 1, name + "_conv2"), name + "_bn2", eps)
-    x = _bn_relu(t, b, _conv(t, b, x, cout, 1, 1, 0, name + "_conv3"), name + "_bn3", eps)
-    x = t.add(x, identity)
+    x = _bn_relu(t, b, _conv(t, b, x, cout, 1, 1, 0, name + "_conv3"), name + "_bn3", eps, identity)
     for i in range(1, num_blocks):
         identity = x
         x = _bn_relu(t, b, _conv(t, b, x, mid, 1, 1, 0, name + "_conv%d" % (3 * i + 1)), name + "_bn%d" % (3 * i + 1), eps)
         x = _bn_relu(t, b, _conv(t, b, x, mid, 3, 1, 1, name + "_conv%d" % (3 * i + 2)), name + "_bn%d" % (3 * i + 2), eps)
-        x = _bn_relu(t, b, _conv(t, b, x, cout, 1, 1, 0, name + "_conv%d" % (3 * i + 3)), name + "_bn%d" % (3 * i + 3), eps)
-        x = t.add(x, identity)
+        x = _bn_relu(t, b, _conv(t, b, x, cout, 1, 1, 0, name + "_conv%d" % (3 * i + 3)), name + "_bn%d" % (3 * i + 3), eps, identity)
     return x
 
 
