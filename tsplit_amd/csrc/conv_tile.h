@@ -262,6 +262,46 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
     if (j == 0) together = together && 2 * (static_cast<int>(c) + TN) <= P.out_w;
   }
   const bool words = __all(together || n >= F.N), ragged = m + 16 * TM > P.M;
+  if (words) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      float v[4][TN / 2][2][4];   // of four rows at a time: a pair of columns' words, this row of positions' and the next one's
+      auto place = [&](int e, int j, int below_it, unsigned &o, int &soff) {
+        const int row = step_row(tm, e);
+        const bool past = ragged && m + row + lane_row >= P.M;
+        soff = past ? 0 : row * plane_bytes;   // (past M the product may leave 32 bits)
+        o = past || (below_it && !below[j]) ? kOobOffset : off[j] + (below_it ? down : 0u);
+      };
+      unsigned o;
+      int soff;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < TN; j += 2)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            float(&w)[4] = v[e][j / 2][u];
+            w[0] = w[1] = w[2] = w[3] = 0.f;
+            place(e, j, u, o, soff);
+            if constexpr (ADD) gt::load_words<4>(from, o, soff, w);
+          }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int j = 0; j < TN; j += 2)
+#pragma unroll
+          for (int u = 0; u < 2; ++u) {
+            float(&w)[4] = v[e][j / 2][u];
+            if (u == 0) {
+              w[0] = ADD ? w[0] + acc[tm][j][e] : acc[tm][j][e];
+              w[2] = ADD ? w[2] + acc[tm][j + 1][e] : acc[tm][j + 1][e];
+            }
+            place(e, j, u, o, soff);
+            gt::store_words<4>(to, o, soff, w);
+          }
+    }
+    return;
+  }
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
@@ -269,35 +309,25 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
       const int row = step_row(tm, e);
       const bool past = ragged && m + row + lane_row >= P.M;
       const int soff = past ? 0 : row * plane_bytes;   // (past M the product may leave 32 bits)
-      if (words) {
+      unsigned o[TN][4];
+      float v[TN][4] = {};
 #pragma unroll
-        for (int j = 0; j < TN; j += 2) {
-          const unsigned o = past ? kOobOffset : off[j], under = past || !below[j] ? kOobOffset : off[j] + down;
-          float v[4] = {0.f, 0.f, 0.f, 0.f}, w[4] = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (ADD) {
-            gt::load_words<4>(from, o, soff, v);
-            gt::load_words<4>(from, under, soff, w);
-          }
-          v[0] = ADD ? v[0] + acc[tm][j][e] : acc[tm][j][e];
-          v[2] = ADD ? v[2] + acc[tm][j + 1][e] : acc[tm][j + 1][e];
-          gt::store_words<4>(to, o, soff, v);
-          gt::store_words<4>(to, under, soff, w);
+      for (int j = 0; j < TN; ++j) {
+        const bool none = past || off[j] == kOobOffset;
+        o[j][0] = none ? kOobOffset : off[j];
+        o[j][1] = none || !beside[j] ? kOobOffset : off[j] + 4u;
+        o[j][2] = none || !below[j] ? kOobOffset : off[j] + down;
+        o[j][3] = none || !below[j] || !beside[j] ? kOobOffset : off[j] + down + 4u;
+        if constexpr (ADD) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[j][i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, o[j][i] + soff, 0, 0));
         }
-      } else {
+      }
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const bool none = past || off[j] == kOobOffset;
-          const unsigned o[4] = {none ? kOobOffset : off[j], none || !beside[j] ? kOobOffset : off[j] + 4u, none || !below[j] ? kOobOffset : off[j] + down,
-                                 none || !below[j] || !beside[j] ? kOobOffset : off[j] + down + 4u};
-          float v[4] = {0.f, 0.f, 0.f, 0.f};
-          if constexpr (ADD) {
+      for (int j = 0; j < TN; ++j) {
+        v[j][0] = ADD ? v[j][0] + acc[tm][j][e] : acc[tm][j][e];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, o[i] + soff, 0, 0));
-          }
-          v[0] = ADD ? v[0] + acc[tm][j][e] : acc[tm][j][e];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[i]), to, o[i] + soff, 0, 0);
-        }
+        for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j][i]), to, o[j][i] + soff, 0, 0);
       }
     }
 }
@@ -345,6 +375,31 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
   const bool words = __all(together || n >= F.N);
   auto store = [&](auto ragged, auto in_words) {   // ragged: the wave's rows run past M
     constexpr bool kRagged = decltype(ragged)::value;
+    // ADD: all of it is asked for before the first store, which the compiler would keep behind the loads above it alone
+    // (1024 channels of 17 x 17: one at a time 50-63 us, without ADD 29)
+    if constexpr (ADD) {
+      float more[TM][4][TN];
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int row = C::step_row(tm, e);
+          const bool past = kRagged && m + row + C::lane_row() >= P.M;
+          const int soff = past ? 0 : row * plane_bytes;
+          if constexpr (decltype(in_words)::value) {
+            gt::load_words<TN>(from, past ? kOobOffset : off[0], soff, more[tm][e]);
+          } else {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) more[tm][e][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, (past ? kOobOffset : off[j]) + soff, 0, 0));
+          }
+        }
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int j = 0; j < TN; ++j) acc[tm][j][e] = more[tm][e][j] + acc[tm][j][e];
+    }
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
@@ -353,20 +408,13 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
         const bool past = kRagged && m + row + C::lane_row() >= P.M;
         const int soff = past ? 0 : row * plane_bytes;   // (past M the product may leave 32 bits)
         if constexpr (decltype(in_words)::value) {
-          float v[TN], more[TN] = {};
-          if constexpr (ADD) gt::load_words<TN>(from, past ? kOobOffset : off[0], soff, more);
-#pragma unroll
-          for (int j = 0; j < TN; ++j) v[j] = ADD ? more[j] + acc[tm][j][e] : acc[tm][j][e];
-          gt::store_words<TN>(to, past ? kOobOffset : off[0], soff, v);
-        } else {
           float v[TN];
 #pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            v[j] = acc[tm][j][e];
-            if constexpr (ADD) v[j] += __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, (past ? kOobOffset : off[j]) + soff, 0, 0));
-          }
+          for (int j = 0; j < TN; ++j) v[j] = acc[tm][j][e];
+          gt::store_words<TN>(to, past ? kOobOffset : off[0], soff, v);
+        } else {
 #pragma unroll
-          for (int j = 0; j < TN; ++j) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j]), to, (past ? kOobOffset : off[j]) + (kRagged ? soff : 0), kRagged ? 0 : soff, 0);
+          for (int j = 0; j < TN; ++j) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[tm][j][e]), to, (past ? kOobOffset : off[j]) + (kRagged ? soff : 0), kRagged ? 0 : soff, 0);
         }
       }
   };
