@@ -68,6 +68,7 @@ template <int BN, int T, bool BWD, int TAPS, bool BLOCKS>
 struct Gathered {
   static constexpr bool kDense = false;
   static constexpr int kFloats = BK * BN, H = BN / 64;
+  static constexpr int kParts = TAPS && BLOCKS ? 4 : 1;   // in which a step's loads may be asked for: prepare() and part(0) to part(3), or load()
   using Mask = typename std::conditional<(TAPS > 32), uint64_t, uint32_t>::type;
   unsigned voff[H];
   Mask inside[H];
@@ -110,12 +111,13 @@ struct Gathered {
     const int u = kw.div(tap), v = tap - u * kw.d, at = u * src_w + v;
     return BWD ? bias - at : at;
   }
-  __device__ __forceinline__ void load(int k0, int kend, unsigned lds) const {
-    lds += 8 * wave * BN * 4;
-    if constexpr (BLOCKS || !TAPS) {
+  unsigned at[H], to;
+  int soff, have;
+  __device__ __forceinline__ void prepare(int k0, int kend, unsigned lds) {
+    to = lds + 8 * wave * BN * 4;
+    {
       const int k = k0 + 8 * wave;
-      int ch = k, soff;
-      unsigned at[H];
+      int ch = k;
       if (TAPS) {
         const int block = k >> 3, cb = taps.div(block), tap = block - cb * taps.d;
         ch = 8 * cb;
@@ -127,12 +129,22 @@ struct Gathered {
 #pragma unroll
         for (int h = 0; h < H; ++h) at[h] = voff[h];
       }
-      const int have = k < kend ? chans - ch : 0;   // channels of this block
+      have = k < kend ? chans - ch : 0;   // channels of this block
+    }
+  }
+  __device__ __forceinline__ void part(int i) const {
 #pragma unroll
-      for (int r = 0; r < 8; ++r, soff += plane)
+    for (int r = 2 * i; r < 2 * i + 2; ++r)
 #pragma unroll
-        for (int h = 0; h < H; ++h) gt::load_word_to_lds(rsrc, at[h], r < have ? soff : nowhere, lds + (r * BN + 64 * h) * 4);
+      for (int h = 0; h < H; ++h) gt::load_word_to_lds(rsrc, at[h], r < have ? soff + r * plane : nowhere, to + (r * BN + 64 * h) * 4);
+  }
+  __device__ __forceinline__ void load(int k0, int kend, unsigned lds) {
+    if constexpr (BLOCKS || !TAPS) {
+      prepare(k0, kend, lds);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part(i);
     } else {
+      lds += 8 * wave * BN * 4;
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
         const int k = k0 + 8 * wave + r, ch = taps.div(k), tap = k - ch * taps.d;
@@ -154,6 +166,7 @@ struct Gathered {
 template <int BN, int T>
 struct Pointwise {
   static constexpr bool kDense = false;
+  static constexpr int kParts = 1;
   static constexpr int kFloats = BK * BN;
   static constexpr int kLoads = BN / 32, kWords = BN / 4, kRows = 64 / kWords;
   unsigned voff;
@@ -194,13 +207,14 @@ struct Pointwise {
 enum Gather { kWords, kOneTap, kBlocks32, kBlocks64, kTaps64 };
 
 // ACROSS: A is the filter in memory, [depth][M] (data gradient of one tap); else [M][depth]
-template <int TM, int TN, bool BWD, int GATHER, bool ACROSS>
+template <int TM, int TN, bool BWD, int GATHER, bool ACROSS, bool PAIR = false>
 struct Pass {
   static constexpr int BM = 32 * TM, BN = 32 * TN;
   using BL = typename std::conditional<GATHER == kWords, Pointwise<BN, TN>,
                                        Gathered<BN, TN, BWD, GATHER == kOneTap ? 0 : GATHER == kBlocks32 ? 32 : 64, GATHER != kTaps64>>::type;
   using AL = typename std::conditional<ACROSS, gt::MnContig<BM, TM>, gt::KContig<BM, TM, false>>::type;
-  using C = gt::Core<TM, TN, 2, 2, AL, BL>;
+  // (a pair's 128 x 128 tiles have no registers left for loads between products)
+  using C = gt::Core<TM, TN, 2, 2, AL, BL, (BL::kParts > 1 && !(PAIR && TM * TN == 16))>;
 
   static __device__ __forceinline__ void run(const Params &P, const Phase &F, int m0, int n0, int z, float *lds, f32x4 (&acc)[TM][TN]) {
     AL la;
@@ -456,7 +470,7 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
 // Data gradient of stride 2: phases 2 q and 2 q + 1 are the even and the odd columns of the same rows of positions.
 template <int TM, int TN>
 __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_pair_kernel(Params P, int total) {
-  using X = Pass<TM, TN, true, kBlocks32, false>;
+  using X = Pass<TM, TN, true, kBlocks32, false, true>;
   using C = typename X::C;
   __shared__ __attribute__((aligned(1024))) float lds[C::kLdsFloats];
   int z, ip, tile_m, tile_n;

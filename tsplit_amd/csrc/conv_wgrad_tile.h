@@ -64,6 +64,7 @@ __device__ __forceinline__ i32x4 from_image(const float *p, int64_t bytes, int i
 template <int MN, int T>
 struct Words {
   static constexpr bool kDense = false, kDealt = false;
+  static constexpr int kParts = 1;
   static constexpr int kGroup = 272, kLoads = MN / 32, kFloats = MN / 8 * kGroup;
   i32x4 rsrc;
   FastDiv image;
@@ -128,6 +129,7 @@ struct Words {
 template <int BN, int T, int G>
 struct Taps {
   static constexpr bool kDense = false;
+  static constexpr int kParts = 4;
   static constexpr int kPair = 68, kGroups = BN / 4 / G, kFloats = BN / 2 * kPair;   // a wave's groups
   i32x4 rsrc;
   FastDiv image, width;
@@ -175,16 +177,15 @@ struct Taps {
     at = static_cast<unsigned>((img - img0) * img_values + static_cast<int>(threadIdx.x >> 5 & 1) * x_plane + row * x_w + col) * 4u;
   }
   // steps come in order
-  __device__ __forceinline__ void load(int k0, int kend, unsigned lds) {
+  unsigned from[kGroups], to;
+  __device__ __forceinline__ void prepare(int k0, int kend, unsigned lds) {
     const bool ok = k0 + static_cast<int>(threadIdx.x & 31) < kend && pos < plane;
-    lds += wave * kGroups * (G / 2) * kPair * 4;
+    to = lds + wave * kGroups * (G / 2) * kPair * 4;
 #pragma unroll
     for (int g = 0; g < kGroups; ++g) {
       const bool in = ok && static_cast<unsigned>(row + down[g]) < static_cast<unsigned>(x_h) &&
                       static_cast<unsigned>(col + right[g]) < static_cast<unsigned>(x_w);
-      const unsigned from = in ? at + shift[g] : kOobOffset;
-#pragma unroll
-      for (int j = 0; j < G / 2; ++j) gt::load_word_to_lds(rsrc, from, chan_at[g] + 2 * j * x_plane * 4, lds + (G / 2 * g + j) * kPair * 4);
+      from[g] = in ? at + shift[g] : kOobOffset;
     }
     pos += BK;
     row += row_step;
@@ -196,6 +197,17 @@ struct Taps {
       at += at_wrap;
     }
     if (pos >= static_cast<int>(image.d)) place(k0 + BK + (threadIdx.x & 31));
+  }
+  __device__ __forceinline__ void part(int i) const {
+    constexpr int kLoads = kGroups * (G / 2);
+#pragma unroll
+    for (int l = kLoads / 4 * i; l < kLoads / 4 * (i + 1); ++l)
+      gt::load_word_to_lds(rsrc, from[l / (G / 2)], chan_at[l / (G / 2)] + 2 * (l % (G / 2)) * x_plane * 4, to + l * kPair * 4);
+  }
+  __device__ __forceinline__ void load(int k0, int kend, unsigned lds) {
+    prepare(k0, kend, lds);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) part(i);
   }
   __device__ __forceinline__ bool cut(int, int) const { return false; }
   __device__ __forceinline__ void clear_tail(int, int, float *) const {}

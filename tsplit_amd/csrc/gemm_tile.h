@@ -72,6 +72,7 @@ __device__ __forceinline__ void lds_ready() {
 template <int MN, int T, bool PERM>
 struct KContig {
   static constexpr bool kDense = true;
+  static constexpr int kParts = 1;
   static constexpr bool kDealt = PERM;   // tile t's lane r supplies index T r + t, not 16 t + r
   static constexpr int kFloats = MN * BK;
   static constexpr int kLoads = MN / 32;   // a wave's loads a step, 8 rows each
@@ -143,6 +144,7 @@ struct KContig {
 template <int MN, int T>
 struct MnContig {
   static constexpr bool kDense = true, kDealt = true;
+  static constexpr int kParts = 1;
   static constexpr int kFloats = BK * MN;
   static constexpr int kLoads = MN / 32;
   static constexpr int kWords = MN / 4;            // 16-byte words of a row
@@ -187,6 +189,20 @@ __device__ __forceinline__ void products(const float (&a)[TM][4], const float (&
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tm][i], b[tn][i], acc[tm][tn], 0, 0, 0);
 }
+// the same with between(i) behind each quarter
+template <int TM, int TN, class Between>
+__device__ __forceinline__ void products_and(const float (&a)[TM][4], const float (&b)[TN][4], f32x4 (&acc)[TM][TN], Between between) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[tm][i], b[tn][i], acc[tm][tn], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    between(i);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
 
 // Output words: T neighbouring columns of a row, at voff + step bytes (kOobOffset: nowhere).  The step is added to the lane's
 // offset and not passed as the scalar offset: with a scalar register there, 16-byte stores whose data registers the next
@@ -217,7 +233,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t output_buffer(float *p, int64_
 }
 
 // The k-loop of one tile with operand loaders AL, BL: acc = sum over [kbegin, kend).
-template <int TM, int TN, int WM, int WN, class AL, class BL>
+template <int TM, int TN, int WM, int WN, class AL, class BL, bool SPREAD = (BL::kParts > 1)>
 struct Core {
   static_assert(WM * WN == 4, "four waves");
   static constexpr int BM = 16 * TM * WM, BN = 16 * TN * WN;
@@ -262,6 +278,54 @@ struct Core {
     la.load(kbegin, kend, lds_at);
     lb.load(kbegin, kend, lds_at + AL::kFloats * 4);
     int stage = 0;
+    if constexpr (SPREAD) {
+      // What is said above of a step, with the next step's loads between the products (see kParts).  The first step has no products to put
+      // them between, the last none to ask for: forms of their own, since a branch between products costs registers.
+      auto step = [&](int k0, auto first, auto more) {
+        if (la.cut(k0, kend) || lb.cut(k0, kend)) {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          la.clear_tail(k0, kend, lds + stage * kStage);
+          lb.clear_tail(k0, kend, lds + stage * kStage + AL::kFloats);
+        }
+        lds_ready();
+        const float *sa = lds + stage * kStage, *sb = sa + AL::kFloats;
+        stage ^= 1;
+        auto part = [&](int i) {
+          if constexpr (decltype(more)::value) {
+            if (i == 0) la.load(k0 + BK, kend, lds_at + stage * kStage * 4);
+            lb.part(i);
+          }
+        };
+        if constexpr (decltype(more)::value) lb.prepare(k0 + BK, kend, lds_at + (stage * kStage + AL::kFloats) * 4);
+        AL::frag(sa, wm0, 0, lane, a0);
+        BL::frag(sb, wn0, 0, lane, b0);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (decltype(first)::value) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) part(i);
+        } else {
+          products_and<TM, TN>(a1, b1, acc, part);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        AL::frag(sa, wm0, 1, lane, a1);
+        BL::frag(sb, wn0, 1, lane, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        products<TM, TN>(a0, b0, acc);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      const std::true_type yes{};
+      const std::false_type no{};
+      int k0 = kbegin;
+      if (k0 + BK >= kend) {
+        step(k0, yes, no);
+      } else {
+        step(k0, yes, yes);
+        for (k0 += BK; k0 + BK < kend; k0 += BK) step(k0, no, yes);
+        step(k0, no, no);
+      }
+      products<TM, TN>(a1, b1, acc);
+      return;
+    }
     for (int k0 = kbegin; k0 < kend; k0 += BK) {
       if (la.cut(k0, kend) || lb.cut(k0, kend)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
