@@ -22,8 +22,8 @@
 // What bounds it is the matrix pipe where the tiles fill the chip (1x1 layers: 64 x 512 x 28 x 28 -> 128 in 62 us, 106 TFLOP/s) and
 // the gathered loads, 4 bytes a lane, elsewhere.  Against 16-deep steps whose operands went through vector registers: 1x1 layers of
 // ResNet-50 66, 62, 76, 76 us (were 90, 87, 90, 90), its first layer 259 (411), 1x7 of 256 -> 256 at 17x17 93 (96), 3x3 of 512 -> 512 at
-// 4x4 71 (79), 3x3 stride 2 of 96 -> 200 channels 17 (32); but 3x3 of 512 -> 512 at 28x28, 18 images, 570 (549), where the loads count
-// most.
+// 4x4 71 (79), 3x3 stride 2 of 96 -> 200 channels 17 (32); 3x3 of 512 -> 512 at 28x28, 18 images, 570 (549), where the loads count
+// most.  With the gathered loads between the products (gt::Core) the last two take 14 and 525.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -282,7 +282,7 @@ struct Core {
       // A step with the next step's loads between the products.  A load takes the memory pipeline 16 clocks whatever its width, and a wave
       // issues in order: 8 to 16 loads of 4 bytes a lane in one burst behind the barrier kept it from its next product until the last
       // was taken.  Two to four behind each quarter of the products: 3x3 of 35 x 35 70.1 -> 63.5 us, 17 x 17 of several taps 69.1 -> 59.5,
-      // 512 -> 512 of 28 x 28, 18 images 559 -> 472, stride-2 data gradients 0.91-0.94 of the time, filter gradients 0.92-0.97.
+      // 512 -> 512 of 28 x 28, 18 images 558 -> 497, its filter gradient 570 -> 525, stride-2 data gradients 0.91-0.94 of the time, filter gradients 0.92-0.97.
       // Operands in words (2 to 8 loads a step) and one-tap gathers, which have no choice of offsets to make, gained nothing either
       // way, nor did the LDS reads between products.  The first step has no products to put loads between, the last none to ask for:
       // forms of their own, since a branch between products costs registers (108 -> 149 on 128 x 64).
