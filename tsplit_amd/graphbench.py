@@ -41,12 +41,14 @@ WORK = {
     "conv2d": lambda x, w, xs, ws, ph, pw, s: ("conv_fwd", 2.0 * xs[0] * ws[0] * ((xs[2] + 2 * ph - ws[2]) // s + 1)
                                                 * ((xs[3] + 2 * pw - ws[3]) // s + 1) * ws[1] * ws[2] * ws[3], "flop"),
     "conv2d_grad_data": lambda w, dy, xs, ph, pw, s: ("conv_bwd_data", 2.0 * _n(dy.shape) * _n(w.shape[1:]), "flop"),
+    "conv2d_grad_data_add": lambda w, dy, xs, ph, pw, s, addend, out=None: ("conv_bwd_data", 2.0 * _n(dy.shape) * _n(w.shape[1:]), "flop"),
     "conv2d_grad_filter": lambda x, dy, ws, ph, pw, s: ("conv_bwd_filter", 2.0 * _n(dy.shape) * _n(ws[1:]), "flop"),
     "matmul": lambda a, ta, b, tb, out: ("matmul", 2.0 * _n(out) * (a.shape[0] if ta else a.shape[1]), "flop"),
     "batch_matmul": lambda a, ta, b, tb, out: ("batch_matmul", 2.0 * _n(out) * (a.shape[-2] if ta else a.shape[-1]), "flop"),
     "bn": lambda x, g, b, xs, eps: ("bn_fwd", 8.0 * _n(xs), "byte"),
     "bn_grad": lambda dy, x, g, xs, eps: ("bn_bwd", 12.0 * _n(xs), "byte"),
-    "bn_relu": lambda x, g, b, xs, eps: ("bn_relu_fwd", 8.0 * _n(xs), "byte"),
+    "bn_relu": lambda x, g, b, xs, eps, exact=False: ("bn_relu_fwd", 8.0 * _n(xs), "byte"),
+    "bn_relu_add": lambda x, g, b, addend, xs, eps, exact=False: ("bn_relu_add_fwd", 12.0 * _n(xs), "byte"),
     "bn_relu_grad": lambda dy, x, g, b, m, i, xs, eps: ("bn_relu_bwd", 12.0 * _n(xs), "byte"),
     "relu": lambda x, shape: ("relu_fwd", 8.0 * _n(shape), "byte"),
     "relu_grad": lambda x, dy, shape: ("relu_bwd", 12.0 * _n(shape), "byte"),
