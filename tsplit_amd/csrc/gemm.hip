@@ -5,8 +5,8 @@
 // operand is simply one whose other index is contiguous); nothing is ever transposed in memory.
 // The tile (128x128, 64x128, 128x64 or 64x64) and the number of ranges K is cut into come from a
 // small model of the chip (tile_plan.h); the ranges' results are added in ascending order by a
-// second kernel.  Small products run on the kernel of gemm_waves.h, in one launch.  The batched form runs every leading index as one more grid dimension of the same
-// kernel.  Operands of 2 GiB and more, and results whose 64 rows reach that far, stay on the engine
+// second kernel.  Small products run on the kernel of gemm_waves.h, in one launch.  The batched form runs every leading index
+// as one more grid dimension of the same kernel.  Operands of 2 GiB and more, and results whose 64 rows reach that far, stay on the engine
 // of mfma_gemm.h, which takes 64-bit addresses, with its own tiles and ranges.
 #include <algorithm>
 
@@ -30,32 +30,30 @@ struct Plan {
   WavesPlan waves;   // with waves: one launch of gemm_waves.h instead, S is 1
 };
 
-Plan best_plan(int M, int N, int K, int batch, bool may_split, bool deep_words) {
+Plan best_plan(int M, int N, int K, int batch, bool may_split) {
   const int64_t cols = N;
   const int steps = std::max(1, (K + gt::BK - 1) / gt::BK);
   const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, kProductCost);
-  const WavesPlan waves = plan_waves(M, N, K, batch, deep_words, t.us);
-  if (waves.waves) return {0, 1, K, waves};
+  const WavesPlan waves = plan_waves(M, N, K, batch, t);
+  if (waves.waves) return {0, 1, waves.kchunk, waves};
   Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK, waves};
   p.S = std::max(1, (K + p.kchunk - 1) / p.kchunk);
   if (p.S == 1) p.kchunk = K;
   return p;
 }
 
-// the plans of the shapes this thread asked for last (working one out takes about 2 us of host time); deep_words: K is contiguous in
-// both operands
-Plan plan_product(int M, int N, int K, int batch, bool may_split, bool deep_words) {
+// the plans of the shapes this thread asked for last (working one out takes about 2 us of host time)
+Plan plan_product(int M, int N, int K, int batch, bool may_split) {
   struct Entry {
     int M, N, K, batch;
-    bool may_split, deep_words;
+    bool may_split;
     Plan plan;
   };
   static thread_local Entry known[256] = {};
   // (multiplied through: sums of small multiples put every shape of a net of power-of-two sizes into two places)
   const unsigned mix = ((static_cast<unsigned>(M) * 31u + static_cast<unsigned>(N)) * 31u + static_cast<unsigned>(K)) * 31u + static_cast<unsigned>(batch);
   Entry &e = known[(mix * 2654435769u) >> 24];
-  if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.may_split != may_split || e.deep_words != deep_words)
-    e = {M, N, K, batch, may_split, deep_words, best_plan(M, N, K, batch, may_split, deep_words)};
+  if (e.M != M || e.N != N || e.K != K || e.batch != batch || e.may_split != may_split) e = {M, N, K, batch, may_split, best_plan(M, N, K, batch, may_split)};
   return e.plan;
 }
 
@@ -109,21 +107,21 @@ constexpr gt::BatchOf kOneProduct{1, 0, 0, 0, 0, 0, 0};
 // small products: the depth shared by the waves of a block (gemm_waves.h)
 template <int TM, int TN, bool TA, bool TB, bool SUMS>
 void launch_waves_tile(const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch, int M, int N,
-                       int K, const gt::Epilogue &ep, float *sums, int waves, hipStream_t s) {
+                       int K, const gt::Epilogue &ep, float *sums, const WavesPlan &p, hipStream_t s) {
   const int tm = (M + 16 * TM - 1) / (16 * TM), tn = (N + 16 * TN - 1) / (16 * TN);
   const bool wide = TN > 1 && N % 2 == 0 && ldc % 2 == 0 && zs.co % 2 == 0 && zs.ci % 2 == 0 && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu) && aligned16(ep.gate);
-  const size_t lds = static_cast<size_t>(waves) * (256 * TM * TN + (SUMS ? 16 * TN : 0)) * sizeof(float);
-  hipLaunchKernelGGL((gw::gemm_waves_kernel<TM, TN, TA, TB, SUMS>), dim3(grid_blocks(tm, tn, batch)), dim3(64 * waves), lds, s, DenseParams{A, lda, M, K},
-                     DenseParams{B, ldb, N, K}, out, ldc, zs, ep, sums, wide, M, N, K, TileGrid{tm, tn, tm * tn * batch});
+  const size_t lds = static_cast<size_t>(p.S) * (256 * TM * TN + (SUMS ? 16 * TN : 0)) * sizeof(float);
+  hipLaunchKernelGGL((gw::gemm_waves_kernel<TM, TN, TA, TB, SUMS>), dim3(grid_blocks(tm, tn, batch)), dim3(64 * p.waves), lds, s, DenseParams{A, lda, M, K},
+                     DenseParams{B, ldb, N, K}, out, ldc, zs, ep, sums, wide, M, N, K, p.S, p.kchunk, TileGrid{tm, tn, tm * tn * batch});
 }
 template <bool TA, bool TB, bool SUMS = false>
 void launch_waves(const WavesPlan &p, const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch,
                   int M, int N, int K, const gt::Epilogue &ep, float *sums, hipStream_t s) {
   switch (p.tile) {
-    case 0: return launch_waves_tile<1, 1, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
-    case 1: return launch_waves_tile<1, 2, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
-    case 2: return launch_waves_tile<2, 1, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
-    default: return launch_waves_tile<2, 2, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p.waves, s);
+    case 0: return launch_waves_tile<1, 1, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p, s);
+    case 1: return launch_waves_tile<1, 2, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p, s);
+    case 2: return launch_waves_tile<2, 1, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p, s);
+    default: return launch_waves_tile<2, 2, TA, TB, SUMS>(A, lda, B, ldb, out, ldc, zs, batch, M, N, K, ep, sums, p, s);
   }
 }
 
@@ -138,7 +136,7 @@ int launch_epilogue_fold(const float *part, float *out, int64_t mn, int N, int S
 
 template <bool TA, bool TB>
 int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, hipStream_t s, int64_t *ws_elems) {
-  const Plan plan = plan_product(M, N, K, 1, true, !TA && TB);
+  const Plan plan = plan_product(M, N, K, 1, true);
   if (plan.waves.waves) {
     launch_waves<TA, TB>(plan.waves, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, kNothingMore, nullptr, s);
     return 0;
@@ -170,7 +168,7 @@ void launch_sums_tile(const float *A, int64_t lda, const float *B, int64_t ldb, 
                      DenseParams{B, ldb, N, K}, out, sums, zs, wide, M, N, K, plan.kchunk, TileGrid{tm, tn, tm * tn * plan.S});
 }
 int launch_sums(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, float *sums, int M, int N, int K, hipStream_t s) {
-  const Plan plan = plan_product(M, N, K, 1, true, false);
+  const Plan plan = plan_product(M, N, K, 1, true);
   if (plan.waves.waves) {
     launch_waves<true, false, true>(plan.waves, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, kNothingMore, sums, s);
     return 0;
@@ -298,7 +296,7 @@ template <bool TA, bool TB>
 int dispatch_epilogue(const float *A, int64_t lda, const float *B, int64_t ldb, float *C, int M, int N, int K, const gt::Epilogue &ep, hipStream_t s) {
   const int64_t mn = static_cast<int64_t>(M) * N;
   if (near<TA, TB>(lda, ldb, M, N, K) && rows_reach(N) && !(split_bf16_enabled() && K % 4 == 0 && K >= BK)) {
-    const Plan plan = plan_product(M, N, K, 1, true, !TA && TB);
+    const Plan plan = plan_product(M, N, K, 1, true);
     if (plan.waves.waves) {
       launch_waves<TA, TB>(plan.waves, A, lda, B, ldb, C, N, kOneProduct, 1, M, N, K, ep, nullptr, s);
       return 0;
@@ -332,7 +330,7 @@ int dispatch_batched(const float *A, int64_t lda, int64_t sa, const float *B, in
     if (N <= 64) return launch_far_batched<256, 64, 4, 1, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
     return launch_far_batched<128, 128, 2, 2, TA, TB>(A, lda, sa, B, ldb, sb, C, batch, M, N, K, s);
   }
-  const Plan plan = plan_product(M, N, K, batch, false, !TA && TB);
+  const Plan plan = plan_product(M, N, K, batch, false);
   if (plan.waves.waves) {
     launch_waves<TA, TB>(plan.waves, A, lda, B, ldb, C, N, gt::BatchOf{1, sa, 0, sb, 0, static_cast<int64_t>(M) * N, 0}, batch, M, N, K, kNothingMore, nullptr, s);
     return 0;
@@ -369,7 +367,7 @@ int dispatch_heads(const HeadArray &a, const HeadArray &b, const HeadArray &c, i
   TS_REQUIRE((near<TA, TB>(a.ld, b.ld, M, N, K) && 65ll * 4 * c.ld < (1ll << 31)),
              "TSplit_HeadsMatrixMultiply: a matrix reaches beyond 32-bit byte offsets");
   const int batch = static_cast<int>(c.n) * heads;
-  const Plan plan = plan_product(M, N, K, batch, false, !TA && TB);
+  const Plan plan = plan_product(M, N, K, batch, false);
   const gt::BatchOf zs{heads, a.outer, a.inner, b.outer, b.inner, c.outer, c.inner};
   if (plan.waves.waves)
     launch_waves<TA, TB>(plan.waves, a.p, a.ld, b.p, b.ld, c.p, c.ld, zs, batch, M, N, K, ep, nullptr, s);
@@ -434,7 +432,7 @@ extern "C" int TSplit_MatrixMultiplySums(const DLArrayHandle matA, const DLArray
   TS_REQUIRE(M < (1ll << 31) && N < (1ll << 31) && K < (1ll << 31) - 64, "%s: dimension too large", who);
   const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
   const bool here = M > 0 && N > 0 && K > 0 && near<true, false>(lda, ldb, m, n, k) && rows_reach(n) && !(split_bf16_enabled() && K % 4 == 0 && K >= BK) &&
-                    plan_product(m, n, k, 1, true, false).kchunk <= kSumsRange;
+                    plan_product(m, n, k, 1, true).kchunk <= kSumsRange;
   if (!here) {   // the product by itself, on whichever kernel takes it, and the sums by themselves
     int64_t ashape[2] = {K, M}, bshape[2] = {K, N};
     DLArray A{matA->data, matA->ctx, 2, ashape}, B{matB->data, matB->ctx, 2, bshape};

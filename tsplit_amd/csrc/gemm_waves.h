@@ -2,11 +2,14 @@
 //
 // A product of a few hundred rows and columns has few 64 x 64 tiles, so on the kernel of gemm_tile.h its depth was cut into ranges and a
 // second launch added them; either launch takes what any launch takes, and a range of one or two steps is a chain of memory latencies
-// behind one barrier each.  Here a block owns 16 TM x 16 TN of the result, its two to four waves deal the depth among them 32 values at a time,
-// operands go from memory to the registers the matrix instruction reads (no LDS, no barrier on the way), and the waves' sums are added
-// through LDS in ascending order.  What bounds it is latency: one for the operands, one for LDS, and the launch.
+// behind one barrier each.  Here a block owns 16 TM x 16 TN of the result, its two to four waves take the ranges of the depth in turn (the tile
+// kernel's own ranges: the bits of that kernel and its fold, see plan_waves), 32 values at a time, operands go from memory to the registers
+// the matrix instruction reads (no LDS, no barrier on the way), and the ranges' results are added through LDS in ascending order.  What bounds
+// it is latency: one for the operands, one for LDS, and the launch.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "gemm_tile.h"
 
@@ -15,7 +18,7 @@ namespace gw {
 
 using gt::f32x4;
 using mg::kOobOffset;
-constexpr int kDeep = 32;       // a wave's share of the depth at a time: whole 128-byte lines of an operand with K contiguous
+constexpr int kDeep = 32;       // of the depth at a time: whole 128-byte lines of an operand with K contiguous
 constexpr int kGroups = kDeep / 16;
 
 // What a lane supplies of one operand: index T (lane & 15) + t of tile t, k = 16 u + 4 (lane >> 4) + i of kDeep.
@@ -83,11 +86,12 @@ struct Loader {
   }
 };
 
-// SUMS: the blocks of the first row of tiles also leave the sums of B's columns.
+// SUMS: the blocks of the first row of tiles also leave the sums of B's columns, added as gt::Core adds them.
 template <int TM, int TN, bool TA, bool TB, bool SUMS>
 __global__ __launch_bounds__(256) void gemm_waves_kernel(mg::DenseParams ap, mg::DenseParams bp, float *out, int64_t ldc, gt::BatchOf zs,
-                                                          gt::Epilogue ep, float *sums, bool wide, int M, int N, int K, mg::TileGrid tg) {
-  extern __shared__ __attribute__((aligned(16))) float lds[];   // [wave][tm][e][lane][tn]; with SUMS [wave][16 TN] behind it
+                                                          gt::Epilogue ep, float *sums, bool wide, int M, int N, int K, int S, int kchunk,
+                                                          mg::TileGrid tg) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];   // [range][tm][e][lane][tn]; with SUMS [range][16 TN] behind it
   int z, tile_m, tile_n;
   if (!mg::block_tile(tg, z, tile_m, tile_n)) return;
   const int zo = z / zs.inner, zi = z - zo * zs.inner;
@@ -99,23 +103,38 @@ __global__ __launch_bounds__(256) void gemm_waves_kernel(mg::DenseParams ap, mg:
   Loader<TN, TB> lb;
   la.init(ap, m0);
   lb.init(bp, n0);
+  constexpr int kTile = 256 * TM * TN;
+  typedef float vec __attribute__((ext_vector_type(TN)));
   f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float col[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) col[j] = 0.f;
+  float col[TN], some[TN];
   const bool on = SUMS && tile_m == 0;
-  Operand<TM, !TA> a[2];
-  Operand<TN, TB> b[2];
-  const int stride = kDeep * waves;
-  int k0 = kDeep * wave;
-  auto multiply = [&](int at, Operand<TM, !TA> &x, Operand<TN, TB> &y) {
-    if (at + kDeep > K) {
-      Loader<TM, !TA>::cut(at, K, x);
-      Loader<TN, TB>::cut(at, K, y);
+  auto clear = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < TN; ++j) col[j] = some[j] = 0.f;
+  };
+  // a share of the wave's: k in [k, k + kDeep) of range r, which ends with share `end`
+  struct Share {
+    int k, r, end;
+  };
+  auto first_of = [&](int r) { return Share{r * kchunk, r, min(K, (r + 1) * kchunk)}; };
+  auto behind = [&](const Share &s) { return s.k + kDeep < s.end ? Share{s.k + kDeep, s.r, s.end} : first_of(s.r + waves); };
+  // last: of the wave's (the others end before the depth does)
+  auto multiply = [&](const Share &s, Operand<TM, !TA> &x, Operand<TN, TB> &y, auto last) {
+    if constexpr (decltype(last)::value)
+      if (s.k + kDeep > K) {
+        Loader<TM, !TA>::cut(s.k, K, x);
+        Loader<TN, TB>::cut(s.k, K, y);
+      }
+    if (SUMS && (s.k - s.r * kchunk) % (8 * kDeep) == 0) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        col[j] += some[j];
+        some[j] = 0.f;
+      }
     }
 #pragma unroll
     for (int u = 0; u < kGroups; ++u) {
@@ -127,65 +146,80 @@ __global__ __launch_bounds__(256) void gemm_waves_kernel(mg::DenseParams ap, mg:
           for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.v[u][tm][i], y.v[u][tn][i], acc[tm][tn], 0, 0, 0);
       if (on) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) col[j] += (y.v[u][j][0] + y.v[u][j][1]) + (y.v[u][j][2] + y.v[u][j][3]);
+        for (int j = 0; j < TN; ++j) some[j] += (y.v[u][j][0] + y.v[u][j][1]) + (y.v[u][j][2] + y.v[u][j][3]);
       }
     }
+    if (s.k + kDeep < s.end) return;
+    // the range's result
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        vec v;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) v[j] = acc[tm][j][e];
+        *reinterpret_cast<vec *>(lds + s.r * kTile + ((tm * 4 + e) * 64 + lane) * TN) = v;
+      }
+    if constexpr (SUMS)
+      if (on) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          float v = col[j] + some[j];
+          v += __shfl_xor(v, 16, 64);
+          v += __shfl_xor(v, 32, 64);
+          if (lane < 16) lds[S * kTile + s.r * 16 * TN + TN * lane + j] = v;
+        }
+      }
+    clear();
   };
-  if (k0 < K) {
-    la.load(k0, a[0]);
-    lb.load(k0, b[0]);
-  }
-  while (k0 < K) {   // two shares a turn, the next one's loads in front of either's products
-    const int k1 = k0 + stride, k2 = k1 + stride;
-    if (k1 < K) {
-      la.load(k1, a[1]);
-      lb.load(k1, b[1]);
-    }
+  clear();
+  Operand<TM, !TA> a[2];
+  Operand<TN, TB> b[2];
+  auto load = [&](const Share &s, int to) {
+    la.load(s.k, a[to]);
+    lb.load(s.k, b[to]);
     __builtin_amdgcn_sched_barrier(0);
-    multiply(k0, a[0], b[0]);
+  };
+  auto use = [&](const Share &s, int from, auto last) {
+    multiply(s, a[from], b[from], last);
     __builtin_amdgcn_sched_barrier(0);
-    if (k2 < K) {
-      la.load(k2, a[0]);
-      lb.load(k2, b[0]);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (k1 < K) multiply(k1, a[1], b[1]);
-    __builtin_amdgcn_sched_barrier(0);
-    k0 = k2;
-  }
-
-  constexpr int kTile = 256 * TM * TN;
-  typedef float vec __attribute__((ext_vector_type(TN)));
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      vec v;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) v[j] = acc[tm][j][e];
-      *reinterpret_cast<vec *>(lds + wave * kTile + ((tm * 4 + e) * 64 + lane) * TN) = v;
-    }
-  if constexpr (SUMS)
-    if (on) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        col[j] += __shfl_xor(col[j], 16, 64);
-        col[j] += __shfl_xor(col[j], 32, 64);
-        if (lane < 16) lds[waves * kTile + wave * 16 * TN + TN * lane + j] = col[j];
+  };
+  // Two shares a turn, the next one's loads in front of either's products.  (No load under a condition of its own: where the paths meet the
+  // compiler waits for as many as the shorter one has, which then are the next share's too.)
+  const std::true_type yes{};
+  const std::false_type no{};
+  Share now = first_of(wave);
+  if (now.r < S) {
+    load(now, 0);
+    for (;;) {
+      const Share next = behind(now);
+      if (next.r >= S) {
+        use(now, 0, yes);
+        break;
       }
+      load(next, 1);
+      use(now, 0, no);
+      now = behind(next);
+      if (now.r >= S) {
+        use(next, 1, yes);
+        break;
+      }
+      load(now, 0);
+      use(next, 1, no);
     }
+  }
   __syncthreads();
   if constexpr (SUMS)
     if (on && threadIdx.x < 16 * TN && n0 + static_cast<int>(threadIdx.x) < N) {
-      float s = 0.f;
-      for (int w = 0; w < waves; ++w) s += lds[waves * kTile + w * 16 * TN + threadIdx.x];
+      float s = lds[S * kTile + threadIdx.x];
+      for (int r = 1; r < S; ++r) s += lds[S * kTile + r * 16 * TN + threadIdx.x];
       sums[n0 + threadIdx.x] = s;
     }
   const int64_t c_at = zo * zs.co + zi * zs.ci;
   for (int q = threadIdx.x; q < TM * 256; q += blockDim.x) {
     const int l = q & 63, m = m0 + TM * (4 * (l >> 4) + (q >> 6 & 3)) + (q >> 8), n = n0 + TN * (l & 15);
     vec s = *reinterpret_cast<const vec *>(lds + q * TN);
-    for (int w = 1; w < waves; ++w) s += *reinterpret_cast<const vec *>(lds + w * kTile + q * TN);
+    for (int r = 1; r < S; ++r) s += *reinterpret_cast<const vec *>(lds + r * kTile + q * TN);
     if (m >= M) continue;
     const int64_t at = c_at + m * ldc + n;
     float v[TN];

@@ -98,35 +98,42 @@ inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int
 }
 
 // Small products go to the kernel whose blocks share the depth of one small tile among their waves (gemm_waves.h), where that takes less.
-// A launch there costs what any launch does, and for every block of the busiest CU a part of its own and one for each value of the depth.
-// From 60 shapes, rows 1 to 2048, columns 10 to 5003, depth 16 to 5003, in the four forms on four tiles with 2 to 16 waves: 9 % rms off, the
-// tile kernel's model (launches included) 12 %.  Over those shapes 1.25 times faster than the tile kernel alone, with the best of both by
-// hindsight 1.30: 128 x 256 over 784 7.3 -> 5.1-5.8 us, over 256 6.6 -> 4.3, 784 x 256 over 128 6.0 -> 4.6, 385 x 256 over 1024 9.9 -> 7.2, 32 x
-// 4096 over 1024 11.6 -> 7.3, 1 x 1908 over 308 6.9 -> 4.6; where the tile kernel stays: 250 x 5003 over 256 12.0 (14.5 here), 100 x 4096 over
-// 4096 39 (41-60).
+//
+// The depth is cut into the tile kernel's own ranges, so that a result has the bits that the tile kernel and the fold give it; where those are
+// fewer than the four waves (many tiles, or batches, whose depth that kernel leaves whole) into up to four, whose chains of roundings are
+// shorter.  (Four waves that dealt a whole depth among them 32 values at a time were as fast, but their chains of K / 4 roundings where
+// the tile kernel has K / 16 were 1.6 times further from float64 at 128 x 256 over 784 and 1.9 times at 64 x 1000 over 2048.)
+//
+// A launch there costs what any launch does, and for every block of the busiest CU a part of its own and one for each value of the depth that
+// the busiest wave takes; beyond 2048 of them 8 % more, where loads bound it (with both depths contiguous up to 20 %: 512 x 512 over 4096
+// 32.9 us on 32 x 32, 27.7 on the tile kernel).  From 217 shapes, rows 1 to 2048, columns 10 to 5003, depth 10 to 65536, batches among
+// them, in the four forms on the four tiles: 9 % rms off, the tile kernel's model (launches included) 15 %.  Over those shapes 1.25 times
+// faster than the tile kernel alone, with the best of both by hindsight 1.26: 128 x 256 over 784 7.5 -> 5.3 us, over 256 6.7 -> 4.1, 784 x 256 over
+// 128 5.7 -> 5.0, 385 x 256 over 1024 9.9 -> 7.1-9.0, 32 x 4096 over 1024 11.7 -> 7.3-9.1, 1 x 1908 over 308 7.0 -> 4.0, 16 of 64 x 64 over
+// 2048 45 -> 9; where the tile kernel stays: 250 x 5003 over 256 12.4, 512 x 512 over 64 4.4 (5.3 on 32 x 32 here).  Worst: 1 x 3000
+// over 65536, 231 us for 195.
 constexpr TileKind kWaveTiles[] = {{16, 16}, {16, 32}, {32, 16}, {32, 32}};
 struct WavesPlan {
   int tile, waves;   // waves 0: the tile kernel
+  int S, kchunk;     // the ranges that the waves take in turn
 };
-//
-// Deep products (from 1024 on) and those with the depth contiguous in both operands (`deep_words`: a lane's words lie a row apart) take
-// more a value on the wider tiles, whose loads then bound them; without that line 512 x 512 over 4096 took 29.9-34.5 us here and 27.7-28.4
-// on the tile kernel, over 8192 54-63 and 43-45, with `deep_words` 384 x 512 over 2048 19.4 and 16.7, 256 x 512 over 2048 15.0 and 14.2.
-inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, bool deep_words, double tile_kernel_us) {
-  constexpr double kLaunch = 3.6, kBlock[] = {0.18, 0.40, 0.47, 0.76}, kDepth[] = {0.0022, 0.0031, 0.0031, 0.0045};
-  constexpr double kBeyond[] = {0, 0.0009, 0.0009, 0.0020}, kWords[] = {0, 0.0014, 0.0014, 0.0014};
-  WavesPlan best{0, 0};
-  double least = 2.3 + 1.15 * tile_kernel_us;
+inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, const TilePlan &tile_kernel) {
+  constexpr double kLaunch = 3.56, kBlock[] = {0, 0.186, 0.363, 0.951}, kDepth[] = {0.00245, 0.00345, 0.00337, 0.00513};
+  WavesPlan best{0, 0, 1, 0};
+  if (K <= 0) return best;
+  const int64_t steps = (K + 31) / 32, per = (steps + std::max(4, tile_kernel.S) - 1) / std::max(4, tile_kernel.S), S = (steps + per - 1) / per;
+  const int64_t deep = S > 4 ? (S + 3) / 4 * per * 128 : K;   // four times what the busiest wave takes
+  double least = 2.3 + 1.15 * tile_kernel.us;
   for (int t = 0; t < 4; ++t) {
     const int64_t blocks = ((M + kWaveTiles[t].bm - 1) / kWaveTiles[t].bm) * ((N + kWaveTiles[t].bn - 1) / kWaveTiles[t].bn) * batch;
-    if (blocks > 1024) continue;
+    // (the ranges' results lie in LDS: two blocks a CU)
+    if (blocks > 1024 || S * (kWaveTiles[t].bm + 1) * kWaveTiles[t].bn * 4 > 81920) continue;
     const int64_t n = (blocks + 255) / 256;
-    const double us = kLaunch + n * (kBlock[t] + kDepth[t] * K + (K > 1024 ? kBeyond[t] * (K - 1024) + (deep_words ? kWords[t] * K : 0) : 0));
-    if (us < least && (n == 1 || us < 8)) {   // (of several blocks a CU the tile kernel fills the chip as well: 100 x 4096 over 4096)
+    const double us = (kLaunch + n * (kBlock[t] + kDepth[t] * deep)) * (deep > 2048 ? 1.08 : 1);
+    if (us < least) {
       least = us;
-      // 32 values of the depth a wave; eight or sixteen waves gain nothing on a CU of their own (over the shapes 0.2 %) and lose where
-      // blocks share one
-      best = {t, static_cast<int>(std::max<int64_t>(2, std::min<int64_t>(4, (K + 31) / 32)))};
+      // eight or sixteen waves gain nothing on a CU of their own (over the shapes 0.2 %) and lose where blocks share one
+      best = {t, static_cast<int>(std::max<int64_t>(2, std::min<int64_t>(4, S))), static_cast<int>(S), static_cast<int>(per * 32)};
     }
   }
   return best;
