@@ -49,3 +49,27 @@ def test_calls_refuse_what_they_cannot_take():
         nd.empty("ab")
     with pytest.raises(TypeError):
         nd.empty((2, 3), 5)
+
+
+def test_an_array_of_a_collected_cycle_goes_to_its_recordings_keeper_first():
+    """The keeper lies in the same cycle, older than the array: what it holds must not have been cleared when it is asked."""
+    from tsplit_amd.stream import _Keeper
+    took, h = [], nd.DLArrayHandle()
+
+    class Keeper(_Keeper):
+        def take(self, handle, rule):
+            took.append((super().take(handle, rule), ctypes.addressof(handle.contents)))
+            return took[-1][0]
+    keeper, ring = Keeper(), []
+    assert _LIB.DLArrayAlloc((ctypes.c_int64 * 1)(4), ctypes.c_int64(1), nd.cpu(0), ctypes.byref(h), ctypes.c_int(1)) == 0
+    h.contents.ctx.device_type = 2              # as an array on the device: only those are the keeper's
+    a = nd.NDArray(h)
+    a._keeper, a._owner = keeper, ring
+    ring.extend([keeper, a])
+    address = ctypes.addressof(h.contents)
+    del a, keeper, ring, h
+    gc.collect()
+    assert took == [(True, address)]
+    h = ctypes.cast(address, nd.DLArrayHandle)
+    h.contents.ctx.device_type = 1
+    assert _LIB.DLArrayFree(h, ctypes.c_int(1)) == 0

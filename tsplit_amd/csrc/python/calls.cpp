@@ -60,8 +60,9 @@ int array_traverse(Array *a, visitproc visit, void *arg) {
   Py_VISIT(a->split_dimension);
   return 0;
 }
-// Gives the memory back, once (also where a collected cycle is being taken apart: a view's memory is its owner's, which may go first)
-void give_back(Array *a) {
+// Gives the memory back, once.  A finalizer: it runs for every array of a collected cycle before anything of the cycle is cleared, a
+// recording's keeper among it (a view's memory is its owner's, which may go first).
+void array_finalize(Array *a) {
   DLArray *raw = a->raw;
   a->raw = nullptr;
   int rule = 0;
@@ -87,10 +88,10 @@ void give_back(Array *a) {
     fn_free(raw, rule);
     Py_END_ALLOW_THREADS
   }
+  Py_CLEAR(a->handle);
   PyErr_Restore(type, value, trace);
 }
 int array_clear(Array *a) {
-  give_back(a);
   Py_CLEAR(a->handle);
   Py_CLEAR(a->owner);
   Py_CLEAR(a->keeper);
@@ -104,6 +105,7 @@ int array_clear(Array *a) {
   return 0;
 }
 void array_dealloc(Array *a) {
+  if (PyObject_CallFinalizerFromDealloc(reinterpret_cast<PyObject *>(a))) return;
   PyObject_GC_UnTrack(a);
   array_clear(a);
   Py_TYPE(a)->tp_free(reinterpret_cast<PyObject *>(a));
@@ -441,6 +443,7 @@ PyMODINIT_FUNC PyInit__calls() {
   ArrayType.tp_dealloc = reinterpret_cast<destructor>(array_dealloc);
   ArrayType.tp_traverse = reinterpret_cast<traverseproc>(array_traverse);
   ArrayType.tp_clear = reinterpret_cast<inquiry>(array_clear);
+  ArrayType.tp_finalize = reinterpret_cast<destructor>(array_finalize);
   ArrayType.tp_init = reinterpret_cast<initproc>(array_init);
   ArrayType.tp_new = PyType_GenericNew;
   ArrayType.tp_getset = array_getset;
