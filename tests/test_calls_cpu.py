@@ -1,12 +1,15 @@
 """The extension module that Python's calls go through (csrc/python/calls.cpp): what arrays own, and what operator calls refuse."""
 import ctypes
 import gc
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
 from tsplit_amd import _calls, gpu_links as L, ndarray as nd
-from tsplit_amd._base import _LIB
+from tsplit_amd._base import LIB_PATH, _LIB
 
 
 def test_arrays_own_their_memory_and_views_keep_their_parent():
@@ -73,3 +76,24 @@ def test_an_array_of_a_collected_cycle_goes_to_its_recordings_keeper_first():
     h = ctypes.cast(address, nd.DLArrayHandle)
     h.contents.ctx.device_type = 1
     assert _LIB.DLArrayFree(h, ctypes.c_int(1)) == 0
+
+
+def test_a_library_without_an_operator_is_loaded_and_misses_that_call_alone(tmp_path):
+    names = [line.split()[-1] for line in subprocess.run(["nm", "-D", "--defined-only", LIB_PATH], capture_output=True, text=True, check=True).stdout.splitlines()
+             if " T " in line and not line.split()[-1].startswith("_")]
+    assert "DLGpuTanh" in names and "TSplit_BatchNormReluAdd" in names
+    src, lib = tmp_path / "other.c", str(tmp_path / "other.so")
+    src.write_text("".join("int %s() { return 0; }\n" % name for name in names if name != "TSplit_BatchNormReluAdd"))
+    subprocess.run(["gcc", "-shared", "-fPIC", str(src), "-o", lib], check=True)
+    program = """
+from tsplit_amd import gpu_links as L, ndarray as nd
+a = nd.NDArray(None)
+L.tanh(a, a)
+try:
+    L.batch_norm_relu_add(a, a, a, a, a, a, a)
+except AttributeError as e:
+    print("without", "TSplit_BatchNormReluAdd" in str(e))
+"""
+    done = subprocess.run([sys.executable, "-c", program], env=dict(os.environ, TSPLIT_LIB_PATH=lib), capture_output=True, text=True,
+                          cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+    assert done.stdout.strip() == "without True", done.stderr

@@ -356,7 +356,7 @@ struct Arg<ProfilerHandle> {   // a Profiler structure, or nothing
 template <class Op, class... A, size_t... I>
 PyObject *call(int (*fn)(A...), PyObject *const *args, Py_ssize_t n, std::index_sequence<I...>) {
   if (n != static_cast<Py_ssize_t>(sizeof...(A))) return PyErr_Format(PyExc_TypeError, "%s takes %d arguments", Op::name(), static_cast<int>(sizeof...(A)));
-  if (!fn) return PyErr_Format(PyExc_RuntimeError, "%s is not bound", Op::name());
+  if (!fn) return PyErr_Format(PyExc_AttributeError, "the library has no %s", Op::name());
   std::tuple<A...> v;
   if (!(Arg<A>::get(args[I], Op::optional >> I & 1, std::get<I>(v)) && ...)) return nullptr;
   int rc;
@@ -401,24 +401,24 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   };
 CALLS(DECLARE)
 
-// bind(addresses by name, the module dict with MEMORY_MANAGE_RULE, the one with _recording_keeper, address -> handle)
+// bind(addresses by name, those of operators that the library lacks left out, the module dict with MEMORY_MANAGE_RULE, the one with _recording_keeper, address -> handle)
 PyObject *bind(PyObject *, PyObject *args) {
   PyObject *addresses, *rules, *recording, *handle_of;
   if (!PyArg_ParseTuple(args, "O!O!O!O", &PyDict_Type, &addresses, &PyDict_Type, &rules, &PyDict_Type, &recording, &handle_of)) return nullptr;
   auto look = [&](const char *name, auto &fn) {
     PyObject *a = PyDict_GetItemString(addresses, name);
     void *p = a ? PyLong_AsVoidPtr(a) : nullptr;
-    if (!p) {
-      if (!PyErr_Occurred()) PyErr_Format(PyExc_RuntimeError, "no address of %s", name);
-      return false;
-    }
     fn = reinterpret_cast<typename std::remove_reference<decltype(fn)>::type>(p);
-    return true;
+    return !PyErr_Occurred();
   };
 #define BIND(symbol, mask) \
   if (!look(#symbol, Op_##symbol::fn)) return nullptr;
   CALLS(BIND)
   if (!look("DLArrayAlloc", fn_alloc) || !look("DLArrayFree", fn_free)) return nullptr;
+  if (!fn_alloc || !fn_free) {
+    PyErr_SetString(PyExc_AttributeError, "the library has no DLArrayAlloc or no DLArrayFree");
+    return nullptr;
+  }
   Py_INCREF(rules);
   Py_XSETREF(g_rules, rules);
   Py_INCREF(recording);

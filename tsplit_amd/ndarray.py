@@ -68,8 +68,18 @@ def _c_shape(shape):
         return c
 
 
-_calls.bind({name: ctypes.cast(_LIB[name], ctypes.c_void_p).value for name in _calls.SYMBOLS + ["DLArrayAlloc", "DLArrayFree"]}, globals(),
-            vars(_stream), lambda address: ctypes.cast(address, DLArrayHandle))
+def _addresses(names):
+    """Where the library has them; an operator that another build of it lacks is missed by its own call alone."""
+    found = {}
+    for name in names:
+        try:
+            found[name] = ctypes.cast(_LIB[name], ctypes.c_void_p).value
+        except AttributeError:
+            pass
+    return found
+
+
+_calls.bind(_addresses(_calls.SYMBOLS + ["DLArrayAlloc", "DLArrayFree"]), globals(), vars(_stream), lambda address: ctypes.cast(address, DLArrayHandle))
 
 
 def cpu(dev_id=0):
