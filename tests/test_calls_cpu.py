@@ -97,3 +97,19 @@ except AttributeError as e:
     done = subprocess.run([sys.executable, "-c", program], env=dict(os.environ, TSPLIT_LIB_PATH=lib), capture_output=True, text=True,
                           cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
     assert done.stdout.strip() == "without True", done.stderr
+
+
+def test_eight_bytes_are_no_pointer_and_no_context():
+    a, eight = nd.empty((2, 3)), np.zeros(1)
+    assert eight.nbytes == ctypes.sizeof(nd.DLContext) == ctypes.sizeof(ctypes.c_void_p)
+    for bad in (eight, b"12345678", ctypes.c_double(1)):
+        with pytest.raises(TypeError):
+            nd.NDArray(bad)
+        with pytest.raises(TypeError):
+            nd.empty((2, 3), bad)
+        with pytest.raises(TypeError):
+            a.handle = bad
+    stream = type("Stream", (), {"handle": eight})()
+    with pytest.raises(TypeError):
+        L.relu(a, a, stream)
+    assert a.shape == (2, 3)

@@ -24,6 +24,8 @@ namespace {
 PyObject *g_rules = nullptr;       // the dict with MEMORY_MANAGE_RULE
 PyObject *g_recording = nullptr;   // the dict with _recording_keeper
 PyObject *g_handle_of = nullptr;   // address -> ctypes handle
+PyObject *g_pointers = nullptr;    // the ctypes types that a pointer may be of
+PyObject *g_context = nullptr;     // DLContext
 PyObject *g_rule_name, *g_keeper_name, *g_take_name, *g_handle_name;
 
 // ---------------------------------------------------------------- arrays
@@ -113,6 +115,11 @@ void array_dealloc(Array *a) {
 
 // the address a ctypes pointer holds
 bool pointer_of(PyObject *p, void **out) {
+  const int is = PyObject_IsInstance(p, g_pointers);
+  if (is <= 0) {
+    if (!is) PyErr_Format(PyExc_TypeError, "a pointer, not %R", p);
+    return false;
+  }
   Py_buffer b;
   if (PyObject_GetBuffer(p, &b, PyBUF_SIMPLE)) return false;
   const bool ok = b.len == static_cast<Py_ssize_t>(sizeof(void *));
@@ -234,6 +241,8 @@ PyObject *new_array(PyObject *, PyObject *const *args, Py_ssize_t n) {
     PyErr_SetString(PyExc_RuntimeError, "the library is not bound");
     return nullptr;
   }
+  const int is = PyObject_IsInstance(args[2], g_context);
+  if (is <= 0) return is ? nullptr : PyErr_Format(PyExc_TypeError, "ctx is a DLContext, not %R", args[2]);
   Py_buffer b;
   if (PyObject_GetBuffer(args[2], &b, PyBUF_SIMPLE)) return nullptr;
   DLContext ctx{};
@@ -401,10 +410,13 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   };
 CALLS(DECLARE)
 
-// bind(addresses by name, those of operators that the library lacks left out, the module dict with MEMORY_MANAGE_RULE, the one with _recording_keeper, address -> handle)
+// bind(addresses by name, those of operators that the library lacks left out, the module dict with MEMORY_MANAGE_RULE, the one with
+// _recording_keeper, address -> handle, the types of pointers, DLContext)
 PyObject *bind(PyObject *, PyObject *args) {
-  PyObject *addresses, *rules, *recording, *handle_of;
-  if (!PyArg_ParseTuple(args, "O!O!O!O", &PyDict_Type, &addresses, &PyDict_Type, &rules, &PyDict_Type, &recording, &handle_of)) return nullptr;
+  PyObject *addresses, *rules, *recording, *handle_of, *pointers, *context;
+  if (!PyArg_ParseTuple(args, "O!O!O!OO!O!", &PyDict_Type, &addresses, &PyDict_Type, &rules, &PyDict_Type, &recording, &handle_of, &PyTuple_Type,
+                        &pointers, &PyType_Type, &context))
+    return nullptr;
   auto look = [&](const char *name, auto &fn) {
     PyObject *a = PyDict_GetItemString(addresses, name);
     void *p = a ? PyLong_AsVoidPtr(a) : nullptr;
@@ -425,6 +437,10 @@ PyObject *bind(PyObject *, PyObject *args) {
   Py_XSETREF(g_recording, recording);
   Py_INCREF(handle_of);
   Py_XSETREF(g_handle_of, handle_of);
+  Py_INCREF(pointers);
+  Py_XSETREF(g_pointers, pointers);
+  Py_INCREF(context);
+  Py_XSETREF(g_context, context);
   Py_RETURN_NONE;
 }
 

@@ -79,7 +79,8 @@ def _addresses(names):
     return found
 
 
-_calls.bind(_addresses(_calls.SYMBOLS + ["DLArrayAlloc", "DLArrayFree"]), globals(), vars(_stream), lambda address: ctypes.cast(address, DLArrayHandle))
+_calls.bind(_addresses(_calls.SYMBOLS + ["DLArrayAlloc", "DLArrayFree"]), globals(), vars(_stream), lambda address: ctypes.cast(address, DLArrayHandle),
+            (ctypes._Pointer, ctypes.c_void_p), DLContext)
 
 
 def cpu(dev_id=0):
