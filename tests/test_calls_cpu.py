@@ -113,3 +113,10 @@ def test_eight_bytes_are_no_pointer_and_no_context():
     with pytest.raises(TypeError):
         L.relu(a, a, stream)
     assert a.shape == (2, 3)
+
+
+def test_flags_of_an_array_take_any_truth_value():
+    a = nd.empty((2, 3))
+    for value in (0, 1, None, "", "yes"):
+        a.auto_deleted = value
+        assert bool(a.auto_deleted) == bool(value)

@@ -7,7 +7,6 @@
 // library that _base.py has loaded.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
-#include <structmember.h>
 
 #include <cstddef>
 #include <cstdint>
@@ -210,10 +209,20 @@ Field f_owner{offsetof(Array, owner), kNone}, f_keeper{offsetof(Array, keeper), 
     f_events{offsetof(Array, events), kDict}, f_swap{offsetof(Array, swap), kFalse}, f_in_gpu{offsetof(Array, in_gpu), kTrue},
     f_splitted{offsetof(Array, splitted), kFalse}, f_number{offsetof(Array, split_number), kOne}, f_dimension{offsetof(Array, split_dimension), kNone};
 
+PyObject *get_flag(Array *a, void *at) { return PyBool_FromLong(*(reinterpret_cast<char *>(a) + *static_cast<size_t *>(at))); }
+int set_flag(Array *a, PyObject *value, void *at) {
+  const int t = value ? PyObject_IsTrue(value) : 0;
+  if (t >= 0) *(reinterpret_cast<char *>(a) + *static_cast<size_t *>(at)) = static_cast<char>(t);
+  return t < 0 ? -1 : 0;
+}
+size_t at_auto_deleted = offsetof(Array, auto_deleted), at_is_view = offsetof(Array, is_view);
+
 #define FIELD(name, f) {name, reinterpret_cast<getter>(get_field), reinterpret_cast<setter>(set_field), nullptr, &f}
 PyGetSetDef array_getset[] = {{"handle", reinterpret_cast<getter>(get_handle), reinterpret_cast<setter>(set_handle), nullptr, nullptr},
                               {"shape", reinterpret_cast<getter>(get_shape), nullptr, nullptr, nullptr},
                               {"data_ptr", reinterpret_cast<getter>(get_data_ptr), nullptr, nullptr, nullptr},
+                              {"auto_deleted", reinterpret_cast<getter>(get_flag), reinterpret_cast<setter>(set_flag), nullptr, &at_auto_deleted},
+                              {"_is_view", reinterpret_cast<getter>(get_flag), reinterpret_cast<setter>(set_flag), nullptr, &at_is_view},
                               FIELD("_owner", f_owner),
                               FIELD("_keeper", f_keeper),
                               FIELD("sTensor", f_stensor),
@@ -224,9 +233,6 @@ PyGetSetDef array_getset[] = {{"handle", reinterpret_cast<getter>(get_handle), r
                               FIELD("split_number", f_number),
                               FIELD("split_dimension", f_dimension),
                               {nullptr, nullptr, nullptr, nullptr, nullptr}};
-PyMemberDef array_members[] = {{"auto_deleted", T_BOOL, offsetof(Array, auto_deleted), 0, nullptr},
-                               {"_is_view", T_BOOL, offsetof(Array, is_view), 0, nullptr},
-                               {nullptr, 0, 0, 0, nullptr}};
 
 PyTypeObject ArrayType = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
@@ -463,7 +469,6 @@ PyMODINIT_FUNC PyInit__calls() {
   ArrayType.tp_init = reinterpret_cast<initproc>(array_init);
   ArrayType.tp_new = PyType_GenericNew;
   ArrayType.tp_getset = array_getset;
-  ArrayType.tp_members = array_members;
   if (PyType_Ready(&ArrayType)) return nullptr;
   g_rule_name = PyUnicode_InternFromString("MEMORY_MANAGE_RULE");
   g_keeper_name = PyUnicode_InternFromString("_recording_keeper");
