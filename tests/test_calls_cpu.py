@@ -120,3 +120,12 @@ def test_flags_of_an_array_take_any_truth_value():
     for value in (0, 1, None, "", "yes"):
         a.auto_deleted = value
         assert bool(a.auto_deleted) == bool(value)
+
+
+def test_a_memory_rule_that_is_no_number_is_refused(monkeypatch):
+    a = nd.empty((2, 3))
+    monkeypatch.setattr(nd, "MEMORY_MANAGE_RULE", "pool")
+    with pytest.raises(TypeError):
+        nd.empty((2, 3))
+    monkeypatch.undo()
+    assert nd.empty((2, 3)).shape == a.shape

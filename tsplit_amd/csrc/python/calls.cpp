@@ -40,12 +40,12 @@ extern PyTypeObject ArrayType;
 int (*fn_alloc)(const index_t *, index_t, DLContext, DLArrayHandle *, int) = nullptr;
 int (*fn_free)(DLArrayHandle, int) = nullptr;
 
-// the memory rule; false while the interpreter goes down
+// the memory rule; false while the interpreter goes down, and with an error set where it is no whole number
 bool current_rule(int &rule) {
   PyObject *r = g_rules ? PyDict_GetItem(g_rules, g_rule_name) : nullptr;
   if (!r || r == Py_None) return false;
   rule = static_cast<int>(PyLong_AsLong(r));
-  return true;
+  return !(rule == -1 && PyErr_Occurred());
 }
 
 int array_traverse(Array *a, visitproc visit, void *arg) {
@@ -66,12 +66,15 @@ int array_traverse(Array *a, visitproc visit, void *arg) {
 void array_finalize(Array *a) {
   DLArray *raw = a->raw;
   a->raw = nullptr;
-  int rule = 0;
-  if (!raw || !current_rule(rule)) return;
+  if (!raw) return;
   PyObject *type, *value, *trace;
   PyErr_Fetch(&type, &value, &trace);
+  int rule = 0;
   bool mine = true;
-  if (a->is_view) {
+  if (!current_rule(rule)) {
+    mine = false;
+    if (PyErr_Occurred()) PyErr_WriteUnraisable(reinterpret_cast<PyObject *>(a));
+  } else if (a->is_view) {
     raw->data = nullptr;   // a view owns its struct and shape but not its data
   } else if (!a->auto_deleted) {
     mine = false;
@@ -244,7 +247,7 @@ PyObject *new_array(PyObject *, PyObject *const *args, Py_ssize_t n) {
   }
   int rule = 0;
   if (!fn_alloc || !current_rule(rule)) {
-    PyErr_SetString(PyExc_RuntimeError, "the library is not bound");
+    if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the library is not bound");
     return nullptr;
   }
   const int is = PyObject_IsInstance(args[2], g_context);
