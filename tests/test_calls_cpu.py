@@ -129,3 +129,12 @@ def test_a_memory_rule_that_is_no_number_is_refused(monkeypatch):
         nd.empty((2, 3))
     monkeypatch.undo()
     assert nd.empty((2, 3)).shape == a.shape
+
+
+def test_the_module_is_of_this_python():
+    """Named by its ABI: another Python finds no module, and not one that does not fit it."""
+    import sysconfig
+
+    from tsplit_amd import build
+    assert _calls.__file__ == build.CALLS and _calls.__file__.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
+    assert not os.path.exists(os.path.join(os.path.dirname(build.CALLS), "_calls.so"))

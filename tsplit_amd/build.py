@@ -3,8 +3,8 @@
     python -m tsplit_amd.build            # incremental
     python -m tsplit_amd.build --force    # recompile everything
 
-Also builds the extension module that Python's calls go through (_calls.so, plain g++) and the host-only pool test library
-used by the CPU tests.
+Also builds the extension module that Python's calls go through (_calls.<the Python's ABI tag>.so, plain g++ and Python's headers) and the
+host-only pool test library used by the CPU tests.
 """
 import argparse
 import concurrent.futures
@@ -19,7 +19,7 @@ CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "_obj")
 LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libc_runtime_api.so")
-CALLS = os.path.join(HERE, "_calls.so")
+CALLS = os.path.join(HERE, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))     # of this Python: another finds none and has its own built
 POOL_TEST_LIB = os.path.join(LIBDIR, "libtsplit_pool_host.so")
 
 HIPCC = os.environ.get("HIPCC", shutil.which("hipcc") or "/opt/rocm/bin/hipcc")
@@ -69,6 +69,9 @@ def build(force=False, jobs=8, verbose=True):
         if r.returncode != 0:
             raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     calls_src = os.path.join(CSRC, "python", "calls.cpp")
+    untagged = os.path.join(HERE, "_calls.so")       # as this module was once named: any Python would load it
+    if os.path.exists(untagged):
+        os.remove(untagged)
     if force or not os.path.exists(CALLS) or os.path.getmtime(CALLS) < max(os.path.getmtime(calls_src), hmtime):
         r = subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-Wall",
                             "-I" + sysconfig.get_paths()["include"], calls_src, "-o", CALLS], capture_output=True, text=True)
