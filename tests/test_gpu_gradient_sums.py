@@ -61,3 +61,38 @@ def test_branches_of_a_tape(stride, hw):
         return [q.grad.asnumpy() for q in p]
     for one, two in zip(gradients(True), gradients(False)):
         np.testing.assert_array_equal(one, two)
+
+
+# positions that no tap reaches, in whole words and value by value
+@pytest.mark.parametrize("n,c,h,w,o,s", [(2, 64, 28, 28, 128, 2), (3, 40, 15, 13, 70, 2), (2, 24, 14, 9, 1300, 2), (2, 64, 28, 28, 96, 1), (1, 33, 5, 7, 1500, 1)])
+def test_zeros_have_the_sign_that_the_two_calls_give_them(n, c, h, w, o, s):
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    rng, ctx = np.random.default_rng(n + c + h + o + s), nd.gpu(0)
+    f, dy = rng.standard_normal((o, c, 1, 1), dtype=np.float32), rng.standard_normal((n, o, (h - 1) // s + 1, (w - 1) // s + 1), dtype=np.float32)
+    f[:, ::3], dy[0] = 0, 0
+    a = np.where(rng.random((n, c, h, w)) < 0.5, np.float32(-0.0), np.float32(0.0))
+    f, dy, addend = (nd.array(v, ctx) for v in (f, dy, a))
+    alone, whole, apart = (nd.empty((n, c, h, w), ctx) for _ in range(3))
+    L.CuDNN_conv2d_gradient_of_data(f, dy, alone, 0, 0, s)
+    L.matrix_elementwise_add(addend, alone, whole)
+    L.conv2d_gradient_of_data_add(f, dy, addend, apart, 0, 0, s)
+    L.conv2d_gradient_of_data_add(f, dy, addend, addend, 0, 0, s)
+    for got in (apart, addend):
+        np.testing.assert_array_equal(got.asnumpy().view(np.uint32), whole.asnumpy().view(np.uint32))
+
+
+# images in runs of 3, 3 and 1, of 2, and one by one; not even one in reach: two calls
+@pytest.mark.parametrize("reach", [160_000, 110_000, 60_000, 20_000])
+@pytest.mark.parametrize("s", [1, 2])
+def test_runs_of_images(s, reach, monkeypatch):
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    rng, ctx, (n, c, h, o) = np.random.default_rng(s), nd.gpu(0), (7, 16, 20 * s, 32)
+    f, dy, a = (nd.array(rng.standard_normal(v, dtype=np.float32), ctx) for v in ((o, c, 1, 1), (n, o, 20, 20), (n, c, h, h)))
+    alone, whole, apart = (nd.empty((n, c, h, h), ctx) for _ in range(3))
+    monkeypatch.setenv("TSPLIT_CONV_REACH_BYTES", str(reach))
+    L.CuDNN_conv2d_gradient_of_data(f, dy, alone, 0, 0, s)
+    L.matrix_elementwise_add(a, alone, whole)
+    L.conv2d_gradient_of_data_add(f, dy, a, apart, 0, 0, s)
+    L.conv2d_gradient_of_data_add(f, dy, a, a, 0, 0, s)
+    for got in (apart, a):
+        np.testing.assert_array_equal(got.asnumpy(), whole.asnumpy())

@@ -295,7 +295,6 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             float(&w)[4] = v[e][j / 2][u];
-            w[0] = w[1] = w[2] = w[3] = 0.f;
             place(e, j, u, o, soff);
             if constexpr (ADD) gt::load_words<4>(from, o, soff, w);
           }
@@ -306,10 +305,9 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
 #pragma unroll
           for (int u = 0; u < 2; ++u) {
             float(&w)[4] = v[e][j / 2][u];
-            if (u == 0) {
-              w[0] = ADD ? w[0] + acc[tm][j][e] : acc[tm][j][e];
-              w[2] = ADD ? w[2] + acc[tm][j + 1][e] : acc[tm][j + 1][e];
-            }
+            const float made[4] = {u == 0 ? acc[tm][j][e] : 0.f, 0.f, u == 0 ? acc[tm][j + 1][e] : 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = ADD ? w[i] + made[i] : made[i];   // (zeros too: -0 + 0 is 0)
             place(e, j, u, o, soff);
             gt::store_words<4>(to, o, soff, w);
           }
@@ -324,7 +322,7 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
       const bool past = ragged && m + row + lane_row >= P.M;
       const int soff = past ? 0 : row * plane_bytes;   // (past M the product may leave 32 bits)
       unsigned o[TN][4];
-      float v[TN][4] = {};
+      float v[TN][4];
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const bool none = past || off[j] == kOobOffset;
@@ -339,9 +337,11 @@ __device__ __forceinline__ void spread(const Params &P, const Phase &F, const f3
       }
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
-        v[j][0] = ADD ? v[j][0] + acc[tm][j][e] : acc[tm][j][e];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j][i]), to, o[j][i] + soff, 0, 0);
+        for (int i = 0; i < 4; ++i) {
+          const float made = i == 0 ? acc[tm][j][e] : 0.f;
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ADD ? v[j][i] + made : made), to, o[j][i] + soff, 0, 0);
+        }
       }
     }
 }
