@@ -63,8 +63,9 @@ def test_branches_of_a_tape(stride, hw):
         np.testing.assert_array_equal(one, two)
 
 
-# positions that no tap reaches, in whole words and value by value
-@pytest.mark.parametrize("n,c,h,w,o,s", [(2, 64, 28, 28, 128, 2), (3, 40, 15, 13, 70, 2), (2, 24, 14, 9, 1300, 2), (2, 64, 28, 28, 96, 1), (1, 33, 5, 7, 1500, 1)])
+# positions that no tap reaches, in whole words and value by value, with the depth in one range and in several
+@pytest.mark.parametrize("n,c,h,w,o,s", [(2, 64, 28, 28, 32, 2), (3, 40, 15, 13, 30, 2), (2, 24, 14, 9, 32, 2), (2, 64, 28, 28, 128, 2), (2, 24, 14, 9, 1300, 2),
+                                         (2, 64, 28, 28, 32, 1), (1, 33, 5, 7, 1500, 1)])
 def test_zeros_have_the_sign_that_the_two_calls_give_them(n, c, h, w, o, s):
     from tsplit_amd import gpu_links as L, ndarray as nd
     rng, ctx = np.random.default_rng(n + c + h + o + s), nd.gpu(0)
