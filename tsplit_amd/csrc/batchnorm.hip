@@ -22,7 +22,8 @@
 // 1 us a direction), the stores.  Forward and gradient behind a Relu, against four waves a block
 // that loaded value by value: 16 x 128 x 32 x 32 12.9 and 16.1 -> 7.8 and 9.7 us, 32 x 192 x 17 x 17
 // 11.0 and 13.9 -> 7.6 and 9.2, 64 x 256 x 14 x 14 12.0 and 14.8 -> 8.6 and 11.1, 64 x 1024 x 14 x 14 28.9
-// and 56.6 -> 25.0 and 35.5 (5.8 TB/s of 12 B/elem would be 26.5), 64 x 512 x 7 x 7 6.9 and 9.0 -> 7.5 and 9.2.
+// and 56.6 -> 25.0 and 35.5 (5.8 TB/s of 12 B/elem would be 26.5).  The smallest channels skip the walk (kOwn below): replayed from a
+// graph, 64 x 512 x 7 x 7 6.4 and 8.7 -> 6.2 and 7.1 (through LDS 7.2 and 8.0), 4 x 64 x 7 x 7 3.7 and 4.3 -> 3.4 and 3.3 (4.8 and 5.4).
 #include <algorithm>
 
 #include "activations.h"
@@ -553,9 +554,10 @@ constexpr int kOnePassMax = 64 * kRow;   // elements per channel
 // Loaded that way, with a division and a 64-bit address a value in four waves, the loads were what took the time.  So wave w of W holds the
 // rows w, w + W, ..., four values a lane, and hands them, two rows of every wave at a time, through LDS to the 256 threads that add.
 // A lane's four values are one word where planes are of whole words, else they lie 64 apart (words that run over the edge of a plane into
-// the next, with a second load and a join, took 8.5 us for 7.5 at 32 x 192 x 17 x 17).  kFar: 64 apart, by 64-bit addresses, where a row's
-// planes lie 2 GiB and more apart.
-enum Layout { kWords, kValues, kFar };
+// the next, with a second load and a join, took 8.5 us for 7.5 at 32 x 192 x 17 x 17).  kOwn: of four waves each thread loads the values that
+// it adds, those of four rows a register group, and nothing goes through LDS: the least for up to 8 rows, and for up to 16 of single values.
+// kFar: 64 apart, by 64-bit addresses, where a row's planes (kOwn: those of four rows) lie 2 GiB and more apart.
+enum Layout { kWords, kValues, kOwn, kFar };
 template <int W, int LAYOUT>
 struct Rows {
   FastDiv hw;
@@ -569,11 +571,15 @@ struct Rows {
     lane = threadIdx.x & 63;
     left = static_cast<int64_t>(m) * C - static_cast<int64_t>(c) * hw.d;
   }
-  // the lane's value i of row r of this wave, m and more where there is none
-  __device__ __forceinline__ uint32_t value(uint32_t r, uint32_t i) const { return (r * W + wave) * kRow + (LAYOUT == kWords ? 4 * lane + i : 64 * i + lane); }
+  // of row r of this wave, or of the rows 4 r on (kOwn), the first value
+  __device__ __forceinline__ uint32_t first_of(uint32_t r) const { return (LAYOUT == kOwn ? 4 * r : r * W + wave) * kRow; }
+  // the lane's value i there, m and more where there is none
+  __device__ __forceinline__ uint32_t value(uint32_t r, uint32_t i) const {
+    return first_of(r) + (LAYOUT == kOwn ? kRow * i + threadIdx.x : LAYOUT == kWords ? 4 * lane + i : 64 * i + lane);
+  }
   // a buffer from the first plane of row r on, and the byte offset of value e in it (out of range where there is none)
   __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const float *p, uint32_t r, uint32_t &n0) const {
-    const uint32_t first = (r * W + wave) * kRow;
+    const uint32_t first = first_of(r);
     n0 = hw.div(first < m ? first : 0);
     const int64_t before = static_cast<int64_t>(n0) * C * hw.d, bytes = (left - before) * 4;
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p) + static_cast<int64_t>(c) * hw.d + before, 0,
@@ -627,6 +633,23 @@ struct Rows {
 // threads with each thread's value of every array.
 template <int R, int ARRAYS, int W, int LAYOUT, class Value, class Add>
 __device__ __forceinline__ void in_rows(const Rows<W, LAYOUT> &rows, float (*stage)[ARRAYS][2 * W][kRow], Value value, Add add) {
+  if constexpr (LAYOUT == kOwn) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      if (r >= static_cast<int>(rows.per)) break;
+      f32x4 v[ARRAYS];
+#pragma unroll
+      for (int k = 0; k < ARRAYS; ++k) v[k] = value(k, r);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float u[ARRAYS];
+#pragma unroll
+        for (int k = 0; k < ARRAYS; ++k) u[k] = v[k][i];
+        add(4 * r + i, u);
+      }
+    }
+    return;
+  }
 #pragma unroll
   for (int b = 0; b < R; b += 2) {
     if (b >= static_cast<int>(rows.per)) break;
@@ -830,33 +853,40 @@ __global__ __launch_bounds__(W *kWave) void bn_bwd_onepass_kernel(const float *_
   }
 }
 
-// a one-pass kernel by the size of a channel: four waves of 4 rows, or eight of 4, 5, 7 or 8 (a wave's rows that do not exist cost what others do:
-// 32 x 192 x 17 x 17 as 8 x 8 rows 8.7 us, as 8 x 5 7.6)
-#define BN_ONEPASS_SIZE(LAUNCH, LAYOUT, ...) \
+// a one-pass kernel by the size of a channel: four waves of 1, 2 or 4 rows, or eight of 4 to 8.  A wave's rows that do not exist cost what others
+// do: 32 x 192 x 17 x 17 as 8 x 8 rows 8.7 us, as 8 x 5 7.6; 32 x 256 x 19 x 19 as 8 x 7 9.9, as 8 x 6 9.1; 16 x 200 x 9 x 9 as 4 x 4 4.5, as 4 x 2 4.0.
+// kOwn for words up to 8 rows: 32 x 1536 x 8 x 8 forward 6.7, here 6.2, gradient 9.8, here 8.3; 64 x 512 x 2 x 2 5.6 and 6.5, here 5.1 and 6.1.
+#define BN_ONEPASS_SIZE(LAUNCH, SMALL, LAYOUT, ...) \
   do {                                       \
-    if (m <= 16 * kRow)                      \
-      LAUNCH(4, 4, LAYOUT, __VA_ARGS__);     \
+    if (m <= 4 * kRow)                       \
+      LAUNCH(4, 1, kOwn, __VA_ARGS__);       \
+    else if (m <= 8 * kRow)                  \
+      LAUNCH(4, 2, kOwn, __VA_ARGS__);       \
+    else if (m <= 16 * kRow)                 \
+      LAUNCH(4, 4, SMALL, __VA_ARGS__);      \
     else if (m <= 32 * kRow)                 \
       LAUNCH(8, 4, LAYOUT, __VA_ARGS__);     \
     else if (m <= 40 * kRow)                 \
       LAUNCH(8, 5, LAYOUT, __VA_ARGS__);     \
+    else if (m <= 48 * kRow)                 \
+      LAUNCH(8, 6, LAYOUT, __VA_ARGS__);     \
     else if (m <= 56 * kRow)                 \
       LAUNCH(8, 7, LAYOUT, __VA_ARGS__);     \
     else                                     \
       LAUNCH(8, 8, LAYOUT, __VA_ARGS__);     \
   } while (0)
-#define BN_ONEPASS(LAUNCH, ...)                       \
-  do {                                                \
-    if (rows_far(m, hw, C))                           \
-      LAUNCH(8, 8, kFar, __VA_ARGS__);                \
-    else if (hw % 4 == 0)                             \
-      BN_ONEPASS_SIZE(LAUNCH, kWords, __VA_ARGS__);   \
-    else                                              \
-      BN_ONEPASS_SIZE(LAUNCH, kValues, __VA_ARGS__);  \
+#define BN_ONEPASS(LAUNCH, ...)                             \
+  do {                                                      \
+    if (rows_far(m, hw, C))                                 \
+      LAUNCH(8, 8, kFar, __VA_ARGS__);                      \
+    else if (hw % 4 == 0)                                   \
+      BN_ONEPASS_SIZE(LAUNCH, kWords, kWords, __VA_ARGS__); \
+    else                                                    \
+      BN_ONEPASS_SIZE(LAUNCH, kOwn, kValues, __VA_ARGS__);  \
   } while (0)
-// the last plane of a row beyond 32-bit byte offsets from its first one
+// the last plane of a row, or of kOwn's four, beyond 32-bit byte offsets from its first one
 inline bool rows_far(int64_t m, int64_t hw, int64_t C) {
-  const int64_t planes = std::min(m / hw, kRow / hw + 2);
+  const int64_t values = m <= (hw % 4 ? 16 : 8) * kRow ? 4 * kRow : kRow, planes = std::min(m / hw, values / hw + 2);
   return ((planes - 1) * C + 1) * hw * 4 >= (1ll << 31);
 }
 
