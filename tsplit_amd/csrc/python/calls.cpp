@@ -109,7 +109,8 @@ int array_clear(Array *a) {
   return 0;
 }
 void array_dealloc(Array *a) {
-  if (PyObject_CallFinalizerFromDealloc(reinterpret_cast<PyObject *>(a))) return;
+  // (a subclass's own deallocation has run the finalizer)
+  if (Py_TYPE(a) == &ArrayType && PyObject_CallFinalizerFromDealloc(reinterpret_cast<PyObject *>(a))) return;
   PyObject_GC_UnTrack(a);
   array_clear(a);
   Py_TYPE(a)->tp_free(reinterpret_cast<PyObject *>(a));
@@ -117,9 +118,11 @@ void array_dealloc(Array *a) {
 
 // the address a ctypes pointer holds
 bool pointer_of(PyObject *p, void **out) {
-  const int is = PyObject_IsInstance(p, g_pointers);
-  if (is <= 0) {
-    if (!is) PyErr_Format(PyExc_TypeError, "a pointer, not %R", p);
+  bool is = false;   // (PyObject_IsInstance would look for __instancecheck__ each time)
+  for (Py_ssize_t i = 0; g_pointers && !is && i < PyTuple_GET_SIZE(g_pointers); ++i)
+    is = PyObject_TypeCheck(p, reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(g_pointers, i)));
+  if (!is) {
+    PyErr_Format(PyExc_TypeError, "a pointer, not %R", p);
     return false;
   }
   Py_buffer b;
@@ -250,8 +253,7 @@ PyObject *new_array(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_RuntimeError, "the library is not bound");
     return nullptr;
   }
-  const int is = PyObject_IsInstance(args[2], g_context);
-  if (is <= 0) return is ? nullptr : PyErr_Format(PyExc_TypeError, "ctx is a DLContext, not %R", args[2]);
+  if (!PyObject_TypeCheck(args[2], reinterpret_cast<PyTypeObject *>(g_context))) return PyErr_Format(PyExc_TypeError, "ctx is a DLContext, not %R", args[2]);
   Py_buffer b;
   if (PyObject_GetBuffer(args[2], &b, PyBUF_SIMPLE)) return nullptr;
   DLContext ctx{};
