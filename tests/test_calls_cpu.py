@@ -138,3 +138,12 @@ def test_the_module_is_of_this_python():
     from tsplit_amd import build
     assert _calls.__file__ == build.CALLS and _calls.__file__.endswith(sysconfig.get_config_var("EXT_SUFFIX"))
     assert not os.path.exists(os.path.join(os.path.dirname(build.CALLS), "_calls.so"))
+
+
+def test_a_pointer_may_be_filled_in_after_the_array_was_made():
+    h = nd.DLArrayHandle()
+    a = nd.NDArray(h)
+    with pytest.raises(AttributeError):
+        a.shape
+    assert _LIB.DLArrayAlloc((ctypes.c_int64 * 2)(2, 3), ctypes.c_int64(2), nd.cpu(0), ctypes.byref(h), ctypes.c_int(1)) == 0
+    assert a.shape == (2, 3) and a.data_ptr == h.contents.data

@@ -48,6 +48,34 @@ bool current_rule(int &rule) {
   return !(rule == -1 && PyErr_Occurred());
 }
 
+// the address a ctypes pointer holds
+bool pointer_of(PyObject *p, void **out) {
+  bool is = false;   // (PyObject_IsInstance would look for __instancecheck__ each time)
+  for (Py_ssize_t i = 0; g_pointers && !is && i < PyTuple_GET_SIZE(g_pointers); ++i)
+    is = PyObject_TypeCheck(p, reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(g_pointers, i)));
+  if (!is) {
+    PyErr_Format(PyExc_TypeError, "a pointer, not %R", p);
+    return false;
+  }
+  Py_buffer b;
+  if (PyObject_GetBuffer(p, &b, PyBUF_SIMPLE)) return false;
+  const bool ok = b.len == static_cast<Py_ssize_t>(sizeof(void *));
+  if (ok) *out = *static_cast<void **>(b.buf);
+  PyBuffer_Release(&b);
+  if (!ok) PyErr_SetString(PyExc_TypeError, "not a pointer");
+  return ok;
+}
+
+// the array's DLArray (a pointer object that it was given may have been filled in since)
+DLArray *raw_of(Array *a) {
+  void *p = nullptr;
+  if (!a->raw && a->handle && a->handle != Py_None) {
+    if (pointer_of(a->handle, &p)) a->raw = static_cast<DLArray *>(p);
+    PyErr_Clear();
+  }
+  return a->raw;
+}
+
 int array_traverse(Array *a, visitproc visit, void *arg) {
   Py_VISIT(a->handle);
   Py_VISIT(a->owner);
@@ -64,11 +92,11 @@ int array_traverse(Array *a, visitproc visit, void *arg) {
 // Gives the memory back, once.  A finalizer: it runs for every array of a collected cycle before anything of the cycle is cleared, a
 // recording's keeper among it (a view's memory is its owner's, which may go first).
 void array_finalize(Array *a) {
-  DLArray *raw = a->raw;
-  a->raw = nullptr;
-  if (!raw) return;
   PyObject *type, *value, *trace;
   PyErr_Fetch(&type, &value, &trace);
+  DLArray *raw = raw_of(a);
+  a->raw = nullptr;
+  if (!raw) return PyErr_Restore(type, value, trace);
   int rule = 0;
   bool mine = true;
   if (!current_rule(rule)) {
@@ -80,7 +108,8 @@ void array_finalize(Array *a) {
     mine = false;
   } else if (a->keeper && a->keeper != Py_None && raw->ctx.device_type == kGPU) {
     // an array born inside a recorded step outlives this object: the graph replays into it
-    PyObject *handle = a->handle && a->handle != Py_None ? (Py_INCREF(a->handle), a->handle) : PyObject_CallFunction(g_handle_of, "n", reinterpret_cast<Py_ssize_t>(raw));
+    PyObject *handle = a->handle && a->handle != Py_None ? (Py_INCREF(a->handle), a->handle)
+                                                         : PyObject_CallFunction(g_handle_of, "n", reinterpret_cast<Py_ssize_t>(raw));
     PyObject *taken = handle ? PyObject_CallMethodObjArgs(a->keeper, g_take_name, handle, PyDict_GetItem(g_rules, g_rule_name), nullptr) : nullptr;
     if (!taken) PyErr_WriteUnraisable(a->keeper);
     mine = taken && !PyObject_IsTrue(taken);
@@ -114,24 +143,6 @@ void array_dealloc(Array *a) {
   PyObject_GC_UnTrack(a);
   array_clear(a);
   Py_TYPE(a)->tp_free(reinterpret_cast<PyObject *>(a));
-}
-
-// the address a ctypes pointer holds
-bool pointer_of(PyObject *p, void **out) {
-  bool is = false;   // (PyObject_IsInstance would look for __instancecheck__ each time)
-  for (Py_ssize_t i = 0; g_pointers && !is && i < PyTuple_GET_SIZE(g_pointers); ++i)
-    is = PyObject_TypeCheck(p, reinterpret_cast<PyTypeObject *>(PyTuple_GET_ITEM(g_pointers, i)));
-  if (!is) {
-    PyErr_Format(PyExc_TypeError, "a pointer, not %R", p);
-    return false;
-  }
-  Py_buffer b;
-  if (PyObject_GetBuffer(p, &b, PyBUF_SIMPLE)) return false;
-  const bool ok = b.len == static_cast<Py_ssize_t>(sizeof(void *));
-  if (ok) *out = *static_cast<void **>(b.buf);
-  PyBuffer_Release(&b);
-  if (!ok) PyErr_SetString(PyExc_TypeError, "not a pointer");
-  return ok;
 }
 
 int array_init(Array *a, PyObject *args, PyObject *kwargs) {
@@ -173,17 +184,19 @@ int set_handle(Array *a, PyObject *v, void *) {
   return 0;
 }
 PyObject *get_shape(Array *a, void *) {
-  if (!a->raw) {
+  const DLArray *raw = raw_of(a);
+  if (!raw) {
     PyErr_SetString(PyExc_AttributeError, "the array has no handle");
     return nullptr;
   }
-  PyObject *t = PyTuple_New(a->raw->ndim);
-  for (int i = 0; t && i < a->raw->ndim; ++i) PyTuple_SET_ITEM(t, i, PyLong_FromLongLong(a->raw->shape[i]));
+  PyObject *t = PyTuple_New(raw->ndim);
+  for (int i = 0; t && i < raw->ndim; ++i) PyTuple_SET_ITEM(t, i, PyLong_FromLongLong(raw->shape[i]));
   return t;
 }
 PyObject *get_data_ptr(Array *a, void *) {
-  if (!a->raw || !a->raw->data) Py_RETURN_NONE;
-  return PyLong_FromVoidPtr(a->raw->data);
+  const DLArray *raw = raw_of(a);
+  if (!raw || !raw->data) Py_RETURN_NONE;
+  return PyLong_FromVoidPtr(raw->data);
 }
 // attributes with a default that is made when first read (a list, a dict) or is the same for all
 enum Default { kNone, kFalse, kTrue, kOne, kList, kDict };
@@ -331,7 +344,7 @@ template <>
 struct Arg<DLArrayHandle> {
   static bool get(PyObject *o, bool optional, DLArrayHandle &v) {
     if (PyObject_TypeCheck(o, &ArrayType)) {
-      v = reinterpret_cast<Array *>(o)->raw;
+      v = raw_of(reinterpret_cast<Array *>(o));
       return true;
     }
     v = nullptr;
@@ -409,7 +422,7 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
   X(DLGpuAvgerage_Pooling2d, 0) X(DLGpuAvgerage_Pooling2d_gradient, 0) X(CuDNN_DLGpuAvgerage_Pooling2d, 0)                                     \
   X(CuDNN_DLGpuAvgerage_Pooling2d_gradient, 0) X(DLGpuBroadcastTo, 0) X(DLGpuReduceSumAxisZero, 0) X(DLGpuConv2d_broadcast_to, 0)              \
   X(DLGpuConv2d_reduce_sum, 0) X(DLGpuBatchMatrixMultiply, 0) X(DLGpuOneHot, 0) X(DLGpuWhere, 0) X(DLGpuEmbeddingLookUp, 0)                    \
-  X(DLGpuEmbeddingLookUp_Gradient, 0) X(DLGpuTanh, 0) X(DLGpuSigmoid, 0) X(TSplit_BatchNormRelu, 0) X(TSplit_BatchNormReluAdd, 0)                                            \
+  X(DLGpuEmbeddingLookUp_Gradient, 0) X(DLGpuTanh, 0) X(DLGpuSigmoid, 0) X(TSplit_BatchNormRelu, 0) X(TSplit_BatchNormReluAdd, 0)              \
   X(TSplit_BatchNormThenRelu, 1 << 7 | 1 << 8) X(TSplit_BatchNormThenRelu_gradient, 1 << 9 | 1 << 10) X(TSplit_Conv2dBatchNormStats, 0)        \
   X(TSplit_BatchNormFromStats, 1 << 7 | 1 << 8) X(TSplit_BatchNormRelu_gradient, 0) X(DLGpuConcat, 0) X(DLGpuConcat_gradient, 0)
 
