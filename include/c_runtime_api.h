@@ -500,7 +500,8 @@ int TSplit_BatchNormReluMaxPool_gradient(const DLArrayHandle gradient_Y, const D
 
 /* ---- gradient_x = the convolution's data gradient + addend (of gradient_x's size; it may be gradient_x): a gradient of several
  *      terms without a pass of its own (outside the reference's ABI, whose graph sums them with DLGpuMatrixElementwiseAdd: the
- *      same bits).  In one launch for 1 x 1 filters of stride 1 and 2 without padding, else in the two it stands for. ---- */
+ *      same bits).  1 x 1 filters of stride 1 and 2 without padding: in the gradient's own launches (one, with the depth in ranges their
+ *      fold's; for each run of images that 32-bit offsets reach), else in the two calls it stands for. ---- */
 int TSplit_Conv2dGradientOfDataAdd(const DLArrayHandle input_f, const DLArrayHandle gradient_y, const DLArrayHandle addend,
                                    DLArrayHandle gradient_x, const int padding, const int padding2, const int stride,
                                    DLStreamHandle stream_handle);

@@ -1239,19 +1239,28 @@ static void bn_apply_from(const double *part, int S, int64_t part_c, int64_t par
   if (plane_major_ok(ap, x, pg, blocks)) {
     const f32x4 *xw = reinterpret_cast<const f32x4 *>(x->data);
     f32x4 *yw = reinterpret_cast<f32x4 *>(y->data), *rw = reinterpret_cast<f32x4 *>(r);
-    const auto kernel = relu == kBoth ? bn_apply_plane_kernel<kBoth> : relu == kSum ? bn_apply_plane_kernel<kSum> : relu == kFused ? bn_apply_plane_kernel<kFused> : bn_apply_plane_kernel<kAlone>;
+    const auto kernel = relu == kBoth    ? bn_apply_plane_kernel<kBoth>
+                        : relu == kSum   ? bn_apply_plane_kernel<kSum>
+                        : relu == kFused ? bn_apply_plane_kernel<kFused>
+                                         : bn_apply_plane_kernel<kAlone>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, xw, yw, rw, coef, pg);
     return;
   }
   if (edges_ok(ap, x, aligned16(x->data) && aligned16(y->data) && aligned16(r), pg, blocks)) {
-    const auto kernel = relu == kBoth ? bn_apply_edges_kernel<kBoth> : relu == kSum ? bn_apply_edges_kernel<kSum> : relu == kFused ? bn_apply_edges_kernel<kFused> : bn_apply_edges_kernel<kAlone>;
+    const auto kernel = relu == kBoth    ? bn_apply_edges_kernel<kBoth>
+                        : relu == kSum   ? bn_apply_edges_kernel<kSum>
+                        : relu == kFused ? bn_apply_edges_kernel<kFused>
+                                         : bn_apply_edges_kernel<kAlone>;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), pg);
     return;
   }
   const dim3 ga(ap.S, C);
 #define BN_APPLY(V)                                                                                                                        \
-  hipLaunchKernelGGL((relu == kBoth ? bn_apply_kernel<V, kBoth> : relu == kSum ? bn_apply_kernel<V, kSum>                                  \
-                                    : relu == kFused ? bn_apply_kernel<V, kFused> : bn_apply_kernel<V, kAlone>), ga, dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), ap.g)
+  hipLaunchKernelGGL((relu == kBoth    ? bn_apply_kernel<V, kBoth>                                                                         \
+                      : relu == kSum   ? bn_apply_kernel<V, kSum>                                                                          \
+                      : relu == kFused ? bn_apply_kernel<V, kFused>                                                                        \
+                                       : bn_apply_kernel<V, kAlone>),                                                                      \
+                     ga, dim3(kThreads), 0, s, cf(x), mf(y), r, static_cast<const float *>(coef), ap.g)
   if (ap.vec == 4)
     BN_APPLY(4);
   else
@@ -1271,7 +1280,8 @@ static int bn_forward(const char *who, int relu, const DLArrayHandle input_X, co
   TS_REQUIRE(relu != kBoth || (relu_R && pair_arr && numel(relu_R) == numel(input_X) && numel(pair_arr) == 2 * C &&
                                relu_R->data != output_Y->data && relu_R->data != input_X->data),
              "%s: Relu's result is another array of the input's size, the pair's coefficients take 2 C elements", who);
-  TS_REQUIRE(relu != kSum || (relu_R && numel(relu_R) == numel(input_X) && relu_R->data != output_Y->data), "%s: the addend is another array of the input's size", who);
+  TS_REQUIRE(relu != kSum || (relu_R && numel(relu_R) == numel(input_X) && relu_R->data != output_Y->data),
+             "%s: the addend is another array of the input's size", who);
   float *const r = relu == kBoth || relu == kSum ? mf(relu_R) : nullptr, *const pair = relu == kBoth ? mf(pair_arr) : nullptr;
   TS_REQUIRE(stats_fit(save_mean_arr, save_var_arr, C, fused_of(relu)), "%s: save_mean and save_var must hold C elements each", who);
   TS_REQUIRE(!fused_of(relu) || (save_mean_arr && save_var_arr), "%s: the fused form needs both save arrays", who);

@@ -1487,7 +1487,7 @@ int conv_forward(const char *who, const DLArray *x, const DLArray *w, DLArray *y
   return ps.finish();
 }
 
-// added: what the gradient is added to (it may be dx), or null.  Only one launch of the tile kernel adds: elsewhere 1 is
+// added: what the gradient is added to (it may be dx), or null.  Only the tile kernel's launches add: elsewhere 1 is
 // returned, nothing launched.
 int conv_bwd_data(const char *who, const DLArray *w, const DLArray *dy, DLArray *dx, int ph, int pw, int s,
                   DLStreamHandle sh, ProfilerHandle p, const DLArray *added = nullptr) {

@@ -428,7 +428,9 @@ __global__ __launch_bounds__(gt::kThreads, 2) void conv_tile_kernel(Params P, in
           gt::store_words<TN>(to, past ? kOobOffset : off[0], soff, v);
         } else {
 #pragma unroll
-          for (int j = 0; j < TN; ++j) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[tm][j][e]), to, (past ? kOobOffset : off[j]) + (kRagged ? soff : 0), kRagged ? 0 : soff, 0);
+          for (int j = 0; j < TN; ++j)
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[tm][j][e]), to, (past ? kOobOffset : off[j]) + (kRagged ? soff : 0),
+                                                  kRagged ? 0 : soff, 0);
         }
       }
   };

@@ -109,7 +109,8 @@ template <int TM, int TN, bool TA, bool TB, bool SUMS>
 void launch_waves_tile(const float *A, int64_t lda, const float *B, int64_t ldb, float *out, int64_t ldc, const gt::BatchOf &zs, int batch, int M, int N,
                        int K, const gt::Epilogue &ep, float *sums, const WavesPlan &p, hipStream_t s) {
   const int tm = (M + 16 * TM - 1) / (16 * TM), tn = (N + 16 * TN - 1) / (16 * TN);
-  const bool wide = TN > 1 && N % 2 == 0 && ldc % 2 == 0 && zs.co % 2 == 0 && zs.ci % 2 == 0 && aligned16(out) && aligned16(ep.add) && aligned16(ep.relu) && aligned16(ep.gate);
+  const bool wide = TN > 1 && N % 2 == 0 && ldc % 2 == 0 && zs.co % 2 == 0 && zs.ci % 2 == 0 && aligned16(out) && aligned16(ep.add) &&
+                    aligned16(ep.relu) && aligned16(ep.gate);
   const size_t lds = static_cast<size_t>(p.S) * (256 * TM * TN + (SUMS ? 16 * TN : 0)) * sizeof(float);
   hipLaunchKernelGGL((gw::gemm_waves_kernel<TM, TN, TA, TB, SUMS>), dim3(grid_blocks(tm, tn, batch)), dim3(64 * p.waves), lds, s, DenseParams{A, lda, M, K},
                      DenseParams{B, ldb, N, K}, out, ldc, zs, ep, sums, wide, M, N, K, p.S, p.kchunk, TileGrid{tm, tn, tm * tn * batch});
@@ -153,8 +154,8 @@ int launch_product(const float *A, int64_t lda, const float *B, int64_t ldb, flo
   return 0;
 }
 
-// C = A^T B and the column sums of B on the tile kernel, in ranges of up to kSumsRange rows: a lane's sums of a range are a chain of a
-// rounding every 256 rows, the reduction's are cut finer the more rows there are.  Error of the sums against float64 (normal values, as a share of
+// C = A^T B and the column sums of B, in ranges of up to kSumsRange rows: on either kernel a lane's sums of a range are a chain of a
+// rounding every 256 rows (the same bits), the reduction's are cut finer the more rows there are.  Error of the sums against float64 (normal values, as a share of
 // the root of the rows) in ranges of 11 K rows 1.6e-7, as a reduction 2.4e-7; of 33 K 2.3 and 2.2, of 87 K 3.7 and 3.1.  Nor is there time to be
 // gained beyond: 262144 x 1024 and 1024 columns 4145 us, as two calls 4029.
 constexpr int kSumsRange = 16384;

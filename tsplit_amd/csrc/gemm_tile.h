@@ -278,60 +278,15 @@ struct Core {
     la.load(kbegin, kend, lds_at);
     lb.load(kbegin, kend, lds_at + AL::kFloats * 4);
     int stage = 0;
-    if constexpr (SPREAD) {
-      // A step with the next step's loads between the products.  A load takes the memory pipeline 16 clocks whatever its width, and a wave
-      // issues in order: 8 to 16 loads of 4 bytes a lane in one burst behind the barrier kept it from its next product until the last
-      // was taken.  Two to four behind each quarter of the products: 3x3 of 35 x 35 70.1 -> 63.5 us, 17 x 17 of several taps 69.1 -> 59.5,
-      // 512 -> 512 of 28 x 28, 18 images 558 -> 497, its filter gradient 570 -> 525, stride-2 data gradients 0.91-0.94 of the time, filter gradients 0.92-0.97.
-      // Operands in words (2 to 8 loads a step) and one-tap gathers, which have no choice of offsets to make, gained nothing either
-      // way, nor did the LDS reads between products.  The first step has no products to put loads between, the last none to ask for:
-      // forms of their own, since a branch between products costs registers (108 -> 149 on 128 x 64).
-      auto step = [&](int k0, auto first, auto more) {
-        if (la.cut(k0, kend) || lb.cut(k0, kend)) {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          la.clear_tail(k0, kend, lds + stage * kStage);
-          lb.clear_tail(k0, kend, lds + stage * kStage + AL::kFloats);
-        }
-        lds_ready();
-        const float *sa = lds + stage * kStage, *sb = sa + AL::kFloats;
-        stage ^= 1;
-        auto part = [&](int i) {
-          if constexpr (decltype(more)::value) {
-            if (i == 0) la.load(k0 + BK, kend, lds_at + stage * kStage * 4);
-            lb.part(i);
-          }
-        };
-        if constexpr (decltype(more)::value) lb.prepare(k0 + BK, kend, lds_at + (stage * kStage + AL::kFloats) * 4);
-        AL::frag(sa, wm0, 0, lane, a0);
-        BL::frag(sb, wn0, 0, lane, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        if constexpr (decltype(first)::value) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) part(i);
-        } else {
-          products_and<TM, TN>(a1, b1, acc, part);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        AL::frag(sa, wm0, 1, lane, a1);
-        BL::frag(sb, wn0, 1, lane, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        products<TM, TN>(a0, b0, acc);
-        __builtin_amdgcn_sched_barrier(0);
-      };
-      const std::true_type yes{};
-      const std::false_type no{};
-      int k0 = kbegin;
-      if (k0 + BK >= kend) {
-        step(k0, yes, no);
-      } else {
-        step(k0, yes, yes);
-        for (k0 += BK; k0 + BK < kend; k0 += BK) step(k0, no, yes);
-        step(k0, no, no);
-      }
-      products<TM, TN>(a1, b1, acc);
-      return;
-    }
-    for (int k0 = kbegin; k0 < kend; k0 += BK) {
+    // SPREAD: the next step's loads of B between the products.  A load takes the memory pipeline 16 clocks whatever its width, and a wave
+    // issues in order: 8 to 16 loads of 4 bytes a lane in one burst behind the barrier kept it from its next product until the last
+    // was taken.  Two to four behind each quarter of the products: 3x3 of 35 x 35 70.1 -> 63.5 us, 17 x 17 of several taps 69.1 -> 59.5,
+    // 512 -> 512 of 28 x 28, 18 images 558 -> 497, its filter gradient 570 -> 525, stride-2 data gradients 0.91-0.94 of the time, filter
+    // gradients 0.92-0.97.  Operands in words (2 to 8 loads a step) and one-tap gathers, which have no choice of offsets to make, gained
+    // nothing either way, nor did the LDS reads between products.  The first step has no products to put loads between, the last none to
+    // ask for: forms of their own (`first`, `more` are types then), since a branch between products costs registers (108 -> 149 on 128 x 64).
+    static_assert(!(SPREAD && SUMS), "loads between products leave no column sums");
+    auto step = [&](int k0, auto first, auto more) {
       if (la.cut(k0, kend) || lb.cut(k0, kend)) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         la.clear_tail(k0, kend, lds + stage * kStage);
@@ -340,14 +295,31 @@ struct Core {
       lds_ready();
       const float *sa = lds + stage * kStage, *sb = sa + AL::kFloats;
       stage ^= 1;
-      if (k0 + BK < kend) {
-        la.load(k0 + BK, kend, lds_at + stage * kStage * 4);
-        lb.load(k0 + BK, kend, lds_at + (stage * kStage + AL::kFloats) * 4);
+      const unsigned next_a = lds_at + stage * kStage * 4, next_b = next_a + AL::kFloats * 4;
+      if (more) {
+        if constexpr (SPREAD) {
+          lb.prepare(k0 + BK, kend, next_b);
+        } else {
+          la.load(k0 + BK, kend, next_a);
+          lb.load(k0 + BK, kend, next_b);
+        }
       }
       AL::frag(sa, wm0, 0, lane, a0);
       BL::frag(sb, wn0, 0, lane, b0);
       __builtin_amdgcn_sched_barrier(0);
-      if (k0 != kbegin) {
+      if constexpr (SPREAD) {
+        auto part = [&](int i) {
+          if (!more) return;
+          if (i == 0) la.load(k0 + BK, kend, next_a);
+          lb.part(i);
+        };
+        if (first) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) part(i);
+        } else {
+          products_and<TM, TN>(a1, b1, acc, part);
+        }
+      } else if (!first) {
         products<TM, TN>(a1, b1, acc);
         add(b1);
         if constexpr (SUMS)
@@ -366,6 +338,20 @@ struct Core {
       products<TM, TN>(a0, b0, acc);
       add(b0);
       __builtin_amdgcn_sched_barrier(0);
+    };
+    if constexpr (SPREAD) {
+      const std::true_type yes{};
+      const std::false_type no{};
+      int k0 = kbegin;
+      if (k0 + BK >= kend) {
+        step(k0, yes, no);
+      } else {
+        step(k0, yes, yes);
+        for (k0 += BK; k0 + BK < kend; k0 += BK) step(k0, no, yes);
+        step(k0, no, no);
+      }
+    } else {
+      for (int k0 = kbegin; k0 < kend; k0 += BK) step(k0, k0 == kbegin, k0 + BK < kend);
     }
     // (a depth whose last half step is all zeros: 100 x 4096' x 4096 46 -> 43 us; convolutions' depths are cut and padded otherwise, and gained
     // nothing)

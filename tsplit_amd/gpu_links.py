@@ -28,7 +28,8 @@ __all__ = [
     "matrix_transpose", "batch_matrix_multiply", "one_hot", "where", "embedding_lookup",
     "embedding_lookup_gradient", "matrix_elementwise_divide", "matrix_elementwise_divide_const",
     "matrix_opposite", "matrix_sqrt", "matrix_rsqrt", "tanh", "sigmoid",
-    "batch_norm_relu", "batch_norm_relu_add", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient", "conv2d_batch_norm_stats", "batch_norm_from_stats",
+    "batch_norm_relu", "batch_norm_relu_add", "batch_norm_relu_gradient", "batch_norm_then_relu", "batch_norm_then_relu_gradient",
+    "conv2d_batch_norm_stats", "batch_norm_from_stats",
     "optimizer_update_multi", "conv2d_gradient_of_data_add", "matrix_multiply_add", "matrix_multiply_sums", "heads_matrix_multiply", "heads_scale",
     "softmax_cross_entropy_ids", "softmax_cross_entropy_ids_gradient", "embedding_add", "embedding_add_gradient",
     "join", "part", "lstm_sizes", "lstm", "lstm_gradient",
@@ -236,7 +237,8 @@ def CuDNN_Batch_Normalization(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_m
 def CuDNN_Batch_Normalization_gradient(in_gradient_y, in_arr_x, in_bn_scale, out_gradient_x,
                                        out_gradient_bn_scale, out_gradient_bn_bias, saved_mean, saved_var,
                                        eps=0.001, stream=None, profiler=None):
-    _calls.CuDNN_DLGpuBatch_Normalization_gradient(in_gradient_y, in_arr_x, in_bn_scale, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
+    _calls.CuDNN_DLGpuBatch_Normalization_gradient(in_gradient_y, in_arr_x, in_bn_scale, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias,
+                                                   eps, saved_mean, saved_var, stream, profiler)
 
 
 # ---- MaxPool (gpu_links/MaxPoolLink.py:8,15; gpu_links/CudnnMaxPoolLink.py:8,15) ----
@@ -534,7 +536,8 @@ def batch_norm_then_relu(in_arr, bn_scale_arr, bn_bias_arr, out_arr, relu_arr, p
 def batch_norm_then_relu_gradient(in_gradient, in_arr, in_bn_scale, pair, out_gradient_y, out_gradient_x, out_gradient_bn_scale,
                                   out_gradient_bn_bias, saved_mean=None, saved_var=None, eps=0.01, stream=None, profiler=None):
     """relu_gradient and CuDNN_Batch_Normalization_gradient in one call, with their bits; out_gradient_y: between the two."""
-    _calls.TSplit_BatchNormThenRelu_gradient(in_gradient, in_arr, in_bn_scale, pair, out_gradient_y, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
+    _calls.TSplit_BatchNormThenRelu_gradient(in_gradient, in_arr, in_bn_scale, pair, out_gradient_y, out_gradient_x, out_gradient_bn_scale,
+                                             out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
 
 
 def batch_norm_relu_max_pool(in_arr, bn_scale_arr, bn_bias_arr, out_arr, save_mean, save_var, eps=0.01, stats=None, slots=0,
@@ -574,4 +577,5 @@ def batch_norm_from_stats(in_arr, stats, slots, bn_scale_arr, bn_bias_arr, out_a
 
 def batch_norm_relu_gradient(in_gradient_y, in_arr_x, in_bn_scale, in_bn_bias, out_gradient_x, out_gradient_bn_scale,
                              out_gradient_bn_bias, saved_mean, saved_var, eps=0.01, stream=None, profiler=None):
-    _calls.TSplit_BatchNormRelu_gradient(in_gradient_y, in_arr_x, in_bn_scale, in_bn_bias, out_gradient_x, out_gradient_bn_scale, out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
+    _calls.TSplit_BatchNormRelu_gradient(in_gradient_y, in_arr_x, in_bn_scale, in_bn_bias, out_gradient_x, out_gradient_bn_scale,
+                                         out_gradient_bn_bias, eps, saved_mean, saved_var, stream, profiler)
