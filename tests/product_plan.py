@@ -14,7 +14,7 @@ extern "C" void plan(long long M, long long N, long long K, long long batch, int
   const int64_t cols = N;
   const int steps = std::max(1ll, (K + 31) / 32);
   const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, batch > 1 ? 1 : 64, static_cast<double>(M) * N, kProductCost);
-  const WavesPlan w = plan_waves(M, N, K, batch, t);
+  const WavesPlan w = plan_waves(M, N, K, batch, t, batch > 1);
   const int range = (steps + t.S - 1) / t.S * 32;
   const int values[] = {t.tile, range, w.tile, w.waves, w.S, w.kchunk};
   for (int i = 0; i < 6; ++i) got[i] = values[i];
@@ -42,6 +42,6 @@ def plan(M, N, K, batch=1):
     _library().plan(*(ctypes.c_longlong(v) for v in (M, N, K, batch)), got)
     tile, tile_range, wave_tile, waves, S, kchunk = got
     if waves:
-        assert S == -(-K // kchunk) and 2 <= waves <= 4
+        assert S == -(-K // kchunk) and waves in (4, max(2, min(4, S)))
         return Plan(waves, WAVE_TILES[wave_tile], kchunk, tile_range)
     return Plan(0, TILES[tile], tile_range, tile_range)

@@ -14,15 +14,16 @@ from test_gpu_product_tiles import _device
 EPS = 2.0 ** -24
 WAVES, TILE = "waves", "tile"
 # M, N, K, batch, kernel, its tile, ranges of the depth
-ONE = [(17, 31, 33, 1, WAVES, (16, 16), 2), (33, 67, 163, 1, WAVES, (16, 16), 6), (1, 1102, 2019, 1, WAVES, (16, 16), 64),
-       (1015, 259, 11, 1, WAVES, (16, 32), 1), (231, 1179, 35, 1, WAVES, (16, 32), 2), (51, 1053, 183, 1, WAVES, (16, 32), 6),
-       (887, 417, 113, 1, WAVES, (32, 16), 4), (1027, 97, 271, 1, WAVES, (32, 16), 5),
-       (133, 917, 485, 1, WAVES, (32, 32), 4), (139, 919, 263, 1, WAVES, (32, 32), 5),
+ONE = [(17, 31, 11, 1, WAVES, (16, 16), 1), (17, 31, 133, 1, WAVES, (16, 16), 1), (113, 127, 159, 1, WAVES, (16, 16), 1), (147, 823, 229, 1, WAVES, (16, 16), 4),
+       (33, 67, 163, 1, WAVES, (16, 16), 6), (1, 1102, 2019, 1, WAVES, (16, 16), 64),
+       (449, 145, 33, 1, WAVES, (16, 32), 1), (197, 1189, 271, 1, WAVES, (16, 32), 3), (51, 1053, 183, 1, WAVES, (16, 32), 6),
+       (597, 193, 61, 1, WAVES, (32, 16), 1), (755, 331, 333, 1, WAVES, (32, 16), 3), (1027, 97, 271, 1, WAVES, (32, 16), 5),
+       (393, 483, 263, 1, WAVES, (32, 32), 3), (139, 919, 263, 1, WAVES, (32, 32), 5),
        (363, 1089, 1, 1, TILE, (64, 64), 1), (895, 441, 47, 1, TILE, (64, 64), 1), (515, 2047, 70, 1, TILE, (64, 64), 1),
-       (1, 1, 1545, 1, TILE, (64, 64), 25), (31, 97, 4098, 1, TILE, (64, 64), 43), (129, 66, 2047, 1, TILE, (64, 64), 32),
+       (1, 1, 1545, 1, TILE, (64, 64), 25), (31, 97, 4098, 1, TILE, (64, 64), 43), (129, 66, 2047, 1, TILE, (64, 64), 32), (1, 3000, 16387, 1, TILE, (64, 64), 16),
        (839, 1189, 907, 1, TILE, (64, 128), 5)]
-MANY = [(1, 273, 11, 57, WAVES, (16, 32), 1), (1, 41, 143, 88, WAVES, (16, 32), 3), (149, 1, 41, 104, WAVES, (32, 16), 2), (21, 1, 299, 173, WAVES, (32, 16), 4),
-        (17, 101, 185, 153, WAVES, (32, 32), 3), (17, 79, 97, 219, WAVES, (32, 32), 4), (13, 29, 37, 6, WAVES, (16, 16), 2),
+MANY = [(13, 29, 37, 6, WAVES, (16, 16), 2), (1, 273, 11, 57, WAVES, (16, 32), 1), (1, 41, 143, 88, WAVES, (16, 32), 3), (287, 1, 53, 109, WAVES, (32, 16), 2),
+        (21, 1, 227, 138, WAVES, (32, 16), 4), (1025, 19, 265, 6, WAVES, (32, 32), 3), (55, 17, 337, 100, WAVES, (32, 32), 4),
         (300, 200, 5, 100, TILE, (64, 64), 1), (257, 255, 64, 256, TILE, (64, 64), 1), (257, 255, 67, 40, TILE, (64, 128), 1), (1, 557, 43, 90, TILE, (64, 128), 1),
         (665, 1, 39, 124, TILE, (128, 64), 1), (1043, 1091, 37, 6, TILE, (128, 128), 1), (256, 256, 64, 256, TILE, (128, 128), 1)]
 BOTH_WAYS = [(False, False), (False, True), (True, False), (True, True)]

@@ -1,7 +1,8 @@
-"""Small products (csrc/gemm_waves.h) are no further from float64 than the tile kernel's order of adding is: fused multiply-adds in fp32 along
-each of its ranges of the depth, the ranges' results added one by one.  That order is followed here value by value on the host.
+"""Small products (csrc/gemm_waves.h) have the bits of the tile kernel and its fold, and are no further from float64 than its order of adding is:
+fused multiply-adds in fp32 along each of its ranges of the depth, the ranges' results added one by one.  That order is followed here value by
+value on the host.
 
-Bar: 1.15 times its rms error.  The matrix instruction may add the four products of a step in another order, which moves a single value's
+Bar of the latter: 1.15 times its rms error.  The matrix instruction may add the four products of a step in another order, which moves a single value's
 error and not the rms of thousands; a chain twice as long has 1.4 times the error."""
 import numpy as np
 import pytest
@@ -30,11 +31,11 @@ def _rms(v):
 
 
 # linear layers of the networks that train here: forward, and the gradients whose depth is the batch or the classes
-SHAPES = [(128, 256, 784), (128, 256, 256), (784, 256, 128), (64, 512, 512), (385, 256, 1024), (32, 1000, 1536), (64, 1000, 2048), (96, 130, 1100),
-          (33, 65, 159), (60, 900, 1800)]
+SHAPES = [(128, 256, 784), (128, 256, 256), (64, 512, 512), (385, 256, 1024), (32, 1000, 1536), (64, 1000, 2048), (96, 130, 1100),
+          (33, 65, 159), (60, 900, 1800), (256, 256, 128), (197, 1189, 271)]
 
 
-def test_ranges_are_the_tile_kernels_or_shorter():
+def test_ranges_are_the_tile_kernels_and_of_batches_shorter():
     rng = np.random.RandomState(5)
     drawn = [tuple(int(round(np.exp(rng.uniform(0, np.log(top))))) for top in (2048, 5003, 5003, 64)) for _ in range(3000)]
     seen = 0
@@ -42,11 +43,37 @@ def test_ranges_are_the_tile_kernels_or_shorter():
         p = plan(M, N, K, batch)
         if p.waves:
             seen += 1
-            ranges = -(-K // p.tile_range)
-            assert p.range == p.tile_range if ranges >= 4 else p.range <= p.tile_range and -(-K // p.range) <= 4, (M, N, K, batch, p)
+            assert p.range == p.tile_range if batch == 1 else p.range <= p.tile_range and -(-K // p.range) <= 4, (M, N, K, batch, p)
             lds = -(-K // p.range) * (p.tile[0] + 1) * p.tile[1] * 4
-            assert p.range % 32 == 0 and lds <= 80 * 1024, (M, N, K, batch, p)
+            assert p.range % 32 == 0 and 2 <= p.waves <= 4 and lds <= 80 * 1024, (M, N, K, batch, p)
     assert seen > 500
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_bits_of_the_tile_kernel_and_its_fold(shape, ta, tb):
+    """The tile kernel makes each range's product by itself where the rows are the first of many."""
+    from tsplit_amd import gpu_links as L, ndarray as nd
+    ctx, (M, N, K), rng = nd.gpu(0), shape, np.random.RandomState(4)
+    p = plan(M, N, K)
+    assert p.waves
+    rows = next(m for m in (4096, 16384) if m > M and not plan(m, N, p.range).waves and plan(m, N, p.range).range >= min(K, p.range))
+    a, b = rng.normal(size=(M, K)).astype(np.float32), rng.normal(size=(K, N)).astype(np.float32)
+
+    def product(x, y):
+        c = nd.empty((x.shape[0], N), ctx)
+        x, y = (np.ascontiguousarray(v.T) if t else np.ascontiguousarray(v) for v, t in ((x, ta), (y, tb)))
+        L.matrix_multiply(nd.array(x, ctx), ta, nd.array(y, ctx), tb, c)
+        return c.asnumpy()
+    want = None
+    for k in range(0, K, p.range):
+        many = np.zeros((rows, min(K, k + p.range) - k), np.float32)
+        many[:M] = a[:, k:k + p.range]
+        assert not plan(rows, N, many.shape[1]).waves
+        part = product(many, b[k:k + p.range])[:M]
+        want = part if want is None else want + part
+    np.testing.assert_array_equal(product(a, b), want)
 
 
 @pytest.mark.gpu

@@ -34,7 +34,7 @@ Plan best_plan(int M, int N, int K, int batch, bool may_split) {
   const int64_t cols = N;
   const int steps = std::max(1, (K + gt::BK - 1) / gt::BK);
   const TilePlan t = plan_tiles(M, &cols, &steps, 1, batch, may_split ? 64 : 1, static_cast<double>(M) * N, kProductCost);
-  const WavesPlan waves = plan_waves(M, N, K, batch, t);
+  const WavesPlan waves = plan_waves(M, N, K, batch, t, !may_split);
   if (waves.waves) return {0, 1, waves.kchunk, waves};
   Plan p{t.tile, 1, (steps + t.S - 1) / t.S * gt::BK, waves};
   p.S = std::max(1, (K + p.kchunk - 1) / p.kchunk);

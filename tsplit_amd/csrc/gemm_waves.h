@@ -3,9 +3,9 @@
 // A product of a few hundred rows and columns has few 64 x 64 tiles, so on the kernel of gemm_tile.h its depth was cut into ranges and a
 // second launch added them; either launch takes what any launch takes, and a range of one or two steps is a chain of memory latencies
 // behind one barrier each.  Here a block owns 16 TM x 16 TN of the result, its two to four waves take the ranges of the depth in turn (the tile
-// kernel's own ranges: the bits of that kernel and its fold, see plan_waves), 32 values at a time, operands go from memory to the registers
-// the matrix instruction reads (no LDS, no barrier on the way), and the ranges' results are added through LDS in ascending order.  What bounds
-// it is latency: one for the operands, one for LDS, and the launch.
+// kernel's own ranges: the bits of that kernel and its fold; batches in up to four, see plan_waves), 32 values at a time, operands go from
+// memory to the registers the matrix instruction reads (no LDS, no barrier on the way), and the ranges' results are added through LDS in
+// ascending order.  What bounds it is latency: one for the operands, one for LDS, and the launch.
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -99,30 +99,32 @@ inline TilePlan plan_tiles(int64_t M, const int64_t *cols, const int *steps, int
 
 // Small products go to the kernel whose blocks share the depth of one small tile among their waves (gemm_waves.h), where that takes less.
 //
-// The depth is cut into the tile kernel's own ranges, so that a result has the bits that the tile kernel and the fold give it; where those are
-// fewer than the four waves (many tiles, or batches, whose depth that kernel leaves whole) into up to four, whose chains of roundings are
-// shorter.  (Four waves that dealt a whole depth among them 32 values at a time were as fast, but their chains of K / 4 roundings where
-// the tile kernel has K / 16 were 1.6 times further from float64 at 128 x 256 over 784 and 1.9 times at 64 x 1000 over 2048.)
+// The depth is cut into the tile kernel's own ranges, so that a result has the bits that the tile kernel and the fold give it.  Four waves that
+// dealt a whole depth among them 32 values at a time were as fast, but their chains of K / 4 roundings where the tile kernel has K / 16 were
+// 1.6 times further from float64 at 128 x 256 over 784 and 1.9 times at 64 x 1000 over 2048.  Up to four ranges where the tile kernel has one to
+// three take 0.75-0.9 of the time at depths of 64 to 160 (784 x 256 over 128 4.7-5.0 us, 5.2-5.8 on the tile kernel), but give other bits.
+// `whole`: batches, whose depth that kernel cannot cut; they are cut into up to four, whose chains are shorter.
 //
-// A launch there costs what any launch does, and for every block of the busiest CU a part of its own and one for each value of the depth that
-// the busiest wave takes; beyond 2048 of them 8 % more, where loads bound it (with both depths contiguous up to 20 %: 512 x 512 over 4096
-// 32.9 us on 32 x 32, 27.7 on the tile kernel).  From 217 shapes, rows 1 to 2048, columns 10 to 5003, depth 10 to 65536, batches among
-// them, in the four forms on the four tiles: 9 % rms off, the tile kernel's model (launches included) 15 %.  Over those shapes 1.25 times
-// faster than the tile kernel alone, with the best of both by hindsight 1.26: 128 x 256 over 784 7.5 -> 5.3 us, over 256 6.7 -> 4.1, 784 x 256 over
-// 128 5.7 -> 5.0, 385 x 256 over 1024 9.9 -> 7.1-9.0, 32 x 4096 over 1024 11.7 -> 7.3-9.1, 1 x 1908 over 308 7.0 -> 4.0, 16 of 64 x 64 over
-// 2048 45 -> 9; where the tile kernel stays: 250 x 5003 over 256 12.4, 512 x 512 over 64 4.4 (5.3 on 32 x 32 here).  Worst: 1 x 3000
-// over 65536, 231 us for 195.
+// A launch here costs what any launch does, and for every block of the busiest CU a part of its own and one for each value of the depth that
+// the busiest wave takes; beyond 2048 of them 8 % more, where loads bound it.  The figures are from 217 shapes, rows 1 to 2048, columns 10 to
+// 5003, depth 10 to 65536, batches among them, in the four forms on the four tiles with the depth in four ranges and more: 9 % rms off, the tile
+// kernel's model (launches included) 15 %.  Over 260 other shapes, replayed from a graph, with this rule 1.26 times faster than the tile kernel
+// alone, none slower by more than 6 %.  In the four forms, tile kernel -> here: 128 x 256 over 784 7.1-7.3 -> 5.0-5.3 us, over 256 6.4-6.6 ->
+// 3.7-4.1, 256 x 256 over 128 5.2-5.7 -> 3.7-3.9, 385 x 256 over 1024 9.3-9.8 -> 7.1-8.8, 32 x 4096 over 1024 11.1-12.1 -> 7.1-8.9, 64 x 1000
+// over 2048 10.4-10.8 -> 7.7-10.1, 1 x 1908 over 308 6.3-6.8 -> 3.7-4.1, 16 of 64 x 64 over 2048 41-49 -> 8-10; where the tile kernel stays:
+// 250 x 5003 over 256 12.2-12.8, 512 x 512 over 64 4.1-4.3 (4.9-5.1 on 32 x 32 here), over 4096 26-28 (27-28).  Beyond 16384 values operands
+// come from memory in parts of lines: 1 x 3000 over 16384 53-56 -> 39-59, over 32768 101-107 -> 110-134, so those stay too.
 constexpr TileKind kWaveTiles[] = {{16, 16}, {16, 32}, {32, 16}, {32, 32}};
 struct WavesPlan {
   int tile, waves;   // waves 0: the tile kernel
   int S, kchunk;     // the ranges that the waves take in turn
 };
-inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, const TilePlan &tile_kernel) {
+inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, const TilePlan &tile_kernel, bool whole) {
   constexpr double kLaunch = 3.56, kBlock[] = {0, 0.186, 0.363, 0.951}, kDepth[] = {0.00245, 0.00345, 0.00337, 0.00513};
   WavesPlan best{0, 0, 1, 0};
-  if (K <= 0) return best;
-  const int64_t steps = (K + 31) / 32, per = (steps + std::max(4, tile_kernel.S) - 1) / std::max(4, tile_kernel.S), S = (steps + per - 1) / per;
-  const int64_t deep = S > 4 ? (S + 3) / 4 * per * 128 : K;   // four times what the busiest wave takes
+  if (K <= 0 || (!whole && K > 16384)) return best;
+  const int64_t ranges = whole ? 4 : tile_kernel.S, steps = (K + 31) / 32, per = (steps + ranges - 1) / ranges, S = (steps + per - 1) / per;
+  const int64_t waves = std::min<int64_t>(4, S), deep = (S + waves - 1) / waves * std::min(4 * K, per * 128);   // 4 x what the busiest wave takes
   double least = 2.3 + 1.15 * tile_kernel.us;
   for (int t = 0; t < 4; ++t) {
     const int64_t blocks = ((M + kWaveTiles[t].bm - 1) / kWaveTiles[t].bm) * ((N + kWaveTiles[t].bn - 1) / kWaveTiles[t].bn) * batch;
@@ -132,8 +134,9 @@ inline WavesPlan plan_waves(int64_t M, int64_t N, int64_t K, int64_t batch, cons
     const double us = (kLaunch + n * (kBlock[t] + kDepth[t] * deep)) * (deep > 2048 ? 1.08 : 1);
     if (us < least) {
       least = us;
-      // eight or sixteen waves gain nothing on a CU of their own (over the shapes 0.2 %) and lose where blocks share one
-      best = {t, static_cast<int>(std::max<int64_t>(2, std::min<int64_t>(4, S))), static_cast<int>(S), static_cast<int>(per * 32)};
+      // A wave without a range still adds and stores: with a CU of their own four waves are 3 % faster than two at one or two ranges, where blocks
+      // share one up to 8 % slower.  Eight or sixteen gain nothing (over the shapes 0.2 %).
+      best = {t, n == 1 ? 4 : std::max(2, static_cast<int>(waves)), static_cast<int>(S), static_cast<int>(per * 32)};
     }
   }
   return best;
