@@ -147,3 +147,15 @@ def test_a_pointer_may_be_filled_in_after_the_array_was_made():
         a.shape
     assert _LIB.DLArrayAlloc((ctypes.c_int64 * 2)(2, 3), ctypes.c_int64(2), nd.cpu(0), ctypes.byref(h), ctypes.c_int(1)) == 0
     assert a.shape == (2, 3) and a.data_ptr == h.contents.data
+
+
+def test_a_profiler_may_have_fields_of_its_own():
+    from tsplit_amd.profiler import Profiler
+
+    class Longer(Profiler):
+        _fields_ = [("calls", ctypes.c_int)]
+    a = nd.empty((2, 3))
+    with pytest.raises(RuntimeError):                       # taken: the shapes do not conform, which the library refuses
+        L.matrix_multiply(a, False, a, False, a, profiler=Longer())
+    with pytest.raises(TypeError):
+        L.matrix_multiply(a, False, a, False, a, profiler=bytearray(ctypes.sizeof(Profiler)))

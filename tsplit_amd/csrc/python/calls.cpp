@@ -25,6 +25,7 @@ PyObject *g_recording = nullptr;   // the dict with _recording_keeper
 PyObject *g_handle_of = nullptr;   // address -> ctypes handle
 PyObject *g_pointers = nullptr;    // the ctypes types that a pointer may be of
 PyObject *g_context = nullptr;     // DLContext
+PyObject *g_structure = nullptr;   // ctypes.Structure
 PyObject *g_rule_name, *g_keeper_name, *g_take_name, *g_handle_name;
 
 // ---------------------------------------------------------------- arrays
@@ -371,14 +372,16 @@ struct Arg<DLStreamHandle> {   // an object with a `handle`, or nothing: the def
   }
 };
 template <>
-struct Arg<ProfilerHandle> {   // a Profiler structure, or nothing
+struct Arg<ProfilerHandle> {   // a Profiler structure or one that begins as it does, or nothing
   static bool get(PyObject *o, bool, ProfilerHandle &v) {
     v = nullptr;
     const int given = o == Py_None ? 0 : PyObject_IsTrue(o);
     if (given <= 0) return given == 0;
     Py_buffer b;
-    if (PyObject_GetBuffer(o, &b, PyBUF_WRITABLE)) return false;
-    const bool ok = b.len == static_cast<Py_ssize_t>(sizeof(Profiler));
+    const bool structure = PyObject_TypeCheck(o, reinterpret_cast<PyTypeObject *>(g_structure));
+    if (!structure) PyErr_Format(PyExc_TypeError, "a Profiler, not %R", o);
+    if (!structure || PyObject_GetBuffer(o, &b, PyBUF_WRITABLE)) return false;
+    const bool ok = b.len >= static_cast<Py_ssize_t>(sizeof(Profiler));
     v = static_cast<ProfilerHandle>(b.buf);
     PyBuffer_Release(&b);   // the structure stays where it is: the caller holds it
     if (!ok) PyErr_SetString(PyExc_TypeError, "not a Profiler");
@@ -435,11 +438,11 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
 CALLS(DECLARE)
 
 // bind(addresses by name, those of operators that the library lacks left out, the module dict with MEMORY_MANAGE_RULE, the one with
-// _recording_keeper, address -> handle, the types of pointers, DLContext)
+// _recording_keeper, address -> handle, the types of pointers, DLContext, ctypes.Structure)
 PyObject *bind(PyObject *, PyObject *args) {
-  PyObject *addresses, *rules, *recording, *handle_of, *pointers, *context;
-  if (!PyArg_ParseTuple(args, "O!O!O!OO!O!", &PyDict_Type, &addresses, &PyDict_Type, &rules, &PyDict_Type, &recording, &handle_of, &PyTuple_Type,
-                        &pointers, &PyType_Type, &context))
+  PyObject *addresses, *rules, *recording, *handle_of, *pointers, *context, *structure;
+  if (!PyArg_ParseTuple(args, "O!O!O!OO!O!O!", &PyDict_Type, &addresses, &PyDict_Type, &rules, &PyDict_Type, &recording, &handle_of, &PyTuple_Type,
+                        &pointers, &PyType_Type, &context, &PyType_Type, &structure))
     return nullptr;
   auto look = [&](const char *name, auto &fn) {
     PyObject *a = PyDict_GetItemString(addresses, name);
@@ -465,6 +468,8 @@ PyObject *bind(PyObject *, PyObject *args) {
   Py_XSETREF(g_pointers, pointers);
   Py_INCREF(context);
   Py_XSETREF(g_context, context);
+  Py_INCREF(structure);
+  Py_XSETREF(g_structure, structure);
   Py_RETURN_NONE;
 }
 

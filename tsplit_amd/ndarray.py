@@ -80,7 +80,7 @@ def _addresses(names):
 
 
 _calls.bind(_addresses(_calls.SYMBOLS + ["DLArrayAlloc", "DLArrayFree"]), globals(), vars(_stream), lambda address: ctypes.cast(address, DLArrayHandle),
-            (ctypes._Pointer, ctypes.c_void_p), DLContext)
+            (ctypes._Pointer, ctypes.c_void_p), DLContext, ctypes.Structure)
 
 
 def cpu(dev_id=0):
